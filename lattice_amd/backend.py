@@ -112,6 +112,22 @@ class ChainStep(C.Structure):
 
 
 _lib = None
+_fast = None
+
+
+def _load_fast():
+    """The CPython entry to the library (csrc/lq4_py.cpp), through which the per-launch methods call it: the same
+    functions without ctypes' argument objects.  Built with the library; there is no other path."""
+    global _fast
+    if _fast is None:
+        load_library()
+        try:
+            from . import _lq4_py
+        except ImportError as e:
+            raise Q4LibraryMissing(f"{_HERE}/_lq4_py.so is not built ({e}); run `python -m lattice_amd.build`") from None
+        _lq4_py.set_error(Q4Error)
+        _fast = _lq4_py
+    return _fast
 
 
 def load_library() -> C.CDLL:
@@ -268,6 +284,9 @@ class HipQ4Backend:
         ctx = C.c_void_p()
         _check(self.lib.lq4_ctx_create(device, C.byref(ctx)))
         self.ctx = ctx
+        self._c = ctx.value
+        self._x = _load_fast()
+        self._current_stream = torch._C._cuda_getCurrentRawStream  # (device) -> hipStream_t as an int
         self.model = model
         self._lora: Dict[Tuple[int, str], _LoraProjection] = {}
         self._lora_scale = 0.0
@@ -276,7 +295,7 @@ class HipQ4Backend:
         self.unload_lora_adapter()
         if self.ctx:
             self.lib.lq4_ctx_destroy(self.ctx)
-            self.ctx = None
+            self.ctx = self._c = None
 
     # ------------------------------------------------------------------ helpers
     def _stream(self):
@@ -380,10 +399,11 @@ class HipQ4Backend:
         ``layer_idx``/``module`` fuses that projection's LoRA delta into the same pass."""
         if n == 0:
             return
-        self._assert_k(k, "dispatch_matmul_q4")
-        lora = self._lora_for(layer_idx, module, n, k)
-        _check(self.lib.lq4_gemv(self.ctx, qw.handle, 0, n, k, x.data_ptr(), 1, y.data_ptr(), lora,
-                                 self._lora_scale, self._stream()))
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_matmul_q4")
+        lora = None if layer_idx is None else self._lora_for(layer_idx, module, n, k)
+        self._x.lq4_gemv(self._c, qw.handle, 0, n, k, x.data_ptr(), 1, y.data_ptr(), lora,
+                         self._lora_scale, self._current_stream(self.device))
 
     # ---- Q8_0 sibling format ------------------------------------------------------------------
     def upload_q8_blocks(self, blocks) -> Q4WeightBuf:
@@ -395,18 +415,20 @@ class HipQ4Backend:
         """``dispatch_matmul_q8`` (dispatch.rs:61-84): decode GEMV over Q8_0 blocks, ``m`` ignored."""
         if n == 0:
             return
-        self._assert_k(k, "dispatch_matmul_q8")
-        _check(self.lib.lq4_gemv_q8(self.ctx, qw.handle, 0, n, k, x.data_ptr(), 1, y.data_ptr(), self._stream()))
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_matmul_q8")
+        self._x.lq4_gemv_q8(self._c, qw.handle, 0, n, k, x.data_ptr(), 1, y.data_ptr(), self._current_stream(self.device))
 
     def dispatch_gemm_q8(self, x, x_offset: int, qw: Q4WeightBuf, y, y_offset: int, m: int, n: int, k: int):
         """``dispatch_gemm_q8`` (dispatch.rs:86-146): byte offsets into x and y; ``m == 0 or n == 0``
         is a no-op; ``m <= 1`` takes the GEMV."""
         if m == 0 or n == 0:
             return
-        self._assert_k(k, "dispatch_gemm_q8")
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_gemm_q8")
         dt = _dtype_code(x)
-        _check(self.lib.lq4_gemm_q8(self.ctx, qw.handle, 0, n, k, x.data_ptr() + x_offset, dt, m,
-                                    y.data_ptr() + y_offset, self._stream()))
+        self._x.lq4_gemm_q8(self._c, qw.handle, 0, n, k, x.data_ptr() + x_offset, dt, m,
+                            y.data_ptr() + y_offset, self._current_stream(self.device))
 
     # ---- Q3 sibling format --------------------------------------------------------------------
     def upload_q3_blocks(self, blocks, payload_offset: int = 0) -> Q4WeightBuf:
@@ -417,17 +439,19 @@ class HipQ4Backend:
         """Decode GEMV over Q3 blocks (the ``m <= 1`` arm of ``dispatch_gemm_q3``, dispatch.rs:269-325)."""
         if n == 0:
             return
-        self._assert_k(k, "dispatch_gemm_q3")
-        _check(self.lib.lq4_gemv_q3(self.ctx, qw.handle, 0, n, k, x.data_ptr(), 1, y.data_ptr(), self._stream()))
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_gemm_q3")
+        self._x.lq4_gemv_q3(self._c, qw.handle, 0, n, k, x.data_ptr(), 1, y.data_ptr(), self._current_stream(self.device))
 
     def dispatch_gemm_q3(self, x, x_offset: int, qw: Q4WeightBuf, y, y_offset: int, m: int, n: int, k: int):
         """``dispatch_gemm_q3`` (dispatch.rs:269-325): byte offsets into x and y; ``m == 0 or n == 0``
         is a no-op; ``m <= 1`` takes the GEMV."""
         if m == 0 or n == 0:
             return
-        self._assert_k(k, "dispatch_gemm_q3")
-        _check(self.lib.lq4_gemm_q3(self.ctx, qw.handle, 0, n, k, x.data_ptr() + x_offset, _dtype_code(x), m,
-                                    y.data_ptr() + y_offset, self._stream()))
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_gemm_q3")
+        self._x.lq4_gemm_q3(self._c, qw.handle, 0, n, k, x.data_ptr() + x_offset, _dtype_code(x), m,
+                            y.data_ptr() + y_offset, self._current_stream(self.device))
 
     # ---- elementwise steps either side of the decode GEMVs -----------------------------------
     @staticmethod
@@ -439,21 +463,21 @@ class HipQ4Backend:
         """``dispatch_fused_residual_add_norm`` / ``_batch`` (dispatch.rs:1171-1266):
         ``residual_out = base + delta``, ``normed_out`` = shifted RMSNorm of it.  ``delta=None`` is
         the plain ``dispatch_rms_norm`` (dispatch.rs:525); ``residual_out=None`` skips that store."""
-        _check(self.lib.lq4_residual_add_rmsnorm(self.ctx, base.data_ptr(), self._ptr(delta), gamma.data_ptr(),
-                                                 row_len, num_rows, eps, self._ptr(residual_out),
-                                                 normed_out.data_ptr(), self._stream()))
+        self._x.lq4_residual_add_rmsnorm(self._c, base.data_ptr(), self._ptr(delta), gamma.data_ptr(),
+                                         row_len, num_rows, eps, self._ptr(residual_out),
+                                         normed_out.data_ptr(), self._current_stream(self.device))
 
     def dispatch_silu_mul_fused(self, data, count: int, rows: int = 1, out=None, out_stride=None):
         """``dispatch_silu_mul_fused`` (dispatch.rs:916-930): ``data[i] = silu(data[i]) *
         data[i + count]`` in place, or into ``out`` (rows ``out_stride`` floats apart)."""
         dst = data if out is None else out
         stride = (2 * count if out is None else count) if out_stride is None else out_stride
-        _check(self.lib.lq4_silu_mul(self.ctx, data.data_ptr(), count, rows, dst.data_ptr(), stride, self._stream()))
+        self._x.lq4_silu_mul(self._c, data.data_ptr(), count, rows, dst.data_ptr(), stride, self._current_stream(self.device))
 
     def dispatch_add_and_copy(self, src, residual, dst, count: int):
         """``dispatch_add_and_copy`` (dispatch.rs:1268-1290): ``residual += src; dst = residual``."""
-        _check(self.lib.lq4_add_and_copy(self.ctx, src.data_ptr(), residual.data_ptr(), self._ptr(dst), count,
-                                         self._stream()))
+        self._x.lq4_add_and_copy(self._c, src.data_ptr(), residual.data_ptr(), self._ptr(dst), count,
+                                 self._current_stream(self.device))
 
     def dispatch_matmul_fused(self, x, qw: Q4WeightBuf, y, n: int, k: int, *, norm=None, silu_mul=False,
                               add_residual=None, silu_mul_pairs=False, qw_extra_offset: int = 0, layer_idx=None,
@@ -468,26 +492,27 @@ class HipQ4Backend:
         ``batch`` rows every per-row tensor is ``[batch, ...]`` and dense."""
         if n == 0:
             return
-        self._assert_k(k, "dispatch_matmul_q4")
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_matmul_q4")
         assert not (norm is not None and silu_mul), "one prologue at a time"
-        f = GemvFusion()
-        f.prologue = LQ4_PRO_ADD_RMSNORM if norm is not None else LQ4_PRO_SILU_MUL if silu_mul else LQ4_PRO_NONE
-        keep = []
+        prologue = LQ4_PRO_ADD_RMSNORM if norm is not None else LQ4_PRO_SILU_MUL if silu_mul else LQ4_PRO_NONE
+        ptr = self._ptr
+        base = delta = gamma = residual_out = residual = dst = None
+        eps = 0.0
         if norm is not None:
             base, delta, gamma, eps, residual_out = norm
-            f.base, f.delta, f.gamma = base.data_ptr(), self._ptr(delta), gamma.data_ptr()
-            f.eps, f.residual_out = eps, self._ptr(residual_out)
-            keep += [base, delta, gamma, residual_out]
-        f.epilogue = LQ4_EPI_NONE
+            base, gamma = base.data_ptr(), gamma.data_ptr()
+        epilogue = LQ4_EPI_NONE
         if add_residual is not None:
             residual, dst = add_residual
-            f.epilogue, f.residual, f.copy_dst = LQ4_EPI_ADD_RESIDUAL, residual.data_ptr(), self._ptr(dst)
+            epilogue, residual = LQ4_EPI_ADD_RESIDUAL, residual.data_ptr()
         if silu_mul_pairs:
             assert add_residual is None, "one epilogue at a time"
-            f.epilogue = LQ4_EPI_SILU_MUL_PAIRS
-        lora = self._lora_for(layer_idx, module, n, k)
-        _check(self.lib.lq4_gemv_fused_batch(self.ctx, qw.handle, qw_extra_offset, n, k, self._ptr(x), batch,
-                                             self._ptr(y), C.byref(f), lora, self._lora_scale, self._stream()))
+            epilogue = LQ4_EPI_SILU_MUL_PAIRS
+        lora = None if layer_idx is None else self._lora_for(layer_idx, module, n, k)
+        self._x.gemv_fused_batch(self._c, qw.handle, qw_extra_offset, n, k, ptr(x), batch, ptr(y), prologue, base,
+                                 ptr(delta), gamma, eps, ptr(residual_out), epilogue, residual, ptr(dst), lora,
+                                 self._lora_scale, self._current_stream(self.device))
 
     def chain_step(self, qw: Q4WeightBuf, n: int, k: int, *, x=None, from_previous=False, norm=None, silu_mul=False,
                    add_residual=None, silu_mul_pairs=False, y=None, qw_extra_offset: int = 0) -> ChainStep:
@@ -498,7 +523,8 @@ class HipQ4Backend:
         ``add_residual=residual``: the result is ``residual + W.x``, written back;
         ``silu_mul_pairs=True``: W is gate rows then up rows and the result is ``silu(gate) * up``
         (n/2 values); ``y`` receives the result."""
-        self._assert_k(k, "dispatch_matmul_q4")
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_matmul_q4")
         assert not (norm is not None and silu_mul), "one prologue at a time"
         assert not (add_residual is not None and silu_mul_pairs), "one epilogue at a time"
         st = ChainStep()
@@ -522,8 +548,7 @@ class HipQ4Backend:
     def dispatch_chain(self, steps: Sequence[ChainStep]):
         """The dispatches of one token between two points where the host must look at the result
         (``forward_step`` encodes them into one command buffer, metal_qwen35.rs:6943), as one library call."""
-        arr = (ChainStep * len(steps))(*steps)
-        _check(self.lib.lq4_gemv_chain(self.ctx, arr, len(steps), self._stream()))
+        self._x.gemv_chain(self._c, steps, self._current_stream(self.device))
 
     def dispatch_gemm(self, x, x_offset: int, qw: Q4WeightBuf, y, y_offset: int, m: int, n: int,
                       k: int, *, layer_idx=None, module=None):
@@ -538,21 +563,23 @@ class HipQ4Backend:
         small ``m`` with f32 activations takes the GEMV kernel (m == 1 in the reference)."""
         if m == 0 or n == 0:
             return
-        self._assert_k(k, "dispatch_gemm_q4")
-        lora = self._lora_for(layer_idx, module, n, k)
-        _check(self.lib.lq4_gemm(self.ctx, qw.handle, qw_extra_offset, n, k, x.data_ptr() + x_offset,
-                                 _dtype_code(x), m, y.data_ptr() + y_offset, lora, self._lora_scale,
-                                 self._stream()))
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_gemm_q4")
+        lora = None if layer_idx is None else self._lora_for(layer_idx, module, n, k)
+        self._x.lq4_gemm(self._c, qw.handle, qw_extra_offset, n, k, x.data_ptr() + x_offset,
+                         _dtype_code(x), m, y.data_ptr() + y_offset, lora, self._lora_scale,
+                         self._current_stream(self.device))
 
     def gemv_batch(self, x, qw: Q4WeightBuf, y, batch: int, n: int, k: int, qw_extra_offset: int = 0,
                    *, layer_idx=None, module=None):
         """Small-batch decode: ``y[b] = W . x[b]`` for ``b < batch <= 16`` in one pass over W."""
         if batch == 0 or n == 0:
             return
-        self._assert_k(k, "dispatch_matmul_q4")
-        lora = self._lora_for(layer_idx, module, n, k)
-        _check(self.lib.lq4_gemv(self.ctx, qw.handle, qw_extra_offset, n, k, x.data_ptr(), batch,
-                                 y.data_ptr(), lora, self._lora_scale, self._stream()))
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_matmul_q4")
+        lora = None if layer_idx is None else self._lora_for(layer_idx, module, n, k)
+        self._x.lq4_gemv(self._c, qw.handle, qw_extra_offset, n, k, x.data_ptr(), batch,
+                         y.data_ptr(), lora, self._lora_scale, self._current_stream(self.device))
 
     def gemv_multi(self, x, projections, batch: int, k: int, *, layer_idx=None):
         """Several projections of the same activations in one call (one launch at batch 1): ``projections`` is a
@@ -561,26 +588,18 @@ class HipQ4Backend:
         ``gemv_batch`` does.  The q/k/v run of dispatch_matmul calls on one input (inner/layers/gqa.rs:72-127)."""
         if batch == 0 or not projections:
             return
-        self._assert_k(k, "dispatch_matmul_q4")
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dispatch_matmul_q4")
         if len(projections) > MAX_PROJECTIONS:
             raise ValueError(f"{len(projections)} projections, at most {MAX_PROJECTIONS} a call")
-        arr = (Projection * len(projections))()
-        for i, p in enumerate(projections):
-            qw, n, y = p[0], p[1], p[2]
-            module = p[3] if len(p) > 3 else None
-            lora = self._lora_for(layer_idx, module, n, k) if module is not None else None
-            arr[i].w = qw.handle
-            arr[i].w_extra_offset = p[4] if len(p) > 4 else 0
-            arr[i].n = n
-            arr[i].y_dev = y.data_ptr()
-            arr[i].lora = lora
-            arr[i].lora_scale = self._lora_scale
-        _check(self.lib.lq4_gemv_multi(self.ctx, arr, len(projections), k, x.data_ptr(), batch, self._stream()))
+        self._x.gemv_multi(self._c, projections, k, x.data_ptr(), batch, self._lora, layer_idx, self._lora_scale,
+                           self._current_stream(self.device))
 
     def dequantize(self, qw: Q4WeightBuf, n: int, k: int, qw_extra_offset: int = 0):
         """f32 [n, k] tensor of ``f32(nibble)*scale + bias`` (bit-exactness probe)."""
         import torch
-        self._assert_k(k, "dequantize")
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "dequantize")
         out = torch.empty((n, k), dtype=torch.float32, device=self.torch_device)
         _check(self.lib.lq4_dequant(self.ctx, qw.handle, qw_extra_offset, n, k, out.data_ptr(),
                                     self._stream()))
@@ -593,8 +612,8 @@ class HipQ4Backend:
         import torch
         out_l = torch.empty(k, dtype=torch.float32, device=self.torch_device)
         out_i = torch.empty(k, dtype=torch.int32, device=self.torch_device)  # u32 bit patterns
-        _check(self.lib.lq4_topk(self.ctx, logits.data_ptr(), logits.numel(), k, out_l.data_ptr(),
-                                 out_i.data_ptr(), self._stream()))
+        self._x.lq4_topk(self._c, logits.data_ptr(), logits.numel(), k, out_l.data_ptr(),
+                         out_i.data_ptr(), self._current_stream(self.device))
         return out_l, out_i
 
     def lm_head_topk(self, x, qw: Q4WeightBuf, vocab: int, k: int, top_k: int, qw_extra_offset: int = 0,
@@ -604,14 +623,15 @@ class HipQ4Backend:
         never returned.  ``static_scratch=True`` takes the entry point that allocates nothing
         (pass ``out=(logits, ids)`` tensors as well and the call touches no allocator at all)."""
         import torch
-        self._assert_k(k, "lm_head_topk")
+        if k <= 0 or k % BLOCK_WEIGHTS:
+            self._assert_k(k, "lm_head_topk")
         if out is None:
             out = (torch.empty(top_k, dtype=torch.float32, device=self.torch_device),
                    torch.empty(top_k, dtype=torch.int32, device=self.torch_device))
         out_l, out_i = out
-        fn = self.lib.lq4_lm_head_topk_static if static_scratch else self.lib.lq4_lm_head_topk
-        _check(fn(self.ctx, qw.handle, qw_extra_offset, vocab, k, x.data_ptr(), top_k,
-                  out_l.data_ptr(), out_i.data_ptr(), self._stream()))
+        fn = self._x.lq4_lm_head_topk_static if static_scratch else self._x.lq4_lm_head_topk
+        fn(self._c, qw.handle, qw_extra_offset, vocab, k, x.data_ptr(), top_k, out_l.data_ptr(), out_i.data_ptr(),
+           self._current_stream(self.device))
         return out_l, out_i
 
     # -------------------------------------------------------------------- LoRA
@@ -693,9 +713,9 @@ class HipQ4Backend:
         proj = self._lora.get((layer_idx, module))
         if proj is None:
             return
-        _check(self.lib.lq4_lora_apply(self.ctx, proj.handle, self._lora_scale,
-                                       x.data_ptr() + x_byte_offset, _dtype_code(x), rows,
-                                       y.data_ptr() + y_byte_offset, self._stream()))
+        self._x.lq4_lora_apply(self._c, proj.handle, self._lora_scale,
+                               x.data_ptr() + x_byte_offset, _dtype_code(x), rows,
+                               y.data_ptr() + y_byte_offset, self._current_stream(self.device))
 
     # --------------------------------------------------------------------- MoE
     def moe_route(self, logits, top_k: int):
@@ -705,8 +725,8 @@ class HipQ4Backend:
         t, e = logits.shape
         ids = torch.empty((t, top_k), dtype=torch.int32, device=self.torch_device)
         wts = torch.empty((t, top_k), dtype=torch.float32, device=self.torch_device)
-        _check(self.lib.lq4_moe_route(self.ctx, logits.data_ptr(), t, e, top_k, ids.data_ptr(),
-                                      wts.data_ptr(), self._stream()))
+        self._x.lq4_moe_route(self._c, logits.data_ptr(), t, e, top_k, ids.data_ptr(),
+                              wts.data_ptr(), self._current_stream(self.device))
         return ids, wts
 
     def moe_shared_expert(self, gate_up: Q4WeightBuf, down: Q4WeightBuf, shared_gate, shared_inter: int,
@@ -714,9 +734,9 @@ class HipQ4Backend:
         """``apply_shared_expert`` (moe.rs:194-250): ``y += sigmoid(x . shared_gate) * FFN_shared(x)``
         per token; ``y`` normally holds the routed experts' sum already."""
         tokens = x.shape[0] if x.dim() > 1 else 1
-        _check(self.lib.lq4_moe_shared_expert(self.ctx, gate_up.handle, down.handle, shared_gate.data_ptr(),
-                                              shared_inter, hidden, x.data_ptr(), tokens, y.data_ptr(),
-                                              self._stream()))
+        self._x.lq4_moe_shared_expert(self._c, gate_up.handle, down.handle, shared_gate.data_ptr(),
+                                      shared_inter, hidden, x.data_ptr(), tokens, y.data_ptr(),
+                                      self._current_stream(self.device))
 
     def moe_ffn(self, router_logits, gate_up: Q4WeightBuf, down: Q4WeightBuf, num_experts: int, top_k: int,
                 inter: int, shared_gate_up: Q4WeightBuf, shared_down: Q4WeightBuf, shared_gate, shared_inter: int,
@@ -724,14 +744,14 @@ class HipQ4Backend:
         """``moe_ffn_step`` (moe.rs:8-36) from the router logits on: route, routed experts, shared expert;
         ``y`` is overwritten."""
         tokens = x.shape[0] if x.dim() > 1 else 1
-        _check(self.lib.lq4_moe_ffn(self.ctx, router_logits.data_ptr(), gate_up.handle, down.handle, num_experts,
-                                    top_k, inter, shared_gate_up.handle, shared_down.handle, shared_gate.data_ptr(),
-                                    shared_inter, hidden, x.data_ptr(), tokens, y.data_ptr(), self._stream()))
+        self._x.lq4_moe_ffn(self._c, router_logits.data_ptr(), gate_up.handle, down.handle, num_experts,
+                            top_k, inter, shared_gate_up.handle, shared_down.handle, shared_gate.data_ptr(),
+                            shared_inter, hidden, x.data_ptr(), tokens, y.data_ptr(), self._current_stream(self.device))
 
     def moe_experts(self, gate_up: Q4WeightBuf, down: Q4WeightBuf, num_experts: int, inter: int,
                     hidden: int, x, ids, weights, y):
         """Routed-expert FFN over Q4 expert tensors (moe.rs:127-190); ``y`` is overwritten."""
         tokens, top_k = ids.shape
-        _check(self.lib.lq4_moe_grouped_gemv(self.ctx, gate_up.handle, down.handle, num_experts, inter,
-                                             hidden, x.data_ptr(), tokens, ids.data_ptr(),
-                                             weights.data_ptr(), top_k, y.data_ptr(), self._stream()))
+        self._x.lq4_moe_grouped_gemv(self._c, gate_up.handle, down.handle, num_experts, inter,
+                                     hidden, x.data_ptr(), tokens, ids.data_ptr(),
+                                     weights.data_ptr(), top_k, y.data_ptr(), self._current_stream(self.device))

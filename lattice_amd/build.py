@@ -1,4 +1,5 @@
-"""Builds ``liblattice_hip_q4.so`` for gfx950 with hipcc, in-tree, next to this file.
+"""Builds ``liblattice_hip_q4.so`` for gfx950 with hipcc, and ``_lq4_py.so`` (its CPython entry), in-tree, next to this
+file.
 
 ``python -m lattice_amd.build`` compiles every translation unit under ``csrc/``
 (in parallel) and links them.  hipcc cross-compiles, so no GPU is needed to build.
@@ -9,11 +10,13 @@ import os
 import shlex
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblattice_hip_q4.so")
+PY_EXT = os.path.join(HERE, "_lq4_py.so")
 SOURCES = ["lq4_api.hip", "lq4_gemv.hip", "lq4_gemv_b1.hip", "lq4_gemv_dma.hip", "lq4_gemv_multi.hip", "lq4_gemv_i8.hip", "lq4_gemv_mfma.hip", "lq4_gemm.hip", "lq4_gemm_wreg.hip", "lq4_gemm_skinny.hip", "lq4_moe.hip", "lq4_moe_i8.hip", "lq4_moe_b1.hip", "lq4_topk.hip", "lq4_elementwise.hip", "lq4_q8.hip", "lq4_q3.hip"]
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32 out of scalar float code.
@@ -46,6 +49,13 @@ def build(verbose: bool = False) -> str:
     with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as ex:
         list(ex.map(compile_one, zip(SOURCES, objs)))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
+    # the CPython entry: host code only, resolves the library next to itself
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "lq4_py.cpp"), "-o", PY_EXT, "-L" + HERE,
+           "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    _run(cmd)
     return LIB
 
 

@@ -92,9 +92,9 @@ int fail(int code, const char* fmt, ...) {
     } while (0)
 
 struct DeviceGuard {
-    int prev = -1;
+    int prev = -1, dev;
     bool ok = true;
-    explicit DeviceGuard(int dev) {
+    explicit DeviceGuard(int d) : dev(d) {
         if (hipGetDevice(&prev) != hipSuccess) prev = -1;
         if (prev != dev) ok = hipSetDevice(dev) == hipSuccess;
         // An error some earlier, unrelated runtime call left behind in this thread must not be
@@ -102,7 +102,7 @@ struct DeviceGuard {
         if (ok) (void)hipGetLastError();
     }
     ~DeviceGuard() {
-        if (prev >= 0) (void)hipSetDevice(prev);
+        if (prev >= 0 && prev != dev) (void)hipSetDevice(prev);
     }
 };
 
