@@ -205,7 +205,9 @@ int lq4_moe_route(lq4_ctx* ctx, const float* logits_dev, uint32_t tokens, uint32
  * expert share one pass over that expert's weights.  x_dev f32 [tokens, hidden];
  * y_dev f32 [tokens, hidden] (overwritten).  tokens*top_k <= 4096.  Up to 8 tokens (hidden <= 8192,
  * top_k * inter <= 8192) every pair is served as a one-token GEMV and the weighted sum over a
- * token's slots is formed inside the down pass; larger steps group the pairs by expert. */
+ * token's slots is formed inside the down pass; larger steps group the pairs by expert, and from 14 pairs
+ * per expert on (num_experts < 1024, hidden and inter at least 128) an expert's blocks are read once for
+ * up to 64 pairs at a time. */
 int lq4_moe_grouped_gemv(lq4_ctx* ctx, const lq4_weight* gate_up, const lq4_weight* down,
                          uint32_t num_experts, uint32_t inter, uint32_t hidden,
                          const float* x_dev, uint32_t tokens, const int32_t* ids_dev,
@@ -241,7 +243,9 @@ int lq4_moe_shared_expert(lq4_ctx* ctx, const lq4_weight* gate_up, const lq4_wei
  *   - from 9 to 384 tokens (num_experts < 1024): the shared expert is one more expert of the grouped
  *     kernels, chosen by every token with sigmoid(x . shared_gate) as its routing weight, which the
  *     router launch computes: four launches (five above 512 (token, slot) pairs, where a grouping
- *     launch runs first), none of the shared expert's own. */
+ *     launch runs first), none of the shared expert's own;
+ *   - from 14 (token, slot) pairs per expert on (num_experts < 1024, all three sizes at least 128), where
+ *     a shared expert of any width is one more expert of the grouped GEMM. */
 int lq4_moe_ffn(lq4_ctx* ctx, const float* router_logits_dev, const lq4_weight* gate_up, const lq4_weight* down,
                 uint32_t num_experts, uint32_t top_k, uint32_t inter, const lq4_weight* shared_gate_up,
                 const lq4_weight* shared_down, const float* shared_gate_dev, uint32_t shared_inter,

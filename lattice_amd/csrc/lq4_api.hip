@@ -828,6 +828,16 @@ int lq4_moe_route(lq4_ctx* ctx, const float* logits_dev, uint32_t tokens, uint32
     return LQ4_OK;
 }
 
+// Where the grouped GEMM (lq4_moe_gemm.hip) serves a step instead of the grouped GEMV: from 14 pairs per expert on (64 experts,
+// top 8, whole layer: 96 tokens = 12 per expert 106 us there, 111 here; 128 tokens 131 / 121; 512 tokens 411 / 147).
+static bool moe_takes_gemm(const MoeGemmShape& m) {
+    static const uint32_t per_expert = [] {
+        const char* env = getenv("LQ4_MOE_GEMM_PAIRS");
+        return env ? static_cast<uint32_t>(strtoul(env, nullptr, 10)) : 14u;
+    }();
+    return static_cast<uint64_t>(m.tokens) * m.top_k >= static_cast<uint64_t>(per_expert) * m.experts && moe_gemm_serves(m);
+}
+
 // Scratch of the grouped expert kernels for `pairs` (token, slot) pairs over `experts` experts.
 static int grouped_scratch(lq4_ctx* ctx, uint32_t experts, size_t pairs, uint32_t inter, uint32_t hidden,
                            hipStream_t stream, MoeScratch* s) {
@@ -883,6 +893,17 @@ int lq4_moe_grouped_gemv(lq4_ctx* ctx, const lq4_weight* gate_up, const lq4_weig
         launch_moe_b1(gu, dn, num_experts, inter, hidden, x_dev, tokens, ids_dev, weights_dev, top_k, y_dev,
                       reinterpret_cast<float*>(ctx->moe_scratch), nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, false,
                       static_cast<hipStream_t>(stream));
+        ctx->counters.moe_gate_up++;
+        ctx->counters.moe_down++;
+        LQ4_HIP(hipGetLastError());
+        return LQ4_OK;
+    }
+    const MoeGemmShape shape{num_experts, top_k, inter, 0, hidden, tokens};
+    if (moe_takes_gemm(shape)) {
+        rc = ensure_scratch(ctx, moe_gemm_scratch_bytes(shape), static_cast<hipStream_t>(stream));
+        if (rc) return rc;
+        launch_moe_gemm(shape, gu, dn, nullptr, nullptr, x_dev, ids_dev, weights_dev, y_dev, ctx->moe_scratch,
+                        static_cast<hipStream_t>(stream));
         ctx->counters.moe_gate_up++;
         ctx->counters.moe_down++;
         LQ4_HIP(hipGetLastError());
@@ -1078,6 +1099,24 @@ int lq4_moe_ffn(lq4_ctx* ctx, const float* router_logits_dev, const lq4_weight* 
         launch_moe_b1(rgu, rdn, num_experts, inter, hidden, x_dev, tokens, ids, wts, top_k, y_dev,
                       reinterpret_cast<float*>(ctx->moe_scratch), gu, dn, shared_gate_dev,
                       route_inside ? router_logits_dev : nullptr, ids, wts, false, s);
+        ctx->counters.moe_gate_up++;
+        ctx->counters.moe_down++;
+        LQ4_HIP(hipGetLastError());
+        return LQ4_OK;
+    }
+    const MoeGemmShape shape{num_experts, top_k, inter, shared_inter, hidden, tokens};
+    if (inter && tokens > b1_tokens && moe_takes_gemm(shape) && static_cast<uint64_t>(num_experts) * 2 * inter <= UINT32_MAX &&
+        static_cast<uint64_t>(num_experts) * hidden <= UINT32_MAX) {
+        // Many tokens per expert: route, then the grouped GEMM with the shared expert (of any width) as one more expert.
+        rc = resolve_weight(gate_up, 0, num_experts * 2 * inter, hidden, &rgu);
+        if (rc) return rc;
+        rc = resolve_weight(down, 0, num_experts * hidden, inter, &rdn);
+        if (rc) return rc;
+        rc = ensure_scratch(ctx, moe_gemm_scratch_bytes(shape), s);
+        if (rc) return rc;
+        launch_moe_route(router_logits_dev, tokens, num_experts, top_k, ids, wts, s, x_dev, shared_gate_dev, hidden);
+        ctx->counters.moe_route++;
+        launch_moe_gemm(shape, rgu, rdn, gu, dn, x_dev, ids, wts, y_dev, ctx->moe_scratch, s);
         ctx->counters.moe_gate_up++;
         ctx->counters.moe_down++;
         LQ4_HIP(hipGetLastError());

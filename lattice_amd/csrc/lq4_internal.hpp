@@ -304,6 +304,18 @@ void launch_moe_down_i8(const uint8_t* down, uint32_t num_experts, uint32_t inte
                         const int32_t* ids, float* o, hipStream_t stream, const uint8_t* last_expert = nullptr);
 // (`last_expert`: the tensor of expert num_experts - 1 when it does not follow the others in `gate_up` / `down`)
 
+// Many tokens per expert (lq4_moe_gemm.hip): grouped GEMM over the experts' blocks, the shared expert (of any width; 0 =
+// none) as one more expert that every token chose.  ids / weights [tokens, slots], slots = top_k, or top_k + 1 with the
+// shared expert's weight in the last one (launch_moe_route with a shared gate).  Scratch from the caller.
+struct MoeGemmShape {
+    uint32_t experts, top_k, inter, shared_inter, hidden, tokens;
+};
+bool moe_gemm_serves(const MoeGemmShape& m);
+size_t moe_gemm_scratch_bytes(const MoeGemmShape& m);
+void launch_moe_gemm(const MoeGemmShape& m, const uint8_t* gate_up, const uint8_t* down, const uint8_t* shared_gate_up,
+                     const uint8_t* shared_down, const float* x, const int32_t* ids, const float* weights, float* y,
+                     uint8_t* scratch, hipStream_t stream);
+
 // Exact top-k over n logits (k <= 256): out_logits / out_ids receive the k best in rank order.
 // `scratch` must hold topk_scratch_bytes(n, k) bytes; `ticket` is one device word that is zero
 // between launches (the kernel counts finished workgroups in it and puts it back to zero).
