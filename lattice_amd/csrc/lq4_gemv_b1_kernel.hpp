@@ -274,10 +274,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
 
     // Loads unit u's blocks.  Lanes past the end of a row and rows past N re-read a valid
     // block; their contribution is zeroed or dropped later.
-    auto load_unit = [&](Q4BlockRaw (&buf)[RW][SG], uint32_t u) {
+    auto load_unit = [&](Q4BlockRaw (&buf)[RW][SG], uint32_t u, int from = 0, int to = RW) {
         const uint32_t chunk = u / slab_groups, sgi = u - chunk * slab_groups;
 #pragma unroll
         for (int j = 0; j < RW; ++j) {
+            if (j < from || j >= to) continue;
             uint32_t wrow = wrow_of(chunk * RW + j);  // scalar
             if (wrow >= n_wrows) wrow = n_wrows - 1;
             uint32_t row = wrow * RPW + sub;
@@ -343,7 +344,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
     }
 
     Q4BlockRaw buf_a[RW][SG], buf_b[RW][SG];
-    load_unit(buf_a, 0);
+    // Fused launches request one row before the staging and the others behind it: a wave whose requests the memory
+    // pipeline does not take yet stands in front of its staging, and with all four gate||up rows of a 12288 x 2048
+    // launch requested first the median wave started its norm after 1.8 us, the last after 3.1 (time stamps).  Token
+    // of 24 layers at hidden 2048: all rows first 445 us, half of them 440, one 429.  A plain launch stages x in a
+    // third of the time and keeps all of them in front.
+    constexpr int kAhead = FUSED ? 1 : RW;
+    load_unit(buf_a, 0, 0, kAhead);
     // residual values of the first chunk's rows, requested now so the final store does not wait
     float res_first[RW];
     if constexpr (FUSED) {
@@ -356,6 +363,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
     }
     __builtin_amdgcn_sched_barrier(0);  // nothing below is scheduled above these loads
 
+    __shared__ float red[FUSED ? WAVES : 1];  // the waves' sums of squares
+    float x_factor = 1.0f;                    // what the staged activations still lack (kAddNorm: 1 / rms)
     // ---- stage x: thread handles (block, dword j) = 8 activations ---------------------------
     auto stage = [&](uint32_t g, const float4 a, const float4 b, bool store) { stage_x8(xsl, g, a, b, store); };
     if constexpr (!FUSED) {
@@ -366,7 +375,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
             stage(g, xp[0], xp[1], true);
         }
     } else {
-        __shared__ float red[WAVES];
         const uint32_t n_units = nb * 4;
         auto unit_at = [](uint32_t g) { return (g >> 2) * kBlockWeights + (g & 3) * 8; };
         auto add4 = [](float4 a, const float4 b) {
@@ -374,9 +382,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
             return a;
         };
         auto sq4 = [](const float4 a) { return (a.x * a.x + a.y * a.y) + (a.z * a.z + a.w * a.w); };
-        auto norm4 = [](float4 v, float inv, const float4 g) {
-            v.x = v.x * inv * (1.0f + g.x); v.y = v.y * inv * (1.0f + g.y);
-            v.z = v.z * inv * (1.0f + g.z); v.w = v.w * inv * (1.0f + g.w);
+        auto gain4 = [](float4 v, const float4 g) {
+            v.x *= 1.0f + g.x; v.y *= 1.0f + g.y; v.z *= 1.0f + g.z; v.w *= 1.0f + g.w;
             return v;
         };
         // v = base + delta for unit g (8 activations)
@@ -391,47 +398,32 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
             }
         };
         if (fz.prologue == GemvFusion::kAddNorm) {
-            // The hoisted units of a thread stay in registers between the sum of squares and the
-            // scaling, with their gamma; longer vectors re-read the rest.
+            // What is staged is v * (1 + gamma); the factor 1 / rms, one number for the whole vector, multiplies the
+            // finished sums instead (the fixed point is relative to each block's largest value, so staging before
+            // or after the factor is the same precision).  Staging so needs no sum of squares first: one barrier
+            // and one pass where the other order has two (the token above 457 -> 445 us).
             float ss = 0.0f;
-#pragma unroll
-            for (int i = 0; i < HF; ++i) {
-                const uint32_t g = tid + i * WAVES * 64;
-                if (g < n_units) {
-                    ss += sq4(xa[i]) + sq4(xb[i]);
+            auto take = [&](uint32_t g, const float4 a, const float4 b, const float4 ga, const float4 gb, bool live) {
+                if (live) {
+                    ss += sq4(a) + sq4(b);
                     if (blockIdx.x == 0 && fz.residual_out) {
                         float4* rp = reinterpret_cast<float4*>(fz.residual_out + unit_at(g));
-                        rp[0] = xa[i];
-                        rp[1] = xb[i];
+                        rp[0] = a;
+                        rp[1] = b;
                     }
                 }
-            }
-            for (uint32_t g = tid + HF * WAVES * 64; g < n_units; g += WAVES * 64) {
-                float4 a, b;
-                load_v(g, a, b);
-                ss += sq4(a) + sq4(b);
-                if (blockIdx.x == 0 && fz.residual_out) {
-                    float4* rp = reinterpret_cast<float4*>(fz.residual_out + unit_at(g));
-                    rp[0] = a;
-                    rp[1] = b;
-                }
-            }
-            ss = wave_sum(ss);
-            if (lane == 0) red[tid >> 6] = ss;
-            __syncthreads();
-            float total = (red[0] + red[1]) + (red[2] + red[3]);
-            if constexpr (WAVES == 8) total += (red[4] + red[5]) + (red[6] + red[7]);
-            static_assert(WAVES == 4 || WAVES == 8, "the sum of squares is combined for four or eight waves");
-            const float inv_rms = 1.0f / sqrtf(total / static_cast<float>(k) + fz.eps);
+                stage(g, gain4(a, ga), gain4(b, gb), live);
+            };
 #pragma unroll
-            for (int i = 0; i < HF; ++i)
-                stage(gx[i], norm4(xa[i], inv_rms, ya[i]), norm4(xb[i], inv_rms, yb[i]), tid + i * WAVES * 64 < n_units);
+            for (int i = 0; i < HF; ++i) take(gx[i], xa[i], xb[i], ya[i], yb[i], tid + i * WAVES * 64 < n_units);
             for (uint32_t g = tid + HF * WAVES * 64; g < n_units; g += WAVES * 64) {
                 float4 a, b;
                 load_v(g, a, b);
                 const float4* gp = reinterpret_cast<const float4*>(fz.gamma + unit_at(g));
-                stage(g, norm4(a, inv_rms, gp[0]), norm4(b, inv_rms, gp[1]), true);
+                take(g, a, b, gp[0], gp[1], true);
             }
+            ss = wave_sum(ss);
+            if (lane == 0) red[tid >> 6] = ss;
         } else if (fz.prologue == GemvFusion::kSiluMul) {
             // silu through the hardware exp2 and reciprocal (about 1 ulp each): every workgroup
             // evaluates the whole vector, so the library expf and an IEEE divide would sit on
@@ -466,7 +458,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
             }
         }
     }
+    if constexpr (kAhead < RW) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_unit(buf_a, 0, kAhead, RW);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     __syncthreads();
+    if constexpr (FUSED) {
+        if (fz.prologue == GemvFusion::kAddNorm) {
+            float total = (red[0] + red[1]) + (red[2] + red[3]);
+            if constexpr (WAVES == 8) total += (red[4] + red[5]) + (red[6] + red[7]);
+            static_assert(WAVES == 4 || WAVES == 8, "the sum of squares is combined for four or eight waves");
+            x_factor = 1.0f / sqrtf(total / static_cast<float>(k) + fz.eps);
+        }
+    }
 
     float acc[RW];
 #pragma unroll
@@ -573,6 +578,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q4_b1(const uint8_t* __restri
                     }
                 }
                 v = segment_sum<SEG>(v);
+                if constexpr (FUSED) v *= x_factor;
                 if constexpr (PAIRS) {
                     if (j % 2 == 0) {
                         gate_kept = v;
