@@ -63,7 +63,7 @@ struct lq4_lora {
     void* b;  // [d_out, rank]
     int is_f16;
     uint32_t rank, d_in, d_out;
-    void* a_packed;  // A as the few-token GEMM's operand (ranks it accepts; else null): that kernel's in-launch A . X
+    void* a_packed;  // A as the few-token GEMM's operand (ranks it accepts; else null): that kernel's own A . X
 };
 
 namespace {
@@ -447,16 +447,13 @@ static bool gemv_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k
 
 // The routing of lq4_gemv once the LoRA factor t (if any) is in ep, or ep.a says that the kernel which serves the
 // shape computes it: which kernel serves (batch, n, k).
-// `x_packed` (may be null): calls in a row on the same x, K and batch share the few-token GEMM's packed activations;
-// true once a call has packed them into the context's scratch.
 static int gemv_dispatch(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, uint32_t k, const float* x_dev, uint32_t batch,
-                         float* y_dev, const LoraEpilogue& ep, hipStream_t s, bool* x_packed = nullptr) {
+                         float* y_dev, const LoraEpilogue& ep, hipStream_t s) {
     int rc;
     if (gemv_takes_few_token_gemm(ctx, n, k, batch)) {
         rc = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, batch), s);
         if (rc) return rc;
-        launch_gemm_skinny(wp, n, k, x_dev, 0, batch, y_dev, ep, ctx->moe_scratch, s, 0, !(x_packed && *x_packed));
-        if (x_packed) *x_packed = true;
+        launch_gemm_skinny(wp, n, k, x_dev, 0, batch, y_dev, ep, ctx->moe_scratch, s);
         ctx->counters.gemm++;
     } else if (batch == 1 && !ep.rank) {
         plain_gemv_one_token(ctx, wp, n, k, x_dev, y_dev, s);
@@ -505,7 +502,7 @@ int lq4_gemv(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
         ep.sync = ctx->lora_sync;
         ep.spin_limit = ctx->lora_spin_limit;
     } else if (ep.rank && batch > 1 && gemv_takes_few_token_gemm(ctx, n, k, batch) && gemm_skinny_computes_t(ep.rank, batch, n)) {
-        ep.a = lora->a_packed;  // the few-token GEMM computes A.x for its token tile itself
+        ep.a = lora->a_packed;  // the few-token GEMM's packing launch computes A.x
     } else if (ep.rank && ctx->lora_in_kernel && gemv_takes_i8(ctx, n, k, batch) &&
                gemv_i8_lora_in_launch(n, k, batch, ep.rank, ctx->cu_count)) {
         // 2..8 rows: `rank` producer workgroups of the launch, on CUs the matrix leaves idle
@@ -522,6 +519,26 @@ int lq4_gemv(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
     LQ4_HIP(hipGetLastError());
     return LQ4_OK;
 }
+
+namespace {
+// lq4_gemv_multi: one more projection for the stacked few-token launch (`a`: that launch computes its A . x).
+void few_token_view(SkinnyViews* few, uint32_t n, const uint8_t* w, float* y, LoraEpilogue e, const void* a) {
+    const uint32_t v = few->count++;
+    e.a = a;
+    few->n[v] = n;
+    few->w[v] = w;
+    few->y[v] = y;
+    few->lora[v] = e;
+}
+
+int launch_few_token_views(lq4_ctx* ctx, const SkinnyViews& few, uint32_t k, const float* x, uint32_t batch, hipStream_t s) {
+    const int rc = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, batch), s);
+    if (rc) return rc;
+    launch_gemm_skinny_views(few, k, x, batch, ctx->moe_scratch, s);
+    ctx->counters.gemm += few.count;
+    return LQ4_OK;
+}
+}  // namespace
 
 int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uint32_t k, const float* x_dev,
                    uint32_t batch, void* stream) {
@@ -574,38 +591,45 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
     hipStream_t s = static_cast<hipStream_t>(stream);
     DeviceGuard g(ctx->device);
     if (batch > kMaxGemvBatch) {
-        // 17..128 rows: lq4_gemm's routing projection by projection.  Those the few-token GEMM serves share one packed
-        // image of x (packed by the first of them) and compute their A . X themselves where that kernel can.
-        if (with_lora) {
+        // 17..128 rows: lq4_gemm's routing.  The projections that the few-token GEMM serves go into one launch of it
+        // (behind one packing launch), the others each into their own.  q, k and v of the 2B model at 64 tokens with
+        // rank-16 adapters on q and v: 18.6 us projection by projection, 12.1 so.
+        SkinnyViews few{};
+        for (uint32_t i = 0, v = 0; i < count; ++i) {
+            const lq4_projection& p = proj[i];
+            if (p.n == 0) continue;
+            if (gemm_takes_few_token_kernel(p.n, k, batch, 0, ctx->gemm_kernel)) {
+                const bool computes_t = ep[i].rank && gemm_skinny_computes_t(ep[i].rank, batch, p.n);
+                few_token_view(&few, p.n, wp[i], p.y_dev, ep[i], computes_t ? p.lora->a_packed : nullptr);
+                if (computes_t) {
+                    av.rank[v] = 0;
+                    --with_lora;
+                }
+            }
+            ++v;
+        }
+        if (with_lora || few.count) {
             const int rc = enter_shared_state(ctx, s);
             if (rc) return rc;
         }
-        bool x_packed = false;
+        if (with_lora) {  // the A . x of the other adapters, in one launch
+            launch_lora_a_views(av, k, x_dev, k, batch, s);
+            ctx->counters.lora_a += with_lora;
+        }
+        if (few.count) {
+            const int rc = launch_few_token_views(ctx, few, k, x_dev, batch, s);
+            if (rc) return rc;
+        }
         for (uint32_t i = 0; i < count; ++i) {
             const lq4_projection& p = proj[i];
-            if (p.n == 0) continue;
-            const bool few = gemm_takes_few_token_kernel(p.n, k, batch, 0, ctx->gemm_kernel);
-            LoraEpilogue e = ep[i];
-            if (e.rank && few && gemm_skinny_computes_t(e.rank, batch, p.n)) {
-                e.a = p.lora->a_packed;
-            } else if (e.rank) {
-                e.t = ctx->lora_t;  // one after the other on this stream
-                launch_lora_a(p.lora->a, p.lora->is_f16, e.rank, k, x_dev, 0, k, batch, ctx->lora_t, s);
-                ctx->counters.lora_a++;
-            }
-            const size_t scratch_bytes = gemm_scratch_floats(p.n, k, batch, 0, e.rank != 0, ctx->gemm_kernel) * sizeof(float);
+            if (p.n == 0 || gemm_takes_few_token_kernel(p.n, k, batch, 0, ctx->gemm_kernel)) continue;
+            const size_t scratch_bytes = gemm_scratch_floats(p.n, k, batch, 0, ep[i].rank != 0, ctx->gemm_kernel) * sizeof(float);
             if (scratch_bytes) {
                 const int rc = ensure_scratch(ctx, scratch_bytes, s);
                 if (rc) return rc;
             }
-            if (few) {
-                launch_gemm_skinny(wp[i], p.n, k, x_dev, 0, batch, p.y_dev, e, ctx->moe_scratch, s, 0, !x_packed);
-                x_packed = true;
-            } else {
-                launch_gemm(wp[i], p.n, k, x_dev, 0, batch, p.y_dev, e,
-                            scratch_bytes ? reinterpret_cast<float*>(ctx->moe_scratch) : nullptr, ctx->gemm_kernel, s);
-                x_packed = false;  // (that kernel's partial tiles share the scratch)
-            }
+            launch_gemm(wp[i], p.n, k, x_dev, 0, batch, p.y_dev, ep[i],
+                        scratch_bytes ? reinterpret_cast<float*>(ctx->moe_scratch) : nullptr, ctx->gemm_kernel, s);
             ctx->counters.gemm++;
         }
         LQ4_HIP(hipGetLastError());
@@ -620,7 +644,7 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
                               (ctx->gemv_i8 == 2 || (k <= 2048 && mv.begin[mv.count] <= 4096)) &&
                               gemv_i8_multi_serves(mv, k, batch, ctx->cu_count);
     if (with_lora && !stacked && !stacked_rows) {
-        // projection by projection: those that go to the few-token GEMM get their A . x there
+        // those that go to the few-token GEMM get their A . x with its packing launch
         for (uint32_t i = 0, v = 0; i < count; ++i) {
             if (proj[i].n == 0) continue;
             if (ep[i].rank && gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch) && gemm_skinny_computes_t(ep[i].rank, batch, proj[i].n)) {
@@ -663,11 +687,20 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
         launch_gemv_multi(mv, k, x_dev, in_launch ? &hand : nullptr, s);
         ctx->counters.gemv_multi++;
     } else {
-        // several rows (or a shape the stacked launch does not take): each projection through lq4_gemv's routing
-        bool x_packed = false;  // the few-token GEMM's packed activations serve every projection that takes it
+        // several rows (or a shape the stacked launch does not take): lq4_gemv's routing, the projections that go to
+        // the few-token GEMM in one launch of it
+        SkinnyViews few{};
         for (uint32_t i = 0; i < count; ++i) {
             if (proj[i].n == 0) continue;
-            int rc = gemv_dispatch(ctx, wp[i], proj[i].n, k, x_dev, batch, proj[i].y_dev, ep[i], s, &x_packed);
+            if (gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch)) {
+                few_token_view(&few, proj[i].n, wp[i], proj[i].y_dev, ep[i], ep[i].a);
+                continue;
+            }
+            const int rc = gemv_dispatch(ctx, wp[i], proj[i].n, k, x_dev, batch, proj[i].y_dev, ep[i], s);
+            if (rc) return rc;
+        }
+        if (few.count) {
+            const int rc = launch_few_token_views(ctx, few, k, x_dev, batch, s);
             if (rc) return rc;
         }
     }
@@ -795,7 +828,7 @@ int lq4_gemm(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
         if (rc) return rc;
     }
     if (ep.rank && gemm_takes_few_token_kernel(n, k, m, x_dtype == LQ4_F16, ctx->gemm_kernel) && gemm_skinny_computes_t(ep.rank, m, n)) {
-        ep.a = lora->a_packed;  // the few-token GEMM computes A.X for its token tile itself
+        ep.a = lora->a_packed;  // the few-token GEMM's packing launch computes A.X
     } else if (ep.rank) {
         launch_lora_a(lora->a, lora->is_f16, lora->rank, k, x_dev, x_dtype == LQ4_F16, k, m, ctx->lora_t, s);
         ctx->counters.lora_a++;

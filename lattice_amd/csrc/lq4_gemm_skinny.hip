@@ -21,14 +21,18 @@
 //    run-time condition would make the compiler wait for loads it cannot count).
 //    Each wave adds its share of the LoRA delta (ranks w, w + 8, ...) to its partial result in
 //    f32; the eight partial results then meet in LDS in a fixed order and y is stored once.
-//    LA = true (Q4, rank <= 16): the factor t = A . X of the workgroup's token tile is computed here as well, A
-//    riding through the K loop as one more 16-row tile against the same packed operands (f16 inputs, f32
-//    accumulation, like the product itself), so that no launch for t precedes this one.  Every workgroup repeats
-//    it for its token tile: 64 KB of A from L2 beside the 256 KB of packed X it reads anyway.
+//    MULTI = true: the workgroups' row tiles run over several matrices of the same K stacked one under the other
+//    (lq4_gemv_multi at 9..128 rows), each with an output and a LoRA delta of its own.
+//
+// The LoRA factors t = A . X of ranks up to 16 come out of launch 1 as well: every wave of it holds one matrix-core
+// operand of X, so A, packed the same way once at upload, costs one more instruction there (f16 inputs, f32
+// accumulation, like the product itself).  The K slices of t go to memory and launch 2 adds them up.
 //
 // Dequantised value: half(q*d + b) with one rounding (shaders/gemm_q4_tiled.metal:57-66), f32
 // accumulation.
 #include "lq4_internal.hpp"
+
+#include <type_traits>
 
 namespace lq4 {
 
@@ -41,6 +45,8 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 constexpr int kWavesK = 8;   // waves of a workgroup, each a K slice
 constexpr int kTokens = 64;  // tokens per workgroup: four groups of 16
 constexpr int TK = 128;      // K per step: four Q4 blocks
+constexpr int kPackSteps = 4;            // K steps a workgroup of the packing launch holds when it computes t
+constexpr uint32_t kMaxTSlices = 8;      // most K slices of t (the K 2048 of a 2B model: four)
 
 struct __attribute__((packed, aligned(4))) Q4BlockRaw {
     uint32_t sb;    // f16 scale | f16 bias << 16
@@ -138,13 +144,30 @@ __device__ __forceinline__ float load_b(const void* b, int is_f16, size_t idx) {
     return is_f16 ? static_cast<float>(static_cast<const _Float16*>(b)[idx]) : static_cast<const float*>(b)[idx];
 }
 
-// grid (K steps, token groups), 256 threads = 4 instructions x 64 lanes of one (step, group).
-// INTERLEAVE: the x0 x4 x1 x5 .. order of the Q4 decoder; false = memory order (sibling formats).
-template <bool X_F16, bool INTERLEAVE>
-__global__ __launch_bounds__(256) void pack_x_kernel(const void* __restrict__ xv, uint32_t m, uint32_t k,
-                                                     uint4* __restrict__ xp) {
-    const uint32_t s = blockIdx.x, t = blockIdx.y, groups = gridDim.y;
-    const int j = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// Adapters whose t = A . X the packing launch computes: `a` packed by gemm_skinny_pack_lora_a, `part` [K slice][token
+// group][lane] float4, element v of lane (c, g) = t[token 16 group + c][rank 4 g + v] over that slice.
+struct PackLora {
+    uint32_t count;
+    const uint4* a[kMaxViews];
+    float4v* part[kMaxViews];
+};
+
+// grid (K slices, token groups), 256 * STEPS threads: 4 instructions x 64 lanes of STEPS K steps at a time; slice p of P
+// takes the runs of STEPS K steps p, p + P, ...  INTERLEAVE: the x0 x4 x1 x5 .. order of the Q4 decoder; false = memory
+// order (sibling formats).  LA: with adapters; four steps a workgroup, so that K slices of t are few.
+template <bool X_F16, bool INTERLEAVE, bool LA>
+__global__ __launch_bounds__(LA ? 1024 : 256) void pack_x_kernel(const void* __restrict__ xv, uint32_t m, uint32_t k,
+                                                                  uint4* __restrict__ xp, uint32_t steps, PackLora la) {
+    constexpr int STEPS = LA ? kPackSteps : 1;
+    const uint32_t t = blockIdx.y, groups = gridDim.y;
+    const int wave = threadIdx.x >> 6;
+    float4v acc[LA ? kMaxViews : 1];
+    if constexpr (LA) {
+#pragma unroll
+        for (int v = 0; v < kMaxViews; ++v) acc[v] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    for (uint32_t s = blockIdx.x * STEPS + wave / 4; s < steps; s += gridDim.x * STEPS) {
+    const int j = wave & 3, lane = threadIdx.x & 63;
     const uint32_t token = 16 * t + (lane & 15);
     const uint32_t koff = s * TK + 32 * (lane >> 4) + 8 * j;
     uint4 out = make_uint4(0, 0, 0, 0);
@@ -178,6 +201,31 @@ __global__ __launch_bounds__(256) void pack_x_kernel(const void* __restrict__ xv
         }
     }
     xp[((static_cast<size_t>(s) * groups + t) * 4 + j) * 64 + lane] = out;
+    if constexpr (LA) {
+#pragma unroll
+        for (int v = 0; v < kMaxViews; ++v)
+            if (v < static_cast<int>(la.count))
+                acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    __builtin_bit_cast(half8, la.a[v][(static_cast<size_t>(s) * 4 + j) * 64 + lane]), __builtin_bit_cast(half8, out), acc[v], 0, 0, 0);
+    }
+    }
+    if constexpr (LA) {  // the waves' sums, in wave order
+        __shared__ float4v part[4 * STEPS][64];
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int v = 0; v < kMaxViews; ++v) {
+            if (v >= static_cast<int>(la.count)) break;
+            if (v) __syncthreads();
+            part[wave][lane] = acc[v];
+            __syncthreads();
+            if (wave == 0) {
+                float4v sum = part[0][lane];
+#pragma unroll
+                for (int w = 1; w < 4 * STEPS; ++w) sum += part[w][lane];
+                la.part[v][(static_cast<size_t>(blockIdx.x) * groups + t) * 64 + lane] = sum;
+            }
+        }
+    }
 }
 
 // RT: 16-row weight tiles per wave (rows per workgroup = 16 RT).  grid (ceil(N / 16 RT), token tiles).
@@ -187,23 +235,36 @@ __global__ __launch_bounds__(256) void pack_x_kernel(const void* __restrict__ xv
 // (grid.y tiles: four groups a tile, or two where NTG is held at two for a larger batch).  Fixed per instantiation, like the prefetches of the K loop below:
 // a load behind a run-time condition makes the compiler wait for loads it cannot count, and the
 // pipeline collapses to one unit in flight.
-// LA: lora.a is the adapter's A packed by gemm_skinny_pack_lora_a and t = A . X is computed here (rank <= 16, Q4
-// only); lora.t is then not read.
-template <int RT, int FMT, int NTG, bool LA = false>
+// MULTI: w, n, y and lora come from `views`, the view that holds this workgroup's row tile.
+struct NoViews {};
+template <int RT, int FMT, int NTG, bool MULTI = false>
 __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __restrict__ w, uint32_t n, uint32_t k,
                                                                 const uint4* __restrict__ xp, uint32_t m,
                                                                 float* __restrict__ y, LoraEpilogue lora,
-                                                                uint32_t tile_groups) {
-    static_assert(!LA || FMT == 0, "the adapter's A is packed in the Q4 decoder's order");
-    static_assert(!LA || NTG <= 2, "with A in the K loop four token groups do not fit the registers");
-    extern __shared__ float4v red[];  // 4 slots of RT * NTG * 64 accumulators; LA: then 8 * NTG * 64 partial t, then t
+                                                                uint32_t tile_groups,
+                                                                typename std::conditional<MULTI, SkinnyViews, NoViews>::type views) {
+    extern __shared__ float4v red[];  // 4 slots of RT * NTG * 64 accumulators
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15;
     const int g = lane >> 4;
 
-    const uint32_t n0 = blockIdx.x * (16 * RT);
+    uint32_t row_tile = blockIdx.x;
+    if constexpr (MULTI) {
+        uint32_t v = 0, first = 0;  // view and its first row tile
+        for (uint32_t tiles = (views.n[0] + 16 * RT - 1) / (16 * RT); row_tile - first >= tiles;) {  // (grid.x = the views' tiles)
+            first += tiles;
+            ++v;
+            tiles = (views.n[v] + 16 * RT - 1) / (16 * RT);
+        }
+        row_tile -= first;
+        w = views.w[v];
+        n = views.n[v];
+        y = views.y[v];
+        lora = views.lora[v];
+    }
+    const uint32_t n0 = row_tile * (16 * RT);
     const uint32_t groups = (m + 15) / 16;             // token groups in X (and in the packed image)
     const uint32_t tg0 = blockIdx.y * tile_groups;  // first token group of this workgroup
     const uint32_t ntg = groups - tg0 < tile_groups ? groups - tg0 : tile_groups;
@@ -221,8 +282,22 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         w_row[u] = w + static_cast<size_t>(row) * (nb * kBytes);
     }
 
-    // LA: A packed like the activations (lq4_pack_lora_a): the operands of step s, instruction j at [(4 s + j) * 64 + lane]
-    const uint4* const a_lane = static_cast<const uint4*>(lora.a) + lane;
+    // The K slices of t (LoraEpilogue::a set: t comes in slices): thread (e, sub) takes slices sub, sub + kSub, ... of float4
+    // e of the tile; requested now for the same reason as B below.
+    constexpr int kSub = 8 / NTG;
+    float4v t_slice[NTG];
+    const uint32_t t_e = threadIdx.x % (NTG * 64), t_sub = threadIdx.x / (NTG * 64);
+    if (lora.a) {
+        uint32_t grp = tg0 + t_e / 64;
+        grp = grp < groups ? grp : groups - 1;
+        const float4v* src = reinterpret_cast<const float4v*>(lora.t) + static_cast<size_t>(grp) * 64 + (t_e & 63);
+#pragma unroll
+        for (int i = 0; i < NTG; ++i) {
+            uint32_t p = t_sub + i * kSub;
+            p = p < lora.t_slices ? p : lora.t_slices - 1;
+            t_slice[i] = src[static_cast<size_t>(p) * groups * 64];
+        }
+    }
     // The LoRA factor B of this wave's first two ranks (w and w + 8) is requested now, as raw bits, and converted in
     // the epilogue: requested there, the loads' whole latency stood between the K loop and the reduction (two token
     // groups of K steps a wave on a 2048-long row: the launch is latency from end to end).
@@ -249,7 +324,6 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     struct Unit {
         WBlock wb[RT];
         uint4 x[NTG][4];  // [token group][instruction]
-        uint4 a[LA ? 4 : 1];  // LA: the lane's operand of A for instruction j
     };
     uint32_t xg[NTG];  // packed-image group of token group t (clamped to the last one)
 #pragma unroll
@@ -261,11 +335,6 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         blk = blk < nb ? blk : nb - 1;
 #pragma unroll
         for (int r = 0; r < RT; ++r) u.wb[r] = *reinterpret_cast<const WBlock*>(w_row[r] + blk * kBytes);
-        if constexpr (LA) {
-            const uint32_t sc = s < steps_total ? s : steps_total - 1;  // (a wave's clamped re-read of its last step)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) u.a[j] = a_lane[(static_cast<size_t>(sc) * 4 + j) * 64];
-        }
         const uint4* xs = xp + static_cast<size_t>(s) * groups * 256 + lane;
 #pragma unroll
         for (int t = 0; t < NTG; ++t)
@@ -278,9 +347,6 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int t = 0; t < NTG; ++t) acc[r][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-    float4v acc_a[NTG];  // LA: element v of lane (lr, g) = t[token 16 (tg0 + t) + lr][rank 4 g + v], this wave's K slice
-#pragma unroll
-    for (int t = 0; t < NTG; ++t) acc_a[t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
     auto compute = [&](const Unit& u, uint32_t i) {
         const bool live = (wave + i * kWavesK) * 4 + g < nb;  // K tail: a block past the end of the row counts as zero
@@ -302,14 +368,6 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
                     acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                         __builtin_bit_cast(half8, a), __builtin_bit_cast(half8, u.x[t][j]), acc[r][t], 0, 0, 0);
             }
-        }
-        if constexpr (LA) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int t = 0; t < NTG; ++t)
-                    acc_a[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                        __builtin_bit_cast(half8, u.a[j]), __builtin_bit_cast(half8, u.x[t][j]), acc_a[t], 0, 0, 0);
         }
     };
 
@@ -358,19 +416,16 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     // ---- LoRA: wave w adds the ranks w, w + 8, ... of scale * B[row, :] . t[token, :] to its own
     //      partial result in f32, so the delta is spread over all waves and joins the same reduction
     constexpr int kSlot = RT * NTG * 64;
-    float* const t_full = reinterpret_cast<float*>(red + 4 * kSlot + kWavesK * NTG * 64);  // [token of the tile][16]
-    if constexpr (LA) {
-        // the eight K slices of t meet in LDS; every (token, rank) is summed in wave order by one thread
-        float4v* const t_part = red + 4 * kSlot;
+    float* const t_full = reinterpret_cast<float*>(red + kMaxTSlices * NTG * 64);  // [token of the tile][16]
+    if (lora.a) {
 #pragma unroll
-        for (int t = 0; t < NTG; ++t) t_part[(wave * NTG + t) * 64 + lane] = acc_a[t];
+        for (int i = 0; i < NTG; ++i)
+            if (t_sub + i * kSub < lora.t_slices) red[(t_sub + i * kSub) * (NTG * 64) + t_e] = t_slice[i];
         __syncthreads();
-        for (uint32_t e = threadIdx.x; e < NTG * 64; e += 64 * kWavesK) {
-            float4v sum = t_part[e];
-#pragma unroll
-            for (int wv = 1; wv < kWavesK; ++wv) sum += t_part[wv * NTG * 64 + e];
-            const uint32_t tg = e >> 6, ln = e & 63;  // token 16 tg + ln % 16, ranks 4 (ln / 16) ..
-            *reinterpret_cast<float4v*>(t_full + (16 * tg + (ln & 15)) * 16 + 4 * (ln >> 4)) = sum;
+        if (t_sub == 0) {  // in slice order, whatever the tile is: t has the same bits in every launch that computes it
+            float4v sum = red[t_e];
+            for (uint32_t p = 1; p < lora.t_slices; ++p) sum += red[p * (NTG * 64) + t_e];
+            *reinterpret_cast<float4v*>(t_full + (16 * (t_e >> 6) + (t_e & 15)) * 16 + 4 * ((t_e & 63) >> 4)) = sum;
         }
         __syncthreads();
     }
@@ -379,13 +434,9 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
             float tv[NTG];
 #pragma unroll
             for (int t = 0; t < NTG; ++t) {
-                if constexpr (LA) {
-                    tv[t] = t_full[(16 * t + lr) * 16 + jj];
-                } else {
-                    uint32_t tok = 16 * (tg0 + t) + lr;
-                    tok = tok < m ? tok : m - 1;
-                    tv[t] = lora.t[static_cast<size_t>(tok) * lora.rank + jj];
-                }
+                uint32_t tok = 16 * (tg0 + t) + lr;
+                tok = tok < m ? tok : m - 1;
+                tv[t] = lora.a ? t_full[(16 * t + lr) * 16 + jj] : lora.t[static_cast<size_t>(tok) * lora.rank + jj];
             }
 #pragma unroll
             for (int r = 0; r < RT; ++r)
@@ -422,6 +473,7 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         }
     }
 
+    if (lora.a) __syncthreads();  // (t in LDS lies where the slots are)
     // ---- the eight K slices meet in LDS in three rounds: (w, w + 4), then (w, w + 2), then (0, 1);
     //      the order is fixed, so the result does not depend on timing
 #pragma unroll
@@ -466,28 +518,30 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     }
 }
 
+// `views`: null, or the matrices of a stacked launch (Q4; w, n, y and lora are then not read).
 template <int RT, int FMT, int NTG>
 void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint32_t m, float* y,
-                const LoraEpilogue& lora, hipStream_t stream) {
+                const LoraEpilogue& lora, const SkinnyViews* views, hipStream_t stream) {
     const uint32_t groups = (m + 15) / 16;
-    const size_t lds = static_cast<size_t>(kWavesK / 2) * RT * NTG * 64 * sizeof(float4v);
-    if constexpr (FMT == 0 && RT == 1 && NTG <= 2) {
-        if (lora.rank && lora.a) {  // t = A . X inside the launch: the waves' partial t and t itself behind the slots
-            const dim3 grid((n + 15) / 16, (groups + NTG - 1) / NTG);
-            const size_t lds_t = lds + static_cast<size_t>(kWavesK) * NTG * 64 * sizeof(float4v) + NTG * 16 * 16 * sizeof(float);
-            hipLaunchKernelGGL((gemm_q4_skinny<RT, FMT, NTG, true>), grid, dim3(64 * kWavesK), lds_t, stream, w, n, k, xp, m,
-                               y, lora, static_cast<uint32_t>(NTG));
+    size_t lds = static_cast<size_t>(kWavesK / 2) * RT * NTG * 64 * sizeof(float4v);
+    const size_t lds_t = kMaxTSlices * NTG * 64 * sizeof(float4v) + NTG * 16 * 16 * sizeof(float);  // slices of t, t
+    if (FMT == 0 && lora.a && lds < lds_t) lds = lds_t;
+    // tiles of two token groups for a batch of more: launch_rt decides when
+    const uint32_t tile_groups = NTG == 2 && groups > 2 ? 2 : kTokens / 16;
+    const uint32_t token_tiles = (groups + tile_groups - 1) / tile_groups;
+    if constexpr (FMT == 0) {
+        if (views) {
+            uint32_t tiles = 0;
+            for (uint32_t v = 0; v < views->count; ++v) tiles += (views->n[v] + 16 * RT - 1) / (16 * RT);
+            for (uint32_t v = 0; v < views->count; ++v)
+                if (views->lora[v].a && lds < lds_t) lds = lds_t;
+            hipLaunchKernelGGL((gemm_q4_skinny<RT, FMT, NTG, true>), dim3(tiles, token_tiles), dim3(64 * kWavesK), lds, stream,
+                               w, n, k, xp, m, y, lora, tile_groups, *views);
             return;
         }
     }
-    if (NTG == 2 && groups > 2) {  // tiles of two token groups (launch_rt decides when)
-        const dim3 grid2((n + 16 * RT - 1) / (16 * RT), (groups + 1) / 2);
-        hipLaunchKernelGGL((gemm_q4_skinny<RT, FMT, NTG>), grid2, dim3(64 * kWavesK), lds, stream, w, n, k, xp, m, y, lora, 2u);
-        return;
-    }
-    const dim3 grid((n + 16 * RT - 1) / (16 * RT), (m + kTokens - 1) / kTokens);
-    hipLaunchKernelGGL((gemm_q4_skinny<RT, FMT, NTG>), grid, dim3(64 * kWavesK), lds, stream, w, n, k, xp, m, y, lora,
-                       static_cast<uint32_t>(kTokens / 16));
+    hipLaunchKernelGGL((gemm_q4_skinny<RT, FMT, NTG>), dim3((n + 16 * RT - 1) / (16 * RT), token_tiles), dim3(64 * kWavesK), lds,
+                       stream, w, n, k, xp, m, y, lora, tile_groups, NoViews{});
 }
 
 // Widest row tile (of 1 or 2) whose two units in flight fit the 256 registers of a wave without spilling.
@@ -499,37 +553,16 @@ constexpr int max_rt(int fmt, int ntg) {
 
 template <int RT, int FMT>
 void launch_rt(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint32_t m, float* y, const LoraEpilogue& lora,
-               hipStream_t stream) {
+               const SkinnyViews* views, hipStream_t stream) {
     const uint32_t groups = (m + 15) / 16;
-    if (lora.rank && lora.a) {
-        // with A as one more tile in the K loop neither a second row tile nor four token groups fit the registers:
-        // one row tile, and tiles of two token groups from 33 tokens on (more workgroups, each re-reading its rows)
-        if constexpr (RT > 1) return launch_rt<1, FMT>(w, n, k, xp, m, y, lora, stream);
-        if (groups > 2) return launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, stream);
-    }
-    if constexpr (RT == 1 && FMT == 0) {  // (measured for Q4 only)
-        // Token tiles of 32 instead of 64 where that fills the chip better: twice the workgroups, each 0.6-0.65 of the
-        // time (its rows are read once more, its fixed parts stay).  One workgroup runs per CU, so it pays when the
-        // workgroups of the 64-token form are at most half the CUs, or leave the second round of workgroups at most
-        // half full (measured at 64 tokens, us: 2048 x 2048 8.15 -> 6.91, 512 x 2048 7.63 -> 6.21, 2048 x 6144 14.9 ->
-        // 11.2, 2048 x 12288 30.7 -> 22.9, 5120 x 5120 26.6 -> 23.0, 6144 x 2048 12.8 -> 11.0; against 3072 x 2048 8.23 ->
-        // 8.72, 4096 x 2048 8.44 -> 8.80, 4096 x 4096 12.5 -> 13.6, which keep 64).
-        const uint32_t wgs = ((n + 15) / 16) * ((m + kTokens - 1) / kTokens);
-        if (groups > 2 && (wgs <= 128 || (wgs > 256 && wgs <= 384)))
-            return launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, stream);
-    }
-    if (groups == 1) launch_ntg<(RT < max_rt(FMT, 1) ? RT : max_rt(FMT, 1)), FMT, 1>(w, n, k, xp, m, y, lora, stream);
-    else if (groups == 2) launch_ntg<(RT < max_rt(FMT, 2) ? RT : max_rt(FMT, 2)), FMT, 2>(w, n, k, xp, m, y, lora, stream);
-    else launch_ntg<(RT < max_rt(FMT, 4) ? RT : max_rt(FMT, 4)), FMT, 4>(w, n, k, xp, m, y, lora, stream);
+    if (groups == 1) launch_ntg<(RT < max_rt(FMT, 1) ? RT : max_rt(FMT, 1)), FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
+    else if (groups == 2) launch_ntg<(RT < max_rt(FMT, 2) ? RT : max_rt(FMT, 2)), FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+    else launch_ntg<(RT < max_rt(FMT, 4) ? RT : max_rt(FMT, 4)), FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
 }
 
 }  // namespace
 
-// The few-token kernel computes t = A . X itself (LoraEpilogue::a set, no launch for t) for Q4, ranks up to 16 and
-// up to 64 tokens (q and v of the 2B model, rank 16, 64 tokens: 13.6 us with a launch for t -> 8.3 / 7.7, against
-// 8.0 / 7.6 without an adapter).  From 65 tokens on its tiles of 32 tokens are three or four to a row tile: taken
-// while those workgroups still find a CU each (512 x 2048 at 128 tokens 10.2 -> 8.0 us; 2048 x 2048, 512 workgroups,
-// 12.8 -> 13.0 and left with the launch for t).
+// Adapters whose t = A . X the packing launch computes (LoraEpilogue::a set, no launch of its own).
 bool gemm_skinny_packs_lora_a(uint32_t rank) { return rank != 0 && rank <= 16; }
 bool gemm_skinny_computes_t(uint32_t rank, uint32_t m, uint32_t n) {
     if (!gemm_skinny_packs_lora_a(rank)) return false;
@@ -580,39 +613,91 @@ bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m) {
 
 size_t gemm_skinny_scratch_bytes(uint32_t k, uint32_t m) {
     const size_t steps = (k / kBlockWeights + 3) / 4, groups = (m + 15) / 16;
-    return steps * groups * 256 * sizeof(uint4);
+    return (steps * groups * 256 + kMaxViews * kMaxTSlices * groups * 64) * sizeof(uint4);  // packed X, slices of t
 }
 
 namespace {
 
 template <int FMT>
 void launch_fmt(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m, float* y,
-                const LoraEpilogue& lora, void* packed_x, hipStream_t stream, bool pack) {
+                LoraEpilogue lora, SkinnyViews* views, void* packed_x, hipStream_t stream) {
     const uint32_t steps = (k / kBlockWeights + 3) / 4, groups = (m + 15) / 16;
     uint4* xp = static_cast<uint4*>(packed_x);
     constexpr bool kInterleave = FMT == 0;
-    if (!pack) {
-    } else if (x_is_f16)
-        hipLaunchKernelGGL((pack_x_kernel<true, kInterleave>), dim3(steps, groups), dim3(256), 0, stream, x, m, k, xp);
-    else
-        hipLaunchKernelGGL((pack_x_kernel<false, kInterleave>), dim3(steps, groups), dim3(256), 0, stream, x, m, k, xp);
+    PackLora la{};
+    const uint32_t runs = (steps + kPackSteps - 1) / kPackSteps, slices = runs < kMaxTSlices ? runs : kMaxTSlices;
+    auto produce_t = [&](LoraEpilogue& e) {  // e.a: packed A; e.t becomes the place of the slices
+        if (!e.rank || !e.a) return;
+        const uint32_t v = la.count++;
+        la.a[v] = static_cast<const uint4*>(e.a);
+        la.part[v] = reinterpret_cast<float4v*>(xp + static_cast<size_t>(steps) * groups * 256) + static_cast<size_t>(v) * kMaxTSlices * groups * 64;
+        e.t = reinterpret_cast<const float*>(la.part[v]);
+        e.t_slices = slices;
+    };
+    uint32_t tiles16 = (n + 15) / 16;
+    if (views) {
+        tiles16 = 0;
+        for (uint32_t v = 0; v < views->count; ++v) {
+            tiles16 += (views->n[v] + 15) / 16;
+            produce_t(views->lora[v]);
+        }
+    } else {
+        produce_t(lora);
+    }
+    if constexpr (FMT == 0) {
+        if (la.count) {
+            const dim3 grid(slices, groups), block(256 * kPackSteps);
+            if (x_is_f16) hipLaunchKernelGGL((pack_x_kernel<true, true, true>), grid, block, 0, stream, x, m, k, xp, steps, la);
+            else hipLaunchKernelGGL((pack_x_kernel<false, true, true>), grid, block, 0, stream, x, m, k, xp, steps, la);
+        }
+    }
+    if (!la.count) {
+        const dim3 grid(steps, groups), block(256);
+        if (x_is_f16) hipLaunchKernelGGL((pack_x_kernel<true, kInterleave, false>), grid, block, 0, stream, x, m, k, xp, steps, la);
+        else hipLaunchKernelGGL((pack_x_kernel<false, kInterleave, false>), grid, block, 0, stream, x, m, k, xp, steps, la);
+    }
     // Every workgroup reads the whole packed X of its token tile, so a wider row tile halves that
     // traffic, at the price of fewer workgroups to balance over the compute units.  Measured over
     // 2048..34816 rows and K 2048..17408 at 16, 32 and 64 tokens: two row tiles pay on tall matrices,
     // on long rows and with four token groups; four never do since the K loop keeps two units in flight.
-    const uint32_t tiles16 = (n + 15) / 16;
+    if constexpr (FMT == 0) {
+        if (groups > 2) {
+            // Q4 at 33..128 tokens: one workgroup runs per CU, so a tile's cost is its rounds of 256 workgroups times
+            // what a workgroup of it takes.  Relative to 16 rows x 64 tokens (8.2 us at K 2048): 16 x 32 0.63, 32 x 32
+            // 1.08, 32 x 64 1.57, the last only where it is one round (a second one takes more than twice that).  us
+            // at 16 x 64 / 16 x 32 / 32 x 32 / 32 x 64, packing included: 64 tokens 4096 x 4096 11.4 / 13.3 / 11.5 /
+            // 15.5, 6144 x 4096 25.3 / 25.3 / 25.9 / 22.4, 1536 x 1024 9.8 / 8.7 / 10.5 / 13.6; 96 tokens 4608 x 2048
+            // 16.7 / 14.9 / 12.6 / 19.4; 128 tokens 4096 x 4096 19.2 / 22.8 / 19.1 / 16.7.
+            const uint32_t t32 = (tiles16 + 1) / 2, q = (groups + 3) / 4, h = (groups + 1) / 2;
+            auto rounds = [](uint32_t wgs) { return (wgs + 255) / 256; };
+            const uint32_t cost[4] = {100 * rounds(tiles16 * q), 63 * rounds(tiles16 * h), 108 * rounds(t32 * h),
+                                      t32 * q <= 256 ? 157u : 0xFFFFFFFFu};
+            int best = 0;
+            for (int i = 1; i < 4; ++i)
+                if (cost[i] < cost[best]) best = i;
+            if (best == 0) launch_ntg<1, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
+            else if (best == 1) launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+            else if (best == 2) launch_ntg<2, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+            else launch_ntg<2, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
+            return;
+        }
+    }
     const bool wide = tiles16 >= 1024 || (k >= 8192 && tiles16 >= 256) || (m > 32 && tiles16 >= 512);
-    if (wide) launch_rt<2, FMT>(w, n, k, xp, m, y, lora, stream);
-    else launch_rt<1, FMT>(w, n, k, xp, m, y, lora, stream);
+    if (wide) launch_rt<2, FMT>(w, n, k, xp, m, y, lora, views, stream);
+    else launch_rt<1, FMT>(w, n, k, xp, m, y, lora, views, stream);
 }
 
 }  // namespace
 
 void launch_gemm_skinny(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m, float* y,
-                        const LoraEpilogue& lora, void* packed_x, hipStream_t stream, int fmt, bool pack) {
-    if (fmt == 1) launch_fmt<1>(w, n, k, x, x_is_f16, m, y, lora, packed_x, stream, pack);
-    else if (fmt == 2) launch_fmt<2>(w, n, k, x, x_is_f16, m, y, lora, packed_x, stream, pack);
-    else launch_fmt<0>(w, n, k, x, x_is_f16, m, y, lora, packed_x, stream, pack);
+                        const LoraEpilogue& lora, void* packed_x, hipStream_t stream, int fmt) {
+    if (fmt == 1) launch_fmt<1>(w, n, k, x, x_is_f16, m, y, lora, nullptr, packed_x, stream);
+    else if (fmt == 2) launch_fmt<2>(w, n, k, x, x_is_f16, m, y, lora, nullptr, packed_x, stream);
+    else launch_fmt<0>(w, n, k, x, x_is_f16, m, y, lora, nullptr, packed_x, stream);
+}
+
+void launch_gemm_skinny_views(SkinnyViews views, uint32_t k, const float* x, uint32_t m, void* packed_x, hipStream_t stream) {
+    launch_fmt<0>(nullptr, 0, k, x, 0, m, nullptr, LoraEpilogue{}, &views, packed_x, stream);
 }
 
 }  // namespace lq4

@@ -52,6 +52,7 @@ struct LoraEpilogue {
     unsigned long long* slots;  // [kMaxLoraRank]
     uint32_t* sync;
     uint32_t spin_limit;
+    uint32_t t_slices;          // the few-token GEMM's own: `t` is that many K slices, still to be added up
 };
 
 // Several matrices with rows of the same K against one activation vector in one batch-1 launch: the rows of the
@@ -246,16 +247,24 @@ void launch_gemm_q3(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int
 // (gemm_skinny_scratch_bytes bytes at `packed_x`), then a kernel without LDS staging.
 bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m);
 size_t gemm_skinny_scratch_bytes(uint32_t k, uint32_t m);
-// For Q4 and a LoRA rank this accepts, the kernel computes t = A . X itself when LoraEpilogue::a points to A as
-// packed (on the host, once) by gemm_skinny_pack_lora_a; t is then not read and no launch for it has to precede.
+// For Q4 and a LoRA rank this accepts the packing launch computes t = A . X when LoraEpilogue::a points to A as packed
+// (on the host, once) by gemm_skinny_pack_lora_a; t is then not read and no launch for it has to precede.
 bool gemm_skinny_computes_t(uint32_t rank, uint32_t m, uint32_t n);
 bool gemm_skinny_packs_lora_a(uint32_t rank);  // an adapter of this rank gets a packed copy of A at upload
 size_t gemm_skinny_packed_lora_a_bytes(uint32_t k);
 void gemm_skinny_pack_lora_a(const void* a_host, int a_is_f16, uint32_t rank, uint32_t k, void* out_host);
 // fmt: 0 = Q4 blocks, 1 = Q8_0, 2 = Q3.
-// pack = false: `packed_x` already holds the packed image of this x (an earlier call with the same x, K, m and format).
 void launch_gemm_skinny(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m, float* y,
-                        const LoraEpilogue& lora, void* packed_x, hipStream_t stream, int fmt = 0, bool pack = true);
+                        const LoraEpilogue& lora, void* packed_x, hipStream_t stream, int fmt = 0);
+// Several Q4 matrices with rows of the same K against one x (f32) in one launch, bit for bit what a launch each gives.
+struct SkinnyViews {
+    uint32_t count;
+    uint32_t n[kMaxViews];
+    const uint8_t* w[kMaxViews];
+    float* y[kMaxViews];
+    LoraEpilogue lora[kMaxViews];  // each with a t of its own
+};
+void launch_gemm_skinny_views(SkinnyViews views, uint32_t k, const float* x, uint32_t m, void* packed_x, hipStream_t stream);
 
 bool launch_probe_read(const void* p, size_t nbytes, uint32_t grid, uint32_t in_flight, bool strided, bool nontemporal,
                        uint32_t* sink, hipStream_t stream);

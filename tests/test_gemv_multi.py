@@ -280,3 +280,29 @@ def test_multi_contract_errors_launch_nothing(be):
     c1 = be.path_counters()
     assert c1["gemv_multi"] == c0["gemv_multi"] and c1["gemv"] == c0["gemv"]
     assert np.all(host(y0) == -3.0)
+
+
+@pytest.mark.parametrize("batch,k,shapes", [(9, 96, (16, 7, 33)), (17, 2080, (40, 129)), (33, 1024, (1040, 24, 16)), (96, 2048, (1000, 1576, 64)),
+                                            (127, 544, (4100, 31)), (128, 4096, (3000, 1096))])
+def test_multi_few_token_views_in_one_launch(be, batch, k, shapes):
+    # views that end inside a row tile, token tiles of 32 and 64, a K that is no whole step: the stacked few-token launch,
+    # adapters (K slices of A . X from one to eight) on every other view
+    import torch
+    print(f"few-token views rows={batch} k={k} shapes={shapes}", flush=True)
+    names = ("q_proj", "k_proj", "v_proj")[:len(shapes)]
+    ws, qs = _views(be, shapes, k, seed=70)
+    mods = {nm: synth.lora_pair(5 + 11 * i, k, shapes[2 * i], seed=4, tag=nm) for i, nm in enumerate(names[::2])}
+    x = synth.activations(batch, k, seed=11)
+    be.load_lora_adapter([backend.LoraLayerData(0, mods)], scale=1.5)
+    try:
+        ys = [torch.full((batch, n), float("nan"), dtype=torch.float32, device="cuda") for n in shapes]
+        be.gemv_multi(dev(x), [(q, n, y, nm) for q, n, y, nm in zip(qs, shapes, ys, names)], batch, k, layer_idx=0)
+        be.synchronize()
+        for w, n, y, nm in zip(ws, shapes, ys, names):
+            want = oracle.gemm_f32(x, w, n, k)
+            if nm in mods:
+                a, b = mods[nm]
+                want = oracle.lora_apply(a.astype(np.float32), b.astype(np.float32), 1.5, x, want)
+            assert rel_err(host(y), want) <= REL_TOL
+    finally:
+        be.unload_lora_adapter()
