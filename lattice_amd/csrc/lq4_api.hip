@@ -1801,7 +1801,7 @@ int lq4_gemm_q8(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
     if (m == 1 && x_dtype == LQ4_F32 && gemv_q8_lds_bytes(k) <= 128 * 1024) {
         launch_gemv_q8_b1(wp, n, k, static_cast<const float*>(x_dev), y_dev, s);
         ctx->counters.gemv++;
-    } else if (m <= 32 || gemm_skinny_wants(n, k, m)) {
+    } else if (m <= 32 || gemm_skinny_wants(n, k, m, 1)) {
         // few rows: operands packed once, the few-token matrix-core kernel with this format's decoder
         // (always up to 32 rows: the large-tile kernels are no match for it there)
         const int src = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, m), static_cast<hipStream_t>(stream));
@@ -1810,7 +1810,7 @@ int lq4_gemm_q8(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
         launch_gemm_skinny(wp, n, k, x_dev, x_dtype == LQ4_F16, m, y_dev, none, ctx->moe_scratch, s, 1);
         ctx->counters.gemm++;
     } else {
-        const int src = ensure_scratch(ctx, gemm_sibling_scratch_floats(1, n, k, m, ctx->gemm_kernel) * sizeof(float), static_cast<hipStream_t>(stream));
+        const int src = ensure_scratch(ctx, gemm_sibling_scratch_floats(1, n, k, m, x_dtype == LQ4_F16, ctx->gemm_kernel) * sizeof(float), static_cast<hipStream_t>(stream));
         if (src) return src;
         launch_gemm_q8(wp, n, k, x_dev, x_dtype == LQ4_F16, m, y_dev, reinterpret_cast<float*>(ctx->moe_scratch), ctx->gemm_kernel, s);
         ctx->counters.gemm++;
@@ -1842,7 +1842,7 @@ int lq4_gemm_q3(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
     if (m == 1 && x_dtype == LQ4_F32 && gemv_q3_lds_bytes(k) <= 128 * 1024) {
         launch_gemv_q3_b1(wp, n, k, static_cast<const float*>(x_dev), y_dev, s);
         ctx->counters.gemv++;
-    } else if (m <= 32 || gemm_skinny_wants(n, k, m)) {
+    } else if (m <= 32 || gemm_skinny_wants(n, k, m, 2)) {
         // few rows: operands packed once, the few-token matrix-core kernel with this format's decoder
         // (always up to 32 rows: the large-tile kernels are no match for it there)
         const int src = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, m), static_cast<hipStream_t>(stream));
@@ -1851,7 +1851,7 @@ int lq4_gemm_q3(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
         launch_gemm_skinny(wp, n, k, x_dev, x_dtype == LQ4_F16, m, y_dev, none, ctx->moe_scratch, s, 2);
         ctx->counters.gemm++;
     } else {
-        const int src = ensure_scratch(ctx, gemm_sibling_scratch_floats(2, n, k, m, ctx->gemm_kernel) * sizeof(float), static_cast<hipStream_t>(stream));
+        const int src = ensure_scratch(ctx, gemm_sibling_scratch_floats(2, n, k, m, x_dtype == LQ4_F16, ctx->gemm_kernel) * sizeof(float), static_cast<hipStream_t>(stream));
         if (src) return src;
         launch_gemm_q3(wp, n, k, x_dev, x_dtype == LQ4_F16, m, y_dev, reinterpret_cast<float*>(ctx->moe_scratch), ctx->gemm_kernel, s);
         ctx->counters.gemm++;

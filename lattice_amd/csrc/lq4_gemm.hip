@@ -539,7 +539,7 @@ size_t gemm_scratch_floats(uint32_t n, uint32_t k, uint32_t m, int x_is_f16, boo
     const GemmPlan p = plan_gemm(n, k, m, x_is_f16, with_lora, forced);
     if (p.skinny) return (gemm_skinny_scratch_bytes(k, m) + sizeof(float) - 1) / sizeof(float);
     if (p.w2) return (gemm_w2_scratch_bytes(n, k, m) + sizeof(float) - 1) / sizeof(float);
-    return p.wreg ? gemm_wreg_scratch_floats(n, k, m) : 0;
+    return p.wreg ? gemm_wreg_scratch_floats(n, k, m, 0, x_is_f16 != 0, with_lora) : 0;
 }
 
 void launch_gemm(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m,
@@ -557,28 +557,30 @@ void launch_gemm(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_
     }
 }
 
-// Sibling formats: the weights-in-registers kernel with the format's decoder, unless the tile
-// kernel is forced (choice 1).  Q8_0 blocks are 1.7 x the bytes and 2-byte aligned, which costs the
-// register kernel more than the tile kernel (measured): it is taken on long, wide matrices only.
+// Sibling formats: the weights-in-registers kernel with the format's decoder, unless the tile kernel is forced (choice
+// 1).  Q8_0 with f16 activations on short rows stays on the tile kernel while its tiles are few: there is too little K
+// for slices or small tiles to pay (908 x 1049 x 608 12.4 against 13.8 us, 1364 x 413 x 1248 14.3 against 16.3; but
+// 1663 x 1158 x 1248 26.0 against 22.0, and with f32 activations 2021 x 506 x 4672 45 against 33).
 namespace {
-bool sibling_wants_wreg(int fmt, uint32_t n, uint32_t k, int forced) {
+bool sibling_wants_wreg(int fmt, uint32_t n, uint32_t k, uint32_t m, int x_is_f16, int forced) {
     if (forced == 1) return false;
-    if (forced == 2) return true;
-    return fmt != 1 || (k >= 4096 && n >= 4096);
+    if (forced == 2 || fmt != 1 || !x_is_f16) return true;
+    const uint32_t tiles = ((n + 127) / 128) * ((m + BM - 1) / BM);
+    return !((k <= 640 && tiles <= 256) || (k <= 1280 && tiles <= 64));
 }
 
 template <int FMT>
 void launch_sibling(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m, float* y,
                     float* scratch, int forced, hipStream_t stream) {
     const LoraEpilogue none{nullptr, nullptr, 0, 0, 0.0f};
-    if (sibling_wants_wreg(FMT, n, k, forced)) return launch_gemm_wreg(w, n, k, x, x_is_f16, m, y, none, scratch, stream, FMT);
+    if (sibling_wants_wreg(FMT, n, k, m, x_is_f16, forced)) return launch_gemm_wreg(w, n, k, x, x_is_f16, m, y, none, scratch, stream, FMT);
     if (x_is_f16) launch_tile<true, 128, false, FMT>(w, n, k, x, m, y, none, stream, scratch);
     else launch_tile<false, 128, false, FMT>(w, n, k, x, m, y, none, stream, scratch);
 }
 }  // namespace
 
-size_t gemm_sibling_scratch_floats(int fmt, uint32_t n, uint32_t k, uint32_t m, int forced) {
-    if (sibling_wants_wreg(fmt, n, k, forced)) return gemm_wreg_scratch_floats(n, k, m);
+size_t gemm_sibling_scratch_floats(int fmt, uint32_t n, uint32_t k, uint32_t m, int x_is_f16, int forced) {
+    if (sibling_wants_wreg(fmt, n, k, m, x_is_f16, forced)) return gemm_wreg_scratch_floats(n, k, m, fmt, x_is_f16 != 0, false);
     const TileSlices ts = plan_tile_slices<128>(n, k, m);
     if (ts.count < 2) return 0;
     return static_cast<size_t>((n + 127) / 128) * ((m + BM - 1) / BM) * ts.count * (BM * 128);

@@ -597,17 +597,22 @@ void gemm_skinny_pack_lora_a(const void* a, int a_is_f16, uint32_t rank, uint32_
             }
 }
 
-bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m) {
-    // Against the large-tile kernel, which wastes the empty part of its 128-token tile but shares the
-    // activations of a tile among 256 rows where this kernel re-reads them for every 16..64 rows
+bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt) {
+    // Against the large-tile kernel, which wastes the empty part of its token tile but shares the
+    // activations of a tile among up to 256 rows where this kernel re-reads them for every 16..64 rows
     // (measured on 6M..500M-weight matrices): up to 16 tokens are always served here; one token tile
     // unless the matrix is large
     // (above 2^26 weights) and either more than 32 tokens, fewer than 8192 rows (too few workgroups
-    // here) or more than 2^28 weights; two token tiles only up to 2^24 weights.
+    // here) or more than 2^28 weights; two token tiles only up to 2^24 weights.  From 33 tokens on a
+    // tall matrix (more rows than 12288) goes to the large tile whatever its K: there are enough of them
+    // (16384 x 1024 at 64 / 128 tokens 15.7 / 27.6 us here, 13.4 / 14.8 there; 12288 x 2048 17.2 / 19.1 at 64).
+    // The sibling formats, whose decoders are longer and run once per 32 or 64 tokens here, leave from 8192 x 2048 on.
     if (k < kBlockWeights) return false;
     const uint64_t weights = static_cast<uint64_t>(n) * k;
     if (m <= 16) return true;
+    if (m > 32 && n > 12288) return false;
     if (m <= kTokens) return weights <= (1ull << 26) || (m <= 32 && n >= 8192 && weights <= (1ull << 28));
+    if (fmt && n >= 8192 && k >= 2048) return false;
     return m <= 2 * kTokens && weights <= (1ull << 24);
 }
 

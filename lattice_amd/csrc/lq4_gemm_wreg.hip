@@ -1,12 +1,12 @@
 // Prefill GEMM, weights-in-registers variant: Y[M,N] = X[M,K] . W[N,K]^T for large shapes.
 //
-// A workgroup of four waves owns 128 tokens x 256 weight rows; wave w owns weight rows
-// 64w .. 64w+63 against all 128 tokens.  Only the activations go through LDS (f16, double
+// A workgroup of four waves owns 16 NT tokens x 64 NU weight rows (128 x 256 the largest, see kWregTiles); wave w owns
+// 16 NU weight rows against all the tokens.  Only the activations go through LDS (f16, double
 // buffered, one barrier per 128-wide K step).  Weights never touch LDS: every lane loads whole
 // Q4 blocks straight from global memory, dequantises them in registers and feeds them to
 // v_mfma_f32_16x16x32_f16 as the A operand.  Compared with staging dequantised weights in LDS
 // this removes 2 bytes of LDS write and 2 x 2 bytes of LDS read per weight, and each weight is
-// dequantised exactly once per 128 tokens.
+// dequantised exactly once per token tile.
 //
 // The K dimension inside one matrix-core instruction is a sum, so its order is free as long as
 // both operands agree.  A K step covers four Q4 blocks; lane (r = lane % 16, g = lane / 16)
@@ -42,7 +42,6 @@ constexpr int TM = 128;                    // tokens per workgroup
 constexpr int TN = 256;                    // weight rows per workgroup
 constexpr int TK = 128;                    // K per step: four Q4 blocks
 constexpr int kPitch16 = TK * 2 / 16 + 1;  // LDS row pitch in 16-byte units (272 bytes)
-constexpr int kBuf16 = TM * kPitch16;      // one activation buffer, in 16-byte units
 constexpr int kGroupM = 16;                // token tiles per rasterisation group
 constexpr int NU = 4;                      // 16-row weight tiles per wave
 constexpr int NT = TM / 16;                // 16-token tiles per workgroup
@@ -53,9 +52,17 @@ struct __attribute__((packed, aligned(4))) Q4BlockRaw {
 };
 
 // Sibling formats (FMT 1 = Q8_0, 2 = Q3).
-struct __attribute__((packed, aligned(2))) Q8BlockRaw {
-    uint16_t d;     // f16 scale
-    uint32_t q[8];  // 32 x i8, weight i in byte i
+// A Q8_0 block (u16 scale, 32 x i8, weight i in byte i) is 34 bytes, so every other block starts in the middle of a
+// dword, and a vector load that does costs the address unit two clocks a lane instead of one.  The registers hold the
+// eight whole dwords of the block and its odd half: a block that starts on a dword keeps the scale in the low half of
+// q[0] and its last two weights in h, one that starts two bytes past one keeps the scale in h.  Both are brought into
+// order by byte-aligns of neighbours (by two bytes or none) as the weights are decoded.
+struct Q8BlockRaw {
+    uint32_t q[8];
+    uint32_t h;
+};
+struct __attribute__((packed, aligned(4))) Dwords8 {
+    uint32_t v[8];
 };
 struct __attribute__((packed, aligned(4))) Q3BlockRaw {
     uint32_t sb;     // f16 scale | f16 bias << 16
@@ -112,7 +119,7 @@ struct DqOps {
 };
 template <>
 struct DqOps<1> {
-    static constexpr int kOps = 14;
+    static constexpr int kOps = 16;
 };
 template <>
 struct DqOps<2> {
@@ -138,17 +145,20 @@ __device__ __forceinline__ void dq_op_q4(int op, uint32_t q, half2v d2, half2v b
 
 // Q8_0, weights 8j..8j+7 in memory order -> half(q * d): a sign-flipped byte (q + 128) under the
 // exponent byte of 1024.0 is 1024 + 128 + q exactly; one subtract, one multiply (a single rounding).
-__device__ __forceinline__ void dq_op_q8(int op, const Q8BlockRaw& blk, int j, half2v d2, DqTmp& tmp, U4& out) {
+// `shift`: 2 where the block starts on a dword, else 0 (see Q8BlockRaw).
+__device__ __forceinline__ void dq_op_q8(int op, const Q8BlockRaw& blk, int j, uint32_t shift, half2v d2, DqTmp& tmp, U4& out) {
     const half2v k1152 = {static_cast<_Float16>(1152.0f), static_cast<_Float16>(1152.0f)};
     switch (op) {
-        case 0: tmp.qa = blk.q[2 * j] ^ 0x80808080u; break;
-        case 1: tmp.q8 = blk.q[2 * j + 1] ^ 0x80808080u; break;
-        case 2: tmp.t[0] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.qa, 0x04010400u)); break;
-        case 3: tmp.t[1] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.qa, 0x04030402u)); break;
-        case 4: tmp.t[2] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.q8, 0x04010400u)); break;
-        case 5: tmp.t[3] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.q8, 0x04030402u)); break;
-        case 6: case 7: case 8: case 9: tmp.t[op - 6] -= k1152; break;
-        default: out.v[op - 10] = as_u32(tmp.t[op - 10] * d2); break;
+        case 0: tmp.qa = __builtin_amdgcn_alignbyte(blk.q[2 * j + 1], blk.q[2 * j], shift); break;
+        case 1: tmp.q8 = __builtin_amdgcn_alignbyte(j < 3 ? blk.q[(2 * j + 2) & 7] : blk.h, blk.q[2 * j + 1], shift); break;
+        case 2: tmp.qa ^= 0x80808080u; break;
+        case 3: tmp.q8 ^= 0x80808080u; break;
+        case 4: tmp.t[0] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.qa, 0x04010400u)); break;
+        case 5: tmp.t[1] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.qa, 0x04030402u)); break;
+        case 6: tmp.t[2] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.q8, 0x04010400u)); break;
+        case 7: tmp.t[3] = as_h2(__builtin_amdgcn_perm(0x64646464u, tmp.q8, 0x04030402u)); break;
+        case 8: case 9: case 10: case 11: tmp.t[op - 8] -= k1152; break;
+        default: out.v[op - 12] = as_u32(tmp.t[op - 12] * d2); break;
     }
 }
 
@@ -185,9 +195,9 @@ __device__ __forceinline__ void dq_op_q3(int op, const Q3BlockRaw& blk, int j, h
 }
 
 template <int FMT, typename WBlock>
-__device__ __forceinline__ void dq_op(int op, const WBlock& blk, int j, half2v d2, half2v b2, DqTmp& tmp, U4& out) {
+__device__ __forceinline__ void dq_op(int op, const WBlock& blk, int j, uint32_t shift, half2v d2, half2v b2, DqTmp& tmp, U4& out) {
     if constexpr (FMT == 0) dq_op_q4(op, blk.q[j], d2, b2, tmp, out);
-    else if constexpr (FMT == 1) dq_op_q8(op, blk, j, d2, tmp, out);
+    else if constexpr (FMT == 1) dq_op_q8(op, blk, j, shift, d2, tmp, out);
     else dq_op_q3(op, blk, j, d2, b2, tmp, out);
 }
 
@@ -221,13 +231,36 @@ struct WregPlan {
     float* partial;        // [tail tile][slice][TM * TN] when tail_slices > 1
 };
 
+// Workgroup -> item of its range.  Workgroups that land on one XCD (blockIdx % 8) take a contiguous run of items, and
+// items that need the same weights at the same time, the token tiles of one weight tile and K slice, are next to each
+// other: each XCD's L2 then streams an eighth of W instead of all of it.
+__device__ __forceinline__ void place_workgroup(const WregPlan& plan, uint32_t tiles_m, bool& in_tail, uint32_t& tile, uint32_t& slice) {
+    const uint32_t n_tail = gridDim.x - plan.full;
+    in_tail = blockIdx.x >= plan.full;
+    const uint32_t pos = in_tail ? blockIdx.x - plan.full : blockIdx.x, count = in_tail ? n_tail : plan.full;
+    const uint32_t xcd = pos & 7u, per = count >> 3, rem = count & 7u;
+    const uint32_t item = xcd * per + (xcd < rem ? xcd : rem) + (pos >> 3);
+    tile = item;
+    slice = 0;
+    if (in_tail) {
+        const uint32_t rest = n_tail / plan.tail_slices;  // tiles
+        const uint32_t run = tiles_m < kGroupM ? tiles_m : kGroupM;
+        const uint32_t first = item / (run * plan.tail_slices) * run;
+        const uint32_t here = rest - first < run ? rest - first : run;
+        const uint32_t in = item - first * plan.tail_slices;
+        slice = in / here;
+        tile = plan.full + first + (in - slice * here);
+    }
+}
+
 // FMT: 0 = Q4 blocks, 1 = Q8_0, 2 = Q3 (the siblings have no LoRA step; Q8_0 keeps its activations in
 // memory order, the other two in the x0 x4 x1 x5 .. order of their decoders).
-template <bool X_F16, bool LORA, int FMT = 0>
+template <bool X_F16, bool LORA, int FMT, int NT, int NU>
 __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict__ w, uint32_t n, uint32_t k,
                                                        const void* __restrict__ xv, uint32_t m,
                                                        float* __restrict__ y, LoraEpilogue lora, WregPlan plan) {
     extern __shared__ uint4 lds16[];  // two activation buffers of kBuf16 units
+    constexpr int TM = 16 * NT, TN = 64 * NU, kBuf16 = TM * kPitch16;
     constexpr int XU = TM * (TK / 8) / 256;  // 8-activation units staged per thread per step
     constexpr int XL = X_F16 ? 1 : 2;        // 16-byte global loads per unit
     typedef typename WBlockOf<FMT>::type WBlock;
@@ -240,15 +273,14 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
     const int lr = lane & 15;  // row inside a 16-row tile
     const int g = lane >> 4;   // K group: block g of the step
 
-    // ---- tile id -> (token tile, weight tile), grouped so co-resident tiles share activations
-    // workgroup -> (tile, K slice): whole tiles first, then the slices of the tail tiles
-    const bool in_tail = blockIdx.x >= plan.full;
-    const uint32_t tail_idx = in_tail ? blockIdx.x - plan.full : 0;
-    const uint32_t tile = in_tail ? plan.full + tail_idx / plan.tail_slices : blockIdx.x;
-    const uint32_t nslices = in_tail ? plan.tail_slices : 1;
-    const uint32_t slice = in_tail ? tail_idx % plan.tail_slices : 0;
-
     const uint32_t tiles_m = (m + TM - 1) / TM, tiles_n = (n + TN - 1) / TN;
+    // ---- workgroup -> (tile, K slice): whole tiles first, then the slices of the tail tiles
+    bool in_tail;
+    uint32_t tile, slice;
+    place_workgroup(plan, tiles_m, in_tail, tile, slice);
+    const uint32_t nslices = in_tail ? plan.tail_slices : 1;
+
+    // tile id -> (token tile, weight tile), token tiles fastest
     const uint32_t per_group = kGroupM * tiles_n;
     const uint32_t group = tile / per_group;
     const uint32_t first_m = group * kGroupM;
@@ -284,10 +316,14 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
     const WUnit* w_row[NU];
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-        uint32_t row = n0 + wave * 64 + u * 16 + lr;
+        uint32_t row = n0 + wave * (16 * NU) + u * 16 + lr;
         row = row < n ? row : n - 1;
         w_row[u] = reinterpret_cast<const WUnit*>(w) + static_cast<size_t>(row) * (nb_total * kUnits) + s_begin * (4 * kUnits);
     }
+    // Q8_0: how the lane's blocks of tile u lie (four blocks from step to step: every step alike)
+    uint32_t w_shift[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) w_shift[u] = FMT == 1 && (reinterpret_cast<uintptr_t>(w_row[u] + g * kUnits) & 2) == 0 ? 2 : 0;
     // activation unit i of this thread: token row tid/16 + 16 i, K offset 8 * (tid % 16) of the step
     const int x_part = tid & 15;
     const uint8_t* x_row[XU];
@@ -333,16 +369,25 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
     auto load_w_one = [&](WBlock (&wr)[NU], uint32_t s, int u) {
         uint32_t blk = s * 4 + g;
         blk = blk < nb ? blk : nb - 1;
-        wr[u] = *reinterpret_cast<const WBlock*>(w_row[u] + blk * kUnits);
+        if constexpr (FMT == 1) {
+            const WUnit* at = w_row[u] + blk * kUnits;
+            const bool even = (reinterpret_cast<uintptr_t>(at) & 2) == 0;
+            const Dwords8 d = *reinterpret_cast<const Dwords8*>(at + (even ? 0 : 1));
+#pragma unroll
+            for (int i = 0; i < 8; ++i) wr[u].q[i] = d.v[i];
+            wr[u].h = at[even ? 16 : 0];
+        } else {
+            wr[u] = *reinterpret_cast<const WBlock*>(w_row[u] + blk * kUnits);
+        }
     };
     auto load_w = [&](WBlock (&wr)[NU], uint32_t s) {
 #pragma unroll
         for (int u = 0; u < NU; ++u) load_w_one(wr, s, u);
     };
 
-    auto scale_pair = [&](const WBlock& blk, bool live, half2v& d2, half2v& b2) {
+    auto scale_pair = [&](const WBlock& blk, int u, bool live, half2v& d2, half2v& b2) {
         uint32_t sb;
-        if constexpr (FMT == 1) sb = live ? static_cast<uint32_t>(blk.d) : 0u;  // scale only
+        if constexpr (FMT == 1) sb = live ? (w_shift[u] ? blk.q[0] : blk.h) : 0u;  // scale only (the low half)
         else sb = live ? blk.sb : 0u;
         d2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x01000100u));  // (d, d)
         b2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x03020302u));  // (b, b)
@@ -354,7 +399,7 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
     half2v d2[NU], b2[NU];
     XRegs xr;
 
-    // One K step = 4 quarters x 8 token tiles x 4 weight tiles = 128 matrix-core instructions,
+    // One K step = 4 quarters x NT token tiles x NU weight tiles of matrix-core instructions,
     // issued in a fixed order.  In the shadow of each instruction go one or two steps of the
     // dequantisation of the NEXT quarter (for the last quarter: the first quarter of step s+1,
     // from `wnext`), and every fourth token tile one activation unit of step s+1 is written to the
@@ -379,24 +424,27 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
                 const int p = j * NT + t;  // slot: (quarter, token tile)
                 // one weight tile's loads every other token tile rather than all eight at the step's
                 // start: a burst from every wave right after the barrier fills the address unit's queue
-                if (j == 0 && (t & 1) == 0) load_w_one(wfree, s + 2, t / 2);
+                if (j == 0) {
+#pragma unroll
+                    for (int u = t * NU / NT; u < (t + 1) * NU / NT; ++u) load_w_one(wfree, s + 2, u);
+                }
                 if (p + 2 < 4 * NT) {
                     const int pj = (p + 2) / NT, pt = (p + 2) % NT;
                     bx[(p + 2) % 3] = xbuf[pt * 16 * kPitch16 + pj];
                 }
 #pragma unroll
                 for (int u = 0; u < NU; ++u) {
-                    const int c = t * NU + u;  // instruction index inside the quarter, 0..31
+                    const int c = t * NU + u;  // instruction index inside the quarter
                     acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                         __builtin_bit_cast(half8, a_cur[u]), __builtin_bit_cast(half8, bx[p % 3]), acc[u][t], 0, 0,
                         0);
 #pragma unroll
-                    for (int e = c * (NU * kDqOps) / 32; e < (c + 1) * (NU * kDqOps) / 32; ++e) {
+                    for (int e = c * kDqOps / NT; e < (c + 1) * kDqOps / NT; ++e) {
                         const int uu = e / kDqOps, op = e % kDqOps;
-                        if (j < 3) dq_op<FMT>(op, wr[uu], j + 1, d2[uu], b2[uu], tmp, a_nxt[uu]);
-                        else dq_op<FMT>(op, wnext[uu], 0, d2n[uu], b2n[uu], tmp, a_nxt[uu]);
+                        if (j < 3) dq_op<FMT>(op, wr[uu], j + 1, w_shift[uu], d2[uu], b2[uu], tmp, a_nxt[uu]);
+                        else dq_op<FMT>(op, wnext[uu], 0, w_shift[uu], d2n[uu], b2n[uu], tmp, a_nxt[uu]);
                     }
-                    if (j == 2 && t == NT - 1) scale_pair(wnext[u], live_next, d2n[u], b2n[u]);
+                    if (j == 2 && t == NT - 1) scale_pair(wnext[u], u, live_next, d2n[u], b2n[u]);
                     if (u == NU - 1 && (p & 3) == 1) {
                         store_x_unit(xr, p >> 2, xnext);
                         load_x_unit(xr, p >> 2, s + 2);
@@ -429,9 +477,9 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
         DqTmp tmp;
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            scale_pair(wa[u], g < nb, d2[u], b2[u]);
+            scale_pair(wa[u], u, g < nb, d2[u], b2[u]);
 #pragma unroll
-            for (int op = 0; op < kDqOps; ++op) dq_op<FMT>(op, wa[u], 0, d2[u], b2[u], tmp, a_cur[u]);
+            for (int op = 0; op < kDqOps; ++op) dq_op<FMT>(op, wa[u], 0, w_shift[u], d2[u], b2[u], tmp, a_cur[u]);
         }
     }
     __syncthreads();
@@ -455,7 +503,7 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
             half8 b_hi[NU], b_his[NU], b_lo[NU];
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
-                uint32_t row = n0 + wave * 64 + u * 16 + lr;
+                uint32_t row = n0 + wave * (16 * NU) + u * 16 + lr;
                 row = row < n ? row : n - 1;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
@@ -497,7 +545,7 @@ __global__ __launch_bounds__(256, 1) void gemm_q4_wreg(const uint8_t* __restrict
     const bool vec_ok = (n & 3u) == 0;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-        const uint32_t gn = n0 + wave * 64 + u * 16 + 4 * g;
+        const uint32_t gn = n0 + wave * (16 * NU) + u * 16 + 4 * g;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const uint32_t gm = m0 + t * 16 + lr;
@@ -621,19 +669,12 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_w2(const uint8_t* __restrict__
     const int lr = lane & 15;  // row inside a 16-row tile
     const int g = lane >> 4;   // K group: block g of the step
 
-    // ---- workgroup -> (tile, K slice).  Whole tiles first, then the slices of the tail tiles; inside
-    // either range, workgroups that land on one XCD (blockIdx % 8) take a contiguous run of tile ids,
-    // i.e. neighbouring weight tiles: each XCD's L2 then streams an eighth of W instead of all of it.
-    const uint32_t n_whole = plan.full, n_tail = gridDim.x - plan.full;
-    const bool in_tail = blockIdx.x >= n_whole;
-    const uint32_t pos = in_tail ? blockIdx.x - n_whole : blockIdx.x, count = in_tail ? n_tail : n_whole;
-    const uint32_t xcd = pos & 7u, per = count >> 3, rem = count & 7u;
-    const uint32_t item = xcd * per + (xcd < rem ? xcd : rem) + (pos >> 3);
-    const uint32_t tile = in_tail ? plan.full + item / plan.tail_slices : item;
-    const uint32_t nslices = in_tail ? plan.tail_slices : 1;
-    const uint32_t slice = in_tail ? item % plan.tail_slices : 0;
-
     const uint32_t tiles_m = (m + TM - 1) / TM, tiles_n = (n + TN - 1) / TN;
+    bool in_tail;
+    uint32_t tile, slice;
+    place_workgroup(plan, tiles_m, in_tail, tile, slice);
+    const uint32_t nslices = in_tail ? plan.tail_slices : 1;
+
     const uint32_t per_group = kGroupM * tiles_n;
     const uint32_t group = tile / per_group;
     const uint32_t first_m = group * kGroupM;
@@ -808,7 +849,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_w2(const uint8_t* __restrict__
 // consecutive weight rows of one token.
 __global__ __launch_bounds__(256) void gemm_reduce_tail(const float* __restrict__ partial, uint32_t first_tile,
                                                         uint32_t slices, uint32_t m, uint32_t n,
-                                                        float* __restrict__ y, LoraEpilogue lora) {
+                                                        float* __restrict__ y, LoraEpilogue lora, uint32_t TM, uint32_t TN) {
     const uint32_t tile = first_tile + blockIdx.x;
     const uint32_t tiles_m = (m + TM - 1) / TM, tiles_n = (n + TN - 1) / TN;
     const uint32_t per_group = kGroupM * tiles_n;
@@ -870,40 +911,70 @@ __global__ __launch_bounds__(256) void gemm_reduce_tail(const float* __restrict_
 
 constexpr uint32_t kCus = 256;
 constexpr uint32_t kMaxTailSlices = 16;
-// Cost of one K slice of one tail tile, in K steps of a tile: its 128 KB partial tile is written and
-// read back once (~0.06 us of memory time against ~2.4 us per step).
-#ifndef LQ4_SLICE_CHARGE
-#define LQ4_SLICE_CHARGE 0.027
-#endif
 
 // How the tiles of a shape are scheduled: `full` whole tiles, the rest in `slices` K slices each.
 struct HostPlan {
     uint32_t tiles, full, slices;
+    uint32_t nt, nu;  // 16-token tiles of a workgroup, 16-row tiles of a wave
+    double us;        // what the model below makes of it
 };
 
-HostPlan plan_tiles(uint32_t n, uint32_t k, uint32_t m, uint32_t slots = kCus) {
-    const uint32_t tiles = ((n + TN - 1) / TN) * ((m + TM - 1) / TM);
+// A tile of 16 nt tokens x 64 nu rows takes `step_us` per K step and about 5 us besides; a K slice writes its partial
+// tile and reads it back (at about 8 TB/s, mostly beside other slices' arithmetic), and a reduction launch follows.
+constexpr double kTileUs = 5.0, kReduceUs = 3.0, kPartialBytesPerUs = 8e6;
+
+HostPlan plan_tiles(uint32_t n, uint32_t k, uint32_t m, uint32_t slots, uint32_t nt, uint32_t nu, double step_us,
+                    double partial_rate = kPartialBytesPerUs) {
+    const uint32_t tiles = ((n + 64 * nu - 1) / (64 * nu)) * ((m + 16 * nt - 1) / (16 * nt));
     const uint32_t steps = (k / kBlockWeights + 3) / 4;
     const uint32_t rest = tiles % slots;
-    HostPlan p{tiles, tiles - rest, 1};
-    if (rest == 0 || steps < 4) return HostPlan{tiles, tiles, 1};
-    // pick the slice count that minimises the time of the last round in K steps,
-    // ceil(rest * s / CUs) * steps-per-slice plus the traffic of the partial tiles,
-    // with at least two steps per slice and no empty slice
-    double best = steps;  // s = 1: one round of whole tiles
+    const double whole = steps * step_us + kTileUs;
+    const double rounds_whole = tiles / slots * whole;
+    HostPlan p{tiles, tiles, 1, nt, nu, rounds_whole + (rest ? whole : 0.0)};
+    if (rest == 0 || steps < 4) return p;
+    // the slice count with the shortest last round, with at least two steps per slice and no empty slice
     for (uint32_t s = 2; s <= kMaxTailSlices && s * 2 <= steps; ++s) {
         const uint32_t per = (steps + s - 1) / s;
         if ((s - 1) * per >= steps) continue;  // would leave the last slice empty
-        const double rounds = static_cast<double>((rest * s + slots - 1) / slots);
-        const double t = rounds * per + LQ4_SLICE_CHARGE * rest * s;
-        if (t < best - 1e-9) {
-            best = t;
+        const double us = rounds_whole + (rest * s + slots - 1) / slots * (per * step_us + kTileUs) + kReduceUs +
+                          2.0 * rest * s * (nt * nu * 4096.0) / partial_rate;
+        if (us < p.us) {
+            p.us = us;
             p.slices = s;
+            p.full = tiles - rest;
         }
     }
-    if (p.slices == 1) p.full = tiles;
     return p;
 }
+
+// Tiles of gemm_q4_wreg and what a K step of one takes with a tile on every CU (us; K 4096, one round of 256 tiles).
+// Smaller tiles do less per step's worth of waiting (one wave per SIMD: a step is bound by the address unit, the LDS
+// reads and the gaps between them rather than by its matrix instructions), so the large tile is taken where its last
+// round is full: 2048 x 4096 tokens x rows 72 us against 79 with the next best, but 777 x 5120 x 5120 93 -> 57 us and 333 x
+// 12288 x 2048 39 -> 29 us with 96 x 192, both one round of 243..256 tiles instead of slices of 140 or a half-empty round.
+struct WregTile {
+    uint32_t nt, nu;
+    double step_us[3][2];  // by format (Q4, Q8_0, Q3) and type of X (f16, f32)
+};
+constexpr WregTile kWregTiles[] = {
+    {8, 4, {{2.10, 2.30}, {2.40, 2.65}, {2.35, 2.45}}}, {8, 3, {{1.65, 1.80}, {1.82, 2.15}, {1.82, 1.90}}},
+    {8, 2, {{1.23, 1.42}, {1.32, 1.65}, {1.35, 1.53}}}, {6, 4, {{1.72, 1.88}, {2.03, 2.20}, {1.80, 2.00}}},
+    {6, 3, {{1.33, 1.52}, {1.56, 1.75}, {1.52, 1.63}}}, {7, 3, {{1.44, 1.60}, {1.66, 1.95}, {1.62, 1.74}}}};
+
+// `large_only`: the launch needs the LoRA step, which only the large tile has.
+HostPlan plan_wreg(uint32_t n, uint32_t k, uint32_t m, int fmt, bool x_is_f16, bool large_only) {
+    HostPlan best{};
+    for (const WregTile& t : kWregTiles) {
+        const HostPlan p = plan_tiles(n, k, m, kCus, t.nt, t.nu, t.step_us[fmt][x_is_f16 ? 0 : 1]);
+        // (the large tile comes first; another one has to promise more than the model's error)
+        if (best.tiles == 0 || p.us < best.us * (best.nu == NU && best.nt == NT ? 0.96 : 1.0)) best = p;
+        if (large_only) break;
+    }
+    return best;
+}
+
+// (two tiles a CU: twice as many slices in flight, whose partial tiles are hidden behind less)
+HostPlan plan_w2(uint32_t n, uint32_t k, uint32_t m) { return plan_tiles(n, k, m, 2 * kCus, NT, NU, 3.1, kPartialBytesPerUs / 2); }
 
 }  // namespace
 
@@ -917,31 +988,50 @@ bool gemm_w2_wants(uint32_t n, uint32_t k, uint32_t m) {
     return k >= kBlockWeights && gemm_wreg_tiles(n, m) >= 2 * kCus;
 }
 
-size_t gemm_wreg_scratch_floats(uint32_t n, uint32_t k, uint32_t m) {
-    const HostPlan p = plan_tiles(n, k, m);
-    return p.slices > 1 ? static_cast<size_t>(p.tiles - p.full) * p.slices * (TM * TN) : 0;
+size_t gemm_wreg_scratch_floats(uint32_t n, uint32_t k, uint32_t m, int fmt, bool x_is_f16, bool with_lora) {
+    const HostPlan p = plan_wreg(n, k, m, fmt, x_is_f16, with_lora);
+    return p.slices > 1 ? static_cast<size_t>(p.tiles - p.full) * p.slices * (p.nt * p.nu * 1024) : 0;
 }
 
 namespace {
 
+template <bool X_F16, bool LORA, int FMT, int NT, int NU>
+void launch_wreg_tile(const uint8_t* w, uint32_t n, uint32_t k, const void* x, uint32_t m, float* y,
+                      const LoraEpilogue& lora, const HostPlan& hp, float* partial, hipStream_t stream) {
+    static LdsCapOnce lds_cap;
+    lds_cap.raise(reinterpret_cast<const void*>(gemm_q4_wreg<X_F16, LORA, FMT, NT, NU>), 160 * 1024);
+    const size_t lds = 2 * 16 * NT * kPitch16 * sizeof(uint4);
+    const WregPlan plan{hp.full, hp.slices, partial};
+    const uint32_t wgs = hp.full + (hp.tiles - hp.full) * hp.slices;
+    hipLaunchKernelGGL((gemm_q4_wreg<X_F16, LORA, FMT, NT, NU>), dim3(wgs), dim3(256), lds, stream, w, n, k, x, m, y, lora,
+                       plan);
+}
+
 template <bool X_F16, bool LORA, int FMT>
 void launch_wreg_t(const uint8_t* w, uint32_t n, uint32_t k, const void* x, uint32_t m, float* y,
                    const LoraEpilogue& lora, const HostPlan& hp, float* partial, hipStream_t stream) {
-    static LdsCapOnce lds_cap;
-    lds_cap.raise(reinterpret_cast<const void*>(gemm_q4_wreg<X_F16, LORA, FMT>), 160 * 1024);
-    const size_t lds = 2 * kBuf16 * sizeof(uint4);
-    const WregPlan plan{hp.full, hp.slices, partial};
-    const uint32_t wgs = hp.full + (hp.tiles - hp.full) * hp.slices;
-    hipLaunchKernelGGL((gemm_q4_wreg<X_F16, LORA, FMT>), dim3(wgs), dim3(256), lds, stream, w, n, k, x, m, y, lora,
-                       plan);
+    if constexpr (!LORA) {
+#define LQ4_TILE(NT_, NU_) \
+    if (hp.nt == NT_ && hp.nu == NU_) return launch_wreg_tile<X_F16, LORA, FMT, NT_, NU_>(w, n, k, x, m, y, lora, hp, partial, stream)
+        LQ4_TILE(8, 3);
+        LQ4_TILE(8, 2);
+        LQ4_TILE(6, 4);
+        LQ4_TILE(6, 3);
+        LQ4_TILE(7, 3);
+#undef LQ4_TILE
+    }
+    launch_wreg_tile<X_F16, LORA, FMT, 8, 4>(w, n, k, x, m, y, lora, hp, partial, stream);
 }
 
 }  // namespace
 
 void launch_gemm_wreg(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m,
                       float* y, const LoraEpilogue& lora, float* partial, hipStream_t stream, int fmt) {
-    HostPlan hp = plan_tiles(n, k, m);
-    if (!partial) hp = HostPlan{hp.tiles, hp.tiles, 1};
+    HostPlan hp = plan_wreg(n, k, m, fmt, x_is_f16 != 0, lora.rank != 0);
+    if (!partial) {
+        hp.full = hp.tiles;
+        hp.slices = 1;
+    }
     if (fmt == 1) {
         if (x_is_f16) launch_wreg_t<true, false, 1>(w, n, k, x, m, y, lora, hp, partial, stream);
         else launch_wreg_t<false, false, 1>(w, n, k, x, m, y, lora, hp, partial, stream);
@@ -960,13 +1050,12 @@ void launch_gemm_wreg(const uint8_t* w, uint32_t n, uint32_t k, const void* x, i
         }
     }
     if (hp.slices > 1)
-        hipLaunchKernelGGL(gemm_reduce_tail, dim3(hp.tiles - hp.full, TM * TN / 1024), dim3(256), 0, stream, partial,
-                           hp.full, hp.slices, m, n, y, lora);
+        hipLaunchKernelGGL(gemm_reduce_tail, dim3(hp.tiles - hp.full, hp.nt * hp.nu), dim3(256), 0, stream, partial,
+                           hp.full, hp.slices, m, n, y, lora, 16 * hp.nt, 64 * hp.nu);
 }
 
 // ---- gemm_q4_w2: scratch = [packed X | partial tiles of the sliced tail] ----------------------------
 namespace {
-constexpr uint32_t kW2Slots = 2 * kCus;  // two workgroups per CU
 inline uint32_t w2_kc_pad(uint32_t k) { return (k / 8 + 15) / 16 * 16; }
 inline size_t w2_packed_bytes(uint32_t k, uint32_t m) {
     return static_cast<size_t>((m + TM - 1) / TM) * TM * w2_kc_pad(k) * 16;
@@ -974,7 +1063,7 @@ inline size_t w2_packed_bytes(uint32_t k, uint32_t m) {
 }  // namespace
 
 size_t gemm_w2_scratch_bytes(uint32_t n, uint32_t k, uint32_t m) {
-    const HostPlan p = plan_tiles(n, k, m, kW2Slots);
+    const HostPlan p = plan_w2(n, k, m);
     const size_t partial = p.slices > 1 ? static_cast<size_t>(p.tiles - p.full) * p.slices * (TM * TN) * sizeof(float) : 0;
     return w2_packed_bytes(k, m) + partial;
 }
@@ -982,7 +1071,7 @@ size_t gemm_w2_scratch_bytes(uint32_t n, uint32_t k, uint32_t m) {
 void launch_gemm_w2(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m, float* y,
                     uint8_t* scratch, hipStream_t stream) {
     const LoraEpilogue lora{nullptr, nullptr, 0, 0, 0.0f};  // no LoRA step in this kernel
-    const HostPlan hp = plan_tiles(n, k, m, kW2Slots);
+    const HostPlan hp = plan_w2(n, k, m);
     const uint32_t kc_pad = w2_kc_pad(k);
     uint4* packed = reinterpret_cast<uint4*>(scratch);
     float* partial = reinterpret_cast<float*>(scratch + w2_packed_bytes(k, m));
@@ -997,7 +1086,7 @@ void launch_gemm_w2(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int
     hipLaunchKernelGGL(gemm_q4_w2, dim3(wgs), dim3(256), lds, stream, w, n, k, packed, kc_pad, m, y, plan);
     if (hp.slices > 1)
         hipLaunchKernelGGL(gemm_reduce_tail, dim3(hp.tiles - hp.full, TM * TN / 1024), dim3(256), 0, stream, partial,
-                           hp.full, hp.slices, m, n, y, lora);
+                           hp.full, hp.slices, m, n, y, lora, static_cast<uint32_t>(TM), static_cast<uint32_t>(TN));
 }
 
 }  // namespace lq4

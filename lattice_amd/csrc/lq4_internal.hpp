@@ -211,13 +211,13 @@ void launch_gemm(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_
 int gemm_kernel_choice_default();  // from the environment variable LQ4_GEMM_KERNEL
 
 // Large-shape variant: weights dequantised in registers, only activations staged in LDS.
-// Tile 128 tokens x 256 weight rows; gemm_wreg_tiles = workgroups it would launch;
+// gemm_wreg_tiles = tiles of 128 tokens x 256 weight rows (its largest);
 // gemm_wreg_supports = the kernel can run the shape at all.
 uint32_t gemm_wreg_tiles(uint32_t n, uint32_t m);
 bool gemm_wreg_supports(uint32_t n, uint32_t k, uint32_t m, int x_is_f16);
 // A last, partly filled round of tiles is cut into K slices that meet in `partial`
 // (gemm_wreg_scratch_floats floats; null = no slicing) and are summed by a second kernel.
-size_t gemm_wreg_scratch_floats(uint32_t n, uint32_t k, uint32_t m);
+size_t gemm_wreg_scratch_floats(uint32_t n, uint32_t k, uint32_t m, int fmt, bool x_is_f16, bool with_lora);
 // The same tile at two workgroups per CU, Q4 only: activations packed into scratch first (f16, tile order),
 // then the tail's partial tiles behind them; gemm_w2_scratch_bytes covers both.
 size_t gemm_w2_scratch_bytes(uint32_t n, uint32_t k, uint32_t m);
@@ -235,7 +235,7 @@ void launch_gemm_q8(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int
                     float* scratch, int forced, hipStream_t stream);
 // Floats of scratch the sibling tile GEMMs use to cut K on shapes with few tiles (0 = none; a null
 // scratch pointer keeps K whole).
-size_t gemm_sibling_scratch_floats(int fmt, uint32_t n, uint32_t k, uint32_t m, int forced);  // fmt: 1 = Q8_0, 2 = Q3
+size_t gemm_sibling_scratch_floats(int fmt, uint32_t n, uint32_t k, uint32_t m, int x_is_f16, int forced);  // fmt: 1 = Q8_0, 2 = Q3
 
 // Q3 sibling format (16-byte blocks: f16 scale, f16 bias, 2-bit and 1-bit planes): same pair of paths.
 size_t gemv_q3_lds_bytes(uint32_t k);
@@ -245,7 +245,7 @@ void launch_gemm_q3(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int
 
 // Few-token variant (up to 128 tokens): activations packed once into matrix-core operand order
 // (gemm_skinny_scratch_bytes bytes at `packed_x`), then a kernel without LDS staging.
-bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m);
+bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt = 0);
 size_t gemm_skinny_scratch_bytes(uint32_t k, uint32_t m);
 // For Q4 and a LoRA rank this accepts the packing launch computes t = A . X when LoraEpilogue::a points to A as packed
 // (on the host, once) by gemm_skinny_pack_lora_a; t is then not read and no launch for it has to precede.
