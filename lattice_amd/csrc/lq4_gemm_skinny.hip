@@ -81,9 +81,15 @@ __device__ __forceinline__ U4 dequant8(uint32_t q, half2v d2, half2v b2) {
 
 // Sibling formats (FMT 1 = Q8_0, 2 = Q3): their decoders emit the eight weights of an instruction
 // in memory order, so their activations are packed without the interleave.
-struct __attribute__((packed, aligned(2))) Q8BlockRaw {
-    uint16_t d;
-    uint32_t q[8];  // weight i in byte i
+// A Q8_0 block as loaded: eight whole dwords and the odd half beside them (a load that starts inside a dword costs the
+// address unit twice as much).  On a dword boundary: scale and weights 0, 1 in q[0], weights 30, 31 in h, and q[i + 1] : q[i]
+// shifted by two bytes are weights 4 i ..; two bytes past one: the scale in h, the weights in q.
+struct Q8BlockRaw {
+    uint32_t q[8];
+    uint32_t h;
+};
+struct __attribute__((packed, aligned(4))) Dwords8 {
+    uint32_t v[8];
 };
 struct __attribute__((packed, aligned(4))) Q3BlockRaw {
     uint32_t sb;
@@ -321,6 +327,9 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
                 }
         }
     }
+    uint32_t w_shift[RT];  // Q8_0: how the lane's blocks lie (every step alike)
+#pragma unroll
+    for (int r = 0; r < RT; ++r) w_shift[r] = FMT == 1 && (reinterpret_cast<uintptr_t>(w_row[r] + g * kBytes) & 2) == 0 ? 2 : 0;
     struct Unit {
         WBlock wb[RT];
         uint4 x[NTG][4];  // [token group][instruction]
@@ -334,7 +343,18 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         uint32_t blk = s * 4 + g;
         blk = blk < nb ? blk : nb - 1;
 #pragma unroll
-        for (int r = 0; r < RT; ++r) u.wb[r] = *reinterpret_cast<const WBlock*>(w_row[r] + blk * kBytes);
+        for (int r = 0; r < RT; ++r) {
+            const uint8_t* at = w_row[r] + blk * kBytes;
+            if constexpr (FMT == 1) {
+                const bool whole = (reinterpret_cast<uintptr_t>(at) & 2) == 0;
+                const Dwords8 d = *reinterpret_cast<const Dwords8*>(at + (whole ? 0 : 2));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) u.wb[r].q[i] = d.v[i];
+                u.wb[r].h = *reinterpret_cast<const uint16_t*>(at + (whole ? 32 : 0));
+            } else {
+                u.wb[r] = *reinterpret_cast<const WBlock*>(at);
+            }
+        }
         const uint4* xs = xp + static_cast<size_t>(s) * groups * 256 + lane;
 #pragma unroll
         for (int t = 0; t < NTG; ++t)
@@ -353,7 +373,7 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             uint32_t sb;
-            if constexpr (FMT == 1) sb = live ? static_cast<uint32_t>(u.wb[r].d) : 0u;  // scale only
+            if constexpr (FMT == 1) sb = live ? (w_shift[r] ? u.wb[r].q[0] : u.wb[r].h) : 0u;  // scale only (the low half)
             else sb = live ? u.wb[r].sb : 0u;
             const half2v d2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x01000100u));
             const half2v b2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x03020302u));
@@ -361,7 +381,9 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
             for (int j = 0; j < 4; ++j) {
                 U4 a;
                 if constexpr (FMT == 0) a = dequant8(live ? u.wb[r].q[j] : 0u, d2, b2);
-                else if constexpr (FMT == 1) a = dequant8_q8(u.wb[r].q[2 * j], u.wb[r].q[2 * j + 1], d2);
+                else if constexpr (FMT == 1)
+                    a = dequant8_q8(__builtin_amdgcn_alignbyte(u.wb[r].q[2 * j + 1], u.wb[r].q[2 * j], w_shift[r]),
+                                    __builtin_amdgcn_alignbyte(j < 3 ? u.wb[r].q[(2 * j + 2) & 7] : u.wb[r].h, u.wb[r].q[2 * j + 1], w_shift[r]), d2);
                 else a = dequant8_q3(u.wb[r], j, d2, b2);
 #pragma unroll
                 for (int t = 0; t < NTG; ++t)

@@ -4,8 +4,11 @@
 // then times f32(d), all f32).
 //
 // Same work layout as the Q4 kernel: lane l owns block 64 s + l of every row its wave
-// processes, so a wave reads 2176 contiguous bytes per row and slab (blocks are only 2-byte
-// aligned; the vector memory path takes unaligned 16-byte loads).
+// processes, so a wave reads 2176 contiguous bytes per row and slab.  A block is 34 bytes, so every other one starts in
+// the middle of a dword, where a vector load costs the address unit two clocks a lane instead of one: a lane loads the
+// eight whole dwords of its block and the odd half beside them, and brings the weights into place with byte aligns
+// (26.7 MB, 12288 x 2048: 8.0 -> 6.9 us, 3.9 TB/s; non-temporal loads, which the Q4 kernel has, 8.7: two
+// lanes' pieces share a cache line here).
 // Arithmetic: the weight bytes are never converted.  The 32 activations of a block are staged once per
 // workgroup as 23-bit fixed point, t = rint(x * 2^22 / S) with S the power of two above the block's largest
 // magnitude (the accuracy of an f32 at that magnitude, the range of f32), cut into three signed bytes
@@ -28,10 +31,13 @@ constexpr int kXPitch = 36;  // dwords of LDS per block of x: byte plane p of we
 constexpr int kPlanes = 3;
 constexpr int kQ8BlockBytes = 34;
 
-struct __attribute__((packed, aligned(2))) Q8BlockRaw {
-    uint16_t d;     // f16 scale
-    uint32_t q[8];  // 32 x i8, weight i in byte i
+// The block [u16 scale][32 x i8] as loaded.  On a dword boundary: scale and weights 0, 1 in q[0], weights 30, 31 in h
+// (shift 2 brings q[i + 1] : q[i] to weights 4 i ..); two bytes past one: the scale in h, the weights in q (shift 0).
+struct Q8BlockRaw {
+    uint32_t q[8];
+    uint32_t h, shift;
 };
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ float dpp_add(float v) {
@@ -51,8 +57,11 @@ __device__ __forceinline__ float wave_total(float v) {
 }
 
 // sum_i q_i * t_i over one block, t the block's fixed-point activations
-__device__ __forceinline__ float block_dot(const uint32_t (&q)[8], const uint32_t (&xn)[8 * kPlanes]) {
+__device__ __forceinline__ float block_dot(const Q8BlockRaw& b, const uint32_t (&xn)[8 * kPlanes]) {
     int32_t part[kPlanes] = {0, 0, 0};
+    uint32_t q[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) q[w] = __builtin_amdgcn_alignbyte(w < 7 ? b.q[w + 1] : b.h, b.q[w], b.shift);
 #pragma unroll
     for (int w = 0; w < 8; ++w)
 #pragma unroll
@@ -87,7 +96,14 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_q8_b1(const uint8_t* __restr
         for (int j = 0; j < RW; ++j) {
             uint32_t row = (chunk * RW + j) * n_waves + wid;
             if (row >= n) row = n - 1;
-            buf[j] = *reinterpret_cast<const Q8BlockRaw*>(w + row * row_bytes + blk * static_cast<uint32_t>(kQ8BlockBytes));
+            const uint8_t* at = w + row * row_bytes + blk * static_cast<uint32_t>(kQ8BlockBytes);
+            const bool whole = (reinterpret_cast<uintptr_t>(at) & 2) == 0;
+            const u32x4u* qp = reinterpret_cast<const u32x4u*>(at + (whole ? 0 : 2));
+            const u32x4u lo = qp[0], hi = qp[1];
+            buf[j].q[0] = lo.x; buf[j].q[1] = lo.y; buf[j].q[2] = lo.z; buf[j].q[3] = lo.w;
+            buf[j].q[4] = hi.x; buf[j].q[5] = hi.y; buf[j].q[6] = hi.z; buf[j].q[7] = hi.w;
+            buf[j].h = *reinterpret_cast<const uint16_t*>(at + (whole ? 32 : 0));
+            buf[j].shift = whole ? 2u : 0u;
         }
     };
 
@@ -189,8 +205,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_q8_b1(const uint8_t* __restr
         const float scale_x = __builtin_bit_cast(float, xs[blk * kXPitch + 33]);
 #pragma unroll
         for (int j = 0; j < RW; ++j) {
-            const float p = block_dot(cur[j].q, xn);
-            const float d = live ? f16_bits_to_f32(cur[j].d) : 0.0f;
+            const float p = block_dot(cur[j], xn);
+            const float d = live ? f16_bits_to_f32((cur[j].shift ? cur[j].q[0] : cur[j].h) & 0xffffu) : 0.0f;
             acc[j] = fmaf(d * p, scale_x, acc[j]);
         }
         if (slab + 1 == slabs) {  // chunk complete
