@@ -432,6 +432,11 @@ static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t b
            gemv_i8_serves(n, k, batch, ctx->cu_count);
 }
 
+// Few, long rows: K slices on the 4x4x4 matrix-core kernel (no LoRA step there).
+static bool gemv_takes_slices(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch, bool with_lora, bool fused) {
+    return !with_lora && gemv_mfma_sliced_wants(n, k, batch, fused);
+}
+
 // Above four activation rows the few-token matrix-core kernel (operands packed once, eight K
 // slices per workgroup) overtakes the 4x4x4 GEMV kernel: always from nine rows; from five for
 // mid-sized matrices only (measured: behind for 512 x 2048, where its two launches dominate,
@@ -450,7 +455,12 @@ static bool gemv_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k
 static int gemv_dispatch(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, uint32_t k, const float* x_dev, uint32_t batch,
                          float* y_dev, const LoraEpilogue& ep, hipStream_t s) {
     int rc;
-    if (gemv_takes_few_token_gemm(ctx, n, k, batch)) {
+    if (gemv_takes_slices(ctx, n, k, batch, ep.rank != 0, false)) {
+        rc = ensure_scratch(ctx, gemv_mfma_sliced_scratch_bytes(n, k, batch), s);
+        if (rc) return rc;
+        launch_gemv_mfma_sliced(wp, n, k, x_dev, false, batch, y_dev, nullptr, nullptr, reinterpret_cast<float*>(ctx->moe_scratch), s);
+        ctx->counters.gemv++;
+    } else if (gemv_takes_few_token_gemm(ctx, n, k, batch)) {
         rc = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, batch), s);
         if (rc) return rc;
         launch_gemm_skinny(wp, n, k, x_dev, 0, batch, y_dev, ep, ctx->moe_scratch, s);
@@ -1556,6 +1566,19 @@ int lq4_gemv_fused_batch(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_off
         const char* env = getenv("LQ4_FUSED_PROLOGUE_BYTES");
         return env ? static_cast<size_t>(strtoull(env, nullptr, 10)) : kFusedPrologueBytes;
     }();
+    if ((f.prologue == LQ4_PRO_NONE || (f.prologue == LQ4_PRO_SILU_MUL && pro_bytes > pro_limit)) &&
+        gemv_takes_slices(ctx, n, k, batch, ep.rank != 0, true)) {
+        // the prologue as each slice is staged, the epilogue where the slices are added up (an elementwise launch)
+        rc = ensure_scratch(ctx, gemv_mfma_sliced_scratch_bytes(n, k, batch), s);
+        if (rc) return rc;
+        const bool add = f.epilogue == LQ4_EPI_ADD_RESIDUAL;
+        launch_gemv_mfma_sliced(wp, n, k, x_dev, f.prologue == LQ4_PRO_SILU_MUL, batch, y_dev, add ? f.residual : nullptr,
+                              add ? f.copy_dst : nullptr, reinterpret_cast<float*>(ctx->moe_scratch), s);
+        ctx->counters.gemv_fused++;
+        ctx->counters.elementwise++;
+        LQ4_HIP(hipGetLastError());
+        return LQ4_OK;
+    }
     if (!ep.rank && batch <= 8 && gemv_fused_batch_fits(k, batch)) {
         GemvFusion gf;
         const float* act_in = x_dev;

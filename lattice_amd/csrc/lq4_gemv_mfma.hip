@@ -94,6 +94,9 @@ struct GemvArgs {
     // [batch, 2K] rows of [gate | up] (x_stride apart), residual and copy_dst are [batch, N] rows
     // (y_stride apart).  kPlain / kStore: the plain product.
     GemvFusion fz;
+    // K slices (launch_gemv_mfma_sliced): workgroup row blockIdx.y works on blocks [y * slice_blocks, ...) of every row and
+    // stores plain partial results to y + slice * batch * n.  0: all of K.
+    uint32_t slice_blocks;
 };
 
 // NSETS: groups of four activation columns (1 or 2).  HILO: two columns per activation row.
@@ -114,7 +117,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_q4_mfma(GemvArgs p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 2;   // block within the step
     const int j = lane & 3;    // weight row within the tile / activation column within a set
-    const uint32_t nb = p.k / kBlockWeights;
+    uint32_t nb = p.k / kBlockWeights;
+    const uint32_t row_dwords = nb * 5;
+    if (p.slice_blocks) {  // from here on blocks and activations are counted from the start of the slice
+        const uint32_t b0 = blockIdx.y * p.slice_blocks;
+        p.w += b0 * static_cast<uint32_t>(kBlockBytes);
+        p.x += b0 * static_cast<uint32_t>(kBlockWeights);
+        p.y += static_cast<size_t>(blockIdx.y) * p.batch * p.n;
+        nb = nb - b0 < p.slice_blocks ? nb - b0 : p.slice_blocks;
+    }
     const uint32_t nsteps = (nb + 15) / 16;
     const uint32_t batch = p.batch;
     const int ncols = HILO ? 2 * static_cast<int>(batch) : static_cast<int>(batch);
@@ -170,7 +181,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_q4_mfma(GemvArgs p) {
             uint32_t row = row0 + 4 * t + j;
             if (row >= p.n) row = p.n - 1;
             buf[t] = *reinterpret_cast<const Q4BlockRaw*>(reinterpret_cast<const uint32_t*>(p.w) +
-                                                          static_cast<size_t>(row) * (nb * 5) + blk * 5);
+                                                          static_cast<size_t>(row) * row_dwords + blk * 5);
         }
     };
 
@@ -285,8 +296,11 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_q4_mfma(GemvArgs p) {
                 }
             }
             __syncthreads();  // inv_rms has been read by all before the meeting point is written
-        } else {  // kSiluMul: silu through the hardware exp2 and reciprocal, as the one-token kernel does
-            auto silu_mul = [](float gate, float u) {
+        } else {  // kSiluMul: silu through the hardware exp2 and reciprocal, as the one-token kernel does (a slice, in
+                  // the place of a launch of its own: as that one does)
+            const bool sliced = p.slice_blocks != 0;
+            auto silu_mul = [sliced](float gate, float u) {
+                if (sliced) return gate / (1.0f + expf(-gate)) * u;
                 const float e = __builtin_amdgcn_exp2f(gate * -1.44269504088896340736f);
                 return gate * __builtin_amdgcn_rcpf(1.0f + e) * u;
             };
@@ -574,6 +588,28 @@ void launch_shape(const GemvArgs& a, size_t lds, uint32_t t, uint32_t ks, uint32
 #undef LQ4_CASE
 }
 
+// y[b, r] = sum over the slices, in order; with `residual` that is added into residual[b, r] (and copied to copy_dst).
+__global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, uint32_t slices, uint32_t count,
+                                                         float* __restrict__ y, float* __restrict__ residual,
+                                                         float* __restrict__ copy_dst) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    const float r = residual ? residual[i] : 0.0f;
+    float v = 0.0f;
+    for (uint32_t s = 0; s < slices; s += 8) {
+        float t[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) t[j] = part[static_cast<size_t>(s + j < slices ? s + j : slices - 1) * count + i];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) v += s + j < slices ? t[j] : 0.0f;
+    }
+    if (y) y[i] = v;
+    if (residual) {
+        residual[i] = r + v;
+        if (copy_dst) copy_dst[i] = r + v;
+    }
+}
+
 }  // namespace
 
 // the K slices' meeting point: [2][waves][T <= 4][columns <= 8][4] floats
@@ -591,7 +627,7 @@ size_t gemv_mfma_lds_bytes(uint32_t k, uint32_t batch) {
 void launch_gemv_mfma(const uint8_t* w, uint32_t n, uint32_t k, const float* x, uint32_t x_stride,
                       uint32_t batch, float* y, uint32_t y_stride, const LoraEpilogue& lora,
                       hipStream_t stream, const GemvFusion* fusion) {
-    GemvArgs a{w, x, y, n, k, batch, x_stride, y_stride, lora, fusion ? *fusion : GemvFusion{}};
+    GemvArgs a{w, x, y, n, k, batch, x_stride, y_stride, lora, fusion ? *fusion : GemvFusion{}, 0};
     const size_t lds = gemv_mfma_lds_bytes(k, batch);
     const uint32_t nsteps = (k / kBlockWeights + 15) / 16;
     // resident workgroups per CU: up to 8 (32 waves, what the T = 1 kernels' 64 registers allow)
@@ -623,6 +659,46 @@ void launch_gemv_mfma(const uint8_t* w, uint32_t n, uint32_t k, const float* x, 
     } else {
         launch_shape<2, false>(a, lds, t, ks, waves, max_wgs, stream);
     }
+}
+
+// Few, long rows at 3..8 activation rows.  The launches above stage all of a row's activations in every workgroup, which on
+// 4096 x 14336 at eight rows is 459 KB (with silu * up formed on the way, twice that) beside 140 KB of weights a CU.  Here a
+// workgroup has 64 weight rows and a slice of 32 blocks, 32 KB of activations beside 40 KB of weights, and a small launch adds
+// the slices up, with the residual add for free.  Slices of 16 blocks, or of 32 rows, stage more than they save.  us, before
+// -> here, at 4 / 8 rows: plain 2560 x 9728 10.8 / 13.7 -> 9.1 / 12.1, 5120 x 17408 21.9 / 30.7 -> 20.3 / 27.4, 4096 x 14336 15.0 /
+// 25.8 -> 15.1 / 20.1; silu * up and residual add included (expf and the division as in the launch they replace, so that
+// the rounding of the activations to f16 falls as before) 2048 x 6144 9.7 / 12.4 -> 9.5 / 11.0, 4096 x 4096 11.9 / 15.8 -> 9.7 /
+// 11.3, 2560 x 9728 15.9 / 17.9 -> 12.5 / 15.0, 8192 x 8192 18.2 / 27.0 -> 20.9 / 25.9.  Behind on shorter rows (2048 x 4096 at
+// eight rows 10.2 -> 10.5, plain 6.4 -> 8.6).
+namespace {
+constexpr uint32_t kSliceBlocks = 32;
+uint32_t slices_of(uint32_t k) { return (k / kBlockWeights + kSliceBlocks - 1) / kSliceBlocks; }
+}  // namespace
+
+// `fused`: with a silu * up prologue or a residual add.
+bool gemv_mfma_sliced_wants(uint32_t n, uint32_t k, uint32_t batch, bool fused) {
+    if (batch < 3 || batch > 8) return false;
+    if (!fused) return k >= 9216 && n <= 5120;
+    const bool large = static_cast<uint64_t>(n) * k >= (1u << 24) && k > 2048;
+    return batch >= 5 ? n <= 8192 && (k >= 5120 || large) : n <= 5120 && large;
+}
+
+size_t gemv_mfma_sliced_scratch_bytes(uint32_t n, uint32_t k, uint32_t batch) {
+    return static_cast<size_t>(slices_of(k)) * batch * n * sizeof(float);
+}
+
+void launch_gemv_mfma_sliced(const uint8_t* w, uint32_t n, uint32_t k, const float* x, bool silu, uint32_t batch, float* y,
+                             float* residual, float* copy_dst, float* part, hipStream_t stream) {
+    GemvFusion fz{};
+    if (silu) fz.prologue = GemvFusion::kSiluMul;
+    const GemvArgs a{w, x, part, n, k, batch, silu ? 2 * k : k, n, LoraEpilogue{}, fz, kSliceBlocks};
+    const size_t lds = static_cast<size_t>(kSliceBlocks) * x_pitch_bytes(static_cast<int>(batch), static_cast<int>(batch)) + 64 + kRedBytes4;
+    constexpr uint32_t kRows = 64;  // of a workgroup: eight waves of two 4-row tiles
+    const dim3 grid((n + kRows - 1) / kRows, slices_of(k)), block(512);
+    if (batch <= 4) hipLaunchKernelGGL((gemv_q4_mfma<1, false, 2, 1, false, 8, false>), grid, block, lds, stream, a);
+    else hipLaunchKernelGGL((gemv_q4_mfma<2, false, 2, 1, false, 8, false>), grid, block, lds, stream, a);
+    const uint32_t count = batch * n;
+    hipLaunchKernelGGL(sum_slices_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, part, slices_of(k), count, y, residual, copy_dst);
 }
 
 }  // namespace lq4

@@ -141,6 +141,14 @@ bool gemv_i8_lora_in_launch(uint32_t n, uint32_t k, uint32_t batch, uint32_t ran
 void launch_gemv_i8(const uint8_t* w, uint32_t n, uint32_t k, const float* x, uint32_t x_stride, uint32_t batch,
                     float* y, uint32_t y_stride, const LoraEpilogue& lora, uint32_t cu_count, hipStream_t stream);
 
+// 3..8 rows of few, long weight rows: the 4x4x4 matrix-core kernel over K slices (partial results in `part`,
+// gemv_mfma_sliced_scratch_bytes), then a launch that adds the slices up.  silu: x = [gate(k) | up(k)] per row.  y may be null
+// where `residual` ([batch, n], added into; copied to copy_dst if set) is not.
+bool gemv_mfma_sliced_wants(uint32_t n, uint32_t k, uint32_t batch, bool fused);
+size_t gemv_mfma_sliced_scratch_bytes(uint32_t n, uint32_t k, uint32_t batch);
+void launch_gemv_mfma_sliced(const uint8_t* w, uint32_t n, uint32_t k, const float* x, bool silu, uint32_t batch, float* y,
+                           float* residual, float* copy_dst, float* part, hipStream_t stream);
+
 // Batch-1 kernel whose weights go from memory straight into a per-wave ring of LDS slots (lq4_gemv_dma.hip): plain
 // y = W . x only.  gemv_dma_serves: the shape fits (K <= 24576 and LDS for the activations plus two slots a wave).
 bool gemv_dma_serves(uint32_t n, uint32_t k, uint32_t cu_count);
