@@ -1592,6 +1592,13 @@ int lq4_gemv_fused_batch(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_off
             ctx->counters.elementwise++;
             act_in = xs;
             pro = LQ4_PRO_NONE;
+            if (f.epilogue == LQ4_EPI_NONE && gemv_takes_i8(ctx, n, k, batch)) {
+                // what is left is a plain product: the kernel that lq4_gemv takes for it (FUSEDFIGURES)
+                launch_gemv_i8(wp, n, k, xs, k, batch, y_dev, n, LoraEpilogue{}, ctx->cu_count, s);
+                ctx->counters.gemv_fused++;
+                LQ4_HIP(hipGetLastError());
+                return LQ4_OK;
+            }
         }
         gf.prologue = pro;
         gf.base = f.base;

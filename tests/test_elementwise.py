@@ -325,6 +325,31 @@ def test_fused_decode_mlp_for_several_rows(be, hidden, inter, batch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,k,batch,delta", [(8177, 1792, 5, True), (12291, 2048, 8, True), (37, 2048, 5, True),
+                                             (8200, 2304, 8, False)])
+def test_norm_as_its_own_launch_before_the_integer_kernel(be, n, k, batch, delta):
+    """Prologue inputs of more than 64 KB: the norm runs once and the plain product behind it goes to the kernel the plain call
+    takes (bit for bit its result)."""
+    import torch
+    print(f"norm + integer gemv n={n} k={k} batch={batch}", flush=True)
+    g = np.random.default_rng(31)
+    base, d = (g.normal(size=(batch, k)).astype(np.float32) for _ in range(2))
+    gamma = (g.normal(size=k) * 0.2).astype(np.float32)
+    w = synth.q4_weight(n, k, seed=31)
+    qw = be.upload_q4_blocks(w)
+    y, y2 = (torch.full((batch, n), float("nan"), device="cuda") for _ in range(2))
+    res, normed = (torch.full((batch, k), float("nan"), device="cuda") for _ in range(2))
+    dd = dev(d) if delta else None
+    be.dispatch_matmul_fused(None, qw, y, n, k, norm=(dev(base), dd, dev(gamma), 1e-6, res), batch=batch)
+    res_ref, normed_ref = oracle.residual_add_norm(base, d if delta else np.zeros_like(d), gamma, 1e-6)
+    assert np.array_equal(res.cpu().numpy(), res_ref)
+    assert rel_err(y.cpu().numpy(), oracle.gemm_f32(normed_ref, w, n, k)) <= 1e-4
+    be.dispatch_fused_residual_add_norm(dev(base), dd, None, normed, dev(gamma), k, 1e-6, num_rows=batch)
+    be.gemv_batch(normed, qw, y2, batch, n, k)
+    assert torch.equal(y, y2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("batch", [3, 8, 12])
 def test_fused_rows_with_a_lora_adapter_run_step_by_step(be, batch):
     """lq4_gemv_fused_batch with an adapter on the projection: the prologue, the GEMV with its LoRA delta
