@@ -13,12 +13,15 @@
 //    handling on this operand.
 //
 // 2. gemm_q4_skinny<RT, FMT, NTG>: a workgroup of eight waves owns 16 RT weight rows against a tile
-//    of NTG groups of 16 tokens.  Wave w takes K steps w, w + 8, ...; per step it loads its own Q4 blocks
-//    (lane (r, g) owns block g of row r of the step, as in the large prefill kernel) and the
-//    packed operands with fully coalesced 16-byte loads, dequantises in registers and issues
-//    v_mfma_f32_16x16x32_f16.  No LDS staging and no barrier in the K loop: nothing is shared
-//    between waves.  Two steps are in flight per wave; every load is unconditional (a load behind a
-//    run-time condition would make the compiler wait for loads it cannot count).
+//    of NTG groups of 16 tokens.  Wave w takes K steps w, w + 8, ...; per step the load unit puts its 16 RT pieces of rows
+//    (four Q4 blocks, 80 bytes) into the wave's own part of LDS, where lane (r, g) picks up block g of row r; the packed
+//    operands come with fully coalesced 16-byte loads; it dequantises in registers and issues
+//    v_mfma_f32_16x16x32_f16.  No barrier in the K loop: nothing is shared between waves.  Two steps are in flight per wave;
+//    every load is unconditional (a load behind a run-time condition would make the compiler wait for loads it cannot count).
+//    Blocks straight from memory to the lanes (20 bytes at a row's stride) cost the address unit a clock a lane and load, as much
+//    as all the activations of a 64-token step; as dense 16-byte pieces a quarter of that (17408 x 5120 at 20 tokens 29.0 -> 22.0
+//    us, 4096 x 4096 at 128 tokens 15.6 -> 13.6, 2048 x 6144 at 100 14.7 -> 12.7; 64 x 2048 x 2048 is latency, 6.9 both ways).  What
+//    is left of a step is its activations, four loads of 1 KB a token group through the CU's 64 bytes a clock.
 //    Each wave adds its share of the LoRA delta (ranks w, w + 8, ...) to its partial result in
 //    f32; the eight partial results then meet in LDS in a fixed order and y is stored once.
 //    MULTI = true: the workgroups' row tiles run over several matrices of the same K stacked one under the other
@@ -34,6 +37,7 @@
 
 #include <cmath>
 #include <type_traits>
+#include <utility>
 
 namespace lq4 {
 
@@ -46,13 +50,11 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 constexpr int kWavesK = 8;   // waves of a workgroup, each a K slice
 constexpr int kTokens = 64;  // tokens per workgroup: four groups of 16
 constexpr int TK = 128;      // K per step: four Q4 blocks
+// LDS of the waves' meeting at the end: 4 slots of RT * NTG * 64 accumulators
+template <int RT, int NTG>
+constexpr uint32_t kRedBytes = kWavesK / 2 * RT * NTG * 1024;
 constexpr uint32_t kMaxTSlices = 16;     // most K slices of t
 constexpr float kRestScale = 2048.0f;    // of what an f32 value loses as f16
-
-struct __attribute__((packed, aligned(4))) Q4BlockRaw {
-    uint32_t sb;    // f16 scale | f16 bias << 16
-    uint32_t q[4];  // 32 nibbles, nibble i of dword j = weight 8j + i
-};
 
 struct U4 {
     uint32_t v[4];
@@ -82,36 +84,84 @@ __device__ __forceinline__ U4 dequant8(uint32_t q, half2v d2, half2v b2) {
 
 // Sibling formats (FMT 1 = Q8_0, 2 = Q3): their decoders emit the eight weights of an instruction
 // in memory order, so their activations are packed without the interleave.
-// A Q8_0 block as loaded: eight whole dwords and the odd half beside them (a load that starts inside a dword costs the
-// address unit twice as much).  On a dword boundary: scale and weights 0, 1 in q[0], weights 30, 31 in h, and q[i + 1] : q[i]
-// shifted by two bytes are weights 4 i ..; two bytes past one: the scale in h, the weights in q.
-struct Q8BlockRaw {
-    uint32_t q[8];
-    uint32_t h;
+// A block as a lane reads it from LDS, and the 16-byte pieces a row's four blocks of a step take there.
+// A Q8_0 block as read: eight whole dwords and the odd half beside them (34-byte blocks: every other one starts inside a dword;
+// the first of a step's may, so 136 bytes take nine pieces).  On a dword boundary: scale and weights 0, 1 in dword 0, weights
+// 30, 31 in e, and dwords i + 1 : i shifted by two bytes are weights 4 i ..; two bytes past one: the scale in e, the weights in
+// the dwords.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+struct Q4Block {
+    u32x4 a;     // f16 scale | f16 bias << 16, weights 0..23 (nibble i of dword j = weight 8j + i)
+    uint32_t e;  // weights 24..31
 };
-struct __attribute__((packed, aligned(4))) Dwords8 {
-    uint32_t v[8];
+struct Q8Block {
+    u32x4 a, b;
+    uint32_t e;
 };
-struct __attribute__((packed, aligned(4))) Q3BlockRaw {
-    uint32_t sb;
-    uint32_t lo[2];  // weight i of 16-weight half h at bits 2i of lo[h]
-    uint32_t hi;     // weight i at bit i
+struct Q3Block {
+    u32x4 a;  // scale | bias; weight i of 16-weight half h at bits 2i of dword 1 + h; high bits: weight i at bit i of dword 3
 };
 template <int FMT>
 struct WBlockOf {
-    typedef Q4BlockRaw type;
-    static constexpr uint32_t kBytes = 20;
+    typedef Q4Block type;
+    static constexpr uint32_t kBytes = 20, kPieces = 5;
+    static constexpr int kReads = 2;
 };
 template <>
 struct WBlockOf<1> {
-    typedef Q8BlockRaw type;
-    static constexpr uint32_t kBytes = 34;
+    typedef Q8Block type;
+    static constexpr uint32_t kBytes = 34, kPieces = 9;
+    static constexpr int kReads = 3;
 };
 template <>
 struct WBlockOf<2> {
-    typedef Q3BlockRaw type;
-    static constexpr uint32_t kBytes = 16;
+    typedef Q3Block type;
+    static constexpr uint32_t kBytes = 16, kPieces = 4;
+    static constexpr int kReads = 1;
 };
+
+// LDS reads by hand, with their waits: one the compiler knows of is made to wait for every global_load_lds in flight.
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef __attribute__((address_space(1))) const void global_void_t;
+template <int OFF>
+__device__ __forceinline__ u32x4 lds_read128(uint32_t addr) {
+    u32x4 r;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF) : "memory");
+    return r;
+}
+template <int OFF>
+__device__ __forceinline__ uint32_t lds_read32(uint32_t addr) {
+    uint32_t r;
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF) : "memory");
+    return r;
+}
+template <int OFF>
+__device__ __forceinline__ uint32_t lds_read_u16(uint32_t addr) {
+    uint32_t r;
+    asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF) : "memory");
+    return r;
+}
+// At most N LDS operations of the wave are outstanding; no use of the block moves ahead of it.
+template <int N>
+__device__ __forceinline__ void wait_w(Q4Block& b) {
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b.a), "+v"(b.e) : "n"(N) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_w(Q8Block& b) {
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b.a), "+v"(b.b), "+v"(b.e) : "n"(N) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_w(Q3Block& b) {
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(b.a) : "n"(N) : "memory");
+}
+template <int... I, typename F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
+}
 
 // Q8_0: two packed dwords (weights 8j..8j+7) -> half(q * d).  A sign-flipped byte (q + 128) under the
 // exponent byte of 1024.0 is 1024 + 128 + q exactly; subtract, then one multiply with one rounding.
@@ -127,10 +177,10 @@ __device__ __forceinline__ U4 dequant8_q8(uint32_t qa, uint32_t qb, half2v d2) {
 }
 
 // Q3: weights 8j..8j+7 -> half(q * d + b), q = low2 | hi << 2.
-__device__ __forceinline__ U4 dequant8_q3(const Q3BlockRaw& b, int j, half2v d2, half2v b2) {
+__device__ __forceinline__ U4 dequant8_q3(uint32_t lo, uint32_t hi, int j, half2v d2, half2v b2) {
     const half2v k1024 = {static_cast<_Float16>(1024.0f), static_cast<_Float16>(1024.0f)};
-    const uint32_t lw = (b.lo[j >> 1] >> (16 * (j & 1))) & 0xffffu;  // 8 two-bit fields
-    const uint32_t hw = (b.hi >> (8 * j)) & 0xffu;                   // 8 bits
+    const uint32_t lw = (lo >> (16 * (j & 1))) & 0xffffu;  // 8 two-bit fields
+    const uint32_t hw = (hi >> (8 * j)) & 0xffu;                   // 8 bits
     U4 out;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
@@ -331,7 +381,7 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
                                                                 float* __restrict__ y, LoraEpilogue lora,
                                                                 uint32_t tile_groups,
                                                                 typename std::conditional<MULTI, SkinnyViews, NoViews>::type views) {
-    extern __shared__ float4v red[];  // 4 slots of RT * NTG * 64 accumulators
+    extern __shared__ float4v red[];  // the meeting of the waves, then two steps of weights for each wave
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -360,15 +410,73 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     const uint32_t steps_total = (nb + 3) / 4;
     const uint32_t cnt = steps_total > static_cast<uint32_t>(wave) ? (steps_total - wave + kWavesK - 1) / kWavesK : 0;
 
+    // ---- weights: a wave's step is 16 RT rows of kPieces 16-byte pieces, which the load unit puts into the wave's part of LDS
     typedef typename WBlockOf<FMT>::type WBlock;
-    constexpr uint32_t kBytes = WBlockOf<FMT>::kBytes;
-    const uint8_t* w_row[RT];
+    constexpr uint32_t kBytes = WBlockOf<FMT>::kBytes, kPieces = WBlockOf<FMT>::kPieces;
+    constexpr int kLoads = (16 * RT * kPieces + 63) / 64;
+    const size_t row_bytes = static_cast<size_t>(nb) * kBytes;
+    const uintptr_t w_first = reinterpret_cast<uintptr_t>(w) + n0 * row_bytes;
+    const uint32_t w_odd = static_cast<uint32_t>(w_first & 3);  // (a piece starts on a dword)
+    const uint8_t* const w_base = reinterpret_cast<const uint8_t*>(w_first - w_odd);
+    const size_t w_rest = ((n - n0) * row_bytes + w_odd + 3) & ~static_cast<size_t>(3);  // bytes from w_base to the end
+    const uint32_t w_left = w_rest < 0xfffffffcu ? static_cast<uint32_t>(w_rest) : 0xfffffffcu;
+    auto piece_off = [&](uint32_t unit) {  // of the wave's unit-th piece, at step 0
+        unit = unit < 16 * RT * kPieces ? unit : 16 * RT * kPieces - 1;
+        uint32_t row = unit / kPieces;
+        row = n0 + row < n ? row : n - 1 - n0;
+        return ((w_odd + row * static_cast<uint32_t>(row_bytes)) & ~3u) + unit % kPieces * 16;
+    };
+    uint32_t w_off[kLoads];
 #pragma unroll
-    for (int u = 0; u < RT; ++u) {
-        uint32_t row = n0 + 16 * u + lr;
-        row = row < n ? row : n - 1;
-        w_row[u] = w + static_cast<size_t>(row) * (nb * kBytes);
+    for (int i = 0; i < kLoads; ++i) w_off[i] = piece_off(i * 64 + lane);
+    const uint32_t w_reach = ((w_odd + (n - n0 < 16 * RT ? n - n0 - 1 : 16 * RT - 1) * static_cast<uint32_t>(row_bytes)) & ~3u) + kPieces * 16;
+    uint8_t* const w_lds = reinterpret_cast<uint8_t*>(red) + kRedBytes<RT, NTG> + wave * (2 * kLoads * 1024);
+    const uint32_t w_lds_at = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) uint8_t*)w_lds));
+    uint32_t w_read[RT], w_shift[RT];  // where the lane's block of row tile r lies in a step; Q8_0: how
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        w_read[r] = (16 * r + lr) * (kPieces * 16) + g * kBytes;
+        w_shift[r] = 0;
+        if constexpr (FMT == 1) {
+            const uint32_t row = n0 + 16 * r + lr < n ? 16 * r + lr : n - 1 - n0;
+            const uint32_t at = ((w_odd + row * static_cast<uint32_t>(row_bytes)) & 2) + g * kBytes;  // 2 bytes past a dword or on it
+            w_read[r] += (w_odd + row * static_cast<uint32_t>(row_bytes)) & 2;
+            w_shift[r] = (at & 2) == 0 ? 2 : 0;
+        }
+        w_read[r] += w_lds_at;
     }
+    auto load_w = [&](uint32_t s, int stage) {
+        const uint32_t at = s * (4 * kBytes);
+        uint8_t* const to = w_lds + stage * (kLoads * 1024);
+        if (at + w_reach <= w_left) {
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i)
+                __builtin_amdgcn_global_load_lds((global_void_t*)(w_base + (w_off[i] + at)), (lds_void_t*)(to + i * 1024), 16, 0, 0);
+        } else {
+            // its last pieces would reach past the end of the matrix: dword by dword, those past it read its last one
+#pragma unroll 1
+            for (int i = 0; i < 4 * kLoads; ++i) {
+                uint32_t off = piece_off(i * 16 + (lane >> 2)) + (lane & 3) * 4 + at;
+                off = off < w_left ? off : w_left - 4;
+                __builtin_amdgcn_global_load_lds((global_void_t*)(w_base + off), (lds_void_t*)(to + i * 256), 4, 0, 0);
+            }
+        }
+    };
+    // the lane's blocks of a step; read_w is followed by wait_w<reads of later row tiles> before a use
+    auto read_w = [&](WBlock& b, int r, auto stage_c) {
+        constexpr int off = decltype(stage_c)::value * kLoads * 1024;
+        if constexpr (FMT == 0) {
+            b.a = lds_read128<off>(w_read[r]);
+            b.e = lds_read32<off + 16>(w_read[r]);
+        } else if constexpr (FMT == 1) {
+            const uint32_t at = w_read[r] + (w_shift[r] ? 0 : 2);
+            b.a = lds_read128<off>(at);
+            b.b = lds_read128<off + 16>(at);
+            b.e = lds_read_u16<off>(w_read[r] + (w_shift[r] ? 32 : 0));
+        } else {
+            b.a = lds_read128<off>(w_read[r]);
+        }
+    };
 
     // ---- LoRA: wave w adds the ranks w, w + 8, ... of scale * B[row, :] . t[token, :] to its own partial result in f32, so the
     // delta is spread over all waves and joins their reduction.  The factors of its first two ranks are requested ahead of
@@ -426,34 +534,17 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         if constexpr (kEarlyT) load_t();
         if constexpr (kEarlyB) load_b_raw();
     }
-    uint32_t w_shift[RT];  // Q8_0: how the lane's blocks lie (every step alike)
-#pragma unroll
-    for (int r = 0; r < RT; ++r) w_shift[r] = FMT == 1 && (reinterpret_cast<uintptr_t>(w_row[r] + g * kBytes) & 2) == 0 ? 2 : 0;
     struct Unit {
-        WBlock wb[RT];
         uint4 x[NTG][4];  // [token group][instruction]
     };
     uint32_t xg[NTG];  // packed-image group of token group t (clamped to the last one)
 #pragma unroll
     for (int t = 0; t < NTG; ++t) xg[t] = tg0 + t < groups ? tg0 + t : groups - 1;
     // i-th step of this wave
-    auto load = [&](Unit& u, uint32_t i) {
+    auto load = [&](Unit& u, uint32_t i, int stage) {
         const uint32_t s = wave + i * kWavesK;
-        uint32_t blk = s * 4 + g;
-        blk = blk < nb ? blk : nb - 1;
-#pragma unroll
-        for (int r = 0; r < RT; ++r) {
-            const uint8_t* at = w_row[r] + blk * kBytes;
-            if constexpr (FMT == 1) {
-                const bool whole = (reinterpret_cast<uintptr_t>(at) & 2) == 0;
-                const Dwords8 d = *reinterpret_cast<const Dwords8*>(at + (whole ? 0 : 2));
-#pragma unroll
-                for (int i = 0; i < 8; ++i) u.wb[r].q[i] = d.v[i];
-                u.wb[r].h = *reinterpret_cast<const uint16_t*>(at + (whole ? 32 : 0));
-            } else {
-                u.wb[r] = *reinterpret_cast<const WBlock*>(at);
-            }
-        }
+        load_w(s, stage);
+        __builtin_amdgcn_sched_barrier(0);
         const uint4* xs = xp + static_cast<size_t>(s) * groups * 256 + lane;
 #pragma unroll
         for (int t = 0; t < NTG; ++t)
@@ -512,31 +603,40 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         }
     };
 
-    auto compute = [&](const Unit& u, uint32_t i) {
+    // LATER: loads issued behind this unit's
+    auto compute = [&](const Unit& u, uint32_t i, auto stage_c, auto later_c) {
         const bool live = (wave + i * kWavesK) * 4 + g < nb;  // K tail: a block past the end of the row counts as zero
+        WBlock blk[RT];
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(later_c)::value) : "memory");  // this unit has landed
 #pragma unroll
-        for (int r = 0; r < RT; ++r) {
-            WBlock wb = u.wb[r];
-            if constexpr (FMT == 2) asm volatile("" : "+v"(wb.lo[0]), "+v"(wb.lo[1]), "+v"(wb.hi));  // (or two units' decoding overlaps, and spills)
+        for (int r = 0; r < RT; ++r) read_w(blk[r], r, stage_c);
+        static_for<RT>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            wait_w<WBlockOf<FMT>::kReads * (RT - 1 - r)>(blk[r]);
+            const WBlock& wb = blk[r];
             uint32_t sb;
-            if constexpr (FMT == 1) sb = live ? (w_shift[r] ? wb.q[0] : wb.h) : 0u;  // scale only (the low half)
-            else sb = live ? wb.sb : 0u;
+            if constexpr (FMT == 1) sb = live ? (w_shift[r] ? wb.a[0] : wb.e) : 0u;  // scale only (the low half)
+            else sb = live ? wb.a[0] : 0u;
             const half2v d2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x01000100u));
             const half2v b2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x03020302u));
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 U4 a;
-                if constexpr (FMT == 0) a = dequant8(live ? wb.q[j] : 0u, d2, b2);
-                else if constexpr (FMT == 1)
-                    a = dequant8_q8(__builtin_amdgcn_alignbyte(wb.q[2 * j + 1], wb.q[2 * j], w_shift[r]),
-                                    __builtin_amdgcn_alignbyte(j < 3 ? wb.q[(2 * j + 2) & 7] : wb.h, wb.q[2 * j + 1], w_shift[r]), d2);
-                else a = dequant8_q3(wb, j, d2, b2);
+                if constexpr (FMT == 0) {
+                    a = dequant8(j < 3 ? wb.a[j < 3 ? j + 1 : 0] : wb.e, d2, b2);
+                } else if constexpr (FMT == 1) {
+                    const uint32_t q0 = j < 2 ? wb.a[(2 * j) & 3] : wb.b[(2 * j) & 3], q1 = j < 2 ? wb.a[(2 * j + 1) & 3] : wb.b[(2 * j + 1) & 3];
+                    const uint32_t q2 = j == 3 ? wb.e : j < 1 ? wb.a[2] : wb.b[(2 * j + 2) & 3];
+                    a = dequant8_q8(__builtin_amdgcn_alignbyte(q1, q0, w_shift[r]), __builtin_amdgcn_alignbyte(q2, q1, w_shift[r]), d2);
+                } else {
+                    a = dequant8_q3(wb.a[1 + (j >> 1)], wb.a[3], j, d2, b2);
+                }
 #pragma unroll
                 for (int t = 0; t < NTG; ++t)
                     acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                         __builtin_bit_cast(half8, a), __builtin_bit_cast(half8, u.x[t][j]), acc[r][t], 0, 0, 0);
             }
-        }
+        });
     };
 
     // Two units in flight.  Every unit that has a successor two places on prefetches it without a
@@ -545,42 +645,45 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     // (the scheduling fences keep a unit's arithmetic from being hoisted across the loads around it,
     // which would hold both units' temporaries live at once and spill)
 #define LQ4_FENCE() __builtin_amdgcn_sched_barrier(0)
+    constexpr std::integral_constant<int, 0> s0{}, none{};
+    constexpr std::integral_constant<int, 1> s1{};
+    constexpr std::integral_constant<int, kLoads + 4 * NTG> unit{};
     if (cnt > 1) {
         Unit u0, u1;
-        load(u0, 0);
-        load(u1, 1);
+        load(u0, 0, 0);
+        load(u1, 1, 1);
         LQ4_FENCE();
         if constexpr (LORA == 2) add_requested();
         uint32_t i = 0;
         for (; i + 3 < cnt; i += 2) {
-            compute(u0, i);
+            compute(u0, i, s0, unit);
             LQ4_FENCE();
-            load(u0, i + 2);
+            load(u0, i + 2, 0);
             LQ4_FENCE();
-            compute(u1, i + 1);
+            compute(u1, i + 1, s1, unit);
             LQ4_FENCE();
-            load(u1, i + 3);
+            load(u1, i + 3, 1);
             LQ4_FENCE();
         }
         if (cnt - i == 3) {
-            compute(u0, i);
+            compute(u0, i, s0, unit);
             LQ4_FENCE();
-            load(u0, i + 2);
+            load(u0, i + 2, 0);
             LQ4_FENCE();
-            compute(u1, i + 1);
+            compute(u1, i + 1, s1, unit);
             LQ4_FENCE();
-            compute(u0, i + 2);
+            compute(u0, i + 2, s0, none);
         } else {
-            compute(u0, i);
+            compute(u0, i, s0, unit);
             LQ4_FENCE();
-            compute(u1, i + 1);
+            compute(u1, i + 1, s1, none);
         }
     } else if (cnt == 1) {
         Unit u0;
-        load(u0, 0);
+        load(u0, 0, 0);
         LQ4_FENCE();
         if constexpr (LORA == 2) add_requested();
-        compute(u0, 0);
+        compute(u0, 0, s0, none);
     } else {
         if constexpr (LORA == 2) add_requested();
     }
@@ -651,12 +754,19 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
 // gemm_q4_skinny's LORA: see there.  (Eight waves: K 1024 is one step a wave, 3072 three.)
 inline int lora_form(uint32_t k) { return k > 1024 && k <= 3072 ? 1 : 2; }
 
+// (RT 2 with four token groups, and Q8_0, take more LDS than a kernel gets unasked)
+template <auto Kernel>
+void raise_lds(size_t bytes) {
+    static LdsCapOnce cap;
+    if (bytes > 64 * 1024) cap.raise(reinterpret_cast<const void*>(Kernel), 160 * 1024);
+}
+
 // `views`: null, or the matrices of a stacked launch (Q4; w, n, y and lora are then not read).
 template <int RT, int FMT, int NTG>
 void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint32_t m, float* y,
                 const LoraEpilogue& lora, const SkinnyViews* views, hipStream_t stream) {
     const uint32_t groups = (m + 15) / 16;
-    const size_t lds = static_cast<size_t>(kWavesK / 2) * RT * NTG * 64 * sizeof(float4v);
+    constexpr size_t lds = kRedBytes<RT, NTG> + kWavesK * 2 * ((16 * RT * WBlockOf<FMT>::kPieces + 63) / 64 * 1024);
     // tiles of two token groups for a batch of more: launch_fmt decides when
     const uint32_t tile_groups = NTG == 2 && groups > 2 ? 2 : kTokens / 16;
     const uint32_t token_tiles = (groups + tile_groups - 1) / tile_groups;
@@ -665,10 +775,14 @@ void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint3
         auto launch = [&](uint32_t tiles, uint32_t with_lora, auto multi, auto views_arg) {
             constexpr bool kMulti = decltype(multi)::value;
             const dim3 grid(tiles, token_tiles);
-            auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, lds, stream, w, n, k, xp, m, y, lora, tile_groups, views_arg); };
-            if (!with_lora) go(gemm_q4_skinny<RT, FMT, NTG, kMulti, 0>);
-            else if (lora_form(k) == 1) go(gemm_q4_skinny<RT, FMT, NTG, kMulti, 1>);
-            else go(gemm_q4_skinny<RT, FMT, NTG, kMulti, 2>);
+            auto go = [&](auto lora_c) {
+                constexpr auto kernel = gemm_q4_skinny<RT, FMT, NTG, kMulti, decltype(lora_c)::value>;
+                raise_lds<kernel>(lds);
+                hipLaunchKernelGGL(kernel, grid, block, lds, stream, w, n, k, xp, m, y, lora, tile_groups, views_arg);
+            };
+            if (!with_lora) go(std::integral_constant<int, 0>{});
+            else if (lora_form(k) == 1) go(std::integral_constant<int, 1>{});
+            else go(std::integral_constant<int, 2>{});
         };
         if (views) {
             uint32_t tiles = 0, with_lora = 0;
@@ -681,7 +795,9 @@ void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint3
             launch((n + 16 * RT - 1) / (16 * RT), lora.rank, std::false_type{}, NoViews{});
         }
     } else {
-        hipLaunchKernelGGL((gemm_q4_skinny<RT, FMT, NTG, false, 0>), dim3((n + 16 * RT - 1) / (16 * RT), token_tiles), block, lds,
+        constexpr auto kernel = gemm_q4_skinny<RT, FMT, NTG, false, 0>;
+        raise_lds<kernel>(lds);
+        hipLaunchKernelGGL(kernel, dim3((n + 16 * RT - 1) / (16 * RT), token_tiles), block, lds,
                            stream, w, n, k, xp, m, y, lora, tile_groups, NoViews{});
     }
 }
