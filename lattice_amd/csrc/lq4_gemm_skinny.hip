@@ -90,13 +90,16 @@ __device__ __forceinline__ U4 dequant8(uint32_t q, half2v d2, half2v b2) {
 // 30, 31 in e, and dwords i + 1 : i shifted by two bytes are weights 4 i ..; two bytes past one: the scale in e, the weights in
 // the dwords.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 struct Q4Block {
-    u32x4 a;     // f16 scale | f16 bias << 16, weights 0..23 (nibble i of dword j = weight 8j + i)
+    u32x2 a[2];  // f16 scale | f16 bias << 16, weights 0..23 (nibble i of dword j = weight 8j + i)
     uint32_t e;  // weights 24..31
+    __device__ __forceinline__ uint32_t dword(int i) const { return i < 4 ? a[i >> 1 & 1][i & 1] : e; }
 };
 struct Q8Block {
-    u32x4 a, b;
+    u32x2 a[4];
     uint32_t e;
+    __device__ __forceinline__ uint32_t dword(int i) const { return i < 8 ? a[i >> 1 & 3][i & 1] : e; }
 };
 struct Q3Block {
     u32x4 a;  // scale | bias; weight i of 16-weight half h at bits 2i of dword 1 + h; high bits: weight i at bit i of dword 3
@@ -105,13 +108,13 @@ template <int FMT>
 struct WBlockOf {
     typedef Q4Block type;
     static constexpr uint32_t kBytes = 20, kPieces = 5;
-    static constexpr int kReads = 2;
+    static constexpr int kReads = 3;
 };
 template <>
 struct WBlockOf<1> {
     typedef Q8Block type;
     static constexpr uint32_t kBytes = 34, kPieces = 9;
-    static constexpr int kReads = 3;
+    static constexpr int kReads = 5;
 };
 template <>
 struct WBlockOf<2> {
@@ -129,6 +132,14 @@ __device__ __forceinline__ u32x4 lds_read128(uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF) : "memory");
     return r;
 }
+// two dwords (a 16-byte read that starts on any dword stalls the unit for some 45 clocks)
+template <int OFF>
+__device__ __forceinline__ u32x2 lds_read2x32(uint32_t addr) {
+    static_assert(OFF % 4 == 0 && OFF / 4 + 1 < 256, "offsets are counted in dwords, in a byte");
+    u32x2 r;
+    asm volatile("ds_read2_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(r) : "v"(addr), "n"(OFF / 4), "n"(OFF / 4 + 1) : "memory");
+    return r;
+}
 template <int OFF>
 __device__ __forceinline__ uint32_t lds_read32(uint32_t addr) {
     uint32_t r;
@@ -144,11 +155,11 @@ __device__ __forceinline__ uint32_t lds_read_u16(uint32_t addr) {
 // At most N LDS operations of the wave are outstanding; no use of the block moves ahead of it.
 template <int N>
 __device__ __forceinline__ void wait_w(Q4Block& b) {
-    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(b.a), "+v"(b.e) : "n"(N) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b.a[0]), "+v"(b.a[1]), "+v"(b.e) : "n"(N) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_w(Q8Block& b) {
-    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(b.a), "+v"(b.b), "+v"(b.e) : "n"(N) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(b.a[0]), "+v"(b.a[1]), "+v"(b.a[2]), "+v"(b.a[3]), "+v"(b.e) : "n"(N) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_w(Q3Block& b) {
@@ -420,11 +431,12 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     const uint8_t* const w_base = reinterpret_cast<const uint8_t*>(w_first - w_odd);
     const size_t w_rest = ((n - n0) * row_bytes + w_odd + 3) & ~static_cast<size_t>(3);  // bytes from w_base to the end
     const uint32_t w_left = w_rest < 0xfffffffcu ? static_cast<uint32_t>(w_rest) : 0xfffffffcu;
+    // Q3: sixteen rows of four pieces lie four rows apart in the banks, so a row's pieces change places with its number
+    auto place = [](uint32_t piece, uint32_t row) { return FMT == 2 ? piece ^ (row >> 2 & 3) : piece; };
     auto piece_off = [&](uint32_t unit) {  // of the wave's unit-th piece, at step 0
         unit = unit < 16 * RT * kPieces ? unit : 16 * RT * kPieces - 1;
-        uint32_t row = unit / kPieces;
-        row = n0 + row < n ? row : n - 1 - n0;
-        return ((w_odd + row * static_cast<uint32_t>(row_bytes)) & ~3u) + unit % kPieces * 16;
+        const uint32_t row = unit / kPieces, real = n0 + row < n ? row : n - 1 - n0;
+        return ((w_odd + real * static_cast<uint32_t>(row_bytes)) & ~3u) + place(unit % kPieces, row) * 16;
     };
     uint32_t w_off[kLoads];
 #pragma unroll
@@ -435,7 +447,7 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     uint32_t w_read[RT], w_shift[RT];  // where the lane's block of row tile r lies in a step; Q8_0: how
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-        w_read[r] = (16 * r + lr) * (kPieces * 16) + g * kBytes;
+        w_read[r] = (16 * r + lr) * (kPieces * 16) + (FMT == 2 ? place(g, 16 * r + lr) : g) * kBytes;
         w_shift[r] = 0;
         if constexpr (FMT == 1) {
             const uint32_t row = n0 + 16 * r + lr < n ? 16 * r + lr : n - 1 - n0;
@@ -464,17 +476,21 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     };
     // the lane's blocks of a step; read_w is followed by wait_w<reads of later row tiles> before a use
     auto read_w = [&](WBlock& b, int r, auto stage_c) {
-        constexpr int off = decltype(stage_c)::value * kLoads * 1024;
+        // (offsets of a two-dword read end at 1 KB, so the second step's place goes into the address)
+        const uint32_t at = w_read[r] + decltype(stage_c)::value * kLoads * 1024;
         if constexpr (FMT == 0) {
-            b.a = lds_read128<off>(w_read[r]);
-            b.e = lds_read32<off + 16>(w_read[r]);
+            b.a[0] = lds_read2x32<0>(at);
+            b.a[1] = lds_read2x32<8>(at);
+            b.e = lds_read32<16>(at);
         } else if constexpr (FMT == 1) {
-            const uint32_t at = w_read[r] + (w_shift[r] ? 0 : 2);
-            b.a = lds_read128<off>(at);
-            b.b = lds_read128<off + 16>(at);
-            b.e = lds_read_u16<off>(w_read[r] + (w_shift[r] ? 32 : 0));
+            const uint32_t whole = at + (w_shift[r] ? 0 : 2);
+            b.a[0] = lds_read2x32<0>(whole);
+            b.a[1] = lds_read2x32<8>(whole);
+            b.a[2] = lds_read2x32<16>(whole);
+            b.a[3] = lds_read2x32<24>(whole);
+            b.e = lds_read_u16<0>(at + (w_shift[r] ? 32 : 0));
         } else {
-            b.a = lds_read128<off>(w_read[r]);
+            b.a = lds_read128<0>(at);
         }
     };
 
@@ -615,19 +631,19 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
             wait_w<WBlockOf<FMT>::kReads * (RT - 1 - r)>(blk[r]);
             const WBlock& wb = blk[r];
             uint32_t sb;
-            if constexpr (FMT == 1) sb = live ? (w_shift[r] ? wb.a[0] : wb.e) : 0u;  // scale only (the low half)
-            else sb = live ? wb.a[0] : 0u;
+            if constexpr (FMT == 1) sb = live ? (w_shift[r] ? wb.dword(0) : wb.e) : 0u;  // scale only (the low half)
+            else if constexpr (FMT == 2) sb = live ? wb.a[0] : 0u;
+            else sb = live ? wb.dword(0) : 0u;
             const half2v d2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x01000100u));
             const half2v b2 = as_h2(__builtin_amdgcn_perm(sb, sb, 0x03020302u));
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 U4 a;
                 if constexpr (FMT == 0) {
-                    a = dequant8(j < 3 ? wb.a[j < 3 ? j + 1 : 0] : wb.e, d2, b2);
+                    a = dequant8(wb.dword(j + 1), d2, b2);
                 } else if constexpr (FMT == 1) {
-                    const uint32_t q0 = j < 2 ? wb.a[(2 * j) & 3] : wb.b[(2 * j) & 3], q1 = j < 2 ? wb.a[(2 * j + 1) & 3] : wb.b[(2 * j + 1) & 3];
-                    const uint32_t q2 = j == 3 ? wb.e : j < 1 ? wb.a[2] : wb.b[(2 * j + 2) & 3];
-                    a = dequant8_q8(__builtin_amdgcn_alignbyte(q1, q0, w_shift[r]), __builtin_amdgcn_alignbyte(q2, q1, w_shift[r]), d2);
+                    a = dequant8_q8(__builtin_amdgcn_alignbyte(wb.dword(2 * j + 1), wb.dword(2 * j), w_shift[r]),
+                                    __builtin_amdgcn_alignbyte(wb.dword(2 * j + 2), wb.dword(2 * j + 1), w_shift[r]), d2);
                 } else {
                     a = dequant8_q3(wb.a[1 + (j >> 1)], wb.a[3], j, d2, b2);
                 }
