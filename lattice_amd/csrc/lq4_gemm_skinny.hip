@@ -818,22 +818,6 @@ void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint3
     }
 }
 
-// Widest row tile (of 1 or 2) whose two units in flight fit the 256 registers of a wave without spilling.
-constexpr int max_rt(int fmt, int ntg) {
-    if (fmt == 0) return 2;
-    if (fmt == 1) return ntg == 4 ? 1 : 2;
-    return ntg == 1 ? 2 : 1;
-}
-
-template <int RT, int FMT>
-void launch_rt(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint32_t m, float* y, const LoraEpilogue& lora,
-               const SkinnyViews* views, hipStream_t stream) {
-    const uint32_t groups = (m + 15) / 16;
-    if (groups == 1) launch_ntg<(RT < max_rt(FMT, 1) ? RT : max_rt(FMT, 1)), FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
-    else if (groups == 2) launch_ntg<(RT < max_rt(FMT, 2) ? RT : max_rt(FMT, 2)), FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
-    else launch_ntg<(RT < max_rt(FMT, 4) ? RT : max_rt(FMT, 4)), FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
-}
-
 }  // namespace
 
 // Adapters whose t = A . X the packing launch computes (LoraEpilogue::a set, no launch of its own): one matrix-core operand
@@ -1011,36 +995,41 @@ void launch_fmt(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_i
     }
     // Every workgroup reads the whole packed X of its token tile, so a wider row tile halves that traffic, at the price of
     // fewer workgroups to balance over the compute units.
-    if constexpr (FMT == 0) {
-        if (groups > 2) {
-            // Q4 at 33..128 tokens: a CU runs one workgroup (two of 16 x 32, whence its low cost), so a tile's cost is its rounds
-            // of 256 workgroups times what a workgroup of it takes, relative to 16 rows x 64 tokens.  Over 54 matrices
-            // (1024..32768 rows, K 512..5120, up to 2^26 weights) at 48..128 tokens the tile so chosen is 0.7 % behind the best
-            // of the four on average, 11 % at worst; with an adapter 1.0 and 11 % (q, k and v of four layers at 64 tokens 42.6 us
-            // in tiles of 32 x 32, 41.0 in 16 x 64).  us at 16 x 64 / 16 x 32 / 32 x 32 / 32 x 64, packing included: 2048 x 1024 at
-            // 64 tokens 6.4 / 5.7 / 6.4 / 7.6; 8192 x 2048 14.6 / 15.1 / 13.7 / 11.3; 16384 x 2048 24.9 / 25.5 / 23.0 / 18.8; at 128
-            // tokens 8192 x 5120 45.8 / 48.3 / 40.5 / 33.2.
-            const uint32_t t32 = (tiles16 + 1) / 2, q = (groups + 3) / 4, h = (groups + 1) / 2;
-            auto rounds = [](uint32_t wgs) { return (wgs + 255) / 256; };
-            const uint32_t cost[4] = {100 * rounds(tiles16 * q), 56 * rounds(tiles16 * h), (adapters ? 104 : 96) * rounds(t32 * h),
-                                      (adapters ? 140 : 155) * rounds(t32 * q)};
-            int best = 0;
-            for (int i = 1; i < 4; ++i)
-                if (cost[i] < cost[best]) best = i;
-            if (best == 0) launch_ntg<1, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
-            else if (best == 1) launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
-            else if (best == 2) launch_ntg<2, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
-            else launch_ntg<2, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
-            return;
-        }
+    if (groups > 2) {
+        // 33..128 tokens: a CU runs one workgroup (two of 16 x 32, whence its low cost), so a tile's cost is its rounds
+        // of 256 workgroups times what a workgroup of it takes, relative to 16 rows x 64 tokens.  Over 52 Q4 products (256..17408
+        // rows, K 512..8192) at 33..128 tokens the tile so chosen is 1.3 % behind the best of the four on average, over 30 sets
+        // of q, k and v with adapters 1.0 %.  us at 16 x 64 / 16 x 32 / 32 x 32 / 32 x 64, packing included: 2048 x 6144 at 64
+        // tokens 13.1 / 10.1 / 11.8 / 15.1; 8192 x 2048 12.1 / 11.0 / 9.9 / 9.4; 8192 x 5120 21.3 / 21.7 / 18.4 / 16.3; at 128 tokens
+        // 4096 x 4096 18.8 / 17.7 / 15.4 / 14.0.
+        // The siblings, whose decoders are longer, by figures of their own: 0.2 % over 38 products (Q8_0 2048 x 5120 at 48 tokens 12.1 /
+        // 9.4 / 11.5 / 14.5, 8192 x 2048 at 64 13.7 / 13.2 / 14.0 / 11.1; Q3 8192 x 1280 at 128 18.0 / 16.2 / 14.2 / 14.3).
+        const uint32_t t32 = (tiles16 + 1) / 2, q = (groups + 3) / 4, h = (groups + 1) / 2;
+        auto rounds = [](uint32_t wgs) { return (wgs + 255) / 256; };
+        const uint32_t r32 = rounds(t32 * h);
+        const uint32_t cost[4] = {100 * rounds(tiles16 * q), (FMT ? 50 : 56) * rounds(tiles16 * h),
+                                  FMT ? 80 * r32 + 20 * (r32 & 1) : (adapters ? 104 : 96) * r32, (FMT ? 125 : adapters ? 140 : 155) * rounds(t32 * q)};
+        int best = 0;
+        for (int i = 1; i < 4; ++i)
+            if (cost[i] < cost[best]) best = i;
+        if (best == 0) launch_ntg<1, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
+        else if (best == 1) launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+        else if (best == 2) launch_ntg<2, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+        else launch_ntg<2, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
+        return;
     }
     // Q4 up to 32 tokens: two row tiles where one of them would need a second round of workgroups (at 32 tokens, one / two: 4096 x
     // 2048 8.0 / 8.9 us, 4096 x 10240 18.1 / 22.7; 8192 x 2048 11.2 / 9.5, 5120 x 5120 19.4 / 15.2; 12288 x 2048, three rounds against
     // two, 14.8 / 14.6; 16 tokens and calls with adapters alike).  The siblings: measured over 2048..34816 rows and K
-    // 2048..17408 at 16, 32 and 64 tokens, two row tiles pay on tall matrices, on long rows and with four token groups.
-    const bool wide = FMT == 0 ? tiles16 > 256 : tiles16 >= 1024 || (k >= 8192 && tiles16 >= 256) || (m > 32 && tiles16 >= 512);
-    if (wide) launch_rt<2, FMT>(w, n, k, xp, m, y, lora, views, stream);
-    else launch_rt<1, FMT>(w, n, k, xp, m, y, lora, views, stream);
+    // 2048..17408 at 16 and 32 tokens, two row tiles pay on tall matrices and on long rows.
+    const bool wide = FMT == 0 ? tiles16 > 256 : tiles16 >= 1024 || (k >= 8192 && tiles16 >= 256);
+    if (groups == 1) {
+        if (wide) launch_ntg<2, FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
+        else launch_ntg<1, FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
+    } else {
+        if (wide) launch_ntg<2, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+        else launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+    }
 }
 
 }  // namespace
