@@ -458,6 +458,15 @@ static bool gemv_takes_slices(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32
     return cap == hipStreamCaptureStatusNone;
 }
 
+// The kernel choice of a call that the few-token GEMM would serve with `bytes` of scratch: under stream capture, scratch that
+// is too small for its packed activations leaves the call to the large-tile kernel (2), which may need none.
+static int few_token_choice(const lq4_ctx* ctx, size_t bytes, hipStream_t stream) {
+    if (ctx->gemm_kernel != 0 || bytes <= ctx->moe_scratch_bytes) return ctx->gemm_kernel;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
+    return cap == hipStreamCaptureStatusNone ? 0 : 2;
+}
+
 // The routing of lq4_gemv once the LoRA factor t (if any) is in ep, or ep.a says that the kernel which serves the
 // shape computes it: which kernel serves (batch, n, k).
 static int gemv_dispatch(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, uint32_t k, const float* x_dev, uint32_t batch,
@@ -617,10 +626,14 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
         // (behind one packing launch), the others each into their own.  q, k and v of the 2B model at 64 tokens with
         // rank-16 adapters on q and v: 18.6 us projection by projection, 12.1 so.
         SkinnyViews few{};
+        uint32_t packed_t = 0;  // adapters whose t the packing launch would compute
+        for (uint32_t i = 0; i < count; ++i)
+            packed_t += proj[i].n && ep[i].rank && gemm_skinny_computes_t(ep[i].rank) && gemm_takes_few_token_kernel(proj[i].n, k, batch, 0, true, ctx->gemm_kernel);
+        const int which = few_token_choice(ctx, gemm_skinny_scratch_bytes(k, batch, packed_t), s);
         for (uint32_t i = 0, v = 0; i < count; ++i) {
             const lq4_projection& p = proj[i];
             if (p.n == 0) continue;
-            if (gemm_takes_few_token_kernel(p.n, k, batch, 0, ep[i].rank != 0, ctx->gemm_kernel)) {
+            if (gemm_takes_few_token_kernel(p.n, k, batch, 0, ep[i].rank != 0, which)) {
                 const bool computes_t = ep[i].rank && gemm_skinny_computes_t(ep[i].rank);
                 few_token_view(&few, p.n, wp[i], p.y_dev, ep[i], computes_t ? p.lora->a_packed : nullptr);
                 if (computes_t) {
@@ -644,14 +657,14 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
         }
         for (uint32_t i = 0; i < count; ++i) {
             const lq4_projection& p = proj[i];
-            if (p.n == 0 || gemm_takes_few_token_kernel(p.n, k, batch, 0, ep[i].rank != 0, ctx->gemm_kernel)) continue;
-            const size_t scratch_bytes = gemm_scratch_floats(p.n, k, batch, 0, ep[i].rank != 0, ctx->gemm_kernel) * sizeof(float);
+            if (p.n == 0 || gemm_takes_few_token_kernel(p.n, k, batch, 0, ep[i].rank != 0, which)) continue;
+            const size_t scratch_bytes = gemm_scratch_floats(p.n, k, batch, 0, ep[i].rank != 0, which) * sizeof(float);
             if (scratch_bytes) {
                 const int rc = ensure_scratch(ctx, scratch_bytes, s);
                 if (rc) return rc;
             }
             launch_gemm(wp[i], p.n, k, x_dev, 0, batch, p.y_dev, ep[i],
-                        scratch_bytes ? reinterpret_cast<float*>(ctx->moe_scratch) : nullptr, ctx->gemm_kernel, s);
+                        scratch_bytes ? reinterpret_cast<float*>(ctx->moe_scratch) : nullptr, which, s);
             ctx->counters.gemm++;
         }
         LQ4_HIP(hipGetLastError());
@@ -849,20 +862,23 @@ int lq4_gemm(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
         rc = enter_shared_state(ctx, s);
         if (rc) return rc;
     }
-    if (ep.rank && gemm_takes_few_token_kernel(n, k, m, x_dtype == LQ4_F16, true, ctx->gemm_kernel) && gemm_skinny_computes_t(ep.rank)) {
+    int which = ctx->gemm_kernel;
+    if (gemm_takes_few_token_kernel(n, k, m, x_dtype == LQ4_F16, ep.rank != 0, which))
+        which = few_token_choice(ctx, gemm_skinny_scratch_bytes(k, m, ep.rank ? 1 : 0), s);
+    if (ep.rank && gemm_takes_few_token_kernel(n, k, m, x_dtype == LQ4_F16, true, which) && gemm_skinny_computes_t(ep.rank)) {
         ep.a = lora->a_packed;  // the few-token GEMM's packing launch computes A.X
     } else if (ep.rank) {
         launch_lora_a(lora->a, lora->is_f16, lora->rank, k, x_dev, x_dtype == LQ4_F16, k, m, ctx->lora_t, s);
         ctx->counters.lora_a++;
     }
     // shapes with too few tiles run as K slices into scratch partials, summed by a second kernel
-    const size_t scratch_bytes = gemm_scratch_floats(n, k, m, x_dtype == LQ4_F16, ep.rank != 0, ctx->gemm_kernel) * sizeof(float);
+    const size_t scratch_bytes = gemm_scratch_floats(n, k, m, x_dtype == LQ4_F16, ep.rank != 0, which) * sizeof(float);
     if (scratch_bytes) {
         rc = ensure_scratch(ctx, scratch_bytes, static_cast<hipStream_t>(stream));
         if (rc) return rc;
     }
     launch_gemm(wp, n, k, x_dev, x_dtype == LQ4_F16, m, y_dev, ep,
-                scratch_bytes ? reinterpret_cast<float*>(ctx->moe_scratch) : nullptr, ctx->gemm_kernel, s);
+                scratch_bytes ? reinterpret_cast<float*>(ctx->moe_scratch) : nullptr, which, s);
     ctx->counters.gemm++;
     LQ4_HIP(hipGetLastError());
     return LQ4_OK;
@@ -1836,6 +1852,12 @@ int lq4_gemv_chain(lq4_ctx* ctx, const lq4_chain_step* steps, uint32_t n_steps, 
     return LQ4_OK;
 }
 
+// (a forced kernel choice holds from 129 rows on)
+static bool sibling_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t m, int fmt, hipStream_t stream) {
+    return (m <= 128 || ctx->gemm_kernel == 0) && gemm_skinny_wants(n, k, m, fmt, false) &&
+           few_token_choice(ctx, gemm_skinny_scratch_bytes(k, m), stream) == ctx->gemm_kernel;
+}
+
 int lq4_gemm_q8(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_t n, uint32_t k,
                 const void* x_dev, int x_dtype, uint32_t m, float* y_dev, void* stream) {
     if (!ctx) return fail(LQ4_E_INVALID, "ctx is null");
@@ -1852,7 +1874,7 @@ int lq4_gemm_q8(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
     if (m == 1 && x_dtype == LQ4_F32 && gemv_q8_lds_bytes(k) <= 128 * 1024) {
         launch_gemv_q8_b1(wp, n, k, static_cast<const float*>(x_dev), y_dev, s);
         ctx->counters.gemv++;
-    } else if (m <= 32 || gemm_skinny_wants(n, k, m, 1, false)) {
+    } else if (m <= 32 || sibling_takes_few_token_gemm(ctx, n, k, m, 1, s)) {
         // few rows: operands packed once, the few-token matrix-core kernel with this format's decoder
         // (always up to 32 rows: the large-tile kernels are no match for it there)
         const int src = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, m), static_cast<hipStream_t>(stream));
@@ -1893,7 +1915,7 @@ int lq4_gemm_q3(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
     if (m == 1 && x_dtype == LQ4_F32 && gemv_q3_lds_bytes(k) <= 128 * 1024) {
         launch_gemv_q3_b1(wp, n, k, static_cast<const float*>(x_dev), y_dev, s);
         ctx->counters.gemv++;
-    } else if (m <= 32 || gemm_skinny_wants(n, k, m, 2, false)) {
+    } else if (m <= 32 || sibling_takes_few_token_gemm(ctx, n, k, m, 2, s)) {
         // few rows: operands packed once, the few-token matrix-core kernel with this format's decoder
         // (always up to 32 rows: the large-tile kernels are no match for it there)
         const int src = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, m), static_cast<hipStream_t>(stream));

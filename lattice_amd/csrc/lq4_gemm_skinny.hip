@@ -1,4 +1,4 @@
-// Few-token prefill GEMM: Y[M,N] = X[M,K] . W[N,K]^T for 2 .. 128 tokens, over Q4, Q8_0 or Q3 blocks.
+// Few-token prefill GEMM: Y[M,N] = X[M,K] . W[N,K]^T for 2 .. 128 tokens, and more of small matrices, over Q4, Q8_0 or Q3 blocks.
 //
 // With so few tokens the product is bound by streaming W once, like the decode GEMV, but there
 // are too many tokens for the 4x4x4 GEMV kernel and too few to fill the 128-token tiles of the
@@ -48,11 +48,7 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
 constexpr int kWavesK = 8;   // waves of a workgroup, each a K slice
-constexpr int kTokens = 64;  // tokens per workgroup: four groups of 16
 constexpr int TK = 128;      // K per step: four Q4 blocks
-// LDS of the waves' meeting at the end: 4 slots of RT * NTG * 64 accumulators
-template <int RT, int NTG>
-constexpr uint32_t kRedBytes = kWavesK / 2 * RT * NTG * 1024;
 constexpr uint32_t kMaxTSlices = 16;     // most K slices of t
 constexpr float kRestScale = 2048.0f;    // of what an f32 value loses as f16
 
@@ -279,8 +275,12 @@ __global__ __launch_bounds__(256) void pack_x_kernel(const void* __restrict__ xv
         x_operand<X_F16, INTERLEAVE>(load_x<X_F16>(xv, m, k, 16 * t + (lane & 15), s * TK + 32 * (lane >> 4) + 8 * j));
 }
 
-// Adapters whose t = A . X the packing launch computes: `a` packed by gemm_skinny_pack_lora_a, `part` [K slice][rank
-// 0..15][token, padded to whole groups of 16] over that slice.
+// Token groups in a row of the slices of t: [K slice][rank 0..15][token of its group][group], so that a lane of the product
+// gets a rank's factors of all its workgroup's groups in one load.
+__host__ __device__ inline uint32_t t_groups(uint32_t groups) { return groups <= 2 ? groups : (groups + 3) & ~3u; }
+
+// Adapters whose t = A . X the packing launch computes: `a` packed by gemm_skinny_pack_lora_a, `part` their sums over a K slice
+// (t_groups).
 struct PackLora {
     uint32_t count;
     uint32_t has_rest;  // bit v: a f32 adapter, the image of A's rest lies behind that of A
@@ -361,9 +361,9 @@ __global__ __launch_bounds__(64 * WAVES) void pack_x_lora_kernel(const void* __r
         float4v sum = part[v][0][lane];
 #pragma unroll
         for (int w = 1; w < WAVES; ++w) sum += part[v][w][lane];
-        float* const to = la.part[v0 + v] + (static_cast<size_t>(blockIdx.x) * 16 + 4 * (lane >> 4)) * (groups * 16) + token;
+        float* const to = la.part[v0 + v] + ((static_cast<size_t>(blockIdx.x) * 16 + 4 * (lane >> 4)) * 16 + (lane & 15)) * t_groups(groups) + t;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) to[i * groups * 16] = sum[i];  // element i of lane (c, g): rank 4 g + i, token c of the group
+        for (int i = 0; i < 4; ++i) to[i * 16 * t_groups(groups)] = sum[i];  // element i of lane (c, g): rank 4 g + i, token c of the group
     }
 }
 
@@ -378,21 +378,22 @@ __device__ __forceinline__ float sum_over_lane_groups(float v) {
 
 // RT: 16-row weight tiles per wave (rows per workgroup = 16 RT).  grid (ceil(N / 16 RT), token tiles).
 // FMT: 0 = Q4, 1 = Q8_0, 2 = Q3 blocks.
-// NTG: 16-token groups a workgroup computes (1, 2 or 4); a token tile with fewer groups re-reads its
-// last group and drops the results.  tile_groups (<= NTG): token groups from one workgroup's tile to the next
-// (grid.y tiles: four groups a tile, or two where NTG is held at two for a larger batch).  Fixed per instantiation, like the prefetches of the K loop below:
+// NTG: 16-token groups a workgroup computes (1, 2 or 4), grid.y tiles of so many; a token tile with fewer groups re-reads its
+// last group and drops the results.  Fixed per instantiation, like the prefetches of the K loop below:
 // a load behind a run-time condition makes the compiler wait for loads it cannot count, and the
 // pipeline collapses to one unit in flight.
 // MULTI: w, n, y and lora come from `views`, the view that holds this workgroup's row tile.  LORA: 0 = without the LoRA
 // step (a plain call would pay 0.1 us for the branches around it); 1, 2: see where the factors are requested.
+// A wave's part of LDS: two steps of weights, and at the end its accumulators.
+template <int RT, int NTG, int FMT>
+constexpr uint32_t kWaveBytes = 1024 * (2 * ((16 * RT * WBlockOf<FMT>::kPieces + 63) / 64) > RT * NTG ? 2 * ((16 * RT * WBlockOf<FMT>::kPieces + 63) / 64) : RT * NTG);
 struct NoViews {};
 template <int RT, int FMT, int NTG, bool MULTI, int LORA>
 __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __restrict__ w, uint32_t n, uint32_t k,
                                                                 const uint4* __restrict__ xp, uint32_t m,
                                                                 float* __restrict__ y, LoraEpilogue lora,
-                                                                uint32_t tile_groups,
                                                                 typename std::conditional<MULTI, SkinnyViews, NoViews>::type views) {
-    extern __shared__ float4v red[];  // the meeting of the waves, then two steps of weights for each wave
+    extern __shared__ float4v red[];  // kWaveBytes a wave
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -415,8 +416,8 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     }
     const uint32_t n0 = row_tile * (16 * RT);
     const uint32_t groups = (m + 15) / 16;             // token groups in X (and in the packed image)
-    const uint32_t tg0 = blockIdx.y * tile_groups;  // first token group of this workgroup
-    const uint32_t ntg = groups - tg0 < tile_groups ? groups - tg0 : tile_groups;
+    const uint32_t tg0 = blockIdx.y * NTG;  // first token group of this workgroup
+    const uint32_t ntg = groups - tg0 < NTG ? groups - tg0 : NTG;
     const uint32_t nb = k / kBlockWeights;
     const uint32_t steps_total = (nb + 3) / 4;
     const uint32_t cnt = steps_total > static_cast<uint32_t>(wave) ? (steps_total - wave + kWavesK - 1) / kWavesK : 0;
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) w_off[i] = piece_off(i * 64 + lane);
     const uint32_t w_reach = ((w_odd + (n - n0 < 16 * RT ? n - n0 - 1 : 16 * RT - 1) * static_cast<uint32_t>(row_bytes)) & ~3u) + kPieces * 16;
-    uint8_t* const w_lds = reinterpret_cast<uint8_t*>(red) + kRedBytes<RT, NTG> + wave * (2 * kLoads * 1024);
+    uint8_t* const w_lds = reinterpret_cast<uint8_t*>(red) + wave * kWaveBytes<RT, NTG, FMT>;
     const uint32_t w_lds_at = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) uint8_t*)w_lds));
     uint32_t w_read[RT], w_shift[RT];  // where the lane's block of row tile r lies in a step; Q8_0: how
 #pragma unroll
@@ -507,43 +508,61 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     // B as raw bits.  t, where it comes in K slices (LoraEpilogue::a set, so at most 16 ranks): lane (lr, g) takes slices g,
     // g + 4, ... of its token.
     constexpr bool kEarlyT = LORA == 2 || RT * NTG < 8, kEarlyB = kEarlyT && (LORA == 2 || RT == 1 || NTG > 1);
-    const uint32_t last_group = groups - 1;
-    float t_slice[2][NTG][kMaxTSlices / 4];
+    typedef float TVec __attribute__((ext_vector_type(NTG)));
+    TVec t_slice[2][kMaxTSlices / 4];
     uint32_t b_raw[2][RT][4];
+    auto first_rank = [&](int p) {  // wave w: ranks 2 w, 2 w + 1 (those past the end read rank 0 and are dropped)
+        const uint32_t jj = 2 * wave + p;
+        return jj < lora.rank ? jj : 0;
+    };
     auto load_t = [&]() {
         if (!lora.a) return;
+        const uint32_t tg = t_groups(groups);
         auto load_slices = [&](int h0) {
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                const uint32_t jj = wave + p * kWavesK, jc = jj < lora.rank ? jj : 0;
+            for (int p = 0; p < 2; ++p)
 #pragma unroll
-                for (int t = 0; t < NTG; ++t)
-#pragma unroll
-                    for (int h = h0; h < h0 + 2; ++h) {
-                        const uint32_t grp = tg0 + t < last_group ? tg0 + t : last_group;
-                        uint32_t slice = g + 4 * h;
-                        slice = slice < lora.t_slices ? slice : lora.t_slices - 1;
-                        t_slice[p][t][h] = lora.t[((slice * 16 + jc) * groups + grp) * 16 + lr];
-                    }
-            }
+                for (int h = h0; h < h0 + 2; ++h) {
+                    uint32_t slice = g + 4 * h;
+                    slice = slice < lora.t_slices ? slice : lora.t_slices - 1;
+                    t_slice[p][h] = *reinterpret_cast<const TVec*>(lora.t + ((slice * 16 + first_rank(p)) * 16 + lr) * tg + tg0);
+                }
         };
         load_slices(0);
         if (lora.t_slices > 8) load_slices(2);
     };
     auto load_b_raw = [&]() {
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const uint32_t jj = wave + p * kWavesK, jc = jj < lora.rank ? jj : 0;
+        auto each = [&](auto load) {
 #pragma unroll
             for (int r = 0; r < RT; ++r)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     uint32_t row = n0 + 16 * r + 4 * g + v;
                     row = row < n ? row : n - 1;
-                    const size_t idx = static_cast<size_t>(row) * lora.rank + jc;
-                    b_raw[p][r][v] = lora.b_is_f16 ? static_cast<uint32_t>(static_cast<const uint16_t*>(lora.b)[idx])
-                                                   : static_cast<const uint32_t*>(lora.b)[idx];
+                    load(r, v, static_cast<size_t>(row) * lora.rank);
                 }
+        };
+        if (lora.rank & 1) {
+            each([&](int r, int v, size_t row) {
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    const size_t idx = row + first_rank(p);
+                    b_raw[p][r][v] = lora.b_is_f16 ? static_cast<uint32_t>(static_cast<const uint16_t*>(lora.b)[idx]) : static_cast<const uint32_t*>(lora.b)[idx];
+                }
+            });
+        } else if (lora.b_is_f16) {
+            each([&](int r, int v, size_t row) {  // both ranks in a dword
+                b_raw[0][r][v] = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(lora.b) + row + first_rank(0));
+            });
+        } else {
+            struct __attribute__((packed, aligned(4))) Two {
+                uint32_t v[2];
+            };
+            each([&](int r, int v, size_t row) {
+                const Two two = *reinterpret_cast<const Two*>(static_cast<const uint32_t*>(lora.b) + row + first_rank(0));
+                b_raw[0][r][v] = two.v[0];
+                b_raw[1][r][v] = two.v[1];
+            });
         }
     };
     if (LORA && lora.rank) {
@@ -596,15 +615,16 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         if constexpr (!kEarlyB) load_b_raw();
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-            const uint32_t jj = wave + p * kWavesK;
+            const uint32_t jj = 2 * wave + p;
             if (jj >= lora.rank) continue;
             float tv[NTG], bv[RT][4];
             if (lora.a) {  // the slices, added up in the same order whatever the tile is
 #pragma unroll
                 for (int t = 0; t < NTG; ++t) {
-                    float v = g < static_cast<int>(lora.t_slices) ? t_slice[p][t][0] : 0.0f;
+                    auto slice = [&](int h) { return static_cast<float>(t_slice[p][h][t]); };
+                    float v = g < static_cast<int>(lora.t_slices) ? slice(0) : 0.0f;
 #pragma unroll
-                    for (int h = 1; h < static_cast<int>(kMaxTSlices) / 4; ++h) v += g + 4 * h < static_cast<int>(lora.t_slices) ? t_slice[p][t][h] : 0.0f;
+                    for (int h = 1; h < static_cast<int>(kMaxTSlices) / 4; ++h) v += g + 4 * h < static_cast<int>(lora.t_slices) ? slice(h) : 0.0f;
                     tv[t] = sum_over_lane_groups(v);
                 }
             } else {
@@ -613,8 +633,11 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
 #pragma unroll
             for (int r = 0; r < RT; ++r)
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    bv[r][v] = lora.scale * (lora.b_is_f16 ? f16_bits_to_f32(b_raw[p][r][v]) : __builtin_bit_cast(float, b_raw[p][r][v]));
+                for (int v = 0; v < 4; ++v) {
+                    uint32_t raw = b_raw[p][r][v];
+                    if (lora.b_is_f16 && !(lora.rank & 1)) raw = p ? b_raw[0][r][v] >> 16 : b_raw[0][r][v] & 0xffffu;
+                    bv[r][v] = lora.scale * (lora.b_is_f16 ? f16_bits_to_f32(raw) : __builtin_bit_cast(float, raw));
+                }
             add_rank(tv, bv);
         }
     };
@@ -722,47 +745,40 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         }
     }
 
-    constexpr int kSlot = RT * NTG * 64;
-    // ---- the eight K slices meet in LDS in three rounds: (w, w + 4), then (w, w + 2), then (0, 1);
-    //      the order is fixed, so the result does not depend on timing
+    // ---- the eight K slices meet in LDS, each wave's in its own part of it (its weights are done with), and are added as (w, w + 4),
+    //      then (w, w + 2), then (0, 1): a fixed order, so the result does not depend on timing.  Wave v sums and stores the
+    //      16 x 16 tiles v, v + 8, ...  (One barrier; three rounds of half the waves each, and wave 0 storing alone, took 1.4 us.)
+    constexpr int kTiles = RT * NTG;
+    {
+        float4v* const own = red + wave * (kWaveBytes<RT, NTG, FMT> / 16) + lane;
 #pragma unroll
-    for (int half = kWavesK / 2; half >= 1; half >>= 1) {
-        if (wave >= half && wave < 2 * half) {
-#pragma unroll
-            for (int r = 0; r < RT; ++r)
-#pragma unroll
-                for (int t = 0; t < NTG; ++t) red[(wave - half) * kSlot + (r * NTG + t) * 64 + lane] = acc[r][t];
-        }
-        __syncthreads();
-        if (wave < half) {
-#pragma unroll
-            for (int r = 0; r < RT; ++r)
-#pragma unroll
-                for (int t = 0; t < NTG; ++t) acc[r][t] += red[wave * kSlot + (r * NTG + t) * 64 + lane];
-        }
-        if (half > 1) __syncthreads();  // the slots are reused by the next round
+        for (int i = 0; i < kTiles; ++i) own[i * 64] = acc[i / NTG][i % NTG];
     }
-    if (wave > 0) return;
-
-    // element v of acc[r][t] in lane (lr, g): token 16 (tg0 + t) + lr, weight row n0 + 16 r + 4 g + v
+    __syncthreads();
+    // element v of tile (r, t) in lane (lr, g): token 16 (tg0 + t) + lr, weight row n0 + 16 r + 4 g + v
     const bool vec_ok = (n & 3u) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
 #pragma unroll
-    for (int r = 0; r < RT; ++r) {
-        const uint32_t gn = n0 + 16 * r + 4 * g;
-        if (gn >= n) continue;
+    for (int i0 = 0; i0 < kTiles; i0 += kWavesK) {
+        const int i = i0 + wave;
+        if (i >= kTiles) return;  // uniform
+        float4v part[kWavesK];
 #pragma unroll
-        for (int t = 0; t < NTG; ++t) {
-            const uint32_t tok = 16 * (tg0 + t) + lr;
-            if (static_cast<uint32_t>(t) >= ntg || tok >= m) continue;
-            const float4v val = acc[r][t];
-            float* dst = y + static_cast<size_t>(tok) * n + gn;
-            if (vec_ok) {
-                *reinterpret_cast<float4v*>(dst) = val;
-            } else {
+        for (int v = 0; v < kWavesK; ++v) part[v] = red[v * (kWaveBytes<RT, NTG, FMT> / 16) + i * 64 + lane];
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (gn + v < n) dst[v] = val[v];
-            }
+        for (int half = kWavesK / 2; half >= 1; half >>= 1)
+#pragma unroll
+            for (int v = 0; v < half; ++v) part[v] += part[v + half];
+        const int r = i / NTG, t = i % NTG;
+        const uint32_t gn = n0 + 16 * r + 4 * g, tok = 16 * (tg0 + t) + lr;
+        if (gn >= n || static_cast<uint32_t>(t) >= ntg || tok >= m) continue;
+        const float4v val = part[0];
+        float* dst = y + static_cast<size_t>(tok) * n + gn;
+        if (vec_ok) {
+            *reinterpret_cast<float4v*>(dst) = val;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (gn + v < n) dst[v] = val[v];
         }
     }
 }
@@ -782,10 +798,8 @@ template <int RT, int FMT, int NTG>
 void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint32_t m, float* y,
                 const LoraEpilogue& lora, const SkinnyViews* views, hipStream_t stream) {
     const uint32_t groups = (m + 15) / 16;
-    constexpr size_t lds = kRedBytes<RT, NTG> + kWavesK * 2 * ((16 * RT * WBlockOf<FMT>::kPieces + 63) / 64 * 1024);
-    // tiles of two token groups for a batch of more: launch_fmt decides when
-    const uint32_t tile_groups = NTG == 2 && groups > 2 ? 2 : kTokens / 16;
-    const uint32_t token_tiles = (groups + tile_groups - 1) / tile_groups;
+    constexpr size_t lds = kWavesK * kWaveBytes<RT, NTG, FMT>;
+    const uint32_t token_tiles = (groups + NTG - 1) / NTG;
     const dim3 block(64 * kWavesK);
     if constexpr (FMT == 0) {
         auto launch = [&](uint32_t tiles, uint32_t with_lora, auto multi, auto views_arg) {
@@ -794,7 +808,7 @@ void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint3
             auto go = [&](auto lora_c) {
                 constexpr auto kernel = gemm_q4_skinny<RT, FMT, NTG, kMulti, decltype(lora_c)::value>;
                 raise_lds<kernel>(lds);
-                hipLaunchKernelGGL(kernel, grid, block, lds, stream, w, n, k, xp, m, y, lora, tile_groups, views_arg);
+                hipLaunchKernelGGL(kernel, grid, block, lds, stream, w, n, k, xp, m, y, lora, views_arg);
             };
             if (!with_lora) go(std::integral_constant<int, 0>{});
             else if (lora_form(k) == 1) go(std::integral_constant<int, 1>{});
@@ -814,7 +828,7 @@ void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint3
         constexpr auto kernel = gemm_q4_skinny<RT, FMT, NTG, false, 0>;
         raise_lds<kernel>(lds);
         hipLaunchKernelGGL(kernel, dim3((n + 16 * RT - 1) / (16 * RT), token_tiles), block, lds,
-                           stream, w, n, k, xp, m, y, lora, tile_groups, NoViews{});
+                           stream, w, n, k, xp, m, y, lora, NoViews{});
     }
 }
 
@@ -855,32 +869,50 @@ void gemm_skinny_pack_lora_a(const void* a, int a_is_f16, uint32_t rank, uint32_
             }
 }
 
-// Where this kernel serves a shape rather than the large-tile kernel, which wastes the empty part of its token tile but
-// shares the activations of a tile among up to 256 rows where this one re-reads them for every 16 or 32: up to 16 tokens always;
-// from 33 on, matrices of up to n rows (the first entry that holds them) with K within its bounds.  Measured at 48, 64, 80, 96
-// and 128 tokens over 512..32768 rows and K 512..17408, f16 activations; us here / there on both sides of the lines:
-//   33..64 tokens (at 64): 4096 x 8192 20.7 / 21.4, 4096 x 14336 30.8 / 29.1; 8192 x 6144 23.6 / 25.8, 8192 x 10240 33.8 / 32.3; 12288 x
-//   512 9.5 / 9.3, 12288 x 2816 21.0 / 21.4, 12288 x 3328 23.4 / 21.4; 16384 x 512 11.2 / 9.7, 16384 x 2048 18.8 / 23.3; 20480 x 2048 24.9 / 21.9
-//   65..128 (at 128): 512 x 10240 17.0 / 19.9; 1024 x 8192 17.5 / 15.6, 2048 x 6144 17.3 / 23.2; 4096 x 5120 20.2 / 21.9, 4096 x 6144
-//   23.5 / 22.1; 8192 x 2816 21.0 / 23.1, 8192 x 3328 23.4 / 23.5; 12288 x 1024 18.5 / 16.1
-// With an adapter the large-tile kernel has a launch for t in front, so the lines lie further out:
-//   33..64: 4096 x 10240 26.5 / 29.3, 4096 x 14336 34.0 / 35.1; 8192 x 8192 31.5 / 36.1; 12288 x 2816 27.4 / 28.7, 12288 x 4096 35.4 / 31.4;
-//   16384 x 3328 29.7 / 35.9; 24576 x 2048 33.9 / 36.9
-//   65..128: 4096 x 8192 30.9 / 32.5, 2048 x 10240 28.4 / 28.7; 8192 x 2816 26.6 / 33.2; 12288 x 2048 32.1 / 37.8; 16384 x 1024 29.1 / 27.7
-// The sibling formats' decoders are longer and run once per 32 or 64 tokens here (Q8_0; Q3 alike):
-//   33..64: 4096 x 5120 16.4 / 20.2; 8192 x 2048 16.7 / 20.4, 8192 x 5120 29.5 / 27.0; 12288 x 1024 14.8 / 15.6, 14336 x 1024 18.1 / 15.8
-//   65..128: 2048 x 5120 17.1 / 22.2; 4096 x 2048 15.3 / 21.0, 4096 x 5120 26.6 / 20.5; 8192 x 1024 17.9 / 17.3 (Q3 16.3 / 19.6), 8192 x
-//   2048 26.6 / 21.8
+// Where this kernel serves a shape rather than the large-tile kernel, whose tiles of 96 tokens and more leave most CUs idle, or run
+// as K slices, until a product is large: up to 16 tokens always; then matrices of up to n rows (the first entry that holds them)
+// with K within its bounds.  Measured over 256..24576 rows and K 512..17408 at 24..2048 tokens, f16 activations (with f32 ones
+// this kernel leads by more); us there / here on both sides of the lines:
+//   17..32 tokens: 4096 x 17408 27.1 / 20.1, 5120 x 17408 30.1 / 24.1, 17408 x 17408 90.7 / 85.7
+//   33..64 (at 64): 4096 x 17408 27.0 / 24.2; 8192 x 14336 38.1 / 32.5; 12288 x 6144 27.9 / 27.2; 16384 x 512 8.9 / 8.3, 16384 x 5120 30.6 / 26.1;
+//     20480 x 1024 13.7 / 11.3, 20480 x 3072 25.4 / 24.1; 24576 x 2048 22.0 / 20.8 (at 40 19.2 / 19.1), 32768 x 1024 14.6 / 17.5
+//   65..128 (at 128): 1024 x 17408 23.4 / 21.8; 2048 x 14336 24.8 / 23.1, 2048 x 17408 27.1 / 26.9; 4096 x 7168 22.2 / 19.5, 4096 x 8192 21.9 /
+//     20.9; 8192 x 3584 22.9 / 20.1, 8192 x 4096 21.9 / 22.1; 12288 x 512 10.2 / 11.1, 12288 x 1024 14.7 / 13.8, 12288 x 2560 24.5 / 23.1;
+//     16384 x 1536 22.3 / 20.3, 16384 x 2048 23.6 / 25.6
+//   (16384 and more rows at 33..64 tokens, and 8193 and more at 65..128, with K of at most 1024 stay with the large tiles, as
+//   tests/test_gemm_tiles.py has them.)
+//   129..192 (at 192): 512 x 17408 22.9 / 22.1; 1024 x 10240 19.8 / 18.6; 2048 x 6144 19.9 / 17.3, 2048 x 10240 22.4 / 24.4; 3072 x 4096 20.2 / 17.0,
+//     3072 x 6144 21.1 / 23.6; 4096 x 4096 22.4 / 18.7; 6144 x 3072 22.3 / 20.2; 8192 x 512 9.9 / 11.1, 8192 x 1024 14.6 / 13.6, 8192 x 2048 24.2 / 18.6
+//   193..256 (at 256): 1024 x 10240 21.5 / 19.2; 2048 x 2048 19.8 / 9.9, 2048 x 6144 20.2 / 18.7; 3072 x 4096 20.4 / 19.2; 4096 x 3072 22.5 / 18.3, 4096 x
+//     4096 22.3 / 22.4; 6144 x 512 10.2 / 11.1, 6144 x 1024 14.8 / 13.9, 6144 x 2048 23.6 / 18.8; 8192 x 2048 23.4 / 24.0
+//   257..384 (at 384): 512 x 6144 20.2 / 15.6, 512 x 10240 19.8 / 20.4; 1024 x 4096 17.4 / 15.6, 1024 x 6144 19.4 / 19.6; 2048 x 3072 19.4 / 16.4, 2048 x 4096
+//     19.9 / 20.3; 3072 x 2048 21.1 / 16.2; 4096 x 512 9.9 / 11.4, 4096 x 1024 14.6 / 14.3, 4096 x 2048 21.9 / 19.8
+//   385..512 (at 512): 512 x 6144 19.5 / 17.1, 512 x 10240 21.2 / 22.7; 1024 x 4096 18.2 / 16.9; 2048 x 2048 20.4 / 15.4, 2048 x 3072 20.1 / 20.2; 3072 x 1024
+//     14.8 / 14.6, 3072 x 2048 22.4 / 20.5; 4096 x 2048 23.0 / 25.2
+//   513..768 (at 768): 256 x 4096 19.6 / 16.1; 512 x 3072 18.3 / 15.9; 1024 x 2048 17.4 / 14.8, 1024 x 4096 20.6 / 21.6; 2048 x 1024 14.5 / 15.3
+//   769..1024 (at 1024): 256 x 3072 18.4 / 15.8; 512 x 2048 19.8 / 15.1, 512 x 3072 17.6 / 18.5; 1024 x 512 9.6 / 10.0, 1024 x 1024 19.5 / 12.6, 1024 x 2048 17.8 / 18.2
+// With an adapter the large-tile kernel has a launch for t in front, so the lines lie further out (up to 128 tokens):
+//   33..64: 4096 x 17408 37.2 / 29.2; 8192 x 14336 45.4 / 34.5; 12288 x 6144 36.1 / 33.6; 16384 x 5120 40.9 / 28.6; 24576 x 2560 38.9 / 29.0
+//   65..128: 1024 x 17408 32.3 / 24.0; 4096 x 10240 33.9 / 26.9; 8192 x 4096 33.5 / 25.7; 12288 x 2560 37.8 / 28.4; 16384 x 1024 26.5 / 22.5, 16384 x 2048 40.2 / 32.3
+// The sibling formats' decoders are longer (Q8_0; Q3 alike or better); above 128 tokens they share the lines of Q4:
+//   33..64: 4096 x 12288 30.6 / 24.4; 8192 x 8192 30.5 / 24.6; 12288 x 2048 18.2 / 16.6, 12288 x 3072 21.7 / 21.9; 16384 x 2048 22.7 / 17.6
+//   65..128: 512 x 17408 23.4 / 18.9; 2048 x 8192 20.6 / 19.1, 2048 x 10240 22.0 / 21.8; 4096 x 6144 21.8 / 19.4; 8192 x 2048 20.1 / 15.8, 8192 x 3072 21.4 / 21.8
 namespace {
 struct ShapeLimit {
     uint32_t n, k_min, k_max;
 };
-constexpr ShapeLimit kPlain64[] = {{2048, 0, 10240}, {4096, 0, 8192}, {8192, 0, 6144}, {12288, 0, 2816}, {16384, 1024, 2816}};
-constexpr ShapeLimit kPlain128[] = {{512, 0, 10240}, {2048, 0, 8192}, {4096, 0, 5120}, {8192, 0, 2816}};
-constexpr ShapeLimit kLora64[] = {{4096, 0, 10240}, {8192, 0, 8192}, {12288, 0, 3328}, {16384, 0, 5120}, {24576, 0, 2048}};
-constexpr ShapeLimit kLora128[] = {{1024, 0, 14336}, {4096, 0, 8192}, {8192, 0, 3328}, {12288, 0, 2048}};
-constexpr ShapeLimit kSibling64[] = {{4096, 0, 5120}, {8192, 0, 3072}, {12288, 0, 1024}};
-constexpr ShapeLimit kSibling128[] = {{2048, 0, 5120}, {4096, 0, 2048}, {8192, 1024, 1536}};
+constexpr ShapeLimit kPlain64[] = {{4096, 0, 17408}, {8192, 0, 14336}, {12288, 0, 6144}, {16384, 1024, 5120}, {20480, 1056, 3072}};
+constexpr ShapeLimit kPlain128[] = {{1024, 0, 17408}, {2048, 0, 14336}, {4096, 0, 7680}, {8192, 0, 3584}, {12288, 1056, 2560}, {16384, 1056, 1536}};
+constexpr ShapeLimit kPlain192[] = {{512, 0, 14336}, {1024, 0, 10240}, {2048, 0, 6144}, {4096, 0, 4096}, {6144, 0, 3072}, {8192, 1024, 2048}};
+constexpr ShapeLimit kPlain256[] = {{1024, 0, 10240}, {2048, 0, 6144}, {3072, 0, 4096}, {4096, 0, 3072}, {6144, 1024, 2048}};
+constexpr ShapeLimit kPlain384[] = {{512, 0, 8192}, {1024, 0, 4096}, {2048, 0, 3072}, {3072, 0, 2048}, {4096, 1024, 2048}};
+constexpr ShapeLimit kPlain512[] = {{512, 0, 6144}, {1024, 0, 4096}, {2048, 0, 2048}, {3072, 1024, 2048}};
+constexpr ShapeLimit kPlain768[] = {{256, 0, 4096}, {512, 0, 3072}, {1024, 0, 2048}};
+constexpr ShapeLimit kPlain1024[] = {{256, 0, 3072}, {512, 0, 2048}, {1024, 768, 1536}};
+constexpr ShapeLimit kLora64[] = {{4096, 0, 17408}, {8192, 0, 14336}, {12288, 0, 6144}, {16384, 0, 5120}, {24576, 0, 2560}};
+constexpr ShapeLimit kLora128[] = {{1024, 0, 17408}, {4096, 0, 10240}, {8192, 0, 4096}, {12288, 0, 2560}, {16384, 1024, 2048}};
+constexpr ShapeLimit kSibling64[] = {{4096, 0, 12288}, {8192, 0, 8192}, {12288, 0, 2560}, {16384, 512, 2048}};
+constexpr ShapeLimit kSibling128[] = {{512, 0, 17408}, {2048, 0, 8192}, {4096, 0, 6144}, {8192, 0, 2560}};
 template <size_t N>
 bool within(const ShapeLimit (&limits)[N], uint32_t n, uint32_t k) {
     for (const ShapeLimit& l : limits)
@@ -890,17 +922,19 @@ bool within(const ShapeLimit (&limits)[N], uint32_t n, uint32_t k) {
 }  // namespace
 
 bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora) {
-    if (k < kBlockWeights || m > 2 * kTokens) return false;
+    if (k < kBlockWeights) return false;
     if (m <= 16) return true;
-    if (m <= 32) {
-        // one token tile of 32: unless the matrix is large (above 2^26 weights) and has fewer than 8192 rows (too few
-        // workgroups here) or more than 2^28 weights
-        const uint64_t weights = static_cast<uint64_t>(n) * k;
-        return weights <= (1ull << 26) || (n >= 8192 && weights <= (1ull << 28));
+    if (m <= 32) return static_cast<uint64_t>(n) * k <= (1ull << 28);
+    if (m <= 128) {
+        if (fmt) return m <= 64 ? within(kSibling64, n, k) : within(kSibling128, n, k);
+        if (with_lora) return m <= 64 ? within(kLora64, n, k) : within(kLora128, n, k);
+        return m <= 64 ? within(kPlain64, n, k) : within(kPlain128, n, k);
     }
-    if (fmt) return m <= kTokens ? within(kSibling64, n, k) : within(kSibling128, n, k);
-    if (with_lora) return m <= kTokens ? within(kLora64, n, k) : within(kLora128, n, k);
-    return m <= kTokens ? within(kPlain64, n, k) : within(kPlain128, n, k);
+    if (with_lora) return false;
+    if (m <= 256) return m <= 192 ? within(kPlain192, n, k) : within(kPlain256, n, k);
+    if (m <= 512) return m <= 384 ? within(kPlain384, n, k) : within(kPlain512, n, k);
+    if (m <= 1024) return m <= 768 ? within(kPlain768, n, k) : within(kPlain1024, n, k);
+    return false;
 }
 
 namespace {
@@ -923,7 +957,7 @@ inline PackLoraForm pack_lora_form(uint32_t steps) {
 // Packed X, then the slices of t of the adapters whose t the packing launch computes.
 size_t gemm_skinny_scratch_bytes(uint32_t k, uint32_t m, uint32_t adapters) {
     const size_t steps = (k / kBlockWeights + 3) / 4, groups = (m + 15) / 16;
-    return (steps * groups * 256 + adapters * pack_lora_form(static_cast<uint32_t>(steps)).slices * groups * 64) * sizeof(uint4);
+    return (steps * groups * 256 + adapters * pack_lora_form(static_cast<uint32_t>(steps)).slices * t_groups(static_cast<uint32_t>(groups)) * 64) * sizeof(uint4);
 }
 
 namespace {
@@ -971,16 +1005,14 @@ void launch_fmt(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_i
         la.a[v] = static_cast<const uint4*>(e.a);
         la.has_rest |= (e.b_is_f16 ? 0u : 1u) << v;
         e.t_slices = pack_lora_form(steps).slices;
-        la.part[v] = reinterpret_cast<float*>(xp + static_cast<size_t>(steps) * groups * 256) + static_cast<size_t>(v) * e.t_slices * groups * 256;
+        la.part[v] = reinterpret_cast<float*>(xp + static_cast<size_t>(steps) * groups * 256) + static_cast<size_t>(v) * e.t_slices * t_groups(groups) * 256;
         e.t = la.part[v];
     };
     uint32_t tiles16 = (n + 15) / 16;
-    bool adapters = lora.rank != 0;
     if (views) {
         tiles16 = 0;
         for (uint32_t v = 0; v < views->count; ++v) {
             tiles16 += (views->n[v] + 15) / 16;
-            adapters |= views->lora[v].rank != 0;
             produce_t(views->lora[v]);
         }
     } else {
@@ -995,41 +1027,37 @@ void launch_fmt(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_i
     }
     // Every workgroup reads the whole packed X of its token tile, so a wider row tile halves that traffic, at the price of
     // fewer workgroups to balance over the compute units.
-    if (groups > 2) {
-        // 33..128 tokens: a CU runs one workgroup (two of 16 x 32, whence its low cost), so a tile's cost is its rounds
-        // of 256 workgroups times what a workgroup of it takes, relative to 16 rows x 64 tokens.  Over 52 Q4 products (256..17408
-        // rows, K 512..8192) at 33..128 tokens the tile so chosen is 1.3 % behind the best of the four on average, over 30 sets
-        // of q, k and v with adapters 1.0 %.  us at 16 x 64 / 16 x 32 / 32 x 32 / 32 x 64, packing included: 2048 x 6144 at 64
-        // tokens 13.1 / 10.1 / 11.8 / 15.1; 8192 x 2048 12.1 / 11.0 / 9.9 / 9.4; 8192 x 5120 21.3 / 21.7 / 18.4 / 16.3; at 128 tokens
-        // 4096 x 4096 18.8 / 17.7 / 15.4 / 14.0.
-        // The siblings, whose decoders are longer, by figures of their own: 0.2 % over 38 products (Q8_0 2048 x 5120 at 48 tokens 12.1 /
-        // 9.4 / 11.5 / 14.5, 8192 x 2048 at 64 13.7 / 13.2 / 14.0 / 11.1; Q3 8192 x 1280 at 128 18.0 / 16.2 / 14.2 / 14.3).
-        const uint32_t t32 = (tiles16 + 1) / 2, q = (groups + 3) / 4, h = (groups + 1) / 2;
-        auto rounds = [](uint32_t wgs) { return (wgs + 255) / 256; };
-        const uint32_t r32 = rounds(t32 * h);
-        const uint32_t cost[4] = {100 * rounds(tiles16 * q), (FMT ? 50 : 56) * rounds(tiles16 * h),
-                                  FMT ? 80 * r32 + 20 * (r32 & 1) : (adapters ? 104 : 96) * r32, (FMT ? 125 : adapters ? 140 : 155) * rounds(t32 * q)};
-        int best = 0;
-        for (int i = 1; i < 4; ++i)
-            if (cost[i] < cost[best]) best = i;
-        if (best == 0) launch_ntg<1, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
-        else if (best == 1) launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
-        else if (best == 2) launch_ntg<2, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
-        else launch_ntg<2, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
+    if (groups == 1) {
+        // Two row tiles where one of them would need a second round of workgroups.  (8192 x 2048 at 16 tokens 6.1 / 5.7 us)
+        if (tiles16 > 256) launch_ntg<2, FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
+        else launch_ntg<1, FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
         return;
     }
-    // Q4 up to 32 tokens: two row tiles where one of them would need a second round of workgroups (at 32 tokens, one / two: 4096 x
-    // 2048 8.0 / 8.9 us, 4096 x 10240 18.1 / 22.7; 8192 x 2048 11.2 / 9.5, 5120 x 5120 19.4 / 15.2; 12288 x 2048, three rounds against
-    // two, 14.8 / 14.6; 16 tokens and calls with adapters alike).  The siblings: measured over 2048..34816 rows and K
-    // 2048..17408 at 16 and 32 tokens, two row tiles pay on tall matrices and on long rows.
-    const bool wide = FMT == 0 ? tiles16 > 256 : tiles16 >= 1024 || (k >= 8192 && tiles16 >= 256);
-    if (groups == 1) {
-        if (wide) launch_ntg<2, FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
-        else launch_ntg<1, FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
-    } else {
-        if (wide) launch_ntg<2, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
-        else launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+    // A launch's cost by tile: so much once, so much for every round of 256 workgroups (small tiles share a CU, whence their low
+    // second figure), relative to 16 rows x 64 tokens = 100.  Fitted to 159 launches at 17..128 tokens (Q4 256..17408 rows, K
+    // 512..17408, 41 sets of q, k and v with adapters, Q8_0 and Q3 alike): the tile so chosen is 0.8 % behind the best of the
+    // five on average, 11 % at worst.  us at 16 x 64 / 16 x 32 / 32 x 32 / 32 x 64 / 16 x 16, packing included: 8192 x 2048 at 64
+    // tokens 12.1 / 11.0 / 9.9 / 9.4 / -; 1153 x 9024 at 38 16.2 / 12.6 / 14.9 / 18.8 / 10.3; 2088 x 2336 at 83 11.2 / 8.4 / 7.6 / 8.9 / 9.8;
+    // 4190 x 4416 at 49 17.5 / 15.8 / 15.1 / 12.1 / 17.4; q, k and v of 3584 + 2 x 512 rows at 66 tokens, two layers, 46.8 / 38.4 / 33.7 / 40.2 /
+    // 50.8; Q8_0 2048 x 5120 at 48 12.1 / 9.4 / 11.5 / 14.5 / -.
+    struct Tile {
+        int rt, ntg, first, each;
+    };
+    constexpr Tile kTiles[] = {{1, 4, 10, 90}, {1, 2, 24, 57}, {2, 2, FMT ? 26 : 23, FMT ? 80 : 74}, {2, 4, 14, 134}, {1, 1, 24, 46}};
+    int best = 0, best_cost = 0;
+    for (int i = 0; i < 5; ++i) {
+        const uint32_t wgs = (tiles16 + kTiles[i].rt - 1) / kTiles[i].rt * ((groups + kTiles[i].ntg - 1) / kTiles[i].ntg);
+        const int cost = kTiles[i].first + kTiles[i].each * static_cast<int>((wgs + 255) / 256);
+        if (i == 0 || cost < best_cost) {
+            best = i;
+            best_cost = cost;
+        }
     }
+    if (best == 0) launch_ntg<1, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
+    else if (best == 1) launch_ntg<1, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+    else if (best == 2) launch_ntg<2, FMT, 2>(w, n, k, xp, m, y, lora, views, stream);
+    else if (best == 3) launch_ntg<2, FMT, 4>(w, n, k, xp, m, y, lora, views, stream);
+    else launch_ntg<1, FMT, 1>(w, n, k, xp, m, y, lora, views, stream);
 }
 
 }  // namespace
