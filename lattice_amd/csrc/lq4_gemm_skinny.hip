@@ -894,7 +894,9 @@ void gemm_skinny_pack_lora_a(const void* a, int a_is_f16, uint32_t rank, uint32_
 // With an adapter the large-tile kernel has a launch for t in front, so the lines lie further out (up to 128 tokens):
 //   33..64: 4096 x 17408 37.2 / 29.2; 8192 x 14336 45.4 / 34.5; 12288 x 6144 36.1 / 33.6; 16384 x 5120 40.9 / 28.6; 24576 x 2560 38.9 / 29.0
 //   65..128: 1024 x 17408 32.3 / 24.0; 4096 x 10240 33.9 / 26.9; 8192 x 4096 33.5 / 25.7; 12288 x 2560 37.8 / 28.4; 16384 x 1024 26.5 / 22.5, 16384 x 2048 40.2 / 32.3
-// The sibling formats' decoders are longer (Q8_0; Q3 alike or better); above 128 tokens they share the lines of Q4:
+// The sibling formats' decoders are longer (Q8_0; Q3 alike or better); above 128 tokens they have two thirds of the K of Q4's
+// lines, and not the tallest matrices (at 192 4096 x 4096 24.3 / 24.5, at 256 2048 x 4096 20.2 / 16.3, 3072 x 3072 19.5 / 21.4, 6144 x 1024 14.4 / 15.4, at
+// 384 2048 x 2048 19.3 / 17.6, 2048 x 3072 18.6 / 22.3, 4096 x 1024 13.9 / 16.3, at 768 1024 x 1024 16.9 / 13.9, 1024 x 2048 18.1 / 20.5):
 //   33..64: 4096 x 12288 30.6 / 24.4; 8192 x 8192 30.5 / 24.6; 12288 x 2048 18.2 / 16.6, 12288 x 3072 21.7 / 21.9; 16384 x 2048 22.7 / 17.6
 //   65..128: 512 x 17408 23.4 / 18.9; 2048 x 8192 20.6 / 19.1, 2048 x 10240 22.0 / 21.8; 4096 x 6144 21.8 / 19.4; 8192 x 2048 20.1 / 15.8, 8192 x 3072 21.4 / 21.8
 namespace {
@@ -914,9 +916,9 @@ constexpr ShapeLimit kLora128[] = {{1024, 0, 17408}, {4096, 0, 10240}, {8192, 0,
 constexpr ShapeLimit kSibling64[] = {{4096, 0, 12288}, {8192, 0, 8192}, {12288, 0, 2560}, {16384, 512, 2048}};
 constexpr ShapeLimit kSibling128[] = {{512, 0, 17408}, {2048, 0, 8192}, {4096, 0, 6144}, {8192, 0, 2560}};
 template <size_t N>
-bool within(const ShapeLimit (&limits)[N], uint32_t n, uint32_t k) {
+bool within(const ShapeLimit (&limits)[N], uint32_t n, uint32_t k, bool narrowed = false) {
     for (const ShapeLimit& l : limits)
-        if (n <= l.n) return k >= l.k_min && k <= l.k_max;
+        if (n <= l.n) return narrowed ? l.k_min == 0 && k + k / 2 <= l.k_max : k >= l.k_min && k <= l.k_max;
     return false;
 }
 }  // namespace
@@ -931,9 +933,9 @@ bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lo
         return m <= 64 ? within(kPlain64, n, k) : within(kPlain128, n, k);
     }
     if (with_lora) return false;
-    if (m <= 256) return m <= 192 ? within(kPlain192, n, k) : within(kPlain256, n, k);
-    if (m <= 512) return m <= 384 ? within(kPlain384, n, k) : within(kPlain512, n, k);
-    if (m <= 1024) return m <= 768 ? within(kPlain768, n, k) : within(kPlain1024, n, k);
+    if (m <= 256) return m <= 192 ? within(kPlain192, n, k, fmt) : within(kPlain256, n, k, fmt);
+    if (m <= 512) return m <= 384 ? within(kPlain384, n, k, fmt) : within(kPlain512, n, k, fmt);
+    if (m <= 1024) return m <= 768 ? within(kPlain768, n, k, fmt) : within(kPlain1024, n, k, fmt);
     return false;
 }
 
