@@ -92,8 +92,10 @@ int fail(int code, const char* fmt, ...) {
         if (e_ != hipSuccess) return fail(LQ4_E_HIP, "%s: %s", #call, hipGetErrorString(e_)); \
     } while (0)
 
+thread_local int t_device = -1;  // the device of the innermost DeviceGuard
+
 struct DeviceGuard {
-    int prev = -1, dev;
+    int prev = -1, dev, outer = t_device;
     bool ok = true;
     explicit DeviceGuard(int d) : dev(d) {
         if (hipGetDevice(&prev) != hipSuccess) prev = -1;
@@ -101,8 +103,10 @@ struct DeviceGuard {
         // An error some earlier, unrelated runtime call left behind in this thread must not be
         // reported by the launch check of this entry point.
         if (ok) (void)hipGetLastError();
+        t_device = ok ? dev : -1;
     }
     ~DeviceGuard() {
+        t_device = outer;
         if (prev >= 0 && prev != dev) (void)hipSetDevice(prev);
     }
 };
@@ -172,6 +176,42 @@ int resolve_lora(const lq4_ctx* ctx, const lq4_lora* l, float scale, uint32_t n,
 }
 
 }  // namespace
+
+namespace lq4 {
+
+hipFunction_t kernel_handle(const void* kernel) {
+    // (fixed size, no lock: an entry is claimed once for its kernel, a handle is written once per device; whoever comes
+    // first writes what everyone would)
+    constexpr uint32_t kEntries = 2048, kProbes = 32;
+    constexpr int kDevices = 8;
+    struct Entry {
+        std::atomic<const void*> kernel;
+        std::atomic<hipFunction_t> handle[kDevices];
+    };
+    static Entry table[kEntries];
+    int device = t_device;
+    if (device < 0 && hipGetDevice(&device) != hipSuccess) return nullptr;
+    hipFunction_t f = nullptr;
+    if (device < kDevices) {
+        const uint32_t at = static_cast<uint32_t>((reinterpret_cast<uintptr_t>(kernel) * 0x9E3779B97F4A7C15ull) >> 53);
+        for (uint32_t i = 0; i < kProbes; ++i) {
+            Entry& e = table[(at + i) % kEntries];
+            const void* have = e.kernel.load(std::memory_order_relaxed);
+            if (!have && e.kernel.compare_exchange_strong(have, kernel, std::memory_order_relaxed)) have = kernel;
+            if (have != kernel) continue;
+            f = e.handle[device].load(std::memory_order_acquire);
+            if (f) return f;
+            if (hipGetFuncBySymbol(&f, kernel) != hipSuccess) break;
+            e.handle[device].store(f, std::memory_order_release);
+            return f;
+        }
+    }
+    if (hipGetFuncBySymbol(&f, kernel) == hipSuccess) return f;
+    (void)hipGetLastError();  // (the launch that follows is what counts)
+    return nullptr;
+}
+
+}  // namespace lq4
 
 extern "C" {
 

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void moe_shared_gate_add_kernel(const float* _
 
 void launch_moe_shared_gate_add(const float* x, const float* gate, const float* shared_out, uint32_t hidden,
                                 uint32_t tokens, float* y, hipStream_t stream) {
-    hipLaunchKernelGGL(moe_shared_gate_add_kernel, dim3(tokens), dim3(256), 0, stream, x, gate, shared_out, hidden, y);
+    launch_kernel(moe_shared_gate_add_kernel, dim3(tokens), dim3(256), 0, stream, x, gate, shared_out, hidden, y);
 }
 
 void launch_residual_add_norm(const float* base, const float* delta, const float* gamma, uint32_t hidden,
@@ -140,24 +140,24 @@ void launch_residual_add_norm(const float* base, const float* delta, const float
     const auto aligned = [](const void* p) { return p == nullptr || reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     if (hidden % 4 == 0 && aligned(base) && aligned(delta) && aligned(gamma) && aligned(residual_out) &&
         aligned(normed_out)) {
-        hipLaunchKernelGGL(residual_add_norm_vec_kernel, dim3(rows), dim3(256), 0, stream,
+        launch_kernel(residual_add_norm_vec_kernel, dim3(rows), dim3(256), 0, stream,
                            reinterpret_cast<const float4*>(base), reinterpret_cast<const float4*>(delta),
                            reinterpret_cast<const float4*>(gamma), hidden / 4, static_cast<float>(hidden), eps,
                            reinterpret_cast<float4*>(residual_out), reinterpret_cast<float4*>(normed_out));
         return;
     }
-    hipLaunchKernelGGL(residual_add_norm_kernel, dim3(rows), dim3(256), 0, stream, base, delta, gamma, hidden, eps,
+    launch_kernel(residual_add_norm_kernel, dim3(rows), dim3(256), 0, stream, base, delta, gamma, hidden, eps,
                        residual_out, normed_out);
 }
 
 void launch_silu_mul(const float* gate_up, uint32_t count, uint32_t rows, float* out, uint32_t out_stride,
                      hipStream_t stream) {
-    hipLaunchKernelGGL(silu_mul_kernel, dim3((count + 255) / 256, rows), dim3(256), 0, stream, gate_up, count, out,
+    launch_kernel(silu_mul_kernel, dim3((count + 255) / 256, rows), dim3(256), 0, stream, gate_up, count, out,
                        out_stride);
 }
 
 void launch_add_and_copy(const float* src, float* residual, float* dst, size_t count, hipStream_t stream) {
-    hipLaunchKernelGGL(add_and_copy_kernel, dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0, stream, src,
+    launch_kernel(add_and_copy_kernel, dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0, stream, src,
                        residual, dst, count);
 }
 

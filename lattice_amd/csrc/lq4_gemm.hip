@@ -493,10 +493,10 @@ void launch_tile(const uint8_t* w, uint32_t n, uint32_t k, const void* x, uint32
     const size_t lds = 2 * (BM + BN_) * kPitch * sizeof(_Float16);
     static LdsCapOnce lds_cap;
     lds_cap.raise(reinterpret_cast<const void*>(gemm_q4_mfma<X_F16, BN_, LORA, FMT>), 160 * 1024);
-    hipLaunchKernelGGL((gemm_q4_mfma<X_F16, BN_, LORA, FMT>), dim3(tiles * ts.count), dim3(2 * BN_), lds, stream, w, n,
+    launch_kernel((gemm_q4_mfma<X_F16, BN_, LORA, FMT>), dim3(tiles * ts.count), dim3(2 * BN_), lds, stream, w, n,
                        k, x, m, y, lora, slices);
     if (ts.count > 1)
-        hipLaunchKernelGGL((gemm_sum_slices<BN_>), dim3(tiles, BM * BN_ / 1024), dim3(256), 0, stream, partial, ts.count,
+        launch_kernel((gemm_sum_slices<BN_>), dim3(tiles, BM * BN_ / 1024), dim3(256), 0, stream, partial, ts.count,
                            m, n, y);
 }
 

@@ -808,7 +808,7 @@ void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint3
             auto go = [&](auto lora_c) {
                 constexpr auto kernel = gemm_q4_skinny<RT, FMT, NTG, kMulti, decltype(lora_c)::value>;
                 raise_lds<kernel>(lds);
-                hipLaunchKernelGGL(kernel, grid, block, lds, stream, w, n, k, xp, m, y, lora, views_arg);
+                launch_kernel(kernel, grid, block, lds, stream, w, n, k, xp, m, y, lora, views_arg);
             };
             if (!with_lora) go(std::integral_constant<int, 0>{});
             else if (lora_form(k) == 1) go(std::integral_constant<int, 1>{});
@@ -827,7 +827,7 @@ void launch_ntg(const uint8_t* w, uint32_t n, uint32_t k, const uint4* xp, uint3
     } else {
         constexpr auto kernel = gemm_q4_skinny<RT, FMT, NTG, false, 0>;
         raise_lds<kernel>(lds);
-        hipLaunchKernelGGL(kernel, dim3((n + 16 * RT - 1) / (16 * RT), token_tiles), block, lds,
+        launch_kernel(kernel, dim3((n + 16 * RT - 1) / (16 * RT), token_tiles), block, lds,
                            stream, w, n, k, xp, m, y, lora, NoViews{});
     }
 }
@@ -969,7 +969,7 @@ void launch_pack_lora_form(const void* x, int x_is_f16, uint32_t m, uint32_t k, 
                            uint32_t groups, const PackLora& la, hipStream_t stream) {
     const dim3 grid(slices, groups, (la.count + NV - 1) / NV);
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(64 * WAVES), 0, stream, x, m, k, xp, steps, slices, groups, la);
+        launch_kernel(kernel, grid, dim3(64 * WAVES), 0, stream, x, m, k, xp, steps, slices, groups, la);
     };
     if constexpr (NV * WAVES < 64) {  // (four f32 adapters and sixteen waves: not enough registers, launch_pack_lora)
         if (la.has_rest) return x_is_f16 ? launch(pack_x_lora_kernel<true, NV, true, J, WAVES>) : launch(pack_x_lora_kernel<false, NV, true, J, WAVES>);
@@ -1024,8 +1024,8 @@ void launch_fmt(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_i
         launch_pack_lora(x, x_is_f16, m, k, xp, steps, groups, la, stream);
     } else {
         const dim3 grid(steps, groups), block(256);
-        if (x_is_f16) hipLaunchKernelGGL((pack_x_kernel<true, kInterleave>), grid, block, 0, stream, x, m, k, xp);
-        else hipLaunchKernelGGL((pack_x_kernel<false, kInterleave>), grid, block, 0, stream, x, m, k, xp);
+        if (x_is_f16) launch_kernel((pack_x_kernel<true, kInterleave>), grid, block, 0, stream, x, m, k, xp);
+        else launch_kernel((pack_x_kernel<false, kInterleave>), grid, block, 0, stream, x, m, k, xp);
     }
     // Every workgroup reads the whole packed X of its token tile, so a wider row tile halves that traffic, at the price of
     // fewer workgroups to balance over the compute units.

@@ -1025,7 +1025,7 @@ void launch_wreg_tile(const uint8_t* w, uint32_t n, uint32_t k, const void* x, u
     const size_t lds = 2 * 16 * NT * kPitch16 * sizeof(uint4);
     const WregPlan plan{hp.full, hp.slices, partial, group_tiles((m + 16 * NT - 1) / (16 * NT), hp.tiles, k, X_F16)};
     const uint32_t wgs = hp.full + (hp.tiles - hp.full) * hp.slices;
-    hipLaunchKernelGGL((gemm_q4_wreg<X_F16, LORA, FMT, NT, NU>), dim3(wgs), dim3(256), lds, stream, w, n, k, x, m, y, lora,
+    launch_kernel((gemm_q4_wreg<X_F16, LORA, FMT, NT, NU>), dim3(wgs), dim3(256), lds, stream, w, n, k, x, m, y, lora,
                        plan);
 }
 
@@ -1070,7 +1070,7 @@ void launch_gemm_wreg(const uint8_t* w, uint32_t n, uint32_t k, const void* x, i
         }
     }
     if (hp.slices > 1)
-        hipLaunchKernelGGL(gemm_reduce_tail, dim3(hp.tiles - hp.full, hp.nt * hp.nu), dim3(256), 0, stream, partial,
+        launch_kernel(gemm_reduce_tail, dim3(hp.tiles - hp.full, hp.nt * hp.nu), dim3(256), 0, stream, partial,
                            hp.full, hp.slices, m, n, y, lora, 16 * hp.nt, 64 * hp.nu,
                            group_tiles((m + 16 * hp.nt - 1) / (16 * hp.nt), hp.tiles, k, x_is_f16 != 0));
 }
@@ -1097,16 +1097,16 @@ void launch_gemm_w2(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int
     uint4* packed = reinterpret_cast<uint4*>(scratch);
     float* partial = reinterpret_cast<float*>(scratch + w2_packed_bytes(k, m));
     const uint64_t units = w2_packed_bytes(k, m) / 16;
-    hipLaunchKernelGGL(pack_x_tiles_kernel, dim3(static_cast<uint32_t>((units + 255) / 256)), dim3(256), 0, stream, x,
+    launch_kernel(pack_x_tiles_kernel, dim3(static_cast<uint32_t>((units + 255) / 256)), dim3(256), 0, stream, x,
                        x_is_f16, m, k, kc_pad, packed, units);
     static LdsCapOnce lds_cap;
     lds_cap.raise(reinterpret_cast<const void*>(gemm_q4_w2), 64 * 1024);
     const size_t lds = 2 * kStepUnits * sizeof(uint4);
     const WregPlan plan{hp.full, hp.slices, partial, group_tiles((m + TM - 1) / TM, hp.tiles, k, true)};
     const uint32_t wgs = hp.full + (hp.tiles - hp.full) * hp.slices;
-    hipLaunchKernelGGL(gemm_q4_w2, dim3(wgs), dim3(256), lds, stream, w, n, k, packed, kc_pad, m, y, plan);
+    launch_kernel(gemm_q4_w2, dim3(wgs), dim3(256), lds, stream, w, n, k, packed, kc_pad, m, y, plan);
     if (hp.slices > 1)
-        hipLaunchKernelGGL(gemm_reduce_tail, dim3(hp.tiles - hp.full, TM * TN / 1024), dim3(256), 0, stream, partial,
+        launch_kernel(gemm_reduce_tail, dim3(hp.tiles - hp.full, TM * TN / 1024), dim3(256), 0, stream, partial,
                            hp.full, hp.slices, m, n, y, lora, static_cast<uint32_t>(TM), static_cast<uint32_t>(TN),
                            plan.group);
 }

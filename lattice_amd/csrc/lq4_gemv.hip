@@ -227,13 +227,13 @@ void launch_gemv(const uint8_t* w, uint32_t n, uint32_t k, const float* x, uint3
         LoraEpilogue l = lora;
         if (l.rank) l.t = lora.t + static_cast<size_t>(b0) * lora.rank;
         if (nb == 1)
-            hipLaunchKernelGGL(gemv_q4_rows<1>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
+            launch_kernel(gemv_q4_rows<1>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
         else if (nb == 2)
-            hipLaunchKernelGGL(gemv_q4_rows<2>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
+            launch_kernel(gemv_q4_rows<2>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
         else if (nb <= 4)
-            hipLaunchKernelGGL(gemv_q4_rows<4>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
+            launch_kernel(gemv_q4_rows<4>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
         else
-            hipLaunchKernelGGL(gemv_q4_rows<8>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
+            launch_kernel(gemv_q4_rows<8>, grid, block, 0, stream, w, n, k, xb, x_stride, nb, yb, y_stride, l);
     }
 }
 
@@ -267,22 +267,22 @@ void launch_lora_a(const void* a, int a_is_f16, uint32_t rank, uint32_t d_in, co
                    int x_is_f16, uint32_t x_stride, uint32_t rows, float* t, hipStream_t stream) {
     const dim3 grid(rank, rows), block(256);
     if (a_is_f16 && x_is_f16)
-        hipLaunchKernelGGL((lora_a_kernel<_Float16, _Float16>), grid, block, 0, stream,
+        launch_kernel((lora_a_kernel<_Float16, _Float16>), grid, block, 0, stream,
                            static_cast<const _Float16*>(a), rank, d_in, static_cast<const _Float16*>(x), x_stride, t);
     else if (a_is_f16)
-        hipLaunchKernelGGL((lora_a_kernel<_Float16, float>), grid, block, 0, stream,
+        launch_kernel((lora_a_kernel<_Float16, float>), grid, block, 0, stream,
                            static_cast<const _Float16*>(a), rank, d_in, static_cast<const float*>(x), x_stride, t);
     else if (x_is_f16)
-        hipLaunchKernelGGL((lora_a_kernel<float, _Float16>), grid, block, 0, stream,
+        launch_kernel((lora_a_kernel<float, _Float16>), grid, block, 0, stream,
                            static_cast<const float*>(a), rank, d_in, static_cast<const _Float16*>(x), x_stride, t);
     else
-        hipLaunchKernelGGL((lora_a_kernel<float, float>), grid, block, 0, stream,
+        launch_kernel((lora_a_kernel<float, float>), grid, block, 0, stream,
                            static_cast<const float*>(a), rank, d_in, static_cast<const float*>(x), x_stride, t);
 }
 
 void launch_lora_b_accum(const void* b, int b_is_f16, uint32_t rank, uint32_t d_out, const float* t,
                          float scale, uint32_t rows, float* y, uint32_t y_stride, hipStream_t stream) {
-    hipLaunchKernelGGL(lora_b_accum_kernel, dim3((d_out + 255) / 256, rows), dim3(256), 0, stream, b,
+    launch_kernel(lora_b_accum_kernel, dim3((d_out + 255) / 256, rows), dim3(256), 0, stream, b,
                        b_is_f16, rank, d_out, t, scale, y, y_stride);
 }
 
@@ -297,10 +297,10 @@ bool launch_probe_read(const void* p, size_t nbytes, uint32_t grid, uint32_t in_
     const probe_u32x4* q = static_cast<const probe_u32x4*>(p);
 #define LQ4_PROBE(D_) \
     do { \
-        if (strided && nontemporal) hipLaunchKernelGGL((probe_read_kernel<D_, true, true>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
-        else if (strided) hipLaunchKernelGGL((probe_read_kernel<D_, false, true>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
-        else if (nontemporal) hipLaunchKernelGGL((probe_read_kernel<D_, true, false>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
-        else hipLaunchKernelGGL((probe_read_kernel<D_, false, false>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
+        if (strided && nontemporal) launch_kernel((probe_read_kernel<D_, true, true>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
+        else if (strided) launch_kernel((probe_read_kernel<D_, false, true>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
+        else if (nontemporal) launch_kernel((probe_read_kernel<D_, true, false>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
+        else launch_kernel((probe_read_kernel<D_, false, false>), dim3(grid), dim3(256), 0, stream, q, n16, sink); \
     } while (0)
     switch (in_flight) {
         case 64: LQ4_PROBE(4); break;
@@ -316,14 +316,14 @@ void launch_probe_copy(const void* src, void* dst, size_t nbytes, hipStream_t st
     const size_t n16 = nbytes / 16;
     uint32_t grid = static_cast<uint32_t>((n16 + 255) / 256);
     grid = grid > 4096 ? 4096 : grid < 1 ? 1 : grid;
-    hipLaunchKernelGGL(probe_copy_kernel, dim3(grid), dim3(256), 0, stream, static_cast<const uint4*>(src),
+    launch_kernel(probe_copy_kernel, dim3(grid), dim3(256), 0, stream, static_cast<const uint4*>(src),
                        static_cast<uint4*>(dst), n16);
 }
 
 void launch_dequant(const uint8_t* w, uint32_t n, uint32_t k, float* out, hipStream_t stream) {
     const uint64_t n_blocks = static_cast<uint64_t>(n) * (k / kBlockWeights);
     const uint64_t threads = n_blocks * 16;
-    hipLaunchKernelGGL(dequant_kernel, dim3(static_cast<uint32_t>((threads + 255) / 256)), dim3(256), 0,
+    launch_kernel(dequant_kernel, dim3(static_cast<uint32_t>((threads + 255) / 256)), dim3(256), 0,
                        stream, w, n_blocks, out);
 }
 

@@ -14,34 +14,34 @@ void launch_cfg(const uint8_t* w, uint32_t n, uint32_t k, const float* x, float*
         if (fusion && fusion->epilogue == GemvFusion::kSiluMulPairs) {
             static LdsCapOnce cap_pairs;
             cap_pairs.raise(reinterpret_cast<const void*>(gemv_q4_b1<RW, SG, SEG, kFusedPairsMode, WAVES>), 159 * 1024);
-            hipLaunchKernelGGL((gemv_q4_b1<RW, SG, SEG, kFusedPairsMode, WAVES>), grid, block, lds, stream, w, n, k, x, y,
+            launch_kernel((gemv_q4_b1<RW, SG, SEG, kFusedPairsMode, WAVES>), grid, block, lds, stream, w, n, k, x, y,
                                lora, *fusion);
             return;
         }
     }
     if (fusion) {
         cap[1].raise(reinterpret_cast<const void*>(gemv_q4_b1<RW, SG, SEG, kFusedMode, WAVES>), 159 * 1024);
-        hipLaunchKernelGGL((gemv_q4_b1<RW, SG, SEG, kFusedMode, WAVES>), grid, block, lds, stream, w, n, k, x, y, lora,
+        launch_kernel((gemv_q4_b1<RW, SG, SEG, kFusedMode, WAVES>), grid, block, lds, stream, w, n, k, x, y, lora,
                            *fusion);
         return;
     }
     if (lora.rank && lora.a) {
         cap[2].raise(reinterpret_cast<const void*>(gemv_q4_b1<RW, SG, SEG, kLoraAMode, WAVES>), 160 * 1024);
         const dim3 grid_a(grid.x + lora.rank);  // the rank producer workgroups come first
-        hipLaunchKernelGGL((gemv_q4_b1<RW, SG, SEG, kLoraAMode, WAVES>), grid_a, block, lds, stream, w, n, k, x, y,
+        launch_kernel((gemv_q4_b1<RW, SG, SEG, kLoraAMode, WAVES>), grid_a, block, lds, stream, w, n, k, x, y,
                            lora, NoFusion{});
         return;
     }
     if constexpr (RW > 1) {  // (one row per chunk: both row orders are the same)
         if (persistent) {
             cap[3].raise(reinterpret_cast<const void*>(gemv_q4_b1<RW, SG, SEG, kPlainAdjMode, WAVES>), 160 * 1024);
-            hipLaunchKernelGGL((gemv_q4_b1<RW, SG, SEG, kPlainAdjMode, WAVES>), grid, block, lds, stream, w, n, k, x, y,
+            launch_kernel((gemv_q4_b1<RW, SG, SEG, kPlainAdjMode, WAVES>), grid, block, lds, stream, w, n, k, x, y,
                                lora, NoFusion{});
             return;
         }
     }
     cap[0].raise(reinterpret_cast<const void*>(gemv_q4_b1<RW, SG, SEG, kPlainMode, WAVES>), 160 * 1024);
-    hipLaunchKernelGGL((gemv_q4_b1<RW, SG, SEG, kPlainMode, WAVES>), grid, block, lds, stream, w, n, k, x, y, lora,
+    launch_kernel((gemv_q4_b1<RW, SG, SEG, kPlainMode, WAVES>), grid, block, lds, stream, w, n, k, x, y, lora,
                        NoFusion{});
 }
 

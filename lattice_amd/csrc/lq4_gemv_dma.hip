@@ -504,7 +504,7 @@ void launch_rows(const DmaPlan& p, const uint8_t* w, uint32_t n, uint32_t k, con
     static LdsCapOnce lds_cap;
     lds_cap.raise(reinterpret_cast<const void*>(gemv_q4_dma_rows<D, SLABS>), 160 * 1024);
     const size_t lds = p.lds < 96 * 1024 ? 96 * 1024 : p.lds;  // one workgroup to a CU
-    hipLaunchKernelGGL((gemv_q4_dma_rows<D, SLABS>), dim3(p.grid), dim3(kWaves * 64), lds, stream, w, n, k, x, y);
+    launch_kernel((gemv_q4_dma_rows<D, SLABS>), dim3(p.grid), dim3(kWaves * 64), lds, stream, w, n, k, x, y);
 }
 
 template <int XR, int D>
@@ -513,7 +513,7 @@ void launch_one(const DmaPlan& p, const uint8_t* w, uint32_t n, uint32_t k, cons
     lds_cap.raise(reinterpret_cast<const void*>(gemv_q4_dma<XR, D>), 160 * 1024);
     // at least half a CU's LDS, so that the workgroups spread one to a CU
     const size_t lds = p.lds < 96 * 1024 ? 96 * 1024 : p.lds;
-    hipLaunchKernelGGL((gemv_q4_dma<XR, D>), dim3(p.grid), dim3(kWaves * 64), lds, stream, w, n, k, x, y);
+    launch_kernel((gemv_q4_dma<XR, D>), dim3(p.grid), dim3(kWaves * 64), lds, stream, w, n, k, x, y);
 }
 
 }  // namespace

@@ -608,7 +608,7 @@ void launch_i8(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, const 
     static LdsCapOnce lds_cap;
     lds_cap.raise(reinterpret_cast<const void*>(gemv_q4_i8<CW, TW, WIDE, MULTI>), 160 * 1024);
     const uint32_t producers = lora.slots ? lora.rank : 0;
-    hipLaunchKernelGGL((gemv_q4_i8<CW, TW, WIDE, MULTI>), dim3(producers + p.grid), dim3(64 * CW * TW), p.lds, stream, w, n,
+    launch_kernel((gemv_q4_i8<CW, TW, WIDE, MULTI>), dim3(producers + p.grid), dim3(64 * CW * TW), p.lds, stream, w, n,
                        k, x, x_stride, batch, y, y_stride, lora, mv);
 }
 

