@@ -908,7 +908,7 @@ constexpr ShapeLimit kPlain128[] = {{1024, 0, 17408}, {2048, 0, 14336}, {4096, 0
 constexpr ShapeLimit kPlain192[] = {{512, 0, 14336}, {1024, 0, 10240}, {2048, 0, 6144}, {4096, 0, 4096}, {6144, 0, 3072}, {8192, 1024, 2048}};
 constexpr ShapeLimit kPlain256[] = {{1024, 0, 10240}, {2048, 0, 6144}, {3072, 0, 4096}, {4096, 0, 3072}, {6144, 1024, 2048}};
 constexpr ShapeLimit kPlain384[] = {{512, 0, 8192}, {1024, 0, 4096}, {2048, 0, 3072}, {3072, 0, 2048}, {4096, 1024, 2048}};
-constexpr ShapeLimit kPlain512[] = {{512, 0, 6144}, {1024, 0, 4096}, {2048, 0, 2048}, {3072, 1024, 2048}};
+constexpr ShapeLimit kPlain512[] = {{512, 0, 6144}, {1024, 0, 4096}, {2048, 512, 2048}, {3072, 1024, 2048}};
 constexpr ShapeLimit kPlain768[] = {{256, 0, 4096}, {512, 0, 3072}, {1024, 0, 2048}};
 constexpr ShapeLimit kPlain1024[] = {{256, 0, 3072}, {512, 0, 2048}, {1024, 768, 1536}};
 constexpr ShapeLimit kLora64[] = {{4096, 0, 17408}, {8192, 0, 14336}, {12288, 0, 6144}, {16384, 0, 5120}, {24576, 0, 2560}};
@@ -918,7 +918,7 @@ constexpr ShapeLimit kSibling128[] = {{512, 0, 17408}, {2048, 0, 8192}, {4096, 0
 template <size_t N>
 bool within(const ShapeLimit (&limits)[N], uint32_t n, uint32_t k, bool narrowed = false) {
     for (const ShapeLimit& l : limits)
-        if (n <= l.n) return narrowed ? l.k_min == 0 && k + k / 2 <= l.k_max : k >= l.k_min && k <= l.k_max;
+        if (n <= l.n) return narrowed ? l.k_min <= 512 && k >= l.k_min && k + k / 2 <= l.k_max : k >= l.k_min && k <= l.k_max;
     return false;
 }
 }  // namespace
@@ -932,7 +932,8 @@ bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lo
         if (with_lora) return m <= 64 ? within(kLora64, n, k) : within(kLora128, n, k);
         return m <= 64 ? within(kPlain64, n, k) : within(kPlain128, n, k);
     }
-    if (with_lora) return false;
+    // (shorter rows: a launch of one to three steps of the large tiles is as long as the two here.  256 x 1000 x 128 6.0 / 6.5, x 256 6.9 / 6.5)
+    if (with_lora || k < 256) return false;
     if (m <= 256) return m <= 192 ? within(kPlain192, n, k, fmt) : within(kPlain256, n, k, fmt);
     if (m <= 512) return m <= 384 ? within(kPlain384, n, k, fmt) : within(kPlain512, n, k, fmt);
     if (m <= 1024) return m <= 768 ? within(kPlain768, n, k, fmt) : within(kPlain1024, n, k, fmt);
