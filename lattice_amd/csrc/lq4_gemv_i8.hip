@@ -14,28 +14,33 @@
 //     of activation rows 2 (l / 16) and 2 (l / 16) + 1 (wide: the three digits of row l / 16).  256 hi + lo is one
 //     integer multiply-add, and
 //       y[b, n] += (scale_n * xs_b) * (256 hi + lo) + bias_n * (xs_b * sum of the block's fixed-point x)
-//     needs the block header of the lane's own row only: no value crosses lanes after the instruction, and every
-//     lane owns two outputs of its row from the first block to the last.
-// Per instruction (16 rows x 32 weights = 320 bytes of weights): 3 operations to spread the nibbles, 2 to convert the
-// header, 10 for the two outputs.  Four SIMDs at that rate consume weights several times faster than memory
-// delivers them, which the 4x4x4 f16 kernel (eight instructions and their operand shuffles per block of four rows)
-// does not.
+//     needs the block header of the lane's own row only, and every lane owns two outputs of its row from the first block to
+//     the last.  The bias terms of four blocks are one v_mfma_f32_16x16x4_f32 (sums x biases, K = the four blocks): lane group
+//     g reads the header of the g-th of the four blocks, its bias is that instruction's operand as it stands, and the scales
+//     reach the other groups by three lane swaps.  The xs of a chunk's eight blocks lie one a lane, each row of sixteen lanes
+//     holding those of its two activation rows, and are broadcast by the multiplication that uses them.
+// Per instruction (16 rows x 32 weights = 320 bytes of weights): 13 vector operations, three to spread the nibbles among them,
+// and 10 bytes a lane from LDS.  (With the header and both rows' xs and sums read for every block it was 23 operations and
+// 32 bytes: 1.2 us a unit of 2.5 KB a wave, 0.4 of them the LDS.)
 //
-// Memory.  A unit is 16 rows x 8 blocks (2.5 KB).  Lane l loads block l % 8 of rows l / 8 and l / 8 + 8 as whole
-// 20-byte blocks (dwordx4 + dword, 160 contiguous bytes per row), keeps four units in flight in registers, and
-// passes the blocks through a wave-private LDS tile to reach the operand layout (row pitch 44 dwords: the 16 rows
-// x 4 dwords a read touches fall into 64 different banks).  Nothing is fetched twice; no barrier: a wave's LDS
-// accesses are carried out in order.
+// Memory.  A unit is 16 rows x 8 blocks (2.5 KB): 160 pieces of 16 bytes, which the load unit puts into the wave's own part of
+// LDS, up to four units ahead, so that a workgroup's share of the matrix is on its way while the activations are staged.
+// (Each lane with blocks of its own, 160 contiguous bytes a row, was four times the address work, one unit ahead, and a
+// rewrite into LDS.)  No barrier: what a wave multiplies it has brought itself.
 //
-// Work split.  A workgroup takes tiles of 16 rows (tile = blockIdx, then += gridDim); its waves split K in chunks
+// Work split.  One workgroup a CU takes tiles of 16 rows (tile = blockIdx, then += gridDim); its waves split K in chunks
 // of 8 blocks and add their partial sums through LDS in wave order.  Each wave stages the activations of its own
-// chunks only, once for all tiles of the workgroup, behind its first weight loads.
+// chunks only, once for all tiles of the workgroup; with one tile at a time it multiplies nothing else.
+//
+// Where the time goes (12288 x 2048 at eight rows, 8.7 -> 6.9 us; 2048 x 2048 5.5 -> 4.3): 0.6 us until the activations are asked
+// for, 1 until they arrive, 0.8 to stage them, then 0.7 to 1 a round of units and 0.6 for the meeting; the weights have arrived
+// by then.  A launch is a single pass through its code, so the order of the code (activations first) and its length count.
 //
 // LoRA.  The factor t = A . x of the adapter (of every view's adapter) is either in memory when the launch starts
 // (lora.t / mv.t), or computed by the launch itself (lora.slots set): the first lora.rank workgroups are producers,
 // one per row of A (the views' A stacked), each forming that row's dot products with the batch's activation rows
-// and publishing them as {value, tag of the launch} words; the other workgroups pick them up into LDS after their
-// staging barrier, by which time the producers, who have nothing else to do, are long done.  The launcher adds the
+// and publishing them as {value, tag of the launch} words; the other workgroups pick them up into LDS when their first
+// tile is multiplied, by which time the producers, who have nothing else to do, are done.  The launcher adds the
 // producers only where CUs are idle anyway (tiles + producers <= CUs): a matrix of 2560 rows occupies 160.  A value
 // that has not arrived after the poll limit is computed by the wave that misses it, in the producers' order of
 // summation (same bits), and counted in sync[2].
@@ -57,24 +62,100 @@ namespace {
 typedef int int4v __attribute__((ext_vector_type(4)));
 
 constexpr int kBpw = 8;            // blocks per wave chunk
-constexpr int kTilePitch = 44;     // dwords per row of the LDS tile (40 used; 44 r mod 64 differs for every r < 16)
-constexpr int kTileDwords = 16 * kTilePitch;
+constexpr int kStageBytes = 16 * kBpw * kBlockBytes;  // a unit in LDS: 16 rows x 160 bytes, one behind the other
+constexpr int kStageDwords = kStageBytes / 4, kRowDwords = kBpw * kBlockBytes / 4;
+constexpr uint32_t kMaxStages = 4;  // units a wave has in flight
+constexpr uint32_t kMeet = 4;       // rounds of tiles between two meetings of a workgroup's waves
+constexpr size_t kLdsBytes = 160 * 1024;
 constexpr int kXqBytes = 512;      // per block: [4 k groups][16 operand rows] x 8 bytes
 constexpr int kXfBytes = 64;       // per block: [4 lane groups][xs of rows 2g, 2g + 1, then their sums] f32
 
-struct __attribute__((packed, aligned(4))) Q4BlockRaw {
-    uint32_t sb;    // f16 scale | f16 bias << 16
-    uint32_t q[4];  // 32 nibbles, nibble i of dword j = weight 8j + i
-};
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Memory -> LDS, 16 or 4 bytes a lane: lane l's bytes land at LDS byte address `lds` + 16 l (or + 4 l).  `base` and `lds` are
+// wave-uniform.  By hand, like the loads of the activations: the compiler would make every LDS access wait for the former, and
+// count the latter without them.  The compiler knows of no hazard either: a vector load may read a scalar register five wait
+// states after a vector instruction wrote it (v_readlane, where the compiler keeps scalars in a vector register), so each brings
+// its own.
+__device__ __forceinline__ void dma16(uint32_t lds, const void* base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void dma4(uint32_t lds, const void* base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ f32x4 load16(const void* base, uint32_t off) {
+    f32x4 r;
+    asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %1, %2" : "=v"(r) : "v"(off), "s"(base) : "memory");
+    return r;
+}
+// Until at most `units` units (three loads each, or more) are outstanding.
+__device__ __forceinline__ void wait_units(uint32_t units) {
+    if (units == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (units == 1) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+    else if (units == 2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if (units == 3) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
+}
 
 __device__ __forceinline__ float as_f32(uint32_t u) { return __builtin_bit_cast(float, u); }
 __device__ __forceinline__ uint32_t as_u32(float f) { return __builtin_bit_cast(uint32_t, f); }
 
-__device__ __forceinline__ float half_lo(uint32_t sb) {
-    return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(sb & 0xFFFFu)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float f16_lo(uint32_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h & 0xFFFFu))); }
+__device__ __forceinline__ float f16_hi(uint32_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h >> 16))); }
+// Lane N of the lane's row of sixteen.
+template <int N>
+__device__ __forceinline__ float of_row_lane(float v) {
+    return as_f32(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(as_u32(v)), 0x150 + N, 0xF, 0xF, true)));
 }
-__device__ __forceinline__ float half_hi(uint32_t sb) {
-    return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(sb >> 16)));
+// out[i] = v of row i of the wave's four rows of sixteen, in every row.
+__device__ __forceinline__ void rows_apart(float v, float (&out)[4]) {
+    const auto halves = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);
+    const auto lo = __builtin_amdgcn_permlane16_swap(halves[0], halves[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(halves[1], halves[1], false, false);
+    out[0] = as_f32(lo[0]);
+    out[1] = as_f32(lo[1]);
+    out[2] = as_f32(hi[0]);
+    out[3] = as_f32(hi[1]);
+}
+
+// A lane's part of the dot product of row j of A with an activation row: eight values from 512 to 512, four such steps requested at
+// once (one after the other, 2048 weights were four round trips to memory, and the producers the last
+// to be ready: q, k and v of 2048 + 2 x 512 rows at eight rows, rank 16 on two of them, four layers 29.2 us, 22.9 so).
+__device__ __forceinline__ float a_row_dot(const void* a, int a_is_f16, uint32_t j, uint32_t k, const float* __restrict__ x, int lane) {
+    constexpr int kAhead = 4;
+    float p = 0.0f;
+    for (uint32_t k0 = 0; k0 < k; k0 += kAhead * 512) {
+        f32x4 xv[kAhead][2], av[kAhead][2];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const uint32_t kk = k0 + i * 512 + lane * 8, at = kk < k ? kk : 0;
+            const f32x4* xp = reinterpret_cast<const f32x4*>(x + at);
+            xv[i][0] = xp[0];
+            xv[i][1] = xp[1];
+            const size_t ai = static_cast<size_t>(j) * k + at;
+            const f32x4* ap = reinterpret_cast<const f32x4*>(a_is_f16 ? static_cast<const char*>(a) + ai * 2 : static_cast<const char*>(a) + ai * 4);
+            av[i][0] = ap[0];
+            av[i][1] = ap[a_is_f16 ? 0 : 1];
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            if (a_is_f16) {
+                typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+                const half8 h = __builtin_bit_cast(half8, av[i][0]);
+                av[i][0] = f32x4{static_cast<float>(h[0]), static_cast<float>(h[1]), static_cast<float>(h[2]), static_cast<float>(h[3])};
+                av[i][1] = f32x4{static_cast<float>(h[4]), static_cast<float>(h[5]), static_cast<float>(h[6]), static_cast<float>(h[7])};
+            }
+            if (k0 + i * 512 + lane * 8 < k) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) p = fmaf(av[i][e / 4][e % 4], xv[i][e / 4][e % 4], p);
+            }
+        }
+    }
+    return p;
 }
 
 // WIDE: up to four activation rows at three digits; else up to eight at two.
@@ -82,18 +163,20 @@ __device__ __forceinline__ float half_hi(uint32_t sb) {
 // MULTI: the rows are those of several matrices stacked one under the other (MultiViews: view v = rows [begin[v],
 // begin[v + 1]), every view a whole number of 16-row tiles), each with its own output [batch, rows of the view] and its
 // own LoRA factors; w, y, y_stride and lora are then unused.
-template <int CW, int TW, bool WIDE, bool MULTI>
+// LORA: with adapters (on any view).  Four layers of eight rows, which have none, took 142 us with this code in their way, 134
+// without.
+template <int CW, int TW, bool WIDE, bool MULTI, bool LORA>
 __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __restrict__ w, uint32_t n, uint32_t k,
                                                            const float* __restrict__ x, uint32_t x_stride,
                                                            uint32_t batch, float* __restrict__ y, uint32_t y_stride,
-                                                           LoraEpilogue lora, MultiViews mv) {
+                                                           uint32_t stages, LoraEpilogue lora, MultiViews mv) {
     constexpr int WAVES = CW * TW;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // ---- producers of the LoRA factors (see the head of the file): workgroup p < prod owns stacked row p of A ----
-    const uint32_t prod = lora.slots ? lora.rank : 0;  // (several views: lora.rank is the ranks of all views together)
+    const uint32_t prod = LORA && lora.slots ? lora.rank : 0;  // (several views: lora.rank is the ranks of all views together)
     auto a_row_of = [&](uint32_t p, const void*& a, int& a_is_f16, uint32_t& j) {
         a = lora.a;
         a_is_f16 = lora.b_is_f16;
@@ -114,27 +197,143 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
         a_row_of(blockIdx.x, a, a_is_f16, j);
         // a wave per activation row: no barrier, nothing through LDS, one cross-lane sum before the word goes out
         for (uint32_t b = wave; b < batch; b += WAVES) {
-            const float total = wave_sum(lora_a_row_partial(a, a_is_f16, j, k, x + static_cast<size_t>(b) * x_stride, lane, 64));
+            const float total = wave_sum(a_row_dot(a, a_is_f16, j, k, x + static_cast<size_t>(b) * x_stride, lane));
             const unsigned long long word = (static_cast<unsigned long long>(launch_tag()) << 32) | as_u32(total);
             if (lane == 0) __hip_atomic_store(&lora.slots[blockIdx.x * 8 + b], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
     }
     const uint32_t wg = blockIdx.x - prod, n_wg = gridDim.x - prod;  // this workgroup among those that stream weights
-    const uint32_t tw = wave / CW, cw = wave % CW;
+    const uint32_t tw = TW == 1 ? 0 : wave / CW, cw = TW == 1 ? wave : wave % CW;
     const uint32_t nb = k / kBlockWeights;
     const size_t row_bytes = static_cast<size_t>(nb) * kBlockBytes;
-    // LDS: [nb] activation digits | [nb] activation scales and sums | [WAVES] tiles | [WAVES][64][2] partial sums |
-    // [8][64] LoRA factors
+    // LDS: [whole chunks] activation digits | [whole chunks] activation scales and sums | [WAVES][stages] units |
+    // [kMeet][WAVES][64][2] partial sums | [8][64] LoRA factors
+    const uint32_t chunks = (nb + kBpw - 1) / kBpw;
     uint8_t* const xq = smem;
-    uint8_t* const xf = xq + static_cast<size_t>(nb) * kXqBytes;
-    uint32_t* const tile = reinterpret_cast<uint32_t*>(xf + static_cast<size_t>(nb) * kXfBytes) + wave * kTileDwords;
-    float* const part = reinterpret_cast<float*>(xf + static_cast<size_t>(nb) * kXfBytes) + WAVES * kTileDwords;
-    float* const t_lds = part + WAVES * 64 * 2;  // [8 activation rows][kMaxLoraRank]: the factors picked up from the producers
+    uint8_t* const xf = xq + chunks * (kBpw * kXqBytes);
+    uint32_t* const ring = reinterpret_cast<uint32_t*>(xf + chunks * (kBpw * kXfBytes)) + wave * stages * kStageDwords;
+    float* const part = reinterpret_cast<float*>(xf + chunks * (kBpw * kXfBytes)) + WAVES * stages * kStageDwords;
+    float* const t_lds = part + kMeet * WAVES * 64 * 2;  // [8 activation rows][kMaxLoraRank]: the factors picked up from the producers
+
+    const uint32_t my_chunks = cw < chunks ? (chunks - cw + CW - 1) / CW : 0;  // chunk c * CW + cw
+
+    // ---- stage the activations: the waves of column cw (one: TW = 1) its chunks ----
+    // A lane's task: eight values of one activation row, a k group of a block.  64 lanes = four k groups x kRows rows x kTaskBlocks
+    // blocks, so a chunk is kTasks of them, of which wave tw takes tw, tw + TW, ..
+    constexpr uint32_t kRows = WIDE ? 4 : 8;      // activation rows the operand holds
+    constexpr int kTaskBlocks = 16 / kRows, kTasks = kBpw / kTaskBlocks, kMyTasks = kTasks > TW ? kTasks / TW : 1;
+    // q = rint(x / xs) with xs = block maximum / kQScale: |q| stays below kQScale + 2 whatever the rounding of the
+    // reciprocal, every digit within -128..127; wide: 22 bits and sign, what the float trick below can hold
+    constexpr float kQScale = WIDE ? 4194000.0f : 32639.0f;
+    const uint32_t kg = lane & 3, xb = (static_cast<uint32_t>(lane) >> 2) & (kRows - 1), xblk = static_cast<uint32_t>(lane) / (4 * kRows);
+    auto task_block = [&](uint32_t c, int i) { return (c * CW + cw) * kBpw + (tw + i * TW) * kTaskBlocks + xblk; };
+    // rows and blocks that do not exist re-read an existing one
+    const uint32_t x_lane = ((xb < batch ? xb : 0) * x_stride + kg * 8) * 4;
+    auto x_off = [&](uint32_t c, int i) {
+        const uint32_t blk = task_block(c, i);
+        return x_lane + (blk < nb ? blk : nb - 1) * (kBlockWeights * 4);
+    };
+    auto quad_max = [](uint32_t v) {
+        v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, false)));
+        return max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false)));
+    };
+    auto quad_sum = [](int v) {
+        v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
+        return v + __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
+    };
+    auto stage_chunk = [&](uint32_t c, auto xv_of) {
+        float my_xs = 0.0f, my_sum = 0.0f;  // k group i's lane: of the wave's i-th task
+        uint8_t* const dst = xq + task_block(c, 0) * kXqBytes + kg * 128 + (WIDE ? 4 : 2) * xb * 8;
+#pragma unroll
+        for (int i = 0; i < kMyTasks; ++i) {
+            f32x4 xa, xc;
+            xv_of(i, xa, xc);
+            const float v[8] = {xa.x, xa.y, xa.z, xa.w, xc.x, xc.y, xc.z, xc.w};
+            // largest magnitude as a bit pattern: infinities and NaNs come out on top of every finite value
+            uint32_t abits = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) abits = max(abits, as_u32(v[j]) & 0x7FFFFFFFu);
+            abits = quad_max(abits);
+            const bool none = abits < 0x0D800000u || task_block(c, i) >= nb;  // below 2^-100, or past the end of the row: counts for nothing
+            const float xs_any = as_f32(abits) * (1.0f / kQScale), inv_any = __builtin_amdgcn_rcpf(xs_any);
+            const float inv = none ? 0.0f : inv_any;
+            // (an infinite or NaN activation: the row's outputs become NaN)
+            const float xs = none ? 0.0f : abits >= 0x7F800000u ? as_f32(0x7FC00000u) : xs_any;
+            // 1.5 * 2^23 + q as a float has q in its low 23 bits in two's complement: bits = 0x4B400000 + q
+            uint32_t qb[8], sum_bits = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                qb[j] = as_u32(fmaf(v[j], inv, 12582912.0f));
+                sum_bits += qb[j];
+            }
+            const int sum = quad_sum(static_cast<int>(sum_bits - 8u * 0x4B400000u));
+            my_xs = kg == static_cast<uint32_t>(i) ? xs : my_xs;
+            my_sum = kg == static_cast<uint32_t>(i) ? static_cast<float>(sum) : my_sum;
+            // Digits -128..127 from the lowest up: byte 0 of q, byte 1 of q + 0x80, byte 2 of q + 0x8080 (minus the
+            // 0x40 the float's own bits hold there).  Byte p of an operand word pair = element {0, 2, 4, 6, 1, 3, 5,
+            // 7}[p] of the k group: the order in which the two masks lay out a payload dword's nibbles.
+            constexpr int kDigits = WIDE ? 3 : 2;
+            uint32_t dg[kDigits][2];
+            if constexpr (WIDE) {
+#pragma unroll
+                for (int t = 0; t < kDigits; ++t) {
+                    const uint32_t add = t == 0 ? 0u : t == 1 ? 0x80u : 0xFFC08080u;
+                    // byte t of (qb + add) of four elements into one dword: 0x0c selects a zero byte
+                    const uint32_t sel_lo = 0x0c0c0400u + 0x0101u * t, sel_hi = 0x04000c0cu + 0x01010000u * t;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {  // h = 0: elements 0, 2, 4, 6;  h = 1: elements 1, 3, 5, 7
+                        const uint32_t e0 = qb[h] + add, e1 = qb[2 + h] + add, e2 = qb[4 + h] + add, e3 = qb[6 + h] + add;
+                        dg[t][h] = __builtin_amdgcn_perm(e1, e0, sel_lo) | __builtin_amdgcn_perm(e3, e2, sel_hi);
+                    }
+                }
+            } else {
+                typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+                const u16x2 up = {0x80, 0x80};
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {  // (two 16-bit q side by side)
+                    const uint32_t p0 = __builtin_amdgcn_perm(qb[2 + h], qb[h], 0x05040100u), p1 = __builtin_amdgcn_perm(qb[6 + h], qb[4 + h], 0x05040100u);
+                    const uint32_t h0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, p0) + up);
+                    const uint32_t h1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, p1) + up);
+                    dg[0][h] = __builtin_amdgcn_perm(p1, p0, 0x06040200u);
+                    dg[1][h] = __builtin_amdgcn_perm(h1, h0, 0x07050301u);
+                }
+            }
+            // operand row of (b, digit): the highest digit first
+#pragma unroll
+            for (int t = 0; t < kDigits; ++t)
+                *reinterpret_cast<uint2*>(dst + i * (TW * kTaskBlocks * kXqBytes) + (kDigits - 1 - t) * 8) = make_uint2(dg[t][0], dg[t][1]);
+        }
+        if (kg < static_cast<uint32_t>(kMyTasks)) {
+            // of a chunk: [row pair g][2 block + row of the pair] xs (wide: [row][2 block]), then [block][row] xs * sum
+            const uint32_t blk = task_block(c, kg), j = blk % kBpw;
+            float* f = reinterpret_cast<float*>(xf + (blk - j) * kXfBytes);
+            f[WIDE ? 16 * xb + 2 * j : 16 * (xb >> 1) + 2 * j + (xb & 1)] = my_xs;
+            f[64 + 8 * j + xb] = my_xs * my_sum;
+        }
+    };
+
+    // The values of a wave's first chunks are requested before any weight (loads are answered in the order a CU
+    // issued them: behind the weights the staging would wait for these), all at once.
+    const bool stages_rows = tw < kTasks && my_chunks;  // uniform (more tiles side by side than tasks, or more waves than chunks: not all)
+    constexpr int kAhead = 2 * TW;  // chunks
+    // (out of the way of the usual case, whose code then lies together: one chunk a wave with one tile at a time)
+    auto has_chunk = [&](int c) { return c == 0 || (TW == 1 ? __builtin_expect(static_cast<uint32_t>(c) < my_chunks, 0) : static_cast<uint32_t>(c) < my_chunks); };
+    f32x4 xv[kAhead][kMyTasks][2];
+#pragma unroll
+    for (int c = 0; c < kAhead; ++c) {
+        if (has_chunk(c)) {  // uniform
+#pragma unroll
+            for (int i = 0; i < kMyTasks; ++i) {
+                const uint32_t at = x_off(c, i);
+                xv[c][i][0] = load16(x, at);
+                xv[c][i][1] = load16(x, at + 16);
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // nothing below is scheduled above these loads
 
     const uint32_t n_tiles = (n + 15) / 16;
-    const uint32_t chunks = (nb + kBpw - 1) / kBpw;
-    const uint32_t my_chunks = cw < chunks ? (chunks - cw + CW - 1) / CW : 0;  // chunk c * CW + cw
     // tiles of the workgroup: blockIdx + j * gridDim; of this wave: j = tw, tw + TW, ...; a round = TW tiles
     const uint32_t wg_tiles = wg < n_tiles ? (n_tiles - wg + n_wg - 1) / n_wg : 0;
     const uint32_t rounds = (wg_tiles + TW - 1) / TW;
@@ -152,14 +351,13 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
     };
 
     auto r_of = [](int l) { return static_cast<uint32_t>(l & 15); };  // the weight row of the tile a lane's outputs belong to
-    // load mapping: lane = (block jl, row rq), rows rq + kRowStep * i
-    constexpr int kRowStep = 64 / kBpw, kLoads = 16 / kRowStep;
-    const uint32_t jl = lane % kBpw, rq = lane / kBpw;
-    auto load_unit = [&](Q4BlockRaw (&buf)[kLoads], uint32_t u) {
+    // A unit is 160 pieces of 16 bytes, ten a row: lane l brings pieces l, l + 64 and (half the lanes) l + 128.
+    const uint32_t row32 = static_cast<uint32_t>(row_bytes);
+    auto piece_off = [&](uint32_t i) { return i / 10 * row32 + i % 10 * 16; };
+    const uint32_t off0 = piece_off(lane), off1 = piece_off(lane + 64), off2 = piece_off((lane & 31) + 128);
+    auto load_unit = [&](uint32_t u, uint32_t stage) {
         const uint32_t t = u / my_chunks, c = u - t * my_chunks;
         const uint32_t row0 = first_row(t);
-        uint32_t blk = (c * CW + cw) * kBpw + jl;
-        if (blk >= nb) blk = nb - 1;
         const uint8_t* wv = w;
         uint32_t row_base = 0, row_end = n;
         if constexpr (MULTI) {
@@ -168,101 +366,21 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
             row_base = mv.begin[v];
             row_end = mv.begin[v + 1];
         }
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            uint32_t row = row0 + rq + kRowStep * i;
-            if (row >= row_end) row = row_end - 1;
-            row -= row_base;
-            const uint8_t* bp = wv + row * row_bytes + blk * static_cast<uint32_t>(kBlockBytes);
-            // (plain loads: a unit's 160-byte pieces share their cache lines with the neighbouring waves' pieces)
-            buf[i].sb = *reinterpret_cast<const uint32_t*>(bp);
-            typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
-            const u32x4u q = *reinterpret_cast<const u32x4u*>(bp + 4);
-            buf[i].q[0] = q.x; buf[i].q[1] = q.y; buf[i].q[2] = q.z; buf[i].q[3] = q.w;
-        }
-    };
-
-    // ---- stage the activations, all waves together: task = (block, activation row, k group), 8 values each ----
-    // The values of a thread's first tasks are requested before any weight (loads are answered in the order a CU
-    // issued them: behind the weight prefetch the staging would wait for the weights), all at once.
-    constexpr uint32_t kRows = WIDE ? 4 : 8;      // activation rows the operand holds
-    constexpr int kHoist = WAVES >= 16 ? 2 : 4;   // tasks a thread requests ahead (K = 2048 at eight rows: all of them)
-    // q = rint(x / xs) with xs = block maximum / kQScale: |q| stays below kQScale + 2 whatever the rounding of the
-    // reciprocal, every digit within -128..127; wide: 22 bits and sign, what the float trick below can hold
-    constexpr float kQScale = WIDE ? 4194000.0f : 32639.0f;
-    const uint32_t n_tasks = nb * 4 * kRows;
-    auto task_ptr = [&](uint32_t idx) {
-        const uint32_t kg = idx & 3, b = (idx >> 2) & (kRows - 1), blk = idx / (4 * kRows);
-        // rows and blocks that do not exist re-read an existing one; their digits are zeroed below
-        const uint32_t bb = b < batch ? b : 0, bl = blk < nb ? blk : nb - 1;
-        return reinterpret_cast<const float4*>(x + static_cast<size_t>(bb) * x_stride + bl * kBlockWeights + kg * 8);
-    };
-    auto quad_max = [](uint32_t v) {
-        v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, false)));
-        return max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false)));
-    };
-    auto quad_sum = [](int v) {
-        v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
-        return v + __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
-    };
-    auto stage_task = [&](uint32_t idx, const float4 xa, const float4 xb) {
-        const uint32_t kg = idx & 3, b = (idx >> 2) & (kRows - 1), blk = idx / (4 * kRows);
-        const bool live = blk < nb && b < batch;  // (the four lanes of a (block, row) agree)
-        const float v[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-        // largest magnitude as a bit pattern: infinities and NaNs come out on top of every finite value
-        uint32_t abits = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) abits = max(abits, as_u32(v[i]) & 0x7FFFFFFFu);
-        abits = quad_max(live ? abits : 0u);
-        const bool finite = abits < 0x7F800000u;
-        float inv = 0.0f, xs = 0.0f;
-        if (finite && abits >= 0x0D800000u) {  // 2^-100 and up
-            xs = as_f32(abits) * (1.0f / kQScale);
-            inv = __builtin_amdgcn_rcpf(xs);
-        } else if (!finite) {
-            xs = as_f32(0x7FC00000u);  // infinite or NaN activation: the row's outputs become NaN
-        }
-        // 1.5 * 2^23 + q as a float has q in its low 23 bits in two's complement: bits = 0x4B400000 + q
-        uint32_t qb[8], sum_bits = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            qb[i] = as_u32(fmaf(v[i], inv, 12582912.0f));  // (a row that does not exist: inv = 0, digits 0)
-            sum_bits += qb[i];
-        }
-        const int sum = quad_sum(static_cast<int>(sum_bits - 8u * 0x4B400000u));
-        // Digits -128..127 from the lowest up: byte 0 of q, byte 1 of q + 0x80, byte 2 of q + 0x8080 (minus the
-        // 0x40 the float's own bits hold there).  Byte p of an operand word pair = element {0, 2, 4, 6, 1, 3, 5,
-        // 7}[p] of the k group: the order in which the two masks lay out a payload dword's nibbles.
-        constexpr int kDigits = WIDE ? 3 : 2;
-        uint32_t dg[kDigits][2];
-#pragma unroll
-        for (int t = 0; t < kDigits; ++t) {
-            const uint32_t add = t == 0 ? 0u : t == 1 ? 0x80u : 0xFFC08080u;
-            // byte t of (qb + add) of four elements into one dword: 0x0c selects a zero byte
-            const uint32_t sel_lo = 0x0c0c0400u + 0x0101u * t, sel_hi = 0x04000c0cu + 0x01010000u * t;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {  // h = 0: elements 0, 2, 4, 6;  h = 1: elements 1, 3, 5, 7
-                const uint32_t e0 = qb[h] + add, e1 = qb[2 + h] + add, e2 = qb[4 + h] + add, e3 = qb[6 + h] + add;
-                dg[t][h] = __builtin_amdgcn_perm(e1, e0, sel_lo) | __builtin_amdgcn_perm(e3, e2, sel_hi);
-            }
-        }
-        if (blk < nb) {
-            // operand row of (b, digit): the highest digit first
-            uint2* dst = reinterpret_cast<uint2*>(xq + static_cast<size_t>(blk) * kXqBytes + kg * 128 + ((WIDE ? 4 : 2) * b) * 8);
-#pragma unroll
-            for (int t = 0; t < kDigits; ++t) dst[t] = make_uint2(dg[kDigits - 1 - t][0], dg[kDigits - 1 - t][1]);
-            if (WIDE) dst[3] = make_uint2(0u, 0u);
-            if (kg == 0) {
-                // per lane group g of the product: {xs, xs} then {sum, sum} of rows 2g, 2g + 1; wide: {xs, sum} of row g
-                float* f = reinterpret_cast<float*>(xf + static_cast<size_t>(blk) * kXfBytes);
-                const float sx = xs * static_cast<float>(sum);
-                if (WIDE) {
-                    f[4 * b] = xs;
-                    f[4 * b + 1] = sx;
-                } else {
-                    f[4 * (b >> 1) + (b & 1)] = xs;
-                    f[4 * (b >> 1) + 2 + (b & 1)] = sx;
-                }
+        const uint32_t at = (c * CW + cw) * (kBpw * kBlockBytes);  // of the chunk in a row
+        const uint8_t* const base = wv + (row0 - row_base) * row_bytes + at;
+        const uint32_t to = lds_address(ring + stage * kStageDwords);
+        const uint32_t rows = row_end - row0;  // of the tile and behind it
+        if (__builtin_expect(rows >= 16 && rows * row_bytes >= 15 * row_bytes + at + kBpw * kBlockBytes, 1)) {  // uniform
+            dma16(to, base, off0);
+            dma16(to + 1024, base, off1);
+            if (lane < 32) dma16(to + 2048, base, off2);
+        } else {
+            // the matrix ends inside the unit: dword by dword, rows and bytes past the end read the last ones
+            const uint32_t last = rows * row32 - at - 4;
+#pragma unroll 1
+            for (int i = 0; i < kStageDwords / 64; ++i) {
+                const uint32_t e = i * 64 + lane, r = e / kRowDwords, off = (r < rows ? r : rows - 1) * row32 + e % kRowDwords * 4;
+                dma4(to + i * 256, base, off < last ? off : last);
             }
         }
     };
@@ -271,9 +389,9 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
     // anything else and used in that tile's epilogue: requested there, its whole latency stood between the last
     // matrix instruction and the store, and a workgroup of these launches has one tile or two.
     struct alignas(16) H8 { _Float16 v[8]; };
-    H8 b_pre[2] = {};
+    f32x4 b_pre[2];
     bool use_pre = false;
-    if (cw == 0 && my_tiles) {  // uniform
+    if (LORA && cw == 0 && my_tiles) {  // uniform
         const uint32_t row0 = first_row(0);
         const void* bq = lora.b;
         uint32_t rank = lora.rank, row_end = n, row_base = 0;
@@ -289,56 +407,44 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
         if (rank && b16 && rank % 8 == 0) {
             use_pre = true;
             const uint32_t row = (row0 + r_of(lane) < row_end ? row0 + r_of(lane) : row_end - 1) - row_base;
-            const _Float16* brow = static_cast<const _Float16*>(bq) + static_cast<size_t>(row) * rank;
-            b_pre[0] = *reinterpret_cast<const H8*>(brow);
-            b_pre[1] = *reinterpret_cast<const H8*>(brow + (rank >= 16 ? 8 : 0));
+            b_pre[0] = load16(bq, row * rank * 2);
+            b_pre[1] = load16(bq, row * rank * 2 + (rank >= 16 ? 16 : 0));
         }
     }
-    float4 xv[kHoist][2];
-#pragma unroll
-    for (int it = 0; it < kHoist; ++it) {
-        const float4* xp = task_ptr(tid + it * 64 * WAVES);
-        xv[it][0] = xp[0];
-        xv[it][1] = xp[1];
-    }
-    // kDepth units per wave in registers (beside the one in its LDS tile), in a ring of register buffers that the
-    // unrolled loop below walks with compile-time indices.  One: the next unit is on its way while the current one is
-    // multiplied.  A ring of four was measured slower on the large matrices (12288 x 2048 at 8 / 4 rows 10.0 / 9.2 ->
-    // 9.1 / 8.2 us, 2048 x 6144 11.3 -> 10.5) and level on the small ones, where a wave has one unit anyway: what a
-    // CU asks for beyond its share of the memory system queues in front of the activations the staging waits for.
-    constexpr int kDepth = 1;
-    Q4BlockRaw ring[kDepth][kLoads];
-#pragma unroll
-    for (int i = 0; i < kDepth; ++i) {
-        if (static_cast<uint32_t>(i) < units) load_unit(ring[i], i);
-    }
+    const uint32_t first_units = units < stages ? units : stages;
+    for (uint32_t i = 0; i < first_units; ++i) load_unit(i, i);
     __builtin_amdgcn_sched_barrier(0);  // nothing below is scheduled above these loads
-    // The LoRA factors of the producers: item i = (stacked row of A i / 8, activation row i % 8), thread i looks at
-    // item i while it still has staging to do (the producers need about 2 us, the activations arrive after 1.5),
-    // so that in the usual case the value is there when the staging is, and one barrier publishes both.
-    const uint32_t tag = launch_tag();
-    const unsigned long long none = static_cast<unsigned long long>(tag) << 32;  // lanes without an item: as if published
-    const bool early_mine = static_cast<uint32_t>(tid) < prod * 8 && (static_cast<uint32_t>(tid) & 7) < batch;
-    unsigned long long early = none;
+    wait_units(first_units);
 #pragma unroll
-    for (int it = 0; it < kHoist; ++it) {
-        if (it == kHoist - 1 && early_mine && lora.spin_limit)
-            early = __hip_atomic_load(&lora.slots[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t idx = tid + it * 64 * WAVES;
-        if (idx < n_tasks) stage_task(idx, xv[it][0], xv[it][1]);  // (whole quads: n_tasks is a multiple of 4)
+    for (int c = 0; c < kAhead; ++c)
+#pragma unroll
+        for (int i = 0; i < kMyTasks; ++i) asm volatile("" : "+v"(xv[c][i][0]), "+v"(xv[c][i][1]));
+    if constexpr (LORA) asm volatile("" : "+v"(b_pre[0]), "+v"(b_pre[1]));
+    if (stages_rows) {
+#pragma unroll
+        for (int c = 0; c < kAhead; ++c) {
+            if (has_chunk(c)) stage_chunk(c, [&](int i, f32x4& a, f32x4& b) {
+                a = xv[c][i][0];
+                b = xv[c][i][1];
+            });
+        }
+#pragma unroll 1
+        for (uint32_t c = kAhead; c < my_chunks; ++c)  // (behind the weights)
+            stage_chunk(c, [&](int i, f32x4& a, f32x4& b) {
+                const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const uint8_t*>(x) + x_off(c, i));
+                a = p[0];
+                b = p[1];
+            });
     }
-    for (uint32_t idx = tid + kHoist * 64 * WAVES; idx < n_tasks; idx += 64 * WAVES) {
-        const float4* xp = task_ptr(idx);
-        stage_task(idx, xp[0], xp[1]);
-    }
-    if (prod && static_cast<uint32_t>(tid) < prod * 8)
-        t_lds[(tid & 7) * kMaxLoraRank + (tid >> 3)] = early_mine ? as_f32(static_cast<uint32_t>(early)) : 0.0f;
-    __syncthreads();
-    // A wave some of whose values were not there yet (or that has more items than lanes) goes the patient way.  No
-    // barrier of its own: whoever reads t_lds does so in a tile's epilogue, behind the two barriers of the partial
-    // sums that every wave passes once a round (a workgroup of one wave reads its own writes).
-    const bool early_bad = early_mine && (!lora.spin_limit || static_cast<uint32_t>(early >> 32) != tag);
-    if (prod && (__any(early_bad) || prod * 8 > 64 * WAVES)) {  // uniform in the wave
+    if constexpr (TW > 1) __syncthreads();
+    else asm volatile("" ::: "memory");  // (one tile at a time: a wave multiplies what it staged itself)
+    // The LoRA factors of the producers: item i = (stacked row of A i / 8, activation row i % 8), 64 items a wave.  Picked up once, when
+    // the wave's first tile is multiplied, in front of the barrier of its partial sums, behind which the factors are read: the
+    // producers need some 2.5 us, and the product has begun after 3 (picked up before it, the four layers of a_row_dot's comment
+    // took 31.5 us, 28.4 behind it).
+    auto pick_up = [&] {
+        const uint32_t tag = launch_tag();
+        const unsigned long long none = static_cast<unsigned long long>(tag) << 32;  // lanes without an item: as if published
         for (uint32_t i0 = wave * 64; i0 < prod * 8; i0 += 64 * WAVES) {  // uniform
             const uint32_t i = i0 + lane;
             const bool mine = i < prod * 8 && (i & 7) < batch;
@@ -364,48 +470,49 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                 uint32_t j;
                 a_row_of(item >> 3, a, a_is_f16, j);
                 const float* xr = x + static_cast<size_t>(item & 7) * x_stride;
-                const float total = wave_sum(lora_a_row_partial(a, a_is_f16, j, k, xr, lane, 64));
+                const float total = wave_sum(a_row_dot(a, a_is_f16, j, k, xr, lane));
                 if (static_cast<uint32_t>(lane) == fl) val = total;
                 if (lane == 0) __hip_atomic_fetch_add(&lora.sync[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             if (i < prod * 8) t_lds[(i & 7) * kMaxLoraRank + (i >> 3)] = mine ? val : 0.0f;
         }
-    }
+    };
 
     // ---- the product ----
     const uint32_t r = lane & 15, g = lane >> 4;  // operand mapping: weight row r of the tile, k group / row pair g
     float acc0 = 0.0f, acc1 = 0.0f;
-    auto process = [&](Q4BlockRaw (&cur)[kLoads], uint32_t u) {
-        if (u >= units) return;  // uniform
-        // through the tile: tile[row][5 * block + d]; the buffer is then free for the unit kDepth ahead
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            uint32_t* tp = tile + (rq + kRowStep * i) * kTilePitch + 5 * jl;
-            tp[0] = cur[i].sb;
-            tp[1] = cur[i].q[0]; tp[2] = cur[i].q[1]; tp[3] = cur[i].q[2]; tp[4] = cur[i].q[3];
-        }
-        if (u + kDepth < units) load_unit(cur, u + kDepth);  // uniform
-        const uint32_t t = u / my_chunks, c = u - t * my_chunks;
+    float4v bias_acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](uint32_t u, uint32_t c, uint32_t stage) {
+        const uint32_t behind = units - 1 - u;
+        wait_units(behind < stages - 1 ? behind : stages - 1);
         const uint32_t blk0 = (c * CW + cw) * kBpw;
-        const uint32_t* tr = tile + r * kTilePitch;
+        uint32_t* const unit = ring + stage * kStageDwords;
+        if (__builtin_expect(blk0 + kBpw > nb, 0)) {  // uniform: blocks past the end of the row; their headers become zero (and their activations are)
+            for (uint32_t i = lane; i < 16 * kBpw; i += 64)
+                if (blk0 + i % kBpw >= nb) unit[i / kBpw * kRowDwords + i % kBpw * 5] = 0;
+        }
+        const uint32_t *head = unit + r * kRowDwords, *data = head + 1 + g;
+        const uint8_t* xqp = xq + blk0 * kXqBytes + lane * 8;
+        const float* xfp = reinterpret_cast<const float*>(xf + blk0 * kXfBytes);
+        const float xs = xfp[lane];
         // four blocks at a time, straight-line: their LDS reads, then their four matrix instructions back to back,
-        // then their results (a block past the end of the row re-reads the row's last one and counts for nothing)
-#pragma unroll
-        for (int j0 = 0; j0 < kBpw; j0 += 4) {
-            uint32_t sb[4], qd[4];
+        // then their results
+        auto four = [&](auto j0c) {
+            constexpr int j0 = decltype(j0c)::value;
+            // lane group g: the header of block j0 + g, and of that block the sums of activation row b(r): operands of the matrix
+            // instruction that adds up bias * sum over the four blocks; its results land as those of the integer ones do
+            const uint32_t hd = head[5 * (j0 + g)];
+            const float sx = xfp[64 + 8 * (j0 + g) + (WIDE ? r >> 2 : 2 * (r >> 2) + (r & 1))];
+            uint32_t qd[4];
             long aop[4];
-            float4 f[4];
-            bool live[4];
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
-                const uint32_t blk_raw = blk0 + j0 + jj;
-                live[jj] = blk_raw < nb;  // uniform
-                const uint32_t blk = live[jj] ? blk_raw : nb - 1;
-                sb[jj] = tr[5 * (j0 + jj)];
-                qd[jj] = tr[5 * (j0 + jj) + 1 + g];
-                aop[jj] = *reinterpret_cast<const long*>(xq + static_cast<size_t>(blk) * kXqBytes + lane * 8);
-                f[jj] = *reinterpret_cast<const float4*>(xf + static_cast<size_t>(blk) * kXfBytes + g * 16);
+                qd[jj] = data[5 * (j0 + jj)];
+                aop[jj] = *reinterpret_cast<const long*>(xqp + (j0 + jj) * kXqBytes);
             }
+            float sc[4];
+            rows_apart(f16_lo(hd), sc);
+            bias_acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sx, f16_hi(hd), bias_acc, 0, 0, 0);
             int4v d[4];
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
@@ -414,41 +521,44 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                 const int4v zero = {0, 0, 0, 0};
                 d[jj] = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop[jj], bop, zero, 0, 0, 0);
             }
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-                const float scale = live[jj] ? half_lo(sb[jj]) : 0.0f, bias = live[jj] ? half_hi(sb[jj]) : 0.0f;
+            auto one = [&](auto jc) {
+                constexpr int jj = decltype(jc)::value, j = j0 + jj;
+                const float s0 = of_row_lane<2 * j>(xs) * sc[jj];
                 if constexpr (WIDE) {
                     // the top digit's sum times 2^16 is exact in f32, so is 256 mid + low: one rounding in the add
-                    const float d0 = fmaf(static_cast<float>(d[jj].x), 65536.0f, static_cast<float>(d[jj].y * 256 + d[jj].z));
-                    acc0 = fmaf(scale * f[jj].x, d0, acc0);
-                    acc0 = fmaf(bias, f[jj].y, acc0);
+                    acc0 = fmaf(s0, fmaf(static_cast<float>(d[jj].x), 65536.0f, static_cast<float>(d[jj].y * 256 + d[jj].z)), acc0);
                 } else {
-                    const float d0 = static_cast<float>(d[jj].x * 256 + d[jj].y), d1 = static_cast<float>(d[jj].z * 256 + d[jj].w);
-                    acc0 = fmaf(scale * f[jj].x, d0, acc0);
-                    acc1 = fmaf(scale * f[jj].y, d1, acc1);
-                    acc0 = fmaf(bias, f[jj].z, acc0);
-                    acc1 = fmaf(bias, f[jj].w, acc1);
+                    const float s1 = of_row_lane<2 * j + 1>(xs) * sc[jj];
+                    acc0 = fmaf(s0, static_cast<float>(d[jj].x * 256 + d[jj].y), acc0);
+                    acc1 = fmaf(s1, static_cast<float>(d[jj].z * 256 + d[jj].w), acc1);
                 }
-            }
+            };
+            one(std::integral_constant<int, 0>{});
+            one(std::integral_constant<int, 1>{});
+            one(std::integral_constant<int, 2>{});
+            one(std::integral_constant<int, 3>{});
+        };
+        four(std::integral_constant<int, 0>{});
+        four(std::integral_constant<int, 4>{});
+        asm volatile("" : "+v"(acc0), "+v"(acc1));  // (sunk below the branch, the broadcasts are instructions of their own)
+        if (u + stages < units) {  // uniform; the unit's LDS reads are done
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            load_unit(u + stages, stage);
         }
-        if (c + 1 == my_chunks) {  // the wave's part of the tile is complete: meet the tile's other waves in LDS
-            const uint32_t row = first_row(t) + r;
-            if constexpr (WAVES > 1) {
-                __syncthreads();  // (every wave passes here once a round; waves without work bring zeros)
-                part[(wave * 64 + lane) * 2] = acc0;
-                part[(wave * 64 + lane) * 2 + 1] = acc1;
-                __syncthreads();
-                acc0 = 0.0f;
-                acc1 = 0.0f;
-                if (cw == 0) {
+    };
+    // The sums of round t's tile and what belongs to them, to memory.
+    auto finish = [&](uint32_t t) {
+        const uint32_t row = first_row(t) + r;
+        const float* const mine = part + (t % kMeet) * (WAVES * 64 * 2) + (tw * CW * 64 + lane) * 2;
+        float acc0 = 0.0f, acc1 = 0.0f;
 #pragma unroll
-                    for (int v = 0; v < CW; ++v) {
-                        acc0 += part[((tw * CW + v) * 64 + lane) * 2];
-                        acc1 += part[((tw * CW + v) * 64 + lane) * 2 + 1];
-                    }
-                }
-            }
-            if (cw == 0 && row < n) {
+        for (int v = 0; v < CW; ++v) {
+            const float2 pv = *reinterpret_cast<const float2*>(mine + v * (64 * 2));
+            acc0 += pv.x;
+            acc1 += pv.y;
+        }
+        {
+            if (row < n) {
                 const uint32_t b0 = WIDE ? g : 2 * g, b1 = WIDE ? batch : 2 * g + 1;  // (wide: one row a lane)
                 // this row's adapter and output: the launch's, or (several views) those of the tile's view
                 LoraEpilogue lo = lora;
@@ -488,8 +598,8 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                         };
                         uint32_t i = 0;
                         if (use_pre && t == 0) {  // uniform
-                            eight(b_pre[0], 0);
-                            if (lo.rank >= 16) eight(b_pre[1], 8);
+                            eight(__builtin_bit_cast(H8, b_pre[0]), 0);
+                            if (lo.rank >= 16) eight(__builtin_bit_cast(H8, b_pre[1]), 8);
                             i = lo.rank >= 16 ? 16 : 8;
                         }
                         for (; i < lo.rank; i += 8) eight(*reinterpret_cast<const H8*>(brow + i), i);
@@ -505,7 +615,7 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                     acc0 = fmaf(lo.scale, l0, acc0);
                     acc1 = fmaf(lo.scale, l1, acc1);
                 };
-                if (lo.rank) {
+                if (LORA && lo.rank) {
                     const uint32_t c0 = b0 < batch ? b0 : 0, c1 = b1 < batch ? b1 : 0;
                     if (prod) {
                         uint32_t off = 0;
@@ -518,42 +628,41 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                 if (b0 < batch) yv[static_cast<size_t>(b0) * ys + lrow] = acc0;
                 if (b1 < batch) yv[static_cast<size_t>(b1) * ys + lrow] = acc1;
             }
-            acc0 = 0.0f;
-            acc1 = 0.0f;
         }
     };
 
-    for (uint32_t u = 0; u < units; u += kDepth) {
-#pragma unroll
-        for (int i = 0; i < kDepth; ++i) process(ring[i], u + i);
-    }
-    // a wave meets the others once a round: those with fewer tiles than rounds (or no chunk at all) make up for it
-    if constexpr (WAVES > 1) {
-        const uint32_t met = my_chunks ? my_tiles : 0;
-        for (uint32_t t = met; t < rounds; ++t) {
+    // The waves meet every kMeet rounds (once, where a workgroup has that many tiles or fewer): in between each goes at its own
+    // pace, so that one reads LDS while another computes.  (With a meeting a round the four layers of a_row_dot's comment took 28.4 us, 24.9 so.)
+    for (uint32_t t = 0, u = 0, stage = 0; t < rounds; ++t) {
+        if (t < my_tiles) {  // uniform in the wave
+            acc0 = 0.0f;
+            acc1 = 0.0f;
+            bias_acc = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+            for (uint32_t c = 0; c < my_chunks; ++c, ++u) {
+                multiply(u, c, stage);
+                stage = stage + 1 == stages ? 0 : stage + 1;
+            }
+            *reinterpret_cast<float2*>(part + ((t % kMeet) * WAVES + wave) * (64 * 2) + lane * 2) = make_float2(acc0 + bias_acc.x, acc1 + bias_acc.y);
+        }
+        if (prod && t == 0) pick_up();  // uniform
+        if ((t + 1) % kMeet == 0 || t + 1 == rounds) {
             __syncthreads();
-            part[(wave * 64 + lane) * 2] = 0.0f;
-            part[(wave * 64 + lane) * 2 + 1] = 0.0f;
-            __syncthreads();
+            for (uint32_t q = t - t % kMeet + cw; q <= t && q < my_tiles; q += CW) finish(q);
+            if (t + 1 < rounds) __syncthreads();
         }
     }
 }
 
 struct I8Plan {
-    uint32_t cw, tw, grid;
+    uint32_t cw, tw, grid, stages;
     size_t lds;
 };
 
-size_t lds_eight_waves(uint32_t nb) {
-    return static_cast<size_t>(nb) * (kXqBytes + kXfBytes) + 8 * kTileDwords * 4 + 8 * 64 * 2 * 4 + 8 * kMaxLoraRank * 4;
-}
-
 }  // namespace
 
-// At least two 16-row tiles per CU and rows short enough that two eight-wave workgroups share a CU's LDS.
+// At least two 16-row tiles per CU, of rows of up to 2816 weights.
 bool gemv_i8_many_short_rows(uint32_t n, uint32_t k, uint32_t cu_count) {
-    const uint32_t nb = k / kBlockWeights;
-    return (n + 15) / 16 >= 2 * cu_count && nb >= 4 * kBpw && lds_eight_waves(nb) <= 78 * 1024;
+    return (n + 15) / 16 >= 2 * cu_count && k >= 1024 && k <= 2816;
 }
 
 namespace {
@@ -564,67 +673,74 @@ bool plan_i8(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count, I8Plan* 
     const uint32_t chunks = (nb + kBpw - 1) / kBpw;
     const uint32_t n_tiles = (n + 15) / 16;
     I8Plan p;
-    // waves that split one tile's chunks: a power of two up to sixteen; tiles side by side: as many as fill a
-    // sixteen-wave workgroup, but no more than leaves every CU a workgroup (one workgroup a CU stages the
-    // activations once for all the tiles that CU works on)
-    p.cw = chunks >= 16 ? 16 : chunks >= 8 ? 8 : chunks >= 4 ? 4 : chunks >= 2 ? 2 : 1;
-    p.tw = 16 / p.cw;
-    while (p.tw > 1 && (n_tiles + p.tw - 1) / p.tw < cu_count) p.tw /= 2;
-    for (;;) {
+    // Up to a tile a CU: as many waves as split its chunks, up to eight.  With more, eight waves as 8, 4 or 2 columns of chunks
+    // beside 1, 2 or 4 tiles, whichever leaves a wave the fewest units (12288 x 2560 is 5 as 2 x 4, 6 else; 8 x 1 has
+    // the shorter staging, so it is taken where it is no worse).
+    p.cw = chunks >= 8 ? 8 : chunks >= 4 ? 4 : chunks >= 2 ? 2 : 1;
+    p.tw = 1;
+    if (n_tiles > cu_count && chunks >= 2) {
+        uint32_t best = 0;
+        for (uint32_t cw = 8; cw >= 2; cw /= 2) {
+            const uint32_t tw = 8 / cw, cost = ((n_tiles + tw - 1) / tw + cu_count - 1) / cu_count * ((chunks + cw - 1) / cw);
+            if (cw >= 2 * chunks || (best && cost >= best)) continue;
+            best = cost;
+            p.cw = cw;
+            p.tw = tw;
+        }
+    }
+    auto bytes = [&](uint32_t stages) {
         const uint32_t waves = p.cw * p.tw;
-        p.lds = static_cast<size_t>(nb) * (kXqBytes + kXfBytes) + static_cast<size_t>(waves) * kTileDwords * 4 +
-                static_cast<size_t>(waves) * 64 * 2 * 4 + 8 * kMaxLoraRank * 4;
-        if (p.lds <= 160 * 1024) break;
+        return static_cast<size_t>(chunks) * kBpw * (kXqBytes + kXfBytes) + static_cast<size_t>(waves) * (stages * kStageBytes + kMeet * 64 * 2 * 4) + 8 * kMaxLoraRank * 4;
+    };
+    while (bytes(1) > kLdsBytes) {
         if (p.tw > 1) p.tw /= 2;
         else if (p.cw > 1) p.cw /= 2;
         else return false;
     }
-    // Many tiles of short rows (12288 x 2048: 768 tiles): workgroups of eight waves (two split K, four tiles side by
-    // side), two of which fit a CU, one round each, instead of sixteen-wave workgroups that walk two rounds
-    // (at 8 / 4 rows 9.1 / 8.1 -> 8.8 / 7.9 us).
-    if (gemv_i8_many_short_rows(n, k, cu_count)) {
-        p.cw = 2;
-        p.tw = 4;
-        p.lds = lds_eight_waves(nb);
-        p.grid = (n_tiles + 3) / 4;
-        *out = p;
-        return true;
-    }
     const uint32_t groups = (n_tiles + p.tw - 1) / p.tw;  // rounds of tiles in all
-    if (groups <= cu_count) {
-        p.grid = groups;
-    } else {
-        const uint32_t per = (groups + cu_count - 1) / cu_count;
-        p.grid = (groups + per - 1) / per;  // the same number of rounds for every workgroup, to within one
-    }
+    p.grid = groups <= cu_count ? groups : cu_count;
+    const uint32_t units = (groups + p.grid - 1) / p.grid * ((chunks + p.cw - 1) / p.cw);  // most of a wave
+    p.stages = units < kMaxStages ? units : kMaxStages;
+    while (bytes(p.stages) > kLdsBytes) --p.stages;
+    p.lds = bytes(p.stages);
     *out = p;
     return true;
 }
 
-template <int CW, int TW, bool WIDE, bool MULTI>
+template <int CW, int TW, bool WIDE, bool MULTI, bool LORA>
 void launch_i8(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, const float* x, uint32_t x_stride,
                uint32_t batch, float* y, uint32_t y_stride, const LoraEpilogue& lora, const MultiViews& mv,
                hipStream_t stream) {
     static LdsCapOnce lds_cap;
-    lds_cap.raise(reinterpret_cast<const void*>(gemv_q4_i8<CW, TW, WIDE, MULTI>), 160 * 1024);
+    constexpr auto kernel = gemv_q4_i8<CW, TW, WIDE, MULTI, LORA>;
+    lds_cap.raise(reinterpret_cast<const void*>(kernel), kLdsBytes);
     const uint32_t producers = lora.slots ? lora.rank : 0;
-    launch_kernel((gemv_q4_i8<CW, TW, WIDE, MULTI>), dim3(producers + p.grid), dim3(64 * CW * TW), p.lds, stream, w, n,
-                       k, x, x_stride, batch, y, y_stride, lora, mv);
+    launch_kernel(kernel, dim3(producers + p.grid), dim3(64 * CW * TW), p.lds, stream, w, n,
+                       k, x, x_stride, batch, y, y_stride, p.stages, lora, mv);
 }
 
-template <bool WIDE, bool MULTI>
+template <bool WIDE, bool MULTI, bool LORA>
 void launch_i8_shape(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, const float* x, uint32_t x_stride,
                      uint32_t batch, float* y, uint32_t y_stride, const LoraEpilogue& lora, const MultiViews& mv,
                      hipStream_t stream) {
 #define LQ4_I8(CW_, TW_)                \
     if (p.cw == CW_ && p.tw == TW_)     \
-    return launch_i8<CW_, TW_, WIDE, MULTI>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, mv, stream)
-    LQ4_I8(16, 1);
-    LQ4_I8(8, 2); LQ4_I8(8, 1);
-    LQ4_I8(4, 4); LQ4_I8(4, 2); LQ4_I8(4, 1);
-    LQ4_I8(2, 8); LQ4_I8(2, 4); LQ4_I8(2, 2); LQ4_I8(2, 1);
-    LQ4_I8(1, 16); LQ4_I8(1, 8); LQ4_I8(1, 4); LQ4_I8(1, 2); LQ4_I8(1, 1);
+    return launch_i8<CW_, TW_, WIDE, MULTI, LORA>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, mv, stream)
+    LQ4_I8(8, 1); LQ4_I8(4, 2); LQ4_I8(2, 4); LQ4_I8(4, 1); LQ4_I8(2, 2); LQ4_I8(2, 1); LQ4_I8(1, 1);
 #undef LQ4_I8
+}
+
+template <bool MULTI>
+void launch_i8_rows(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, const float* x, uint32_t x_stride,
+                    uint32_t batch, float* y, uint32_t y_stride, const LoraEpilogue& lora, const MultiViews& mv, bool with_lora,
+                    hipStream_t stream) {
+    auto go = [&](auto wide) {
+        constexpr bool W = decltype(wide)::value;
+        if (with_lora) launch_i8_shape<W, MULTI, true>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, mv, stream);
+        else launch_i8_shape<W, MULTI, false>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, mv, stream);
+    };
+    if (batch <= 4) go(std::true_type{});
+    else go(std::false_type{});
 }
 
 }  // namespace
@@ -639,8 +755,7 @@ void launch_gemv_i8(const uint8_t* w, uint32_t n, uint32_t k, const float* x, ui
     I8Plan p;
     if (!plan_i8(n, k, batch, cu_count, &p)) return;  // the caller asked gemv_i8_serves first
     const MultiViews none{};
-    if (batch <= 4) launch_i8_shape<true, false>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, none, stream);
-    else launch_i8_shape<false, false>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, none, stream);
+    launch_i8_rows<false>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, none, lora.rank != 0, stream);
 }
 
 // The launch can carry `rank_total` producer workgroups for the LoRA factors when they find idle CUs beside the
@@ -667,8 +782,9 @@ void launch_gemv_i8_multi(const MultiViews& mv, uint32_t k, const float* x, uint
     I8Plan p;
     if (!plan_i8(n, k, batch, cu_count, &p)) return;  // the caller asked gemv_i8_multi_serves first
     const LoraEpilogue hand = in_launch ? *in_launch : LoraEpilogue{};  // rank = the views' ranks together, slots, sync
-    if (batch <= 4) launch_i8_shape<true, true>(p, nullptr, n, k, x, x_stride, batch, nullptr, 0, hand, mv, stream);
-    else launch_i8_shape<false, true>(p, nullptr, n, k, x, x_stride, batch, nullptr, 0, hand, mv, stream);
+    bool with_lora = false;
+    for (uint32_t v = 0; v < mv.count; ++v) with_lora |= mv.rank[v] != 0;
+    launch_i8_rows<true>(p, nullptr, n, k, x, x_stride, batch, nullptr, 0, hand, mv, with_lora, stream);
 }
 
 }  // namespace lq4
