@@ -463,15 +463,29 @@ static void plain_gemv_one_token(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, ui
     ctx->counters.gemv++;
 }
 
-// 2..8 rows on the integer matrix-core kernel: three to eight rows of a matrix of up to 4096 x 2048; five to eight
-// rows of a tall matrix of short rows (12288 x 2048 9.6-10.0 -> 8.7-8.8 us, 16384 x 2048 11.0-11.6 -> 8.8-9.0,
-// 9728 x 2560 12.0-12.6 -> 10.0-10.1; at 2..4 rows the 4x4x4 kernel is ahead there, 6.3-7.3 us against 7.8); or, for
-// the tests, whatever it can hold.
-static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch) {
-    const bool small = batch >= 3 && k <= 2048 && n <= 4096;
-    const bool tall = batch >= 5 && gemv_i8_many_short_rows(n, k, ctx->cu_count);
-    return batch >= 2 && batch <= 8 && ctx->gemv_i8 && (ctx->gemv_i8 == 2 || small || tall) &&
-           gemv_i8_serves(n, k, batch, ctx->cu_count);
+// 2..8 rows on the integer matrix-core kernel, which keeps 24 (up to four rows) or 16 bits of every activation below its block's
+// maximum where the others round it to f16: wherever it is the faster one, or, for the tests, whatever it can hold.  us there (4x4x4
+// kernel or few-token GEMM) / here:
+//   up to 4096 rows, K up to 2048: from three rows (512 x 2048 4.2 / 3.6, 2048 x 2048 4.8 / 3.9, at eight 5.5 / 4.3; at two 3.6 / 3.8);
+//   at 2560 rows and more K up to 5120: at three 2560 x 2560 5.4 / 4.5, 4096 x 4096 8.1 / 5.4, 12288 x 2048 8.3 / 6.6, 12288 x
+//     5120 13.7 / 11.4, 24576 x 1024 9.6 / 6.6; at eight 6144 x 1024 5.4 / 4.1, 4096 x 4096 7.5 / 6.5, 12288 x 4096 17.5 / 11.3, 32768 x 3072
+//     21.0 / 17.2.  Not short rows of many (5120 x 512 at four 3.2 / 4.0); not much beyond (16384 x 4608 at three 15.3 / 15.8, x 5632 16.0 /
+//     19.0); and where the waves would stand idle for half of it not instead of the few-token GEMM (5120 x 2560 at five 6.7 / 7.0);
+//   fewer rows: K up to 2816 from 1024 on (1536 x 2560 at three 4.6 / 4.4, at eight 6.0 / 4.9; 512 x 2816 at three 4.1 / 4.3), at seven and
+//     eight K up to 5120 (1536 x 5120 7.5 / 6.7, 512 x 3072 5.6 / 4.9; at five 5.1 / 5.0 and 4.7 / 4.9);
+//   two rows: 2560..4096 rows (4096 x 2048 4.4 / 3.9, 4096 x 5120 7.8 / 6.6, 2560 x 4096 6.1 / 5.3; 4096 x 1536 3.9 / 4.4) and 7168 and more
+//     with K of 2048..4096 (8192 x 2816 10.3 / 7.6, 10240 x 3072 11.9 / 8.7, 24576 x 2048 13.7 / 10.8; 12288 x 2560 8.6 / 9.0, 6144 x 2560 6.0 / 6.3).
+static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch, bool with_lora = false) {
+    if (batch < 2 || batch > 8 || !ctx->gemv_i8 || !gemv_i8_serves(n, k, batch, ctx->cu_count)) return false;
+    if (ctx->gemv_i8 == 2) return true;
+    if (batch >= 3 && k <= 2048 && n <= 4096) return true;
+    if (batch >= 5 && gemv_i8_many_short_rows(n, k, ctx->cu_count)) return true;
+    if (k > 5120) return false;
+    if (batch == 2) return k >= 2048 && ((n >= 2560 && n <= 4096) || (n >= 7168 && k <= 4096 && (n <= 10240 || k == 2048 || k >= 2816)));
+    if (n < 2560) return n >= 512 && k <= (batch >= 7 ? 5120u : n >= 1024 ? 2816u : 2048u);
+    if (k < 1024 || (n > 12288 && k > 4096 && batch < 8)) return false;
+    // (the few-token GEMM computes the factors of an adapter on its way; here they are a launch of their own unless CUs are left)
+    return batch < 5 || n >= 8192 || (gemv_i8_busy(n, k, ctx->cu_count) && !(with_lora && n > 3072));
 }
 
 // Above four activation rows the few-token matrix-core kernel (operands packed once, eight K
@@ -479,12 +493,12 @@ static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t b
 // mid-sized matrices only (measured: behind for 512 x 2048, where its two launches dominate,
 // and for 12288 x 2048, where the GEMV kernel's grid already fills the chip), and not where the integer
 // matrix-core kernel serves (3072 x 2048 at 5..8 rows 5.8-5.9 us here, 5.4-5.5 there; 4096 x 2048 6.2 / 5.5).
-static bool gemv_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch) {
+static bool gemv_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch, bool with_lora) {
     const uint64_t weights = static_cast<uint64_t>(n) * k;
     // (not for up to 2048 rows while the GEMV kernel can stage the activations: its eight-wave
     // workgroups then win, 2048 x 6144 at 5..8 rows 9.5 -> 7.2..8.2 us)
     const bool narrow = n <= 2048 && gemv_mfma_lds_bytes(k, batch < 8 ? batch : 8) <= 150 * 1024;
-    return batch >= 9 || (batch >= 5 && n < 8192 && !narrow && weights >= 6000000 && !gemv_takes_i8(ctx, n, k, batch));
+    return batch >= 9 || (batch >= 5 && n < 8192 && !narrow && weights >= 6000000 && !gemv_takes_i8(ctx, n, k, batch, with_lora));
 }
 
 // K slices on the 4x4x4 matrix-core kernel (no LoRA step there).  Their partial results live in the context's scratch, so only
@@ -512,7 +526,7 @@ static int few_token_choice(const lq4_ctx* ctx, size_t bytes, hipStream_t stream
 static int gemv_dispatch(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, uint32_t k, const float* x_dev, uint32_t batch,
                          float* y_dev, const LoraEpilogue& ep, hipStream_t s) {
     int rc;
-    if (gemv_takes_few_token_gemm(ctx, n, k, batch)) {
+    if (gemv_takes_few_token_gemm(ctx, n, k, batch, ep.rank != 0)) {
         if (gemv_takes_slices(ctx, n, k, batch, ep.rank != 0, false, s)) {
             rc = ensure_scratch(ctx, gemv_mfma_sliced_scratch_bytes(n, k, batch), s);
             if (rc) return rc;
@@ -526,14 +540,7 @@ static int gemv_dispatch(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, uint32_t k
         ctx->counters.gemm++;
     } else if (batch == 1 && !ep.rank) {
         plain_gemv_one_token(ctx, wp, n, k, x_dev, y_dev, s);
-    } else if (gemv_takes_i8(ctx, n, k, batch)) {
-        // Three to eight rows of a matrix of up to 4096 x 2048: the integer matrix-core kernel, which is as fast as
-        // or faster than the 4x4x4 kernel there (512 x 2048: 4.33 -> 4.09 us at four rows, 4.71 -> 4.53 at eight;
-        // 2048 x 2048: 4.67 -> 4.54, 5.09 -> 4.98; 3072 x 2048 at four rows 5.58 -> 4.82) and keeps 24 (up to four rows)
-        // or 16 bits of every activation below its block's maximum instead of rounding it to f16.  Behind on long rows
-        // and many rows (2048 x 6144 at eight rows 8.7 -> 10.4 us, 12288 x 2048 at four 7.8 -> 8.8), which stay where
-        // they were.  With a LoRA epilogue alike (q+v of the 2B model at eight rows 17.6 -> 16.2 us), so that a
-        // projection is served by the same arithmetic with and without its adapter.
+    } else if (gemv_takes_i8(ctx, n, k, batch, ep.rank != 0)) {
         launch_gemv_i8(wp, n, k, x_dev, k, batch, y_dev, n, ep, ctx->cu_count, s);
         ctx->counters.gemv++;
     } else {
@@ -570,9 +577,9 @@ int lq4_gemv(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
         ep.slots = reinterpret_cast<unsigned long long*>(ctx->lora_sync + 64);
         ep.sync = ctx->lora_sync;
         ep.spin_limit = ctx->lora_spin_limit;
-    } else if (ep.rank && batch > 1 && gemv_takes_few_token_gemm(ctx, n, k, batch) && gemm_skinny_computes_t(ep.rank)) {
+    } else if (ep.rank && batch > 1 && gemv_takes_few_token_gemm(ctx, n, k, batch, true) && gemm_skinny_computes_t(ep.rank)) {
         ep.a = lora->a_packed;  // the few-token GEMM's packing launch computes A.x
-    } else if (ep.rank && ctx->lora_in_kernel && gemv_takes_i8(ctx, n, k, batch) &&
+    } else if (ep.rank && ctx->lora_in_kernel && gemv_takes_i8(ctx, n, k, batch, true) &&
                gemv_i8_lora_in_launch(n, k, batch, ep.rank, ctx->cu_count)) {
         // 2..8 rows: `rank` producer workgroups of the launch, on CUs the matrix leaves idle
         ep.a = lora->a;
@@ -715,14 +722,14 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
     // wave holds the factor of stacked row l, hence at most 64 rows of A in all)
     const bool in_launch = stacked && with_lora && ctx->lora_in_kernel && total_rank <= 64;
     // two to eight rows: the integer matrix-core kernel over the stacked rows, where it is the faster one
-    const bool stacked_rows = !stacked && batch >= 2 && batch <= 8 && mv.count > 1 && ctx->gemv_i8 &&
-                              (ctx->gemv_i8 == 2 || (k <= 2048 && mv.begin[mv.count] <= 4096)) &&
+    const bool stacked_rows = !stacked && batch >= 2 && batch <= 8 && mv.count > 1 &&
+                              ((ctx->gemv_i8 && k <= 2048 && mv.begin[mv.count] <= 4096) || gemv_takes_i8(ctx, mv.begin[mv.count], k, batch, with_lora)) &&
                               gemv_i8_multi_serves(mv, k, batch, ctx->cu_count);
     if (with_lora && !stacked && !stacked_rows) {
         // those that go to the few-token GEMM get their A . x with its packing launch
         for (uint32_t i = 0, v = 0; i < count; ++i) {
             if (proj[i].n == 0) continue;
-            if (ep[i].rank && gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch) && gemm_skinny_computes_t(ep[i].rank)) {
+            if (ep[i].rank && gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch, true) && gemm_skinny_computes_t(ep[i].rank)) {
                 ep[i].a = proj[i].lora->a_packed;
                 av.rank[v] = 0;
                 --with_lora;
@@ -767,7 +774,7 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
         SkinnyViews few{};
         for (uint32_t i = 0; i < count; ++i) {
             if (proj[i].n == 0) continue;
-            if (gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch)) {
+            if (gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch, ep[i].rank != 0)) {
                 few_token_view(&few, proj[i].n, wp[i], proj[i].y_dev, ep[i], ep[i].a);
                 continue;
             }

@@ -667,27 +667,32 @@ bool gemv_i8_many_short_rows(uint32_t n, uint32_t k, uint32_t cu_count) {
 
 namespace {
 
+struct I8Split {
+    uint32_t cw, tw, steps;  // columns of chunks, tiles side by side, units a wave is left with
+};
+I8Split split_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count) {
+    // Up to a tile a CU: as many waves as split its chunks, up to eight.  With more, eight waves as 8, 4 or 2 columns of chunks
+    // beside 1, 2 or 4 tiles, whichever leaves a wave the fewest units (12288 x 2560 is 5 as 2 x 4, 6 else; 8 x 1 has
+    // the shorter staging, so it is taken where it is no worse).
+    I8Split best{chunks >= 8 ? 8u : chunks >= 4 ? 4u : chunks >= 2 ? 2u : 1u, 1, 0};
+    auto steps = [&](uint32_t cw, uint32_t tw) { return ((n_tiles + tw - 1) / tw + cu_count - 1) / cu_count * ((chunks + cw - 1) / cw); };
+    best.steps = steps(best.cw, best.tw);
+    if (n_tiles <= cu_count || chunks < 2) return best;
+    best.steps = ~0u;
+    for (uint32_t cw = 8; cw >= 2; cw /= 2)
+        if (cw < 2 * chunks && steps(cw, 8 / cw) < best.steps) best = I8Split{cw, 8 / cw, steps(cw, 8 / cw)};
+    return best;
+}
+
 bool plan_i8(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count, I8Plan* out) {
     if (k == 0 || k % kBlockWeights || n == 0 || batch == 0 || batch > 8) return false;
     const uint32_t nb = k / kBlockWeights;
     const uint32_t chunks = (nb + kBpw - 1) / kBpw;
     const uint32_t n_tiles = (n + 15) / 16;
     I8Plan p;
-    // Up to a tile a CU: as many waves as split its chunks, up to eight.  With more, eight waves as 8, 4 or 2 columns of chunks
-    // beside 1, 2 or 4 tiles, whichever leaves a wave the fewest units (12288 x 2560 is 5 as 2 x 4, 6 else; 8 x 1 has
-    // the shorter staging, so it is taken where it is no worse).
-    p.cw = chunks >= 8 ? 8 : chunks >= 4 ? 4 : chunks >= 2 ? 2 : 1;
-    p.tw = 1;
-    if (n_tiles > cu_count && chunks >= 2) {
-        uint32_t best = 0;
-        for (uint32_t cw = 8; cw >= 2; cw /= 2) {
-            const uint32_t tw = 8 / cw, cost = ((n_tiles + tw - 1) / tw + cu_count - 1) / cu_count * ((chunks + cw - 1) / cw);
-            if (cw >= 2 * chunks || (best && cost >= best)) continue;
-            best = cost;
-            p.cw = cw;
-            p.tw = tw;
-        }
-    }
+    const I8Split split = split_i8(n_tiles, chunks, cu_count);
+    p.cw = split.cw;
+    p.tw = split.tw;
     auto bytes = [&](uint32_t stages) {
         const uint32_t waves = p.cw * p.tw;
         return static_cast<size_t>(chunks) * kBpw * (kXqBytes + kXfBytes) + static_cast<size_t>(waves) * (stages * kStageBytes + kMeet * 64 * 2 * 4) + 8 * kMaxLoraRank * 4;
@@ -744,6 +749,12 @@ void launch_i8_rows(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, c
 }
 
 }  // namespace
+
+// The eight waves of every CU busy for at least 55 % of their steps.
+bool gemv_i8_busy(uint32_t n, uint32_t k, uint32_t cu_count) {
+    const uint32_t n_tiles = (n + 15) / 16, chunks = (k / kBlockWeights + kBpw - 1) / kBpw;
+    return static_cast<uint64_t>(n_tiles) * chunks * 100 >= 55ull * 8 * cu_count * split_i8(n_tiles, chunks, cu_count).steps;
+}
 
 bool gemv_i8_serves(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count) {
     I8Plan p;
