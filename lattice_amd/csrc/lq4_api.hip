@@ -44,7 +44,7 @@ struct lq4_ctx {
     hipEvent_t state_event;  // recorded on the previous stream when a call arrives on another one
     int gemm_kernel;         // lq4_set_gemm_kernel
     int gemv_kernel;         // lq4_set_gemv_kernel: which kernel serves a plain one-token GEMV
-    int gemv_i8;             // LQ4_GEMV_I8: 1 = 3..8 rows of small matrices take the integer matrix-core kernel (default),
+    int gemv_i8;             // LQ4_GEMV_I8: 1 = the integer matrix-core kernel where it is the fastest at 2..8 rows (default),
                              // 0 = never, 2 = 2..8 rows of every matrix it can serve (tests)
     int moe_gemm_pairs;      // LQ4_MOE_GEMM_PAIRS: (token, slot) pairs per expert from which the grouped GEMM serves, -1 = by shape
     lq4_path_counters counters;
@@ -492,7 +492,7 @@ static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t b
 // slices per workgroup) overtakes the 4x4x4 GEMV kernel: always from nine rows; from five for
 // mid-sized matrices only (measured: behind for 512 x 2048, where its two launches dominate,
 // and for 12288 x 2048, where the GEMV kernel's grid already fills the chip), and not where the integer
-// matrix-core kernel serves (3072 x 2048 at 5..8 rows 5.8-5.9 us here, 5.4-5.5 there; 4096 x 2048 6.2 / 5.5).
+// matrix-core kernel serves (3072 x 2048 at 5..8 rows 5.8-5.9 us here, 4.3 there; 4096 x 4096 7.5 / 6.5).
 static bool gemv_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch, bool with_lora) {
     const uint64_t weights = static_cast<uint64_t>(n) * k;
     // (not for up to 2048 rows while the GEMV kernel can stage the activations: its eight-wave
@@ -1677,7 +1677,7 @@ int lq4_gemv_fused_batch(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_off
             act_in = xs;
             pro = LQ4_PRO_NONE;
             if (f.epilogue == LQ4_EPI_NONE && gemv_takes_i8(ctx, n, k, batch)) {
-                // what is left is a plain product: the kernel that lq4_gemv takes for it (12288 x 2048 at eight rows 10.4 -> 8.6 us)
+                // what is left is a plain product: the kernel that lq4_gemv takes for it (12288 x 2048 at eight rows 10.4 -> 6.9 us)
                 launch_gemv_i8(wp, n, k, xs, k, batch, y_dev, n, LoraEpilogue{}, ctx->cu_count, s);
                 ctx->counters.gemv_fused++;
                 LQ4_HIP(hipGetLastError());

@@ -22,7 +22,7 @@
 //    as all the activations of a 64-token step; as dense 16-byte pieces a quarter of that (17408 x 5120 at 20 tokens 29.0 -> 22.0
 //    us, 4096 x 4096 at 128 tokens 15.6 -> 13.6, 2048 x 6144 at 100 14.7 -> 12.7; 64 x 2048 x 2048 is latency, 6.9 both ways).  What
 //    is left of a step is its activations, four loads of 1 KB a token group through the CU's 64 bytes a clock.
-//    Each wave adds its share of the LoRA delta (ranks w, w + 8, ...) to its partial result in
+//    Each wave adds its share of the LoRA delta (ranks 2 w, 2 w + 1, then 16 on) to its partial result in
 //    f32; the eight partial results then meet in LDS in a fixed order and y is stored once.
 //    MULTI = true: the workgroups' row tiles run over several matrices of the same K stacked one under the other
 //    (lq4_gemv_multi at 9..128 rows), each with an output and a LoRA delta of its own.
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         }
     };
 
-    // ---- LoRA: wave w adds the ranks w, w + 8, ... of scale * B[row, :] . t[token, :] to its own partial result in f32, so the
+    // ---- LoRA: wave w adds the ranks 2 w, 2 w + 1 (then 16 on) of scale * B[row, :] . t[token, :] to its own partial result in f32, so the
     // delta is spread over all waves and joins their reduction.  The factors of its first two ranks are requested ahead of
     // everything else (behind the K loop their whole latency would stand: the launch is latency from end to end).
     //   LORA = 2: they are what the accumulators start from.  The first step waits for them, but no register is held: 118

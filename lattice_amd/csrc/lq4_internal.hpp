@@ -147,8 +147,7 @@ void launch_gemv_b1(const uint8_t* w, uint32_t n, uint32_t k, const float* x, fl
                     const LoraEpilogue& lora, hipStream_t stream);
 // 2..8 activation rows on the integer matrix cores (lq4_gemv_i8.hip): y = W . x, optional LoRA epilogue with t in
 // memory or computed by producer workgroups of the launch (gemv_i8_lora_in_launch).  gemv_i8_serves: the staged activations fit the LDS (K up to about 7000).
-// Tall matrices of short rows (at least two 16-row tiles per CU, K up to about 2900), which the kernel serves with
-// two eight-wave workgroups per CU.
+// gemv_i8_many_short_rows: at least two 16-row tiles per CU, K of 1024..2816.  gemv_i8_busy: see there.
 bool gemv_i8_many_short_rows(uint32_t n, uint32_t k, uint32_t cu_count);
 bool gemv_i8_busy(uint32_t n, uint32_t k, uint32_t cu_count);
 bool gemv_i8_serves(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count);
@@ -271,8 +270,8 @@ void launch_gemv_q3_b1(const uint8_t* w, uint32_t n, uint32_t k, const float* x,
 void launch_gemm_q3(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m, float* y,
                     float* scratch, int forced, hipStream_t stream);
 
-// Few-token variant (up to 128 tokens): activations packed once into matrix-core operand order
-// (gemm_skinny_scratch_bytes bytes at `packed_x`), then a kernel without LDS staging.
+// Few-token variant (up to 128 tokens, small matrices up to 1024): activations packed once into matrix-core operand order
+// (gemm_skinny_scratch_bytes bytes at `packed_x`), then a kernel whose weights come through wave-private LDS.
 bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora);
 // `adapters`: those of the launch whose t = A . X it computes.
 size_t gemm_skinny_scratch_bytes(uint32_t k, uint32_t m, uint32_t adapters = 0);

@@ -1,9 +1,9 @@
 // CPython entry to the C ABI of liblattice_hip_q4.so for the calls an engine makes many times a token
 // (built by lattice_amd/build.py next to the library; loaded by lattice_amd/backend.py).
 //
-// A launch costs the HIP runtime 2.4 us on this machine.  Through ctypes (argument objects, a structure filled
+// A launch costs the HIP runtime 2.2 us on this machine.  Through ctypes (argument objects, a structure filled
 // field by field) and torch.cuda.current_stream() a one-row GEMV cost the host 6.8 us, i.e. two thirds of the call were
-// spent before the library saw it; with these wrappers the same call takes 3.6 us (4096 x 1024, one row), an eight-row decode
+// spent before the library saw it; with these wrappers the same call takes 3.3 us (4096 x 1024, one row), an eight-row decode
 // layer's host time falls from 39 to 24 us.
 // The GIL is released around the call, as ctypes does: a call may allocate or wait on a full queue.
 #define PY_SSIZE_T_CLEAN
