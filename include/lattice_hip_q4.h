@@ -138,7 +138,7 @@ int lq4_lora_apply(lq4_ctx* ctx, const lq4_lora* lora, float lora_scale, const v
  * activation makes every output NaN); at batch 2..16 activations are split into unscaled f16 pairs
  * (two rows) or rounded to f16 (more), and |x| >= 65504 becomes infinity -- except where the integer
  * matrix-core kernel serves the call (2..8 rows where it is the fastest, most matrices of K up to 5120, unless
- * the context was created under LQ4_GEMV_I8=0): it keeps 24 bits (up to four rows: an f32 GEMV, as the
+ * the context was created under LQ4_GEMV_I8=0): it keeps 28 bits (up to four rows: an f32 GEMV, as the
  * reference's gemm_q4 is) or 16 bits (five to eight) of every activation below its 32-element block's
  * largest magnitude and takes any finite f32 value; a row that holds an infinity or a NaN comes back
  * NaN.  The guaranteed contract is the weaker one. */

@@ -463,8 +463,8 @@ static void plain_gemv_one_token(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, ui
     ctx->counters.gemv++;
 }
 
-// 2..8 rows on the integer matrix-core kernel, which keeps 24 (up to four rows) or 16 bits of every activation below its block's
-// maximum where the others round it to f16: wherever it is the faster one, or, for the tests, whatever it can hold.  us there (4x4x4
+// 2..8 rows on the integer matrix-core kernel, which keeps 28 (up to four rows) or 16 bits of every activation below its block's
+// maximum where the others round it to f16 (two rows: to pairs of f16): wherever it is the faster one, or, for the tests, whatever it can hold.  us there (4x4x4
 // kernel or few-token GEMM) / here:
 //   up to 4096 rows, K up to 2048: from three rows (512 x 2048 4.2 / 3.6, 2048 x 2048 4.8 / 3.9, at eight 5.5 / 4.3; at two 3.6 / 3.8);
 //   at 2560 rows and more K up to 5120: at three 2560 x 2560 5.4 / 4.5, 4096 x 4096 8.1 / 5.4, 12288 x 2048 8.3 / 6.6, 12288 x

@@ -6,12 +6,12 @@
 // rows with 16 activation columns, and the block's scale and bias are applied to its result in f32 afterwards.
 //   B operand (32 x 16): the weights.  Lane l supplies column n = l % 16 (a weight row), k = 8 * (l / 16) .. + 7:
 //     the eight nibbles of payload dword l / 16 of that row's block, spread into bytes by two masks.
-//   A operand (16 x 32): the activations, staged as fixed point scaled per block (x = xs * q, xs = the block's largest
-//     magnitude / the largest q) and cut into signed byte digits.  Five to eight activation rows: two digits each
-//     (q = 256 hi + lo, 16 bits), operand row m = 2 b + digit, so eight rows fill the operand and nothing of the
-//     instruction is idle.  Up to four rows ("wide"): three digits each (24 bits), m = 4 b + digit.
+//   A operand (16 x 32): the activations, staged as fixed point scaled per block (x = xs * q) and cut into signed byte
+//     digits; either way they fill the operand.  Five to eight activation rows: two digits each (q = 256 hi + lo, xs = the
+//     block's largest magnitude / 32639), operand row m = 2 b + digit.  Up to four rows ("wide"): four digits each (28 bits
+//     and sign, xs a power of two), m = 4 b + digit.
 //   D (16 x 16): lane l receives column n = l % 16, rows m = 4 (l / 16) .. + 3, i.e. for ITS weight row both digits
-//     of activation rows 2 (l / 16) and 2 (l / 16) + 1 (wide: the three digits of row l / 16).  256 hi + lo is one
+//     of activation rows 2 (l / 16) and 2 (l / 16) + 1 (wide: the four digits of row l / 16).  256 hi + lo is one
 //     integer multiply-add, and
 //       y[b, n] += (scale_n * xs_b) * (256 hi + lo) + bias_n * (xs_b * sum of the block's fixed-point x)
 //     needs the block header of the lane's own row only, and every lane owns two outputs of its row from the first block to
@@ -45,11 +45,15 @@
 // that has not arrived after the poll limit is computed by the wave that misses it, in the producers' order of
 // summation (same bits), and counted in sync[2].
 //
-// Precision.  The weights enter exactly, the integer sums are exact.  An activation is rounded to a multiple of its
-// block's largest magnitude / 32639 (two digits: step 3e-5 of the block maximum, against 5e-4 of the element for the
-// f16 rounding of the 4x4x4 kernel and of the reference's tiled kernel, shaders/gemm_q4_tiled.metal:45-48) or
-// / 8355711 (wide: 1.2e-7, the resolution of the f32 activation itself, so up to four rows track an f32 GEMV as the
-// reference's gemm_q4 does).  Any finite f32 activation is in range (the scale is per block); a block whose largest
+// Precision.  The weights enter exactly, the integer sums are exact.  Five to eight rows: an activation is rounded to a
+// multiple of its block's largest magnitude / 32639 (step 3e-5 of the block maximum, against 5e-4 of the element for the
+// f16 rounding of the 4x4x4 kernel and of the reference's tiled kernel, shaders/gemm_q4_tiled.metal:45-48).  Up to four rows
+// it is cut off below 2^-27 .. 2^-28 of the block's largest magnitude: an f32 value of at least a 16th of that, and an f16
+// value of at least a 2^-16th, enters exactly, so they track an f32 GEMV as the reference's gemm_q4 does.  (Two rows are
+// served by pairs of f16 values elsewhere, 22 bits of each element.  Three digits, 22 bits and sign below the block's maximum,
+// kept fewer of elements far below it.  2560 x 4096, rms of the activations' rounding alone, pairs / three digits / four: N(0,1)
+// 4.4e-8 / 1.7e-7 / 2e-9, one channel in 64 a hundred times larger 4.3e-8 / 3.8e-7 / 1.6e-8; of the results against f64 6.5e-6 / 2.2e-7 /
+// 1.5e-7 and 1.5e-5 / 4.1e-7 / 1.5e-7.  The fourth digit is free in the instruction; staging it costs 2048 x 2048 3.86 -> 3.98 us.)  Any finite f32 activation is in range (the scale is per block); a block whose largest
 // magnitude is below 2^-100 counts as zero; an infinite or NaN activation makes the outputs of its row NaN.
 #include "lq4_internal.hpp"
 
@@ -158,7 +162,7 @@ __device__ __forceinline__ float a_row_dot(const void* a, int a_is_f16, uint32_t
     return p;
 }
 
-// WIDE: up to four activation rows at three digits; else up to eight at two.
+// WIDE: up to four activation rows at four digits; else up to eight at two.
 // CW x TW waves: CW waves split the chunks of one tile, TW tiles are worked on side by side.
 // MULTI: the rows are those of several matrices stacked one under the other (MultiViews: view v = rows [begin[v],
 // begin[v + 1]), every view a whole number of 16-row tiles), each with its own output [batch, rows of the view] and its
@@ -224,8 +228,8 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
     constexpr uint32_t kRows = WIDE ? 4 : 8;      // activation rows the operand holds
     constexpr int kTaskBlocks = 16 / kRows, kTasks = kBpw / kTaskBlocks, kMyTasks = kTasks > TW ? kTasks / TW : 1;
     // q = rint(x / xs) with xs = block maximum / kQScale: |q| stays below kQScale + 2 whatever the rounding of the
-    // reciprocal, every digit within -128..127; wide: 22 bits and sign, what the float trick below can hold
-    constexpr float kQScale = WIDE ? 4194000.0f : 32639.0f;
+    // reciprocal, both digits within -128..127.  (Wide: below.)
+    constexpr float kQScale = 32639.0f;
     const uint32_t kg = lane & 3, xb = (static_cast<uint32_t>(lane) >> 2) & (kRows - 1), xblk = static_cast<uint32_t>(lane) / (4 * kRows);
     auto task_block = [&](uint32_t c, int i) { return (c * CW + cw) * kBpw + (tw + i * TW) * kTaskBlocks + xblk; };
     // rows and blocks that do not exist re-read an existing one
@@ -238,9 +242,12 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
         v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, false)));
         return max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false)));
     };
-    auto quad_sum = [](int v) {
-        v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
-        return v + __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
+    auto quad_sum = [](auto v) {
+        auto of = [](auto w, auto ctrl) {
+            return __builtin_bit_cast(decltype(w), __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, w), decltype(ctrl)::value, 0xF, 0xF, false));
+        };
+        v += of(v, std::integral_constant<int, 0xB1>{});
+        return v + of(v, std::integral_constant<int, 0x4E>{});
     };
     auto stage_chunk = [&](uint32_t c, auto xv_of) {
         float my_xs = 0.0f, my_sum = 0.0f;  // k group i's lane: of the wave's i-th task
@@ -256,38 +263,50 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
             for (int j = 0; j < 8; ++j) abits = max(abits, as_u32(v[j]) & 0x7FFFFFFFu);
             abits = quad_max(abits);
             const bool none = abits < 0x0D800000u || task_block(c, i) >= nb;  // below 2^-100, or past the end of the row: counts for nothing
-            const float xs_any = as_f32(abits) * (1.0f / kQScale), inv_any = __builtin_amdgcn_rcpf(xs_any);
-            const float inv = none ? 0.0f : inv_any;
-            // (an infinite or NaN activation: the row's outputs become NaN)
-            const float xs = none ? 0.0f : abits >= 0x7F800000u ? as_f32(0x7FC00000u) : xs_any;
-            // 1.5 * 2^23 + q as a float has q in its low 23 bits in two's complement: bits = 0x4B400000 + q
-            uint32_t qb[8], sum_bits = 0;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                qb[j] = as_u32(fmaf(v[j], inv, 12582912.0f));
-                sum_bits += qb[j];
-            }
-            const int sum = quad_sum(static_cast<int>(sum_bits - 8u * 0x4B400000u));
-            my_xs = kg == static_cast<uint32_t>(i) ? xs : my_xs;
-            my_sum = kg == static_cast<uint32_t>(i) ? static_cast<float>(sum) : my_sum;
-            // Digits -128..127 from the lowest up: byte 0 of q, byte 1 of q + 0x80, byte 2 of q + 0x8080 (minus the
-            // 0x40 the float's own bits hold there).  Byte p of an operand word pair = element {0, 2, 4, 6, 1, 3, 5,
-            // 7}[p] of the k group: the order in which the two masks lay out a payload dword's nibbles.
-            constexpr int kDigits = WIDE ? 3 : 2;
+            constexpr int kDigits = WIDE ? 4 : 2;
             uint32_t dg[kDigits][2];
+            float xs, sum;  // sum: of the block's q, in units of xs
             if constexpr (WIDE) {
+                // q = x * 2^(154 - e), truncated, with e = the maximum's exponent field (27 and more): |q| < 2^28, so that eight
+                // of them add up in 32 bits.  xs is what 2^16 of q stand for, so that it is no denormal.
+                const uint32_t e = abits >> 23;
+                const float inv = none ? 0.0f : as_f32((281u - e) << 23);
+                xs = none ? 0.0f : abits >= 0x7F800000u ? as_f32(0x7FC00000u) : as_f32((e - 11u) << 23);
+                int lane_sum = 0;
+                // Byte i of q + 0x80808080, less 128, is digit i (-128..127) of q.  u: those of element {0, 2, 4, 6}[p] (h = 0) or
+                // {1, 3, 5, 7}[p], as the two masks lay out a payload dword's nibbles; a digit's four go into one dword.
 #pragma unroll
-                for (int t = 0; t < kDigits; ++t) {
-                    const uint32_t add = t == 0 ? 0u : t == 1 ? 0x80u : 0xFFC08080u;
-                    // byte t of (qb + add) of four elements into one dword: 0x0c selects a zero byte
-                    const uint32_t sel_lo = 0x0c0c0400u + 0x0101u * t, sel_hi = 0x04000c0cu + 0x01010000u * t;
+                for (int h = 0; h < 2; ++h) {
+                    uint32_t u[4];
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {  // h = 0: elements 0, 2, 4, 6;  h = 1: elements 1, 3, 5, 7
-                        const uint32_t e0 = qb[h] + add, e1 = qb[2 + h] + add, e2 = qb[4 + h] + add, e3 = qb[6 + h] + add;
-                        dg[t][h] = __builtin_amdgcn_perm(e1, e0, sel_lo) | __builtin_amdgcn_perm(e3, e2, sel_hi);
+                    for (int p = 0; p < 4; ++p) {
+                        const int q = static_cast<int>(v[2 * p + h] * inv);
+                        lane_sum += q;
+                        u[p] = (static_cast<uint32_t>(q) + 0x80808080u) ^ 0x80808080u;
                     }
+                    const uint32_t a0 = __builtin_amdgcn_perm(u[1], u[0], 0x05010400u), a1 = __builtin_amdgcn_perm(u[3], u[2], 0x05010400u);
+                    const uint32_t b0 = __builtin_amdgcn_perm(u[1], u[0], 0x07030602u), b1 = __builtin_amdgcn_perm(u[3], u[2], 0x07030602u);
+                    dg[0][h] = __builtin_amdgcn_perm(a1, a0, 0x05040100u);
+                    dg[1][h] = __builtin_amdgcn_perm(a1, a0, 0x07060302u);
+                    dg[2][h] = __builtin_amdgcn_perm(b1, b0, 0x05040100u);
+                    dg[3][h] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
                 }
+                sum = quad_sum(static_cast<float>(lane_sum) * (1.0f / 65536.0f));
             } else {
+                const float xs_any = as_f32(abits) * (1.0f / kQScale), inv_any = __builtin_amdgcn_rcpf(xs_any);
+                const float inv = none ? 0.0f : inv_any;
+                // (an infinite or NaN activation: the row's outputs become NaN)
+                xs = none ? 0.0f : abits >= 0x7F800000u ? as_f32(0x7FC00000u) : xs_any;
+                // 1.5 * 2^23 + q as a float has q in its low 23 bits in two's complement: bits = 0x4B400000 + q
+                uint32_t qb[8], sum_bits = 0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    qb[j] = as_u32(fmaf(v[j], inv, 12582912.0f));
+                    sum_bits += qb[j];
+                }
+                sum = static_cast<float>(quad_sum(static_cast<int>(sum_bits - 8u * 0x4B400000u)));
+                // Digits -128..127 from the lowest up: byte 0 of q, byte 1 of q + 0x80.  Byte p of an operand word pair = element
+                // {0, 2, 4, 6, 1, 3, 5, 7}[p] of the k group: the order in which the two masks lay out a payload dword's nibbles.
                 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
                 const u16x2 up = {0x80, 0x80};
 #pragma unroll
@@ -299,10 +318,12 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                     dg[1][h] = __builtin_amdgcn_perm(h1, h0, 0x07050301u);
                 }
             }
+            my_xs = kg == static_cast<uint32_t>(i) ? xs : my_xs;
+            my_sum = kg == static_cast<uint32_t>(i) ? sum : my_sum;
             // operand row of (b, digit): the highest digit first
+            uint4* const to = reinterpret_cast<uint4*>(dst + i * (TW * kTaskBlocks * kXqBytes));
 #pragma unroll
-            for (int t = 0; t < kDigits; ++t)
-                *reinterpret_cast<uint2*>(dst + i * (TW * kTaskBlocks * kXqBytes) + (kDigits - 1 - t) * 8) = make_uint2(dg[t][0], dg[t][1]);
+            for (int t = 0; t < kDigits; t += 2) to[t / 2] = make_uint4(dg[kDigits - 1 - t][0], dg[kDigits - 1 - t][1], dg[kDigits - 2 - t][0], dg[kDigits - 2 - t][1]);
         }
         if (kg < static_cast<uint32_t>(kMyTasks)) {
             // of a chunk: [row pair g][2 block + row of the pair] xs (wide: [row][2 block]), then [block][row] xs * sum
@@ -526,8 +547,8 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                 constexpr int jj = decltype(jc)::value, j = j0 + jj;
                 const float s0 = of_row_lane<2 * j>(xs) * sc[jj];
                 if constexpr (WIDE) {
-                    // the top digit's sum times 2^16 is exact in f32, so is 256 mid + low: one rounding in the add
-                    acc.x = fmaf(s0, fmaf(static_cast<float>(d[jj].x), 65536.0f, static_cast<float>(d[jj].y * 256 + d[jj].z)), acc.x);
+                    // the sums of the two digits above and of the two below are exact in f32: one rounding in their add
+                    acc.x = fmaf(s0, fmaf(static_cast<float>(d[jj].z * 256 + d[jj].w), 1.0f / 65536.0f, static_cast<float>(d[jj].x * 256 + d[jj].y)), acc.x);
                 } else {
                     const float s1 = of_row_lane<2 * j + 1>(xs) * sc[jj];
                     acc.x = fmaf(s0, static_cast<float>(d[jj].x * 256 + d[jj].y), acc.x);

@@ -1,0 +1,95 @@
+"""What the integer matrix-core GEMV keeps of the activations at two to four rows: 27 bits and more below their 32-element block's
+largest magnitude, so in sum no fewer than the pairs of f16 (22 bits of each element) that serve two rows elsewhere; and every
+finite f32 in range."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from lattice_amd import backend, synth
+from util import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def context(which):
+    old = os.environ.get("LQ4_GEMV_I8")
+    os.environ["LQ4_GEMV_I8"] = which
+    try:
+        return backend.HipQ4Backend(0)
+    finally:
+        if old is None:
+            del os.environ["LQ4_GEMV_I8"]
+        else:
+            os.environ["LQ4_GEMV_I8"] = old
+
+
+@pytest.fixture(scope="module")
+def contexts():
+    c = {w: context(w) for w in ("0", "1", "2")}  # never, by the rule, wherever it can be held
+    yield c
+    for b in c.values():
+        b.close()
+
+
+def gemv(be, x, wq, n, k):
+    import torch
+    y = torch.full((len(x), n), float("nan"), device="cuda")
+    be.gemv_batch(torch.from_numpy(x).cuda(), be.upload_q4_blocks(wq), y, len(x), n, k)
+    return y.cpu().numpy().astype(np.float64)
+
+
+def norm_err(got, want):
+    return np.linalg.norm(got - want) / np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("small", [1.0, 2.0 ** -5, 2.0 ** -8])
+@pytest.mark.parametrize("n,k", [(48, 2048), (33, 288)])
+@pytest.mark.parametrize("batch", [2, 3, 4])
+def test_elements_far_below_their_blocks_maximum(contexts, n, k, batch, small):
+    """Element 5 of every block has the block's largest magnitude and meets weights of exactly zero (code 0, bias 0, nothing that
+    cancels): the result is made of the others alone."""
+    print(f"i8 precision n={n} k={k} batch={batch} small={small}", flush=True)
+    rng = np.random.default_rng(n + batch)
+    blocks = np.frombuffer(bytes(synth.q4_weight(n, k, seed=n)), np.uint8).reshape(-1, 20).copy()
+    blocks[:, 2:4] = 0                                   # bias
+    blocks[:, 4 + 5 // 2] &= 0x0F if 5 % 2 else 0xF0     # code of element 5
+    x = (rng.normal(size=(batch, k)) * small).astype(np.float32)
+    x[:, 5::32] = rng.uniform(2, 4, size=x[:, 5::32].shape) * np.sign(x[:, 5::32])
+    wq = blocks.tobytes()
+    assert np.all(oracle.dequantize(wq, n * k).reshape(n, k)[:, 5::32] == 0)
+    e = norm_err(gemv(contexts["2"], x, wq, n, k), oracle.gemm_f64(x, wq, n, k))
+    # An element is cut below 2^-26 (maxima of 2..4, 28 bits), i.e. by at most 2^-26 / small of its size, 0.6 of that rms; twice that
+    # for sums over few rows, beside f32 sums.  Three digits, steps of 2^-20, are off by 1e-5 and 1e-4 at the last two sizes.
+    print(f"  {e:.2e}", flush=True)
+    assert e <= 3e-7 + 1.2 * 2.0 ** -26 / small
+
+
+@pytest.mark.parametrize("outliers", [False, True])
+@pytest.mark.parametrize("n,k", [(2560, 4096), (4096, 2048)])
+def test_two_rows_are_no_further_from_f64_than_without_the_kernel(contexts, n, k, outliers):
+    print(f"i8 two rows n={n} k={k} outliers={outliers}", flush=True)
+    wq = synth.q4_weight(n, k, seed=n)
+    x = synth.activations(2, k, seed=k)
+    if outliers:
+        x[:, ::64] *= 100
+    want = oracle.gemm_f64(x, wq, n, k)
+    e = {w: norm_err(gemv(be, x, wq, n, k), want) for w, be in contexts.items()}
+    print(f"  {e}", flush=True)
+    assert e["1"] == e["2"] <= e["0"]
+
+
+def test_range_and_non_finite_rows(contexts):
+    n, k = 64, 256
+    w = synth.q4_weight(n, k, seed=9)
+    for scale in (1e30, 1e-30, 2.0 ** -96):
+        x = synth.activations(4, k, seed=10)
+        x[1] *= np.float32(scale)
+        x[2, 17] = np.inf
+        x[3, 200] = np.nan
+        got = gemv(contexts["2"], x, w, n, k)
+        want = oracle.gemm_f64(x[:2], w, n, k)
+        for b in (0, 1):
+            assert np.all(np.isfinite(got[b])) and rel_err(got[b], want[b].astype(np.float32)) <= 5e-6, (scale, b)
+        assert np.all(np.isnan(got[2])) and np.all(np.isnan(got[3]))
