@@ -1900,8 +1900,8 @@ int lq4_gemv_chain(lq4_ctx* ctx, const lq4_chain_step* steps, uint32_t n_steps, 
 }
 
 // (a forced kernel choice holds from 129 rows on)
-static bool sibling_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t m, int fmt, hipStream_t stream) {
-    return (m <= 128 || ctx->gemm_kernel == 0) && gemm_skinny_wants(n, k, m, fmt, false) &&
+static bool sibling_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t m, int fmt, int x_is_f16, hipStream_t stream) {
+    return (m <= 128 || ctx->gemm_kernel == 0) && gemm_skinny_wants(n, k, m, fmt, false, x_is_f16) &&
            few_token_choice(ctx, gemm_skinny_scratch_bytes(k, m), stream) == ctx->gemm_kernel;
 }
 
@@ -1921,7 +1921,7 @@ int lq4_gemm_q8(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
     if (m == 1 && x_dtype == LQ4_F32 && gemv_q8_lds_bytes(k) <= 128 * 1024) {
         launch_gemv_q8_b1(wp, n, k, static_cast<const float*>(x_dev), y_dev, s);
         ctx->counters.gemv++;
-    } else if (m <= 32 || sibling_takes_few_token_gemm(ctx, n, k, m, 1, s)) {
+    } else if (m <= 32 || sibling_takes_few_token_gemm(ctx, n, k, m, 1, x_dtype == LQ4_F16, s)) {
         // few rows: operands packed once, the few-token matrix-core kernel with this format's decoder
         // (always up to 32 rows: the large-tile kernels are no match for it there)
         const int src = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, m), static_cast<hipStream_t>(stream));
@@ -1962,7 +1962,7 @@ int lq4_gemm_q3(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint
     if (m == 1 && x_dtype == LQ4_F32 && gemv_q3_lds_bytes(k) <= 128 * 1024) {
         launch_gemv_q3_b1(wp, n, k, static_cast<const float*>(x_dev), y_dev, s);
         ctx->counters.gemv++;
-    } else if (m <= 32 || sibling_takes_few_token_gemm(ctx, n, k, m, 2, s)) {
+    } else if (m <= 32 || sibling_takes_few_token_gemm(ctx, n, k, m, 2, x_dtype == LQ4_F16, s)) {
         // few rows: operands packed once, the few-token matrix-core kernel with this format's decoder
         // (always up to 32 rows: the large-tile kernels are no match for it there)
         const int src = ensure_scratch(ctx, gemm_skinny_scratch_bytes(k, m), static_cast<hipStream_t>(stream));

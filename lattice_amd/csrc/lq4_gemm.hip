@@ -521,7 +521,7 @@ struct GemmPlan {
 };
 
 GemmPlan plan_gemm(uint32_t n, uint32_t k, uint32_t m, int x_is_f16, bool with_lora, int forced) {
-    if (forced == 3 || (forced == 0 && gemm_skinny_wants(n, k, m, 0, with_lora))) return {false, true, false};
+    if (forced == 3 || (forced == 0 && gemm_skinny_wants(n, k, m, 0, with_lora, x_is_f16))) return {false, true, false};
     if (forced == 1 || !gemm_wreg_supports(n, k, m, x_is_f16)) return {false, false, false};
     if (!with_lora && (forced == 4 || (forced == 0 && gemm_w2_wants(n, k, m)))) return {false, false, true};
     // The weights-in-registers kernel everywhere else: its scheduling cuts a partly filled last round

@@ -899,12 +899,18 @@ void gemm_skinny_pack_lora_a(const void* a, int a_is_f16, uint32_t rank, uint32_
 // 384 2048 x 2048 19.3 / 17.6, 2048 x 3072 18.6 / 22.3, 4096 x 1024 13.9 / 16.3, at 768 1024 x 1024 16.9 / 13.9, 1024 x 2048 18.1 / 20.5):
 //   33..64: 4096 x 12288 30.6 / 24.4; 8192 x 8192 30.5 / 24.6; 12288 x 2048 18.2 / 16.6, 12288 x 3072 21.7 / 21.9; 16384 x 2048 22.7 / 17.6
 //   65..128: 512 x 17408 23.4 / 18.9; 2048 x 8192 20.6 / 19.1, 2048 x 10240 22.0 / 21.8; 4096 x 6144 21.8 / 19.4; 8192 x 2048 20.1 / 15.8, 8192 x 3072 21.4 / 21.8
+// This kernel packs X into the context's scratch.  The large tiles use none where they run a product whole (rows of fewer than
+// four steps, or a last round that is nearly full): such a call needs nothing of the context, can be captured on a new one, takes
+// the same kernel whether scratch has grown or not, and replays beside other calls.  It keeps that above 128 tokens and in the
+// entries marked `sliced`, also where it would be faster here (us there / here: 129 x 64 x 512 8.1 / 4.4, 256 x 1000 x 384 7.8 / 5.3, 160 x 4096 x
+// 768 12.3 / 8.3, 160 x 8192 x 1024 15.3 / 12.4, 40 x 20196 x 1152 15.5 / 13.8; Q8_0 192 x 6144 x 768 12.8 / 13.8, 104 x 8104 x 64 6.9 / 8.6).
 namespace {
 struct ShapeLimit {
     uint32_t n, k_min, k_max;
+    bool sliced = false;  // only what the large tiles run as K slices
 };
-constexpr ShapeLimit kPlain64[] = {{4096, 0, 17408}, {8192, 0, 14336}, {12288, 0, 6144}, {16384, 1024, 5120}, {20480, 1056, 3072}};
-constexpr ShapeLimit kPlain128[] = {{1024, 0, 17408}, {2048, 0, 14336}, {4096, 0, 7680}, {8192, 0, 3584}, {12288, 1056, 2560}, {16384, 1056, 1536}};
+constexpr ShapeLimit kPlain64[] = {{4096, 0, 17408}, {8192, 0, 14336}, {12288, 0, 6144}, {16384, 1024, 5120}, {20480, 1056, 3072, true}};
+constexpr ShapeLimit kPlain128[] = {{1024, 0, 17408}, {2048, 0, 14336}, {4096, 0, 7680}, {8192, 0, 3584}, {12288, 1056, 2560, true}, {16384, 1056, 1536, true}};
 constexpr ShapeLimit kPlain192[] = {{512, 0, 14336}, {1024, 0, 10240}, {2048, 0, 6144}, {4096, 0, 4096}, {6144, 0, 3072}, {8192, 1024, 2048}};
 constexpr ShapeLimit kPlain256[] = {{1024, 0, 10240}, {2048, 0, 6144}, {3072, 0, 4096}, {4096, 0, 3072}, {6144, 1024, 2048}};
 constexpr ShapeLimit kPlain384[] = {{512, 0, 8192}, {1024, 0, 4096}, {2048, 0, 3072}, {3072, 0, 2048}, {4096, 1024, 2048}};
@@ -913,30 +919,29 @@ constexpr ShapeLimit kPlain768[] = {{256, 0, 4096}, {512, 0, 3072}, {1024, 0, 20
 constexpr ShapeLimit kPlain1024[] = {{256, 0, 3072}, {512, 0, 2048}, {1024, 768, 1536}};
 constexpr ShapeLimit kLora64[] = {{4096, 0, 17408}, {8192, 0, 14336}, {12288, 0, 6144}, {16384, 0, 5120}, {24576, 0, 2560}};
 constexpr ShapeLimit kLora128[] = {{1024, 0, 17408}, {4096, 0, 10240}, {8192, 0, 4096}, {12288, 0, 2560}, {16384, 1024, 2048}};
-constexpr ShapeLimit kSibling64[] = {{4096, 0, 12288}, {8192, 0, 8192}, {12288, 0, 2560}, {16384, 512, 2048}};
-constexpr ShapeLimit kSibling128[] = {{512, 0, 17408}, {2048, 0, 8192}, {4096, 0, 6144}, {8192, 0, 2560}};
-template <size_t N>
-bool within(const ShapeLimit (&limits)[N], uint32_t n, uint32_t k, bool narrowed = false) {
-    for (const ShapeLimit& l : limits)
-        if (n <= l.n) return narrowed ? l.k_min <= 512 && k >= l.k_min && k + k / 2 <= l.k_max : k >= l.k_min && k <= l.k_max;
-    return false;
-}
+constexpr ShapeLimit kSibling64[] = {{4096, 0, 12288}, {8192, 0, 8192}, {12288, 0, 2560}, {16384, 512, 2048, true}};
+constexpr ShapeLimit kSibling128[] = {{512, 0, 17408}, {2048, 0, 8192}, {4096, 0, 6144}, {8192, 0, 2560, true}};
 }  // namespace
 
-bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora) {
+bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora, int x_is_f16) {
     if (k < kBlockWeights) return false;
     if (m <= 16) return true;
     if (m <= 32) return static_cast<uint64_t>(n) * k <= (1ull << 28);
+    auto sliced = [&] { return (fmt ? gemm_sibling_scratch_floats(fmt, n, k, m, x_is_f16, 0) : gemm_wreg_scratch_floats(n, k, m, 0, x_is_f16 != 0)) != 0; };
+    auto within = [&](const auto& limits, bool narrowed = false) {
+        for (const ShapeLimit& l : limits)
+            if (n <= l.n) return (narrowed ? l.k_min <= 512 && k >= l.k_min && k + k / 2 <= l.k_max : k >= l.k_min && k <= l.k_max) && (!l.sliced || sliced());
+        return false;
+    };
     if (m <= 128) {
-        if (fmt) return m <= 64 ? within(kSibling64, n, k) : within(kSibling128, n, k);
-        if (with_lora) return m <= 64 ? within(kLora64, n, k) : within(kLora128, n, k);
-        return m <= 64 ? within(kPlain64, n, k) : within(kPlain128, n, k);
+        if (fmt) return m <= 64 ? within(kSibling64) : within(kSibling128);
+        if (with_lora) return m <= 64 ? within(kLora64) : within(kLora128);
+        return m <= 64 ? within(kPlain64) : within(kPlain128);
     }
-    // (shorter rows: a launch of one to three steps of the large tiles is as long as the two here.  256 x 1000 x 128 6.0 / 6.5, x 256 6.9 / 6.5)
-    if (with_lora || k < 256) return false;
-    if (m <= 256) return m <= 192 ? within(kPlain192, n, k, fmt) : within(kPlain256, n, k, fmt);
-    if (m <= 512) return m <= 384 ? within(kPlain384, n, k, fmt) : within(kPlain512, n, k, fmt);
-    if (m <= 1024) return m <= 768 ? within(kPlain768, n, k, fmt) : within(kPlain1024, n, k, fmt);
+    if (with_lora || !sliced()) return false;
+    if (m <= 256) return m <= 192 ? within(kPlain192, fmt) : within(kPlain256, fmt);
+    if (m <= 512) return m <= 384 ? within(kPlain384, fmt) : within(kPlain512, fmt);
+    if (m <= 1024) return m <= 768 ? within(kPlain768, fmt) : within(kPlain1024, fmt);
     return false;
 }
 

@@ -270,9 +270,9 @@ void launch_gemv_q3_b1(const uint8_t* w, uint32_t n, uint32_t k, const float* x,
 void launch_gemm_q3(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m, float* y,
                     float* scratch, int forced, hipStream_t stream);
 
-// Few-token variant (up to 128 tokens, small matrices up to 1024): activations packed once into matrix-core operand order
+// Few-token variant (up to 128 tokens; up to 1024 small matrices whose large tiles would take scratch too): activations packed once into matrix-core operand order
 // (gemm_skinny_scratch_bytes bytes at `packed_x`), then a kernel whose weights come through wave-private LDS.
-bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora);
+bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora, int x_is_f16);
 // `adapters`: those of the launch whose t = A . X it computes.
 size_t gemm_skinny_scratch_bytes(uint32_t k, uint32_t m, uint32_t adapters = 0);
 // For Q4 and a LoRA rank this accepts the packing launch computes t = A . X when LoraEpilogue::a points to A as packed

@@ -32,8 +32,8 @@ def weights(be, fmt, n, k):
 # tokens, rows, K, served by the few-token kernel
 @pytest.mark.parametrize("fmt", ["q4", "q8", "q3"])
 @pytest.mark.parametrize("xdt", [np.float16, np.float32])
-@pytest.mark.parametrize("m,n,k,few", [(129, 17, 256, True), (129, 513, 1056, True), (176, 1023, 1184, True), (256, 130, 2080, True), (257, 47, 288, True),
-                                       (500, 512, 1056, True), (512, 33, 4064, True), (769, 250, 544, True), (912, 272, 1056, True), (1024, 256, 1056, True),
+@pytest.mark.parametrize("m,n,k,few", [(129, 17, 256, False), (129, 17, 1056, True), (129, 513, 1056, True), (176, 1023, 1184, True), (256, 130, 2080, True), (257, 47, 288, False), (257, 47, 800, True),
+                                       (500, 512, 1056, True), (512, 33, 4064, True), (769, 250, 544, False), (769, 250, 1056, True), (912, 272, 1056, True), (1024, 256, 1056, True),
                                        (1025, 64, 512, False), (192, 100, 224, False), (256, 6160, 1056, False), (1024, 520, 2080, False)])
 def test_edges_and_lines(be, fmt, m, n, k, few, xdt):
     import torch
