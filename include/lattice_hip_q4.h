@@ -422,7 +422,9 @@ int lq4_gemv_chain(lq4_ctx* ctx, const lq4_chain_step* steps, uint32_t n_steps, 
  * GEMVs of a few rows, packed few-token operands and the K slices of their A . X, MoE and shared-expert intermediates, lm_head logits, the results a chain keeps between its steps) to at
  * least `bytes` ahead of time.  The library grows them on demand
  * otherwise, which allocates: a call that would have to grow it while its stream is being captured
- * into a HIP graph returns LQ4_E_UNSUPPORTED instead (GEMVs in K slices excepted, see lq4_gemv).  Outgrown buffers stay allocated until
+ * into a HIP graph returns LQ4_E_UNSUPPORTED instead (GEMVs in K slices excepted, see lq4_gemv, and GEMMs of
+ * 17 rows and more whose large tiles make do with the scratch there is: they take those then, so a graph captured before the
+ * scratch has grown may hold another kernel than one captured after it).  Outgrown buffers stay allocated until
  * lq4_ctx_destroy, so launches already queued or captured keep valid addresses.  No counterpart in
  * the reference. */
 int lq4_ctx_reserve_scratch(lq4_ctx* ctx, size_t bytes);

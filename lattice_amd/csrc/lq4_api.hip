@@ -4,6 +4,7 @@
 // that would launch returns LQ4_E_HIP.
 #include "../../include/lattice_hip_q4.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -512,10 +513,11 @@ static bool gemv_takes_slices(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32
     return cap == hipStreamCaptureStatusNone;
 }
 
-// The kernel choice of a call that the few-token GEMM would serve with `bytes` of scratch: under stream capture, scratch that
-// is too small for its packed activations leaves the call to the large-tile kernel (2), which may need none.
-static int few_token_choice(const lq4_ctx* ctx, size_t bytes, hipStream_t stream) {
-    if (ctx->gemm_kernel != 0 || bytes <= ctx->moe_scratch_bytes) return ctx->gemm_kernel;
+// The kernel choice of a call that the few-token GEMM would serve with `bytes` of scratch and the large-tile kernel (2) with
+// `large_bytes`: under stream capture, scratch that holds the latter's but not the former's leaves it to that one.  (Where it
+// holds neither the call is refused, for want of `bytes`.)
+static int few_token_choice(const lq4_ctx* ctx, size_t bytes, size_t large_bytes, hipStream_t stream) {
+    if (ctx->gemm_kernel != 0 || bytes <= ctx->moe_scratch_bytes || large_bytes > ctx->moe_scratch_bytes) return ctx->gemm_kernel;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
     return cap == hipStreamCaptureStatusNone ? 0 : 2;
@@ -673,10 +675,14 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
         // (behind one packing launch), the others each into their own.  q, k and v of the 2B model at 64 tokens with
         // rank-16 adapters on q and v: 18.6 us projection by projection, 12.1 so.
         SkinnyViews few{};
-        uint32_t packed_t = 0;  // adapters whose t the packing launch would compute
-        for (uint32_t i = 0; i < count; ++i)
-            packed_t += proj[i].n && ep[i].rank && gemm_skinny_computes_t(ep[i].rank) && gemm_takes_few_token_kernel(proj[i].n, k, batch, 0, true, ctx->gemm_kernel);
-        const int which = few_token_choice(ctx, gemm_skinny_scratch_bytes(k, batch, packed_t), s);
+        uint32_t packed_t = 0;   // adapters whose t the packing launch would compute
+        size_t large_floats = 0;  // of the large-tile kernel in its place
+        for (uint32_t i = 0; i < count; ++i) {
+            if (!proj[i].n || !gemm_takes_few_token_kernel(proj[i].n, k, batch, 0, ep[i].rank != 0, ctx->gemm_kernel)) continue;
+            packed_t += gemm_skinny_computes_t(ep[i].rank);
+            large_floats = std::max(large_floats, gemm_scratch_floats(proj[i].n, k, batch, 0, ep[i].rank, 2));
+        }
+        const int which = few_token_choice(ctx, gemm_skinny_scratch_bytes(k, batch, packed_t), large_floats * sizeof(float), s);
         for (uint32_t i = 0, v = 0; i < count; ++i) {
             const lq4_projection& p = proj[i];
             if (p.n == 0) continue;
@@ -705,7 +711,7 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
         for (uint32_t i = 0; i < count; ++i) {
             const lq4_projection& p = proj[i];
             if (p.n == 0 || gemm_takes_few_token_kernel(p.n, k, batch, 0, ep[i].rank != 0, which)) continue;
-            const size_t scratch_bytes = gemm_scratch_floats(p.n, k, batch, 0, ep[i].rank != 0, which) * sizeof(float);
+            const size_t scratch_bytes = gemm_scratch_floats(p.n, k, batch, 0, ep[i].rank, which) * sizeof(float);
             if (scratch_bytes) {
                 const int rc = ensure_scratch(ctx, scratch_bytes, s);
                 if (rc) return rc;
@@ -911,7 +917,8 @@ int lq4_gemm(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
     }
     int which = ctx->gemm_kernel;
     if (gemm_takes_few_token_kernel(n, k, m, x_dtype == LQ4_F16, ep.rank != 0, which))
-        which = few_token_choice(ctx, gemm_skinny_scratch_bytes(k, m, ep.rank ? 1 : 0), s);
+        which = few_token_choice(ctx, gemm_skinny_scratch_bytes(k, m, gemm_skinny_computes_t(ep.rank)),
+                                 gemm_scratch_floats(n, k, m, x_dtype == LQ4_F16, ep.rank, 2) * sizeof(float), s);
     if (ep.rank && gemm_takes_few_token_kernel(n, k, m, x_dtype == LQ4_F16, true, which) && gemm_skinny_computes_t(ep.rank)) {
         ep.a = lora->a_packed;  // the few-token GEMM's packing launch computes A.X
     } else if (ep.rank) {
@@ -919,7 +926,7 @@ int lq4_gemm(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
         ctx->counters.lora_a++;
     }
     // shapes with too few tiles run as K slices into scratch partials, summed by a second kernel
-    const size_t scratch_bytes = gemm_scratch_floats(n, k, m, x_dtype == LQ4_F16, ep.rank != 0, which) * sizeof(float);
+    const size_t scratch_bytes = gemm_scratch_floats(n, k, m, x_dtype == LQ4_F16, ep.rank, which) * sizeof(float);
     if (scratch_bytes) {
         rc = ensure_scratch(ctx, scratch_bytes, static_cast<hipStream_t>(stream));
         if (rc) return rc;
@@ -1902,7 +1909,7 @@ int lq4_gemv_chain(lq4_ctx* ctx, const lq4_chain_step* steps, uint32_t n_steps, 
 // (a forced kernel choice holds from 129 rows on)
 static bool sibling_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t m, int fmt, int x_is_f16, hipStream_t stream) {
     return (m <= 128 || ctx->gemm_kernel == 0) && gemm_skinny_wants(n, k, m, fmt, false, x_is_f16) &&
-           few_token_choice(ctx, gemm_skinny_scratch_bytes(k, m), stream) == ctx->gemm_kernel;
+           few_token_choice(ctx, gemm_skinny_scratch_bytes(k, m), gemm_sibling_scratch_floats(fmt, n, k, m, x_is_f16, 0) * sizeof(float), stream) == ctx->gemm_kernel;
 }
 
 int lq4_gemm_q8(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_t n, uint32_t k,

@@ -535,9 +535,9 @@ bool gemm_takes_few_token_kernel(uint32_t n, uint32_t k, uint32_t m, int x_is_f1
     return plan_gemm(n, k, m, x_is_f16, with_lora, forced).skinny;
 }
 
-size_t gemm_scratch_floats(uint32_t n, uint32_t k, uint32_t m, int x_is_f16, bool with_lora, int forced) {
-    const GemmPlan p = plan_gemm(n, k, m, x_is_f16, with_lora, forced);
-    if (p.skinny) return (gemm_skinny_scratch_bytes(k, m, with_lora ? 1 : 0) + sizeof(float) - 1) / sizeof(float);
+size_t gemm_scratch_floats(uint32_t n, uint32_t k, uint32_t m, int x_is_f16, uint32_t rank, int forced) {
+    const GemmPlan p = plan_gemm(n, k, m, x_is_f16, rank != 0, forced);
+    if (p.skinny) return (gemm_skinny_scratch_bytes(k, m, gemm_skinny_computes_t(rank)) + sizeof(float) - 1) / sizeof(float);
     if (p.w2) return (gemm_w2_scratch_bytes(n, k, m) + sizeof(float) - 1) / sizeof(float);
     return p.wreg ? gemm_wreg_scratch_floats(n, k, m, 0, x_is_f16 != 0) : 0;
 }

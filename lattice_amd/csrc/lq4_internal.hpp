@@ -228,7 +228,7 @@ void launch_lora_b_accum(const void* b, int b_is_f16, uint32_t rank, uint32_t d_
 // gemm_scratch_floats = floats of scratch launch_gemm needs for the shape (0 = none).
 // `forced`: 0 = choose by shape, 1 = LDS-staged kernel, 2 = weights-in-registers kernel where supported,
 // 3 = few-token kernel, 4 = the weights-in-registers tile at two workgroups per CU (a context's setting).
-size_t gemm_scratch_floats(uint32_t n, uint32_t k, uint32_t m, int x_is_f16, bool with_lora, int forced);
+size_t gemm_scratch_floats(uint32_t n, uint32_t k, uint32_t m, int x_is_f16, uint32_t rank, int forced);
 // true = launch_gemm serves the shape (with a LoRA epilogue) with the few-token kernel below
 bool gemm_takes_few_token_kernel(uint32_t n, uint32_t k, uint32_t m, int x_is_f16, bool with_lora, int forced);
 void launch_gemm(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int x_is_f16, uint32_t m,

@@ -78,3 +78,81 @@ def test_products_without_scratch_stay_without(fmt, m, n, k, xdt, whole):
         assert not np.array_equal(got, y.cpu().numpy())
     del call
     be.close()
+
+
+def many(be, wqs, n, k, m):
+    qws = [be.upload_q4_blocks(wq) for wq in wqs]
+    return lambda dx, ys: be.gemv_multi(dx, [(q, n, y, None) for q, y in zip(qws, ys)], m, k)
+
+
+# shapes of the few-token kernel whose large tiles are whole (nothing reserved), or whose K slices fit where the packed
+# activations do not
+@pytest.mark.parametrize("fmt,m,n,k,reserve", [("q4", 17, 2048, 352, 0), ("q4", 100, 512, 352, 0), ("q4", 160, 128, 8192, 2 << 20), ("q8", 40, 1024, 352, 0),
+                                               ("q3", 120, 512, 256, 0), ("multi", 40, 512, 352, 0), ("multi", 128, 128, 8192, 1 << 20)])
+def test_capture_takes_the_large_tiles_where_only_their_scratch_fits(fmt, m, n, k, reserve):
+    import torch
+    print(f"few-token capture {fmt} m={m} n={n} k={k}", flush=True)
+    be = backend.HipQ4Backend(0)
+    wq, deq = blocks("q4" if fmt == "multi" else fmt, n, k)
+    x = synth.activations(m, k, seed=2)
+    dx = torch.from_numpy(x).cuda()
+    y, other = (torch.empty((m, n), device="cuda") for _ in range(2))
+    if fmt == "multi":
+        both = many(be, [wq, wq], n, k, m)
+        go = lambda: both(dx, (y, other))  # noqa: E731
+    else:
+        call = caller(be, fmt, wq)
+        go = lambda: call(dx, y, m, n, k)  # noqa: E731
+    if reserve:
+        be.reserve_scratch(reserve)
+    if fmt in ("q8", "q3"):
+        # (up to 32 rows always, above by the lines: there a forced kernel does not hold, the large tiles are what a capture takes)
+        got = captured(go, y)
+        assert rel_err(got, x @ deq.T) <= REL_TOL
+        go()
+        assert not np.array_equal(got, y.cpu().numpy())
+    else:
+        got = captured(go, y)
+        assert rel_err(got, x @ deq.T) <= REL_TOL
+        be.set_gemm_kernel(2)
+        go()
+        assert np.array_equal(got, y.cpu().numpy())
+        be.set_gemm_kernel(0)
+        go()
+        assert not np.array_equal(got, y.cpu().numpy())
+    go = call = both = None
+    be.close()
+
+
+@pytest.mark.parametrize("fmt,m,n,k,rank,need", [("q4", 100, 2048, 2048, 0, 7 * 16 * 4096), ("q4", 100, 2048, 2048, 32, 7 * 16 * 4096), ("q8", 100, 1024, 2048, 0, 7 * 16 * 4096),
+                                                 ("multi", 64, 1024, 2048, 0, 4 * 16 * 4096)])
+def test_capture_that_fits_neither_names_the_packed_activations(fmt, m, n, k, rank, need):
+    """K slices of the large tiles would take several times the bytes of the packed activations (need: token groups x K steps x 4 KB)."""
+    import torch
+    print(f"few-token refused {fmt} m={m} n={n} k={k} rank={rank}", flush=True)
+    be = backend.HipQ4Backend(0)
+    wq, _ = blocks("q4" if fmt == "multi" else fmt, n, k)
+    dx = torch.from_numpy(synth.activations(m, k, seed=2)).cuda()
+    y, other = (torch.empty((m, n), device="cuda") for _ in range(2))
+    kw = {}
+    if rank:
+        be.load_lora_adapter([backend.LoraLayerData(0, {"q_proj": synth.lora_pair(rank, k, n, seed=3)})], scale=2.0)
+        kw = dict(layer_idx=0, module="q_proj")
+    if fmt == "multi":
+        both = many(be, [wq, wq], n, k, m)
+        go = lambda: both(dx, (y, other))  # noqa: E731
+    elif rank:
+        qw = be.upload_q4_blocks(wq)
+        go = lambda: be.dispatch_gemm(dx, 0, qw, y, 0, m, n, k, **kw)  # noqa: E731
+    else:
+        call = caller(be, fmt, wq)
+        go = lambda: call(dx, y, m, n, k)  # noqa: E731
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with pytest.raises(backend.Q4Error, match=f"to {need} bytes"):
+        with torch.cuda.stream(stream):
+            with torch.cuda.graph(graph, stream=stream):
+                go()
+    be.reserve_scratch(need)
+    assert np.all(np.isfinite(captured(go, y)))  # and what it names is enough
+    go = call = both = qw = None
+    be.close()
