@@ -476,7 +476,7 @@ static void plain_gemv_one_token(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, ui
 //     eight K up to 5120 (1536 x 5120 7.5 / 6.7, 512 x 3072 5.6 / 4.9; at five 5.1 / 5.0 and 4.7 / 4.9);
 //   two rows: 2560..4096 rows (4096 x 2048 4.4 / 3.9, 4096 x 5120 7.8 / 6.6, 2560 x 4096 6.1 / 5.3; 4096 x 1536 3.9 / 4.4) and 7168 and more
 //     with K of 2048..4096 (8192 x 2816 10.3 / 7.6, 10240 x 3072 11.9 / 8.7, 24576 x 2048 13.7 / 10.8; 12288 x 2560 8.6 / 9.0, 6144 x 2560 6.0 / 6.3).
-static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch, bool with_lora = false) {
+static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch) {
     if (batch < 2 || batch > 8 || !ctx->gemv_i8 || !gemv_i8_serves(n, k, batch, ctx->cu_count)) return false;
     if (ctx->gemv_i8 == 2) return true;
     if (batch >= 3 && k <= 2048 && n <= 4096) return true;
@@ -485,8 +485,8 @@ static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t b
     if (batch == 2) return k >= 2048 && ((n >= 2560 && n <= 4096) || (n >= 7168 && k <= 4096 && (n <= 10240 || k == 2048 || k >= 2816)));
     if (n < 2560) return n >= 512 && k <= (batch >= 7 ? 5120u : n >= 1024 ? 2816u : 2048u);
     if (k < 1024 || (n > 12288 && k > 4096 && batch < 8)) return false;
-    // (the few-token GEMM computes the factors of an adapter on its way; here they are a launch of their own unless CUs are left)
-    return batch < 5 || n >= 8192 || (gemv_i8_busy(n, k, ctx->cu_count) && !(with_lora && n > 3072));
+    // (the same line with an adapter, so that a projection is served by the same arithmetic with and without it)
+    return batch < 5 || n >= 8192 || gemv_i8_busy(n, k, ctx->cu_count);
 }
 
 // Above four activation rows the few-token matrix-core kernel (operands packed once, eight K
@@ -494,12 +494,12 @@ static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t b
 // mid-sized matrices only (measured: behind for 512 x 2048, where its two launches dominate,
 // and for 12288 x 2048, where the GEMV kernel's grid already fills the chip), and not where the integer
 // matrix-core kernel serves (3072 x 2048 at 5..8 rows 5.8-5.9 us here, 4.3 there; 4096 x 4096 7.5 / 6.5).
-static bool gemv_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch, bool with_lora) {
+static bool gemv_takes_few_token_gemm(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch) {
     const uint64_t weights = static_cast<uint64_t>(n) * k;
     // (not for up to 2048 rows while the GEMV kernel can stage the activations: its eight-wave
     // workgroups then win, 2048 x 6144 at 5..8 rows 9.5 -> 7.2..8.2 us)
     const bool narrow = n <= 2048 && gemv_mfma_lds_bytes(k, batch < 8 ? batch : 8) <= 150 * 1024;
-    return batch >= 9 || (batch >= 5 && n < 8192 && !narrow && weights >= 6000000 && !gemv_takes_i8(ctx, n, k, batch, with_lora));
+    return batch >= 9 || (batch >= 5 && n < 8192 && !narrow && weights >= 6000000 && !gemv_takes_i8(ctx, n, k, batch));
 }
 
 // K slices on the 4x4x4 matrix-core kernel (no LoRA step there).  Their partial results live in the context's scratch, so only
@@ -528,7 +528,7 @@ static int few_token_choice(const lq4_ctx* ctx, size_t bytes, size_t large_bytes
 static int gemv_dispatch(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, uint32_t k, const float* x_dev, uint32_t batch,
                          float* y_dev, const LoraEpilogue& ep, hipStream_t s) {
     int rc;
-    if (gemv_takes_few_token_gemm(ctx, n, k, batch, ep.rank != 0)) {
+    if (gemv_takes_few_token_gemm(ctx, n, k, batch)) {
         if (gemv_takes_slices(ctx, n, k, batch, ep.rank != 0, false, s)) {
             rc = ensure_scratch(ctx, gemv_mfma_sliced_scratch_bytes(n, k, batch), s);
             if (rc) return rc;
@@ -542,7 +542,7 @@ static int gemv_dispatch(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, uint32_t k
         ctx->counters.gemm++;
     } else if (batch == 1 && !ep.rank) {
         plain_gemv_one_token(ctx, wp, n, k, x_dev, y_dev, s);
-    } else if (gemv_takes_i8(ctx, n, k, batch, ep.rank != 0)) {
+    } else if (gemv_takes_i8(ctx, n, k, batch)) {
         launch_gemv_i8(wp, n, k, x_dev, k, batch, y_dev, n, ep, ctx->cu_count, s);
         ctx->counters.gemv++;
     } else {
@@ -579,9 +579,9 @@ int lq4_gemv(lq4_ctx* ctx, const lq4_weight* w, uint64_t w_extra_offset, uint32_
         ep.slots = reinterpret_cast<unsigned long long*>(ctx->lora_sync + 64);
         ep.sync = ctx->lora_sync;
         ep.spin_limit = ctx->lora_spin_limit;
-    } else if (ep.rank && batch > 1 && gemv_takes_few_token_gemm(ctx, n, k, batch, true) && gemm_skinny_computes_t(ep.rank)) {
+    } else if (ep.rank && batch > 1 && gemv_takes_few_token_gemm(ctx, n, k, batch) && gemm_skinny_computes_t(ep.rank)) {
         ep.a = lora->a_packed;  // the few-token GEMM's packing launch computes A.x
-    } else if (ep.rank && ctx->lora_in_kernel && gemv_takes_i8(ctx, n, k, batch, true) &&
+    } else if (ep.rank && ctx->lora_in_kernel && gemv_takes_i8(ctx, n, k, batch) &&
                gemv_i8_lora_in_launch(n, k, batch, ep.rank, ctx->cu_count)) {
         // 2..8 rows: `rank` producer workgroups of the launch, on CUs the matrix leaves idle
         ep.a = lora->a;
@@ -729,13 +729,13 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
     const bool in_launch = stacked && with_lora && ctx->lora_in_kernel && total_rank <= 64;
     // two to eight rows: the integer matrix-core kernel over the stacked rows, where it is the faster one
     const bool stacked_rows = !stacked && batch >= 2 && batch <= 8 && mv.count > 1 &&
-                              ((ctx->gemv_i8 && k <= 2048 && mv.begin[mv.count] <= 4096) || gemv_takes_i8(ctx, mv.begin[mv.count], k, batch, with_lora)) &&
+                              ((ctx->gemv_i8 && k <= 2048 && mv.begin[mv.count] <= 4096) || gemv_takes_i8(ctx, mv.begin[mv.count], k, batch)) &&
                               gemv_i8_multi_serves(mv, k, batch, ctx->cu_count);
     if (with_lora && !stacked && !stacked_rows) {
         // those that go to the few-token GEMM get their A . x with its packing launch
         for (uint32_t i = 0, v = 0; i < count; ++i) {
             if (proj[i].n == 0) continue;
-            if (ep[i].rank && gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch, true) && gemm_skinny_computes_t(ep[i].rank)) {
+            if (ep[i].rank && gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch) && gemm_skinny_computes_t(ep[i].rank)) {
                 ep[i].a = proj[i].lora->a_packed;
                 av.rank[v] = 0;
                 --with_lora;
@@ -780,7 +780,7 @@ int lq4_gemv_multi(lq4_ctx* ctx, const lq4_projection* proj, uint32_t count, uin
         SkinnyViews few{};
         for (uint32_t i = 0; i < count; ++i) {
             if (proj[i].n == 0) continue;
-            if (gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch, ep[i].rank != 0)) {
+            if (gemv_takes_few_token_gemm(ctx, proj[i].n, k, batch)) {
                 few_token_view(&few, proj[i].n, wp[i], proj[i].y_dev, ep[i], ep[i].a);
                 continue;
             }

@@ -57,6 +57,7 @@
 // magnitude is below 2^-100 counts as zero; an infinite or NaN activation makes the outputs of its row NaN.
 #include "lq4_internal.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace lq4 {
@@ -693,12 +694,15 @@ namespace {
 struct I8Split {
     uint32_t cw, tw, steps;  // columns of chunks, tiles side by side, units a wave is left with
 };
+uint32_t steps_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count, uint32_t cw, uint32_t tw) {
+    return ((n_tiles + tw - 1) / tw + cu_count - 1) / cu_count * ((chunks + cw - 1) / cw);
+}
 I8Split split_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count) {
     // Up to a tile a CU: as many waves as split its chunks, up to eight.  With more, eight waves as 8, 4 or 2 columns of chunks
     // beside 1, 2 or 4 tiles, whichever leaves a wave the fewest units (12288 x 2560 is 5 as 2 x 4, 6 else; 8 x 1 has
     // the shorter staging, so it is taken where it is no worse).
     I8Split best{chunks >= 8 ? 8u : chunks >= 4 ? 4u : chunks >= 2 ? 2u : 1u, 1, 0};
-    auto steps = [&](uint32_t cw, uint32_t tw) { return ((n_tiles + tw - 1) / tw + cu_count - 1) / cu_count * ((chunks + cw - 1) / cw); };
+    auto steps = [&](uint32_t cw, uint32_t tw) { return steps_i8(n_tiles, chunks, cu_count, cw, tw); };
     best.steps = steps(best.cw, best.tw);
     if (n_tiles <= cu_count || chunks < 2) return best;
     best.steps = ~0u;
@@ -707,13 +711,27 @@ I8Split split_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count) {
     return best;
 }
 
-bool plan_i8(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count, I8Plan* out) {
+// producers: workgroups of the launch that compute LoRA factors.  Where they find no idle CU beside the usual split, but do beside
+// more tiles in a workgroup at up to two steps more, that one: the launch for the factors which they save takes three (rank 16, eight
+// rows, us with that launch / so / plain: 5120 x 4096 12.5 / 10.2 / 9.0, 4096 x 2048 7.7 / 6.4 / 4.5, 12288 x 2048 10.8 / 9.9 / 7.2, 4096 x 2560 8.3 / 7.9 /
+// 5.3, 4096 x 4096 10.3 / 9.7 / 7.0).
+bool plan_i8(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count, I8Plan* out, uint32_t producers = 0) {
     if (k == 0 || k % kBlockWeights || n == 0 || batch == 0 || batch > 8) return false;
     const uint32_t nb = k / kBlockWeights;
     const uint32_t chunks = (nb + kBpw - 1) / kBpw;
     const uint32_t n_tiles = (n + 15) / 16;
     I8Plan p;
-    const I8Split split = split_i8(n_tiles, chunks, cu_count);
+    I8Split split = split_i8(n_tiles, chunks, cu_count);
+    auto fits = [&](const I8Split& s) { return std::min((n_tiles + s.tw - 1) / s.tw, cu_count) + producers <= cu_count; };
+    if (producers && split.cw * split.tw == 8 && !fits(split)) {
+        const uint32_t usual = split.steps;
+        for (uint32_t tw = 2 * split.tw; tw <= 4; tw *= 2) {
+            const I8Split s{8 / tw, tw, steps_i8(n_tiles, chunks, cu_count, 8 / tw, tw)};
+            if (!fits(s) || s.steps > usual + 2) continue;
+            split = s;
+            break;
+        }
+    }
     p.cw = split.cw;
     p.tw = split.tw;
     auto bytes = [&](uint32_t stages) {
@@ -787,7 +805,7 @@ bool gemv_i8_serves(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count) {
 void launch_gemv_i8(const uint8_t* w, uint32_t n, uint32_t k, const float* x, uint32_t x_stride, uint32_t batch,
                     float* y, uint32_t y_stride, const LoraEpilogue& lora, uint32_t cu_count, hipStream_t stream) {
     I8Plan p;
-    if (!plan_i8(n, k, batch, cu_count, &p)) return;  // the caller asked gemv_i8_serves first
+    if (!plan_i8(n, k, batch, cu_count, &p, lora.slots ? lora.rank : 0)) return;  // the caller asked gemv_i8_serves first
     const MultiViews none{};
     launch_i8_rows<false>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, none, lora.rank != 0, stream);
 }
@@ -797,7 +815,7 @@ void launch_gemv_i8(const uint8_t* w, uint32_t n, uint32_t k, const float* x, ui
 // 16-byte row of A can be loaded (K a multiple of 8 elements is given: K is a multiple of 32).
 bool gemv_i8_lora_in_launch(uint32_t n, uint32_t k, uint32_t batch, uint32_t rank_total, uint32_t cu_count) {
     I8Plan p;
-    return rank_total != 0 && rank_total <= static_cast<uint32_t>(kMaxLoraRank) && plan_i8(n, k, batch, cu_count, &p) &&
+    return rank_total != 0 && rank_total <= static_cast<uint32_t>(kMaxLoraRank) && plan_i8(n, k, batch, cu_count, &p, rank_total) &&
            p.grid + rank_total <= cu_count;
 }
 
@@ -814,7 +832,7 @@ void launch_gemv_i8_multi(const MultiViews& mv, uint32_t k, const float* x, uint
                           uint32_t cu_count, const LoraEpilogue* in_launch, hipStream_t stream) {
     const uint32_t n = mv.begin[mv.count];
     I8Plan p;
-    if (!plan_i8(n, k, batch, cu_count, &p)) return;  // the caller asked gemv_i8_multi_serves first
+    if (!plan_i8(n, k, batch, cu_count, &p, in_launch ? in_launch->rank : 0)) return;  // the caller asked gemv_i8_multi_serves first
     const LoraEpilogue hand = in_launch ? *in_launch : LoraEpilogue{};  // rank = the views' ranks together, slots, sync
     bool with_lora = false;
     for (uint32_t v = 0; v < mv.count; ++v) with_lora |= mv.rank[v] != 0;

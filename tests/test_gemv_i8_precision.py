@@ -93,3 +93,29 @@ def test_range_and_non_finite_rows(contexts):
         for b in (0, 1):
             assert np.all(np.isfinite(got[b])) and rel_err(got[b], want[b].astype(np.float32)) <= 5e-6, (scale, b)
         assert np.all(np.isnan(got[2])) and np.all(np.isnan(got[3]))
+
+
+@pytest.mark.parametrize("n,k,batch,rank", [(4096, 4096, 5, 16), (4096, 4096, 8, 64), (5120, 4096, 6, 16), (6144, 2560, 8, 8), (8064, 2560, 7, 16),
+                                            (4096, 2560, 5, 16), (4096, 2048, 8, 16), (12288, 2048, 5, 8), (5120, 4096, 3, 4)])
+def test_the_same_arithmetic_with_and_without_an_adapter(contexts, n, k, batch, rank):
+    """An adapter whose B is zero: the same integers, hence the same result to the order of f32 sums (workgroups may be split another
+    way to leave CUs for the factors); f16 activations or weights in its place would show at 1e-4.  With several views alike."""
+    import torch
+    print(f"i8 same arithmetic n={n} k={k} batch={batch} rank={rank}", flush=True)
+    be = contexts["1"]
+    wq = synth.q4_weight(n, k, seed=n)
+    x = synth.activations(batch, k, seed=k)
+    plain = gemv(be, x, wq, n, k)
+    a, b = synth.lora_pair(rank, k, n, seed=1)
+    a2, b2 = synth.lora_pair(rank, k, 64, seed=2)
+    qw, small, dx = be.upload_q4_blocks(wq), be.upload_q4_blocks(synth.q4_weight(64, k, seed=2)), torch.from_numpy(x).cuda()
+    y, z, s = (torch.full((batch, r), float("nan"), device="cuda") for r in (n, n, 64))
+    be.load_lora_adapter([backend.LoraLayerData(0, {"q_proj": (a, np.zeros_like(b)), "v_proj": (a2, b2)})], scale=2.0)
+    try:
+        be.gemv_batch(dx, qw, y, batch, n, k, layer_idx=0, module="q_proj")
+        be.gemv_multi(dx, [(qw, n, z, "q_proj"), (small, 64, s, "v_proj")], batch, k, layer_idx=0)
+        got = y.cpu().numpy(), z.cpu().numpy()
+    finally:
+        be.unload_lora_adapter()
+    for g in got:
+        assert norm_err(g, plain) <= 5e-7
