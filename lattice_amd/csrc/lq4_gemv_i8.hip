@@ -338,7 +338,7 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
     // The values of a wave's first chunks are requested before any weight (loads are answered in the order a CU
     // issued them: behind the weights the staging would wait for these), all at once.
     const bool stages_rows = tw < kTasks && my_chunks;  // uniform (more tiles side by side than tasks, or more waves than chunks: not all)
-    constexpr int kAhead = 2 * TW;  // chunks
+    constexpr int kAhead = TW < 4 ? 2 * TW : 8;  // chunks
     // (out of the way of the usual case, whose code then lies together: one chunk a wave with one tile at a time)
     auto has_chunk = [&](int c) { return c == 0 || (TW == 1 ? __builtin_expect(static_cast<uint32_t>(c) < my_chunks, 0) : static_cast<uint32_t>(c) < my_chunks); };
     f32x4 xv[kAhead][kMyTasks][2];
@@ -697,16 +697,18 @@ struct I8Split {
 uint32_t steps_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count, uint32_t cw, uint32_t tw) {
     return ((n_tiles + tw - 1) / tw + cu_count - 1) / cu_count * ((chunks + cw - 1) / cw);
 }
-I8Split split_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count) {
-    // Up to a tile a CU: as many waves as split its chunks, up to eight.  With more, eight waves as 8, 4 or 2 columns of chunks
-    // beside 1, 2 or 4 tiles, whichever leaves a wave the fewest units (12288 x 2560 is 5 as 2 x 4, 6 else; 8 x 1 has
-    // the shorter staging, so it is taken where it is no worse).
+I8Split split_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count, bool wide) {
+    // Up to a tile a CU: as many waves as split its chunks, up to eight.  With more, eight waves as 8, 4, 2 or 1 columns of chunks
+    // beside 1, 2, 4 or 8 tiles, whichever leaves a wave the fewest units (12288 x 2560 is 5 as 2 x 4, 6 else; 8 x 1 has
+    // the shorter staging, so it is taken where it is no worse).  One column only of short rows, which four of the waves stage (up to four
+    // activation rows: two): us as 2 x 4 / 1 x 8 at five rows 32768 x 1280 11.3 / 10.0, x 1792 13.1 / 12.0, x 2304 15.8 / 15.2, x 2816 17.7 / 18.3,
+    // at three rows 10.1 / 9.7, 12.5 / 12.1, 14.4 / 15.2.
     I8Split best{chunks >= 8 ? 8u : chunks >= 4 ? 4u : chunks >= 2 ? 2u : 1u, 1, 0};
     auto steps = [&](uint32_t cw, uint32_t tw) { return steps_i8(n_tiles, chunks, cu_count, cw, tw); };
     best.steps = steps(best.cw, best.tw);
     if (n_tiles <= cu_count || chunks < 2) return best;
     best.steps = ~0u;
-    for (uint32_t cw = 8; cw >= 2; cw /= 2)
+    for (uint32_t cw = 8; cw >= (chunks <= (wide ? 7u : 9u) ? 1u : 2u); cw /= 2)
         if (cw < 2 * chunks && steps(cw, 8 / cw) < best.steps) best = I8Split{cw, 8 / cw, steps(cw, 8 / cw)};
     return best;
 }
@@ -721,7 +723,7 @@ bool plan_i8(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count, I8Plan* 
     const uint32_t chunks = (nb + kBpw - 1) / kBpw;
     const uint32_t n_tiles = (n + 15) / 16;
     I8Plan p;
-    I8Split split = split_i8(n_tiles, chunks, cu_count);
+    I8Split split = split_i8(n_tiles, chunks, cu_count, batch <= 4);
     auto fits = [&](const I8Split& s) { return std::min((n_tiles + s.tw - 1) / s.tw, cu_count) + producers <= cu_count; };
     if (producers && split.cw * split.tw == 8 && !fits(split)) {
         const uint32_t usual = split.steps;
@@ -772,7 +774,7 @@ void launch_i8_shape(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, 
 #define LQ4_I8(CW_, TW_)                \
     if (p.cw == CW_ && p.tw == TW_)     \
     return launch_i8<CW_, TW_, WIDE, MULTI, LORA>(p, w, n, k, x, x_stride, batch, y, y_stride, lora, mv, stream)
-    LQ4_I8(8, 1); LQ4_I8(4, 2); LQ4_I8(2, 4); LQ4_I8(4, 1); LQ4_I8(2, 2); LQ4_I8(2, 1); LQ4_I8(1, 1);
+    LQ4_I8(8, 1); LQ4_I8(4, 2); LQ4_I8(2, 4); LQ4_I8(1, 8); LQ4_I8(4, 1); LQ4_I8(2, 2); LQ4_I8(2, 1); LQ4_I8(1, 1);
 #undef LQ4_I8
 }
 
@@ -791,10 +793,10 @@ void launch_i8_rows(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, c
 
 }  // namespace
 
-// The eight waves of every CU busy for at least 55 % of their steps.
+// The eight waves of every CU busy for at least 55 % of their steps (five to eight rows).
 bool gemv_i8_busy(uint32_t n, uint32_t k, uint32_t cu_count) {
     const uint32_t n_tiles = (n + 15) / 16, chunks = (k / kBlockWeights + kBpw - 1) / kBpw;
-    return static_cast<uint64_t>(n_tiles) * chunks * 100 >= 55ull * 8 * cu_count * split_i8(n_tiles, chunks, cu_count).steps;
+    return static_cast<uint64_t>(n_tiles) * chunks * 100 >= 55ull * 8 * cu_count * split_i8(n_tiles, chunks, cu_count, false).steps;
 }
 
 bool gemv_i8_serves(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count) {

@@ -29,7 +29,8 @@ def i8():
 
 @pytest.mark.parametrize("lead", [0, 20])
 @pytest.mark.parametrize("n,k", [(1, 32), (3, 160), (16, 224), (17, 256), (31, 288), (40, 1056), (33, 2048), (19, 2304), (24, 4128),
-                                 (4097, 1024), (8200, 1184), (12289, 2080), (300, 6944)])
+                                 (4097, 1024), (8200, 1184), (12289, 2080), (300, 6944),
+                                 (32763, 1184), (28700, 2080), (65530, 224)])  # one column of chunks beside eight tiles
 @pytest.mark.parametrize("batch", [2, 4, 5, 8])
 def test_rows_end_with_the_buffer(i8, lead, n, k, batch):
     import torch
