@@ -467,26 +467,29 @@ static void plain_gemv_one_token(lq4_ctx* ctx, const uint8_t* wp, uint32_t n, ui
 // 2..8 rows on the integer matrix-core kernel, which keeps 28 (up to four rows) or 16 bits of every activation below its block's
 // maximum where the others round it to f16 (two rows: to pairs of f16): wherever it is the faster one, or, for the tests, whatever it can hold.  us there (4x4x4
 // kernel or few-token GEMM) / here:
-//   up to 4096 rows, K up to 2048: from three rows (512 x 2048 4.2 / 3.6, 2048 x 2048 4.8 / 3.9, at eight 5.5 / 4.3; at two 3.6 / 3.8);
-//   at 2560 rows and more K up to 5120: at three 2560 x 2560 5.4 / 4.5, 4096 x 4096 8.1 / 5.4, 12288 x 2048 8.3 / 6.6, 12288 x
-//     5120 13.7 / 11.4, 24576 x 1024 9.6 / 6.6; at eight 6144 x 1024 5.4 / 4.1, 4096 x 4096 7.5 / 6.5, 12288 x 4096 17.5 / 11.3, 32768 x 3072
-//     21.0 / 17.2.  Not short rows of many (5120 x 512 at four 3.2 / 4.0); not much beyond (16384 x 4608 at three 15.3 / 15.8, x 5632 16.0 /
-//     19.0); and where the waves would stand idle for half of it not instead of the few-token GEMM (5120 x 2560 at five 6.7 / 7.0);
-//   fewer rows: K up to 2816 from 1024 on (1536 x 2560 at three 4.6 / 4.4, at eight 6.0 / 4.9; 512 x 2816 at three 4.1 / 4.3), at seven and
+//   up to 4096 rows, K up to 2048: from three rows, for the precision also where it is not (2048 x 2048 4.1 / 4.0, at eight 5.5 / 4.3; 512 x
+//     2048 3.6 / 3.7, 4096 x 512 2.7 / 3.3; at two 3.6 / 4.0);
+//   at 2560 rows and more K up to 5120: at three 2560 x 2560 5.4 / 4.6, 4096 x 4096 8.0 / 5.9, 12288 x 2048 8.2 / 7.0, 12288 x
+//     5120 13.8 / 12.0, 24576 x 1024 9.6 / 6.9 (but 6144 x 2560 6.0 / 6.5, 20480 x 2560 11.5 / 12.2); at eight 6144 x 1024 5.4 / 4.1, 4096 x 4096 7.5 / 6.8, 12288 x
+//     4096 17.5 / 12.0, 32768 x 3072 21.0 / 17.2.  Not short rows of many (5120 x 512 at four 3.2 / 4.0); not much beyond (16384 x 4608 at three
+//     15.3 / 15.8, x 5632 16.0 / 19.0); and where the waves would stand idle for half of it not instead of the few-token GEMM (5120 x 2560 at five 6.7 / 7.0);
+//   fewer rows: K up to 2816 from 1024 on (1536 x 2560 at three 4.6 / 4.5, at eight 6.0 / 4.9; 512 x 2816 at three 4.1 / 4.5), at seven and
 //     eight K up to 5120 (1536 x 5120 7.5 / 6.7, 512 x 3072 5.6 / 4.9; at five 5.1 / 5.0 and 4.7 / 4.9);
-//   two rows: 2560..4096 rows (4096 x 2048 4.4 / 3.9, 4096 x 5120 7.8 / 6.6, 2560 x 4096 6.1 / 5.3; 4096 x 1536 3.9 / 4.4) and 7168 and more
-//     with K of 2048..4096 (8192 x 2816 10.3 / 7.6, 10240 x 3072 11.9 / 8.7, 24576 x 2048 13.7 / 10.8; 12288 x 2560 8.6 / 9.0, 6144 x 2560 6.0 / 6.3).
+//   two rows: 2560..4096 rows (4096 x 2048 4.4 / 4.1, 4096 x 5120 7.9 / 6.7, 2560 x 4096 6.1 / 5.5; 4096 x 1536 3.9 / 4.6) and 7168 and more
+//     with K of 2048..4096 (8192 x 2816 10.2 / 7.3, 10240 x 3072 11.8 / 8.8, 24576 x 2048 13.7 / 11.0; 6144 x 2560 6.0 / 6.3), above 10240 of them
+//     K up to 2816 only where the waves are busy for more than three quarters of their steps (14336 x 2304 10.6 / 9.3, 24576 x 2560 15.0 / 13.5, 12288 x 2048 7.0 /
+//     7.0; 12288 x 2560 8.6 / 9.1, 20480 x 2304 11.6 / 12.1).
 static bool gemv_takes_i8(const lq4_ctx* ctx, uint32_t n, uint32_t k, uint32_t batch) {
     if (batch < 2 || batch > 8 || !ctx->gemv_i8 || !gemv_i8_serves(n, k, batch, ctx->cu_count)) return false;
     if (ctx->gemv_i8 == 2) return true;
     if (batch >= 3 && k <= 2048 && n <= 4096) return true;
     if (batch >= 5 && gemv_i8_many_short_rows(n, k, ctx->cu_count)) return true;
     if (k > 5120) return false;
-    if (batch == 2) return k >= 2048 && ((n >= 2560 && n <= 4096) || (n >= 7168 && k <= 4096 && (n <= 10240 || k == 2048 || k >= 2816)));
+    if (batch == 2) return k >= 2048 && ((n >= 2560 && n <= 4096) || (n >= 7168 && k <= 4096 && (n <= 10240 || k >= 2816 || gemv_i8_busier_than(75, n, k, batch, ctx->cu_count))));
     if (n < 2560) return n >= 512 && k <= (batch >= 7 ? 5120u : n >= 1024 ? 2816u : 2048u);
     if (k < 1024 || (n > 12288 && k > 4096 && batch < 8)) return false;
     // (the same line with an adapter, so that a projection is served by the same arithmetic with and without it)
-    return batch < 5 || n >= 8192 || gemv_i8_busy(n, k, ctx->cu_count);
+    return batch < 5 || n >= 8192 || gemv_i8_busier_than(55, n, k, batch, ctx->cu_count);
 }
 
 // Above four activation rows the few-token matrix-core kernel (operands packed once, eight K

@@ -793,10 +793,10 @@ void launch_i8_rows(const I8Plan& p, const uint8_t* w, uint32_t n, uint32_t k, c
 
 }  // namespace
 
-// The eight waves of every CU busy for at least 55 % of their steps (five to eight rows).
-bool gemv_i8_busy(uint32_t n, uint32_t k, uint32_t cu_count) {
+// The eight waves of every CU have a unit in more than `percent` of their steps.
+bool gemv_i8_busier_than(uint32_t percent, uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count) {
     const uint32_t n_tiles = (n + 15) / 16, chunks = (k / kBlockWeights + kBpw - 1) / kBpw;
-    return static_cast<uint64_t>(n_tiles) * chunks * 100 >= 55ull * 8 * cu_count * split_i8(n_tiles, chunks, cu_count, false).steps;
+    return static_cast<uint64_t>(n_tiles) * chunks * 100 > 8ull * percent * cu_count * split_i8(n_tiles, chunks, cu_count, batch <= 4).steps;
 }
 
 bool gemv_i8_serves(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count) {

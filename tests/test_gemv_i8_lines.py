@@ -36,7 +36,9 @@ def contexts():
     (2048, 2048, 2, False), (2560, 2048, 2, True), (4096, 2016, 2, False), (4097, 2048, 2, False), (7168, 2048, 2, True), (10256, 2304, 2, False),
     (4096, 2048, 3, True), (511, 2080, 3, False), (1024, 2816, 3, True), (1023, 2816, 3, False), (2560, 5120, 4, True), (2560, 5152, 4, False),
     (5120, 992, 4, False), (5120, 1024, 4, True), (12304, 4128, 4, False), (1536, 2848, 6, False), (1536, 2848, 7, True), (5120, 2560, 5, False),
-    (6144, 2560, 5, True), (8192, 3072, 5, True), (65552, 1024, 8, True)])
+    (6144, 2560, 5, True), (8192, 3072, 5, True), (65552, 1024, 8, True),
+    (10240, 2304, 2, True), (12288, 2048, 2, True), (12304, 2048, 2, True), (12288, 2080, 2, False), (12288, 2560, 2, False), (12288, 2816, 2, True), (14336, 2304, 2, True),
+    (20480, 2560, 2, False), (16384, 2784, 2, True)])
 def test_lines(contexts, n, k, batch, served):
     import torch
     print(f"i8 lines n={n} k={k} batch={batch}", flush=True)
