@@ -81,7 +81,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // wave-uniform.  By hand, like the loads of the activations: the compiler would make every LDS access wait for the former, and
 // count the latter without them.  The compiler knows of no hazard either: a vector load may read a scalar register five wait
 // states after a vector instruction wrote it (v_readlane, where the compiler keeps scalars in a vector register), so each brings
-// its own.
+// its own.  m0 cannot be named as written: it is reserved, and set by the compiler in front of whatever of its own reads it.
+// load16's register is filled only when a wait has passed: tests/test_isa.py looks for anything that touches it before.
 __device__ __forceinline__ void dma16(uint32_t lds, const void* base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
 }
