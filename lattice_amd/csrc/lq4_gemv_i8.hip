@@ -603,8 +603,6 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
                 }
                 // t of activation rows b0 and b1, `t0[i]` = factor i: from memory, or (producers) from LDS
                 auto delta = [&](auto* t0, auto* t1) {
-                    // (every load below is unconditional and used where it is made: a load left pending on one path
-                    // would make the compiler wait for the whole weight ring wherever its register is reused)
                     float l0 = 0.0f, l1 = 0.0f;
                     if (lo.b_is_f16 && lo.rank % 8 == 0) {
                         // eight factors a step: one 16-byte load of B[row, i..i+7] (the first two steps of the wave's
@@ -659,6 +657,12 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
 
     // The waves meet every kMeet rounds (once, where a workgroup has that many tiles or fewer): in between each goes at its own
     // pace, so that one reads LDS while another computes.  (With a meeting a round the four layers of a_row_dot's comment took 28.4 us, 24.9 so.)
+    // (with adapters: what finish and pick_up load is waited for at their end, in a form that the compiler sees.  Left to it, it assumes
+    // such loads pending on the registers that every unit of the product uses, and empties the ring in front of each: with rank 16
+    // 10240 x 4096 at eight rows 15.5 -> 14.2 us, 12288 x 4096 16.4 -> 14.7, 5120 x 5120 12.1 -> 11.1.)
+    auto settle = [] {
+        if constexpr (LORA) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    };
     for (uint32_t t = 0, u = 0, stage = 0; t < rounds; ++t) {
         if (t < my_tiles) {  // uniform in the wave
             acc0 = 0.0f;
@@ -669,10 +673,14 @@ __global__ __launch_bounds__(64 * CW * TW) void gemv_q4_i8(const uint8_t* __rest
             }
             *reinterpret_cast<float2*>(part + ((t % kMeet) * WAVES + wave) * (64 * 2) + lane * 2) = make_float2(acc0, acc1);
         }
-        if (prod && t == 0) pick_up();  // uniform
+        if (prod && t == 0) {  // uniform
+            pick_up();
+            settle();
+        }
         if ((t + 1) % kMeet == 0 || t + 1 == rounds) {
             __syncthreads();
             for (uint32_t q = t - t % kMeet + cw; q <= t && q < my_tiles; q += CW) finish(q);
+            settle();
             if (t + 1 < rounds) __syncthreads();
         }
     }

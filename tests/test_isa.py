@@ -2,7 +2,8 @@
 
 The integer matrix-core GEMV loads activations and adapter factors through inline assembly, which returns a register that the compiler
 believes filled, and waits for them through inline assembly further down.  A copy or a spill in between would carry old data; no
-result on the GPU would show it reliably."""
+result on the GPU would show it reliably.  And where the compiler believes loads of its own pending on registers of the product, it
+waits for everything in flight in front of every unit."""
 import os
 import re
 import shutil
@@ -125,3 +126,16 @@ def test_scalar_addresses_of_loads_by_hand_are_settled(kernels):
                 nop = re.match(r"s_nop (\d+)", ins[j][1])
                 states += int(nop[1]) + 1 if nop else 1
                 j -= 1
+
+
+def test_the_product_waits_for_no_load_but_by_hand(kernels):
+    """In the straight-line code of a unit's product: four blocks' matrix instructions twice, from its LDS reads on."""
+    for name, ins in kernels.items():
+        targets = {j for f in successors(ins) if len(f) != 1 for j in f} | {f[0] for i, f in enumerate(successors(ins)) if len(f) == 1 and f[0] != i + 1}
+        products = [i for i, (_, t) in enumerate(ins) if t.startswith("v_mfma_i32")]
+        assert len(products) == 8, name
+        start = products[0]
+        while start not in targets and not ins[start - 1][1].startswith(("s_branch", "s_cbranch")):
+            start -= 1
+        waits = [t for _, t in ins[start:products[-1]] if vmcnt(t) is not None]
+        assert not waits, (name, waits)
