@@ -16,8 +16,10 @@
 //    of NTG groups of 16 tokens.  Wave w takes K steps w, w + 8, ...; per step the load unit puts its 16 RT pieces of rows
 //    (four Q4 blocks, 80 bytes) into the wave's own part of LDS, where lane (r, g) picks up block g of row r; the packed
 //    operands come with fully coalesced 16-byte loads; it dequantises in registers and issues
-//    v_mfma_f32_16x16x32_f16.  No barrier in the K loop: nothing is shared between waves.  Two steps are in flight per wave;
-//    every load is unconditional (a load behind a run-time condition would make the compiler wait for loads it cannot count).
+//    v_mfma_f32_16x16x32_f16.  No barrier in the K loop: nothing is shared between waves.  Two steps are in flight per wave: the
+//    packed operands are loaded without a condition (behind one, the compiler would wait for loads it cannot count), the weights by
+//    hand (see dma16; with the builtin one step was in flight: 4096 x 4096 at 128 tokens 15.1 -> 14.1 us, 17408 x 5120 at 20 27.9 -> 26.7,
+//    2048 x 6144 at 12 9.4 -> 8.9, Q8_0 2048 x 6144 at 128 17.6 -> 16.9, weights from memory).
 //    Blocks straight from memory to the lanes (20 bytes at a row's stride) cost the address unit a clock a lane and load, as much
 //    as all the activations of a 64-token step; as dense 16-byte pieces a quarter of that (17408 x 5120 at 20 tokens 29.0 -> 22.0
 //    us, 4096 x 4096 at 128 tokens 15.6 -> 13.6, 2048 x 6144 at 100 14.7 -> 12.7; 64 x 2048 x 2048 is latency, 6.9 both ways).  What
@@ -119,9 +121,19 @@ struct WBlockOf<2> {
     static constexpr int kReads = 1;
 };
 
-// LDS reads by hand, with their waits: one the compiler knows of is made to wait for every global_load_lds in flight.
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((address_space(1))) const void global_void_t;
+// Memory -> LDS, 16 or 4 bytes a lane: lane l's bytes land at LDS byte address `lds` + 16 l (or + 4 l); `base` and `lds` are
+// wave-uniform.  By hand, like the LDS reads behind them and the waits: while one that the compiler knows of is in flight, it
+// empties the queue in front of every LDS access and of the first use of any other load.  (The builtin's steady state was one
+// unit in flight.)  The waits it places for the packed operands do not count these, so they wait for a few loads more.
+// The compiler knows of no hazard either: a vector load may read a scalar register five wait states after a vector instruction
+// wrote it, so each brings its own.  m0 cannot be named as written: it is reserved, and set by the compiler in front of whatever
+// of its own reads it.
+__device__ __forceinline__ void dma16(uint32_t lds, const void* base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void dma4(uint32_t lds, const void* base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
 template <int OFF>
 __device__ __forceinline__ u32x4 lds_read128(uint32_t addr) {
     u32x4 r;
@@ -460,18 +472,16 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     }
     auto load_w = [&](uint32_t s, int stage) {
         const uint32_t at = s * (4 * kBytes);
-        uint8_t* const to = w_lds + stage * (kLoads * 1024);
+        const uint32_t to = w_lds_at + stage * (kLoads * 1024);
         if (at + w_reach <= w_left) {
 #pragma unroll
-            for (int i = 0; i < kLoads; ++i)
-                __builtin_amdgcn_global_load_lds((global_void_t*)(w_base + (w_off[i] + at)), (lds_void_t*)(to + i * 1024), 16, 0, 0);
+            for (int i = 0; i < kLoads; ++i) dma16(to + i * 1024, w_base, w_off[i] + at);
         } else {
             // its last pieces would reach past the end of the matrix: dword by dword, those past it read its last one
 #pragma unroll 1
             for (int i = 0; i < 4 * kLoads; ++i) {
                 uint32_t off = piece_off(i * 16 + (lane >> 2)) + (lane & 3) * 4 + at;
-                off = off < w_left ? off : w_left - 4;
-                __builtin_amdgcn_global_load_lds((global_void_t*)(w_base + off), (lds_void_t*)(to + i * 256), 4, 0, 0);
+                dma4(to + i * 256, w_base, off < w_left ? off : w_left - 4);
             }
         }
     };
@@ -576,15 +586,19 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
 #pragma unroll
     for (int t = 0; t < NTG; ++t) xg[t] = tg0 + t < groups ? tg0 + t : groups - 1;
     // i-th step of this wave
-    auto load = [&](Unit& u, uint32_t i, int stage) {
-        const uint32_t s = wave + i * kWavesK;
-        load_w(s, stage);
-        __builtin_amdgcn_sched_barrier(0);
-        const uint4* xs = xp + static_cast<size_t>(s) * groups * 256 + lane;
+    auto load_x_of = [&](Unit& u, uint32_t i) {
+        const uint4* xs = xp + static_cast<size_t>(wave + i * kWavesK) * groups * 256 + lane;
 #pragma unroll
         for (int t = 0; t < NTG; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) u.x[t][j] = xs[(xg[t] * 4 + j) * 64];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // (the packed operands first: the loads behind them for which the compiler waits too many, not counting those of the weights, are
+    // then the next unit's operands and not its weights)
+    auto load = [&](Unit& u, uint32_t i, int stage) {
+        load_x_of(u, i);
+        load_w(wave + i * kWavesK, stage);
     };
 
     float4v acc[RT][NTG];
@@ -689,9 +703,11 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
     constexpr std::integral_constant<int, kLoads + 4 * NTG> unit{};
     if (cnt > 1) {
         Unit u0, u1;
-        load(u0, 0, 0);
-        load(u1, 1, 1);
+        load_w(wave, 0);
+        load_w(wave + kWavesK, 1);
         LQ4_FENCE();
+        load_x_of(u0, 0);
+        load_x_of(u1, 1);
         if constexpr (LORA == 2) add_requested();
         uint32_t i = 0;
         for (; i + 3 < cnt; i += 2) {
@@ -719,8 +735,9 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
         }
     } else if (cnt == 1) {
         Unit u0;
-        load(u0, 0, 0);
+        load_w(wave, 0);
         LQ4_FENCE();
+        load_x_of(u0, 0);
         if constexpr (LORA == 2) add_requested();
         compute(u0, 0, s0, none);
     } else {

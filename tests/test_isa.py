@@ -3,7 +3,8 @@
 The integer matrix-core GEMV loads activations and adapter factors through inline assembly, which returns a register that the compiler
 believes filled, and waits for them through inline assembly further down.  A copy or a spill in between would carry old data; no
 result on the GPU would show it reliably.  And where the compiler believes loads of its own pending on registers of the product, it
-waits for everything in flight in front of every unit."""
+waits for everything in flight in front of every unit.  The few-token GEMM's weights go into LDS by hand, beside operands that the
+compiler loads and waits for: its waits count from where those stand among the others, and must not empty the queue."""
 import os
 import re
 import shutil
@@ -32,28 +33,41 @@ def code_objects(path):
         pos = data.find(BUNDLE, pos + 1)
 
 
-@pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
-    """{name: [(address, text)]} of the integer matrix-core GEMV's instantiations."""
+def instantiations(kernel, tmp):
+    """{name: [(address, text)]}"""
     if not OBJDUMP:
         pytest.skip("no llvm-objdump")
     if not os.path.exists(build.LIB):
         build.build()
     out = {}
     for i, obj in enumerate(code_objects(build.LIB)):
-        if b"gemv_q4_i8" not in obj or b"launch" in obj[:64]:
+        if kernel.encode() not in obj:
             continue
-        f = tmp_path_factory.mktemp("isa") / f"{i}.co"
+        f = tmp / f"{i}.co"
         f.write_bytes(obj)
         name = None
         for line in subprocess.run([OBJDUMP, "-d", str(f)], capture_output=True, text=True, check=True).stdout.splitlines():
             head = re.match(r"[0-9a-f]+ <(\S+)>:", line)
             if head:
-                name = head[1] if "gemv_q4_i8" in head[1] else None
+                name = head[1] if kernel in head[1] else None
             elif name and "//" in line:
                 text, _, note = line.partition("//")
                 out.setdefault(name, []).append((int(note.split(":")[0], 16), text.strip()))
+    return out
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """Of the integer matrix-core GEMV."""
+    out = instantiations("gemv_q4_i8", tmp_path_factory.mktemp("i8"))
     assert len(out) == 64
+    return out
+
+
+@pytest.fixture(scope="module")
+def few_token(tmp_path_factory):
+    out = instantiations("gemm_q4_skinny", tmp_path_factory.mktemp("skinny"))
+    assert len(out) == 48
     return out
 
 
@@ -110,13 +124,15 @@ def test_nothing_touches_a_register_between_its_load_and_a_wait(kernels):
     assert loads > 64
 
 
-def test_scalar_addresses_of_loads_by_hand_are_settled(kernels):
+def test_scalar_addresses_of_loads_by_hand_are_settled(kernels, few_token):
     """Five wait states between a vector instruction that writes a scalar register and the load that reads it: the compiler counts
     them for its own instructions only."""
     writes = re.compile(r"v_(?:readlane|readfirstlane)_b32\S*\s+(s\d+)|v_cmp\S+\s+(s\[\d+:\d+\])")
-    for name, ins in kernels.items():
+    for name, ins in (kernels | few_token).items():
         for i, (a, text) in enumerate(ins):
             m = re.match(r"global_load\S*\s.*(s\[(\d+):(\d+)\])", text)
+            if m and name in few_token and "_lds_" not in text:
+                continue  # the compiler's own
             if not m:
                 continue
             base, states, j = {f"s{r}" for r in range(int(m[2]), int(m[3]) + 1)}, 0, i - 1
@@ -139,3 +155,32 @@ def test_the_product_waits_for_no_load_but_by_hand(kernels):
             start -= 1
         waits = [t for _, t in ins[start:products[-1]] if vmcnt(t) is not None]
         assert not waits, (name, waits)
+
+
+def test_the_few_token_loop_keeps_two_units_in_flight(few_token):
+    """The loop over K, two units a round: each unit's product, then the packed operands of the unit two places on, then its weights;
+    in front of a product a wait by hand that leaves what was requested behind the unit, and none of the compiler's that leaves less
+    than the next unit's operands."""
+    for name, ins in few_token.items():
+        rt, fmt, ntg = (int(v) for v in re.search(r"skinnyILi(\d)ELi(\d)ELi(\d)E", name).groups())
+        bodies = []
+        for i, follow in enumerate(successors(ins)):
+            for j in follow:
+                body = [t for _, t in ins[j:i + 1]]
+                if j <= i and any(t.startswith("v_mfma") for t in body) and any("_lds_" in t for t in body):
+                    bodies.append(body)
+        body = min(bodies, key=len)
+        kind = {"v_mfma": "M", "global_load_lds": "D", "global_load": "L"}
+        runs = []
+        for t in body:
+            k = next((v for p, v in kind.items() if t.startswith(p)), None)
+            if k:
+                runs[-1:] = [(k, runs[-1][1] + 1)] if runs and runs[-1][0] == k else runs[-1:] + [(k, 1)]
+        if runs[0][0] == runs[-1][0]:
+            runs[0] = (runs[0][0], runs[0][1] + runs.pop()[1])
+        order = "".join(k for k, _ in runs)
+        assert order in ("MLDMLD", "LDMLDM", "DMLDML"), (name, runs)
+        assert [c for k, c in runs if k == "M"] == [4 * rt * ntg] * 2 and [c for k, c in runs if k == "L"] == [4 * ntg] * 2, (name, runs)
+        loads = -(-16 * rt * (5, 9, 4)[fmt] // 64)
+        waits = [vmcnt(t) for t in body if vmcnt(t) is not None]
+        assert waits.count(loads + 4 * ntg) >= 2 and min(waits) >= 4 * ntg, (name, waits)
