@@ -56,9 +56,35 @@ def test_lines(contexts, n, k, batch, served):
     assert not served or rel_err(got["2"], want) <= max(rel_err(got["0"], want), 5e-6)
 
 
+@pytest.mark.parametrize("n,k,batch,served", [(4096, 4096, 3, True), (12304, 4128, 4, False), (6144, 2560, 5, True), (5120, 2560, 5, False),
+                                              (1536, 2848, 7, True), (1536, 2848, 6, False)])
+def test_lines_behind_a_norm(contexts, n, k, batch, served):
+    """What lq4_gemv_fused_batch leaves of a call once the norm is a launch of its own (more than 64 KB of rows and deltas) is a plain
+    product, by the same lines."""
+    import torch
+    print(f"i8 lines fused n={n} k={k} batch={batch}", flush=True)
+    wq = synth.q4_weight(n, k, seed=n)
+    x, delta, gamma = synth.activations(batch, k, seed=k), synth.activations(batch, k, seed=k + 2), synth.activations(1, k, seed=k + 1)[0] * 0.1
+    (dx, dd, dg), got = (torch.from_numpy(t).cuda() for t in (x, delta, gamma)), {}
+    for w, be in contexts.items():
+        y = torch.full((batch, n), float("nan"), device="cuda")
+        be.dispatch_matmul_fused(None, be.upload_q4_blocks(wq), y, n, k, norm=(dx, dd, dg, 1e-6, torch.empty_like(dx)), batch=batch)
+        got[w] = y.cpu().numpy()
+    x = x.astype(np.float64) + delta
+    normed = (x / np.sqrt(np.mean(x ** 2, axis=1, keepdims=True) + 1e-6) * (1 + gamma.astype(np.float64))).astype(np.float32)
+    assert rel_err(got["1"], oracle.gemm_f32(normed, wq, n, k)) <= REL_TOL
+    assert np.array_equal(got["1"], got["2" if served else "0"]) and not np.array_equal(got["0"], got["2"])
+
+
 @pytest.mark.parametrize("rank", [0, 16])
-@pytest.mark.parametrize("k,shapes,batch", [(4096, (4096, 1024, 1024), 3), (2560, (2560, 512, 512), 8), (3072, (3072, 48, 16), 5), (5120, (5120, 128, 128), 2)])
-def test_views_at_once(contexts, k, shapes, batch, rank):
+@pytest.mark.parametrize("k,shapes,batch,at_once", [
+    (4096, (4096, 1024, 1024), 3, True), (2560, (2560, 512, 512), 8, False), (3072, (3072, 48, 16), 5, True), (5120, (5120, 128, 128), 2, False),
+    (2048, (2048, 512, 512), 2, True),     # up to 4096 rows of K up to 2048 from two rows on, unlike one matrix
+    (4096, (2048, 512, 512), 2, True), (2048, (3072, 512, 528), 2, False),  # two rows: 2560..4096 rows together
+    (2560, (4096, 1024, 1024), 5, True),  # five and more: by how busy the waves are
+    (5152, (2560, 512, 512), 4, False), (2560, (4096, 1024, 1032), 8, False)])  # K; a view that is no whole number of tiles
+def test_views_at_once(contexts, k, shapes, batch, at_once, rank):
+    """By the sum of the views' rows, with and without adapters; elsewhere each view by its own."""
     import torch
     print(f"i8 views k={k} shapes={shapes} batch={batch} rank={rank}", flush=True)
     x = synth.activations(batch, k, seed=3)
@@ -72,8 +98,10 @@ def test_views_at_once(contexts, k, shapes, batch, rank):
         be.load_lora_adapter([backend.LoraLayerData(0, pairs)], scale=2.0)
         kw = dict(layer_idx=0)
     try:
+        before = be.path_counters()["gemv_multi"]
         ys = [torch.full((batch, n), float("nan"), device="cuda") for n in shapes]
         be.gemv_multi(dx, [(be.upload_q4_blocks(w), n, y, m) for w, n, y, m in zip(ws, shapes, ys, names)], batch, k, **kw)
+        assert be.path_counters()["gemv_multi"] - before == int(at_once)
     finally:
         be.unload_lora_adapter()
     for w, n, y, m in zip(ws, shapes, ys, names):
