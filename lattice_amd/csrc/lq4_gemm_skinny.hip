@@ -893,8 +893,8 @@ void gemm_skinny_pack_lora_a(const void* a, int a_is_f16, uint32_t rank, uint32_
 //   17..32 tokens: 4096 x 17408 27.1 / 20.1, 5120 x 17408 30.1 / 24.1, 17408 x 17408 90.7 / 85.7
 //   33..64 (at 64): 4096 x 17408 27.0 / 24.2; 8192 x 14336 38.1 / 32.5; 12288 x 6144 27.9 / 27.2; 16384 x 512 8.9 / 8.3, 16384 x 5120 30.6 / 26.1;
 //     20480 x 1024 13.7 / 11.3, 20480 x 3072 25.4 / 24.1; 24576 x 2048 22.0 / 20.8 (at 40 19.2 / 19.1), 32768 x 1024 14.6 / 17.5
-//   65..128 (at 128): 1024 x 17408 23.4 / 21.8; 2048 x 14336 24.8 / 23.1, 2048 x 17408 27.1 / 26.9; 4096 x 7168 22.2 / 19.5, 4096 x 8192 21.9 /
-//     20.9; 8192 x 3584 22.9 / 20.1, 8192 x 4096 21.9 / 22.1; 12288 x 512 10.2 / 11.1, 12288 x 1024 14.7 / 13.8, 12288 x 2560 24.5 / 23.1;
+//   65..128 (at 128): 1024 x 17408 23.4 / 21.8; 2048 x 14336 24.8 / 23.1, 2048 x 17408 27.1 / 26.9; 2080 x 8192 19.5 / 19.9 (at 72 19.6 / 15.0), 2560 x 9728 20.9 / 22.1;
+//     4096 x 7168 21.5 / 18.8, 4096 x 8192 22.4 / 20.4; 8192 x 3584 22.9 / 20.1, 8192 x 4096 21.9 / 22.1; 12288 x 512 10.2 / 11.1, 12288 x 1024 14.7 / 13.8, 12288 x 2560 24.5 / 23.1;
 //     16384 x 1536 22.3 / 20.3, 16384 x 2048 23.6 / 25.6
 //   (16384 and more rows at 33..64 tokens, and 8193 and more at 65..128, with K of at most 1024 stay with the large tiles, as
 //   tests/test_gemm_tiles.py has them.)
@@ -927,7 +927,7 @@ struct ShapeLimit {
     bool sliced = false;  // only what the large tiles run as K slices
 };
 constexpr ShapeLimit kPlain64[] = {{4096, 0, 17408}, {8192, 0, 14336}, {12288, 0, 6144}, {16384, 1024, 5120}, {20480, 1056, 3072, true}};
-constexpr ShapeLimit kPlain128[] = {{1024, 0, 17408}, {2048, 0, 14336}, {4096, 0, 7680}, {8192, 0, 3584}, {12288, 1056, 2560, true}, {16384, 1056, 1536, true}};
+constexpr ShapeLimit kPlain128[] = {{1024, 0, 17408}, {2048, 0, 14336}, {4096, 0, 8192}, {8192, 0, 3584}, {12288, 1056, 2560, true}, {16384, 1056, 1536, true}};
 constexpr ShapeLimit kPlain192[] = {{512, 0, 14336}, {1024, 0, 10240}, {2048, 0, 6144}, {4096, 0, 4096}, {6144, 0, 3072}, {8192, 1024, 2048}};
 constexpr ShapeLimit kPlain256[] = {{1024, 0, 10240}, {2048, 0, 6144}, {3072, 0, 4096}, {4096, 0, 3072}, {6144, 1024, 2048}};
 constexpr ShapeLimit kPlain384[] = {{512, 0, 8192}, {1024, 0, 4096}, {2048, 0, 3072}, {3072, 0, 2048}, {4096, 1024, 2048}};

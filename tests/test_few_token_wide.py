@@ -62,6 +62,25 @@ def test_edges_and_lines(be, fmt, m, n, k, few, xdt):
         assert np.array_equal(got[0][:m], y.cpu().numpy()) == few
 
 
+@pytest.mark.parametrize("m,n,k,few", [(128, 4096, 8192, True), (65, 2080, 8192, True), (128, 4096, 8224, False), (128, 2049, 14336, False)])
+def test_lines_up_to_128(be, m, n, k, few):
+    import torch
+    print(f"few-token lines m={m} n={n} k={k}", flush=True)
+    qw, deq, call = weights(be, "q4", n, k)
+    x = synth.activations(m, k, seed=3, dtype=np.float16)
+    dx, got = torch.from_numpy(x).cuda(), {}
+    try:
+        for which in (0, 3):
+            y = torch.full((m, n), float("nan"), device="cuda")
+            be.set_gemm_kernel(which)
+            call(dx, 0, qw, y, 0, m, n, k)
+            got[which] = y.cpu().numpy()
+    finally:
+        be.set_gemm_kernel(0)
+    assert rel_err(got[0], x.astype(np.float32) @ deq.T) <= REL_TOL
+    assert np.array_equal(got[0], got[3]) == few
+
+
 @pytest.mark.parametrize("m,n,k", [(100, 2048, 2048), (512, 512, 1024)])
 def test_capture_with_scratch_for_the_packed_activations(m, n, k):
     """Reserved scratch comes in whole MiB; the packed activations of the second shape fill one.  (Less of it, and none:
