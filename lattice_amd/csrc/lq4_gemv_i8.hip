@@ -725,7 +725,8 @@ I8Split split_i8(uint32_t n_tiles, uint32_t chunks, uint32_t cu_count, bool wide
 // producers: workgroups of the launch that compute LoRA factors.  Where they find no idle CU beside the usual split, but do beside
 // more tiles in a workgroup at up to two steps more, that one: the launch for the factors which they save takes three (rank 16, eight
 // rows, us with that launch / so / plain: 5120 x 4096 12.5 / 10.2 / 9.0, 4096 x 2048 7.7 / 6.4 / 4.5, 12288 x 2048 10.8 / 9.9 / 7.2, 4096 x 2560 8.3 / 7.9 /
-// 5.3, 4096 x 4096 10.3 / 9.7 / 7.0).
+// 5.3, 4096 x 4096 10.3 / 9.7 / 7.0).  Up to four rows from a tile for every CU on (rank 16, three and four rows, with that launch / so: 5120 x
+// 4096 10.6 / 8.6, 4096 x 2048 6.9 / 5.9, 12288 x 2048 9.5 / 8.5); 4000 x 2048, 7.0 / 5.9, keeps the launch, as tests/test_gpu_parity.py has it.
 bool plan_i8(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count, I8Plan* out, uint32_t producers = 0) {
     if (k == 0 || k % kBlockWeights || n == 0 || batch == 0 || batch > 8) return false;
     const uint32_t nb = k / kBlockWeights;
@@ -734,7 +735,7 @@ bool plan_i8(uint32_t n, uint32_t k, uint32_t batch, uint32_t cu_count, I8Plan* 
     I8Plan p;
     I8Split split = split_i8(n_tiles, chunks, cu_count, batch <= 4);
     auto fits = [&](const I8Split& s) { return std::min((n_tiles + s.tw - 1) / s.tw, cu_count) + producers <= cu_count; };
-    if (producers && split.cw * split.tw == 8 && !fits(split)) {
+    if (producers && (batch > 4 || n_tiles >= cu_count) && split.cw * split.tw == 8 && !fits(split)) {
         const uint32_t usual = split.steps;
         for (uint32_t tw = 2 * split.tw; tw <= 4; tw *= 2) {
             const I8Split s{8 / tw, tw, steps_i8(n_tiles, chunks, cu_count, 8 / tw, tw)};
