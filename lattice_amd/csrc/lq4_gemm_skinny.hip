@@ -477,11 +477,18 @@ __global__ __launch_bounds__(64 * kWavesK) void gemm_q4_skinny(const uint8_t* __
 #pragma unroll
             for (int i = 0; i < kLoads; ++i) dma16(to + i * 1024, w_base, w_off[i] + at);
         } else {
-            // its last pieces would reach past the end of the matrix: dword by dword, those past it read its last one
-#pragma unroll 1
-            for (int i = 0; i < 4 * kLoads; ++i) {
-                uint32_t off = piece_off(i * 16 + (lane >> 2)) + (lane & 3) * 4 + at;
-                dma4(to + i * 256, w_base, off < w_left ? off : w_left - 4);
+            // Its last pieces would reach past the end of the matrix.  The last row dword by dword, those past the end read its last
+            // one; of the rows before it (at least 16 bytes a row) only pieces of blocks past the end of K do, which are dropped: as
+            // far back as they must.  (Everything dword by dword, 0.15 us: 96 x 300 x 3104 6.4 us, K 3072 6.1.)
+            const uint32_t last = n - 1 - n0;  // (of a tile in front of the last one: none of its rows)
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                const uint32_t off = w_off[i] + at;
+                if ((i * 64 + lane) / kPieces != last) dma16(to + i * 1024, w_base, off + 16 <= w_left ? off : w_left - 16);
+            }
+            if (last < 16 * RT && lane < static_cast<int>(4 * kPieces)) {
+                const uint32_t off = ((w_odd + last * static_cast<uint32_t>(row_bytes)) & ~3u) + place(lane >> 2, last) * 16 + (lane & 3) * 4 + at;
+                dma4(to + last * (kPieces * 16), w_base, off < w_left ? off : w_left - 4);
             }
         }
     };

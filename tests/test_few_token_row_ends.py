@@ -18,7 +18,8 @@ def be():
 
 
 @pytest.mark.parametrize("fmt,lead", [("q4", 0), ("q4", 20), ("q8", 0), ("q8", 34), ("q3", 0), ("q3", 16)])
-@pytest.mark.parametrize("m,n,k", [(17, 1, 32), (20, 3, 64), (33, 17, 96), (128, 47, 160), (50, 33, 1056), (24, 4097, 224), (64, 31, 2048)])
+@pytest.mark.parametrize("m,n,k", [(17, 1, 32), (20, 3, 64), (33, 17, 96), (128, 47, 160), (50, 33, 1056), (24, 4097, 224), (64, 31, 2048),
+                                   (20, 17, 32), (40, 33, 32), (18, 16, 96), (96, 300, 3104)])  # (a tile in front of the last that cannot load whole steps either)
 def test_rows_end_with_the_buffer(be, fmt, lead, m, n, k):
     import torch
     print(f"few-token row ends {fmt} lead={lead} m={m} n={n} k={k}", flush=True)

@@ -167,7 +167,7 @@ def test_the_few_token_loop_keeps_two_units_in_flight(few_token):
         for i, follow in enumerate(successors(ins)):
             for j in follow:
                 body = [t for _, t in ins[j:i + 1]]
-                if j <= i and any(t.startswith("v_mfma") for t in body) and any("_lds_" in t for t in body):
+                if j <= i and sum(t.startswith("v_mfma") for t in body) == 8 * rt * ntg and any("_lds_" in t for t in body):
                     bodies.append(body)
         body = min(bodies, key=len)
         kind = {"v_mfma": "M", "global_load_lds": "D", "global_load": "L"}
