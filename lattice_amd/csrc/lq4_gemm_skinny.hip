@@ -926,7 +926,7 @@ void gemm_skinny_pack_lora_a(const void* a, int a_is_f16, uint32_t rank, uint32_
 // This kernel packs X into the context's scratch.  The large tiles use none where they run a product whole (rows of fewer than
 // four steps, or a last round that is nearly full): such a call needs nothing of the context, can be captured on a new one, takes
 // the same kernel whether scratch has grown or not, and replays beside other calls.  It keeps that above 128 tokens and in the
-// entries marked `sliced`, also where it would be faster here (us there / here: 129 x 64 x 512 8.1 / 4.4, 256 x 1000 x 384 7.8 / 5.3, 160 x 4096 x
+// entries marked `sliced`, but for a product inside a call that works in the scratch anyway, also where it would be faster here (us there / here: 129 x 64 x 512 8.1 / 4.4, 256 x 1000 x 384 7.8 / 5.3, 160 x 4096 x
 // 768 12.3 / 8.3, 160 x 8192 x 1024 15.3 / 12.4, 40 x 20196 x 1152 15.5 / 13.8; Q8_0 192 x 6144 x 768 12.8 / 13.8, 104 x 8104 x 64 6.9 / 8.6).
 namespace {
 struct ShapeLimit {
@@ -947,11 +947,11 @@ constexpr ShapeLimit kSibling64[] = {{4096, 0, 12288}, {8192, 0, 8192}, {12288, 
 constexpr ShapeLimit kSibling128[] = {{512, 0, 17408}, {2048, 0, 8192}, {4096, 0, 6144}, {8192, 0, 2560, true}};
 }  // namespace
 
-bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora, int x_is_f16) {
+bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora, int x_is_f16, bool in_state) {
     if (k < kBlockWeights) return false;
     if (m <= 16) return true;
     if (m <= 32) return static_cast<uint64_t>(n) * k <= (1ull << 28);
-    auto sliced = [&] { return (fmt ? gemm_sibling_scratch_floats(fmt, n, k, m, x_is_f16, 0) : gemm_wreg_scratch_floats(n, k, m, 0, x_is_f16 != 0)) != 0; };
+    auto sliced = [&] { return in_state || (fmt ? gemm_sibling_scratch_floats(fmt, n, k, m, x_is_f16, 0) : gemm_wreg_scratch_floats(n, k, m, 0, x_is_f16 != 0)) != 0; };
     auto within = [&](const auto& limits, bool narrowed = false) {
         for (const ShapeLimit& l : limits)
             if (n <= l.n) return (narrowed ? l.k_min <= 512 && k >= l.k_min && k + k / 2 <= l.k_max : k >= l.k_min && k <= l.k_max) && (!l.sliced || sliced());

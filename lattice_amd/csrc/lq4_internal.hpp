@@ -272,7 +272,8 @@ void launch_gemm_q3(const uint8_t* w, uint32_t n, uint32_t k, const void* x, int
 
 // Few-token variant (up to 128 tokens; up to 1024 small matrices whose large tiles would take scratch too): activations packed once into matrix-core operand order
 // (gemm_skinny_scratch_bytes bytes at `packed_x`), then a kernel whose weights come through wave-private LDS.
-bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora, int x_is_f16);
+// `in_state`: the call works in the context's scratch anyway (there), so also what the large tiles would run without.
+bool gemm_skinny_wants(uint32_t n, uint32_t k, uint32_t m, int fmt, bool with_lora, int x_is_f16, bool in_state = false);
 // `adapters`: those of the launch whose t = A . X it computes.
 size_t gemm_skinny_scratch_bytes(uint32_t k, uint32_t m, uint32_t adapters = 0);
 // For Q4 and a LoRA rank this accepts the packing launch computes t = A . X when LoraEpilogue::a points to A as packed

@@ -156,3 +156,28 @@ def test_capture_that_fits_neither_names_the_packed_activations(fmt, m, n, k, ra
     assert np.all(np.isfinite(captured(go, y)))  # and what it names is enough
     go = call = both = qw = None
     be.close()
+
+
+def test_the_shared_expert_works_in_the_scratch_anyway():
+    """A product that the large tiles would run whole (hidden 1408 x 576 and 1152 x 1408 at 174 tokens), inside a call that works in the
+    context's scratch and is ordered by it: the few-token kernel's bits; of the plain call, the large tiles'."""
+    import torch
+    print("few-token context shared expert", flush=True)
+    be = backend.HipQ4Backend(0)
+    try:
+        tokens, hidden, inter = 174, 1408, 576
+        gu, dn = synth.q4_weight(2 * inter, hidden, seed=1), synth.q4_weight(hidden, inter, seed=2)
+        x, sg = synth.activations(tokens, hidden, seed=3), synth.activations(1, hidden, seed=4)[0] / hidden ** 0.5
+        qgu, qdn, dx, dsg = be.upload_q4_blocks(gu), be.upload_q4_blocks(dn), torch.from_numpy(x).cuda(), torch.from_numpy(sg).cuda()
+        got, plain = {}, {}
+        for which in (0, 2, 3):
+            be.set_gemm_kernel(which)
+            y, z = torch.zeros((tokens, hidden), device="cuda"), torch.empty((tokens, hidden), device="cuda")
+            be.moe_shared_expert(qgu, qdn, dsg, inter, hidden, dx, y)
+            be.dispatch_gemm(dx[:, :inter].contiguous(), 0, qdn, z, 0, tokens, hidden, inter)
+            got[which], plain[which] = y.cpu().numpy(), z.cpu().numpy()
+        assert rel_err(got[0], oracle.moe_shared_expert(gu, dn, sg, inter, hidden, x, np.zeros_like(got[0]))) <= REL_TOL
+        assert np.array_equal(got[0], got[3]) and not np.array_equal(got[0], got[2])
+        assert np.array_equal(plain[0], plain[2]) and not np.array_equal(plain[0], plain[3])
+    finally:
+        be.close()
