@@ -41,7 +41,7 @@
 // one per row of A (the views' A stacked), each forming that row's dot products with the batch's activation rows
 // and publishing them as {value, tag of the launch} words; the other workgroups pick them up into LDS when their first
 // tile is multiplied, by which time the producers, who have nothing else to do, are done.  The launcher adds the
-// producers only where CUs are idle anyway (tiles + producers <= CUs): a matrix of 2560 rows occupies 160.  A value
+// producers only where CUs are idle beside the others (workgroups + producers <= CUs: a matrix of 2560 rows occupies 160; see plan_i8).  A value
 // that has not arrived after the poll limit is computed by the wave that misses it, in the producers' order of
 // summation (same bits), and counted in sync[2].
 //
